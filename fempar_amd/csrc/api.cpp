@@ -293,6 +293,7 @@ int femhip_operator_set_physics(femhip_operator_t *op, const femhip_physics_t *p
   FH_HIP(hipSetDevice(op->ctx->device));
   op->phys = *phys;
   op->has_physics = true;
+  ++op->phys_version;
   upload_physics(*op);
   op->computed = false;
   return FEMHIP_OK;

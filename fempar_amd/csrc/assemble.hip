@@ -981,6 +981,10 @@ constexpr int kGatherRows = 128;
 
 }  // namespace
 
+void ensure_trig(femhip_operator &op) {
+  if (op.trig.n == 0) build_trig(op);
+}
+
 // The owner-computes rows can fill the symmetric-diagonal solver copy too when
 // the column offset of each neighbour code is the same on every row (the
 // structured numberings for which that copy exists).  The offsets are read off

@@ -39,6 +39,7 @@
 #include <type_traits>
 
 #include "femhip_internal.h"
+#include "lattice.h"
 
 namespace femhip {
 namespace {
@@ -66,6 +67,7 @@ struct CgState {
   double ru_rz, ru_rmax, ru_rnorm, ru_beta;
   double rscale, ru_rscale;    // ||S r|| / ||r|| at the last update (scaled inner residual)
   int iter, done, converged, maxit, crit, ru, updates, ru_conv, ru_done, first;
+  int set, pad;                // lattice FP32 passes: which of the two vector sets holds r, p, s
 };
 
 struct CgResult {
@@ -451,6 +453,7 @@ __global__ __launch_bounds__(kThreads) void k_init_fin(const double *part, int g
   s.ru = 0;
   s.updates = 0;
   s.rmax = rnorm;
+  s.first = 1;
   S[1] = s;
   R->est = 0.0;
   R->rhs_test = t;
@@ -533,6 +536,56 @@ __global__ __launch_bounds__(kThreads) void k_update(int32_t n, T *__restrict__ 
   write_partials<2>(out, part);
 }
 
+// Stopping test (cg.f90:323-407) after the iteration whose <r,z>, ||r||^2 are
+// red[0], red[1]; `lead` (one thread of the launch) writes the next state, the
+// history and the result blocks.  Returns done, beta for the next direction.
+__device__ __forceinline__ bool cg_decide(const CgState &cur, const double (&red)[2], bool lead, CgState &next,
+                                          double *hist, CgResult *R, CgResult *Rh, double &beta_out) {
+  const int it = cur.iter + 1;
+  const int c = cur.crit;
+  const double rnorm = sqrt(red[1]);
+  double est = cur.est, rhs_test = cur.rhs_test;
+  if (it == 1 && is_delta(c)) {
+    est = cur.alpha * sqrt(cur.pp);
+    if (is_delta_delta(c)) rhs_test = cur.rtol * est + cur.atol;
+  }
+  if (c == FEMHIP_RES_RES || c == FEMHIP_RES_RHS) est = rnorm;
+  else if (is_delta(c)) {
+    if (it != 1) est = cur.alpha * sqrt(cur.pp);
+  } else est = cur.rnrm_m;
+  int conv = est <= rhs_test;
+  if (c >= FEMHIP_DELTA_RHS_AND_RES_RES && conv) conv = rnorm <= cur.rhs_extra;
+  const bool done = conv || it >= cur.maxit;
+  double beta = 1.0 / cur.rz;
+  beta = beta * red[0];
+  if (lead) {
+    CgState nx = cur;
+    nx.first = 0;
+    nx.iter = it;
+    nx.est = est;
+    nx.rhs_test = rhs_test;
+    nx.rnorm = rnorm;
+    nx.converged = conv;
+    nx.done = done;
+    nx.beta = beta;
+    nx.rz = red[0];
+    nx.rnrm_m = sqrt(red[0]);
+    next = nx;
+    if (hist) hist[it - 1] = est;
+    R->iter = it;
+    R->est = est;
+    R->rhs_test = rhs_test;
+    R->rnorm = rnorm;
+    R->converged = conv;
+    R->done = done;
+    R->prog = est;
+    R->prog_it = it;
+    if (Rh) *Rh = *R;
+  }
+  beta_out = beta;
+  return done;
+}
+
 // stopping test (cg.f90:323-407) ; beta ; x += alpha p ; p = z + beta p
 // (the last iteration: x += alpha p only).  Rh (the last iteration of a chunk
 // only): host-mapped copy of the result block, read by the host after the
@@ -564,46 +617,8 @@ __global__ __launch_bounds__(kThreads) void k_dir(int32_t n, T *__restrict__ x, 
   }
   double red[2];
   reduce_partials<2>(part_u, gu, red);
-  const int it = cur.iter + 1;
-  const int c = cur.crit;
-  const double rnorm = sqrt(red[1]);
-  double est = cur.est, rhs_test = cur.rhs_test;
-  if (it == 1 && is_delta(c)) {
-    est = cur.alpha * sqrt(cur.pp);
-    if (is_delta_delta(c)) rhs_test = cur.rtol * est + cur.atol;
-  }
-  if (c == FEMHIP_RES_RES || c == FEMHIP_RES_RHS) est = rnorm;
-  else if (is_delta(c)) {
-    if (it != 1) est = cur.alpha * sqrt(cur.pp);
-  } else est = cur.rnrm_m;
-  int conv = est <= rhs_test;
-  if (c >= FEMHIP_DELTA_RHS_AND_RES_RES && conv) conv = rnorm <= cur.rhs_extra;
-  const bool done = conv || it >= cur.maxit;
-  double beta = 1.0 / cur.rz;
-  beta = beta * red[0];
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    CgState nx = cur;
-    nx.iter = it;
-    nx.est = est;
-    nx.rhs_test = rhs_test;
-    nx.rnorm = rnorm;
-    nx.converged = conv;
-    nx.done = done;
-    nx.beta = beta;
-    nx.rz = red[0];
-    nx.rnrm_m = sqrt(red[0]);
-    S[par ^ 1] = nx;
-    if (hist) hist[it - 1] = est;
-    R->iter = it;
-    R->est = est;
-    R->rhs_test = rhs_test;
-    R->rnorm = rnorm;
-    R->converged = conv;
-    R->done = done;
-    R->prog = est;
-    R->prog_it = it;
-    if (Rh) *Rh = *R;
-  }
+  double beta = 0.0;
+  const bool done = cg_decide(cur, red, blockIdx.x == 0 && threadIdx.x == 0, S[par ^ 1], hist, R, Rh, beta);
   const T a = (T)cur.alpha;
   if (done) {
 #pragma unroll
@@ -941,27 +956,17 @@ __global__ __launch_bounds__(kThreads) void k_ru_dir(int32_t n, float *__restric
 
 constexpr int kRfbGroup = 8;   // slices of a wave whose r and q loads k_rf_b keeps in flight together
 
-template <typename A>
-__global__ __launch_bounds__(kThreads, 4) void k_rf_a(SlicedDev m, SlicedDev m32, const float *__restrict__ v32,
-                                                   const float *__restrict__ r, float *__restrict__ p,
-                                                   float *__restrict__ q, float *__restrict__ d,
-                                                   double *__restrict__ x, const double *__restrict__ sc,
-                                                   CgState *S, int par, const double *part_b, int gb, double *part,
-                                                   CgResult *R, CgResult *Rh, int rev) {
-  const CgState &cur = S[par];
-  if (cur.done) {   // keep `done` sticky in both parity slots
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-      S[par ^ 1].done = 1;
-      if (Rh) *Rh = *R;
-    }
-    return;
-  }
-  double red[2] = {0.0, 0.0};
-  if (!cur.first) reduce_partials<2>(part_b, gb, red);
-  const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
+// What a slot A does: the decision after the previous slot B, whose <r,r> (and
+// after a fold the FP64 ||b - A x||^2) are red; `lead` writes the next state.
+struct RfStep {
+  int fold, upd_d, done;
+  double beta;
+};
+__device__ __forceinline__ RfStep rf_decide(const CgState &cur, const double (&red)[2], bool lead, CgState &next,
+                                            CgResult *R) {
   if (lead) {
-    S[par ^ 1] = cur;
-    S[par ^ 1].first = 0;
+    next = cur;
+    next.first = 0;
   }
   int fold = 0, upd_d = 0, done = 0;
   double beta = 0.0;
@@ -978,7 +983,7 @@ __global__ __launch_bounds__(kThreads, 4) void k_rf_a(SlicedDev m, SlicedDev m32
       upd_d = 1;
     }
     if (lead) {
-      CgState &w = S[par ^ 1];
+      CgState &w = next;
       w.iter = it;
       w.rnorm = rnorm;
       w.ru = fold;
@@ -998,7 +1003,7 @@ __global__ __launch_bounds__(kThreads, 4) void k_rf_a(SlicedDev m, SlicedDev m32
     beta = beta * red[0];
     done = conv || cur.iter >= cur.maxit;
     if (lead) {
-      CgState &w = S[par ^ 1];
+      CgState &w = next;
       w.ru = 0;
       w.rz = red[0];
       w.beta = beta;
@@ -1019,6 +1024,30 @@ __global__ __launch_bounds__(kThreads, 4) void k_rf_a(SlicedDev m, SlicedDev m32
       R->prog_it = cur.iter;
     }
   }
+  return {fold, upd_d, done, beta};
+}
+
+template <typename A>
+__global__ __launch_bounds__(kThreads, 4) void k_rf_a(SlicedDev m, SlicedDev m32, const float *__restrict__ v32,
+                                                   const float *__restrict__ r, float *__restrict__ p,
+                                                   float *__restrict__ q, float *__restrict__ d,
+                                                   double *__restrict__ x, const double *__restrict__ sc,
+                                                   CgState *S, int par, const double *part_b, int gb, double *part,
+                                                   CgResult *R, CgResult *Rh, int rev) {
+  const CgState &cur = S[par];
+  if (cur.done) {   // keep `done` sticky in both parity slots
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      S[par ^ 1].done = 1;
+      if (Rh) *Rh = *R;
+    }
+    return;
+  }
+  double red[2] = {0.0, 0.0};
+  if (!cur.first) reduce_partials<2>(part_b, gb, red);
+  const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
+  const RfStep step = rf_decide(cur, red, lead, S[par ^ 1], R);
+  const int fold = step.fold, upd_d = step.upd_d, done = step.done;
+  const double beta = step.beta;
   if (lead && Rh) *Rh = *R;
   if (done) return;
   const int lane = threadIdx.x & 63;
@@ -1338,6 +1367,8 @@ __global__ __launch_bounds__(kThreads) void k_true_res(SlicedDev m, const double
   write_partials<1>(acc, part);
 }
 
+#include "cg_lattice.h"
+
 }  // namespace
 }  // namespace femhip
 
@@ -1351,6 +1382,14 @@ struct femhip_solver {
   int g_mat = 8, g_vec = 8;      // grid sizes of the matrix and vector kernels
   DevBuf<double> x, b, r, p, q, invd, part_i, part_s, part_u, part_r, hist;
   DevBuf<float> r32, p32, q32, d32;
+  // products from the cells (lattice.h): r, p and q alternate between two
+  // vectors; the coefficient and kernels the chunk graphs were built with
+  bool lat = false;
+  DevBuf<double> r_alt, p_alt, q_alt;
+  DevBuf<float> r32_alt, p32_alt, q32_alt;
+  CoefDev coef;
+  Q2Tab q2tab{};
+  LatticeKernels lk{};
   DevBuf<CgState> st;            // S[2]
   DevBuf<CgResult> res;
   int *h_flag = nullptr, *d_flag = nullptr;    // zero-pivot flag of the Jacobi setup (pinned, mapped)
@@ -1453,9 +1492,111 @@ bool fp32_integration() {
   return e && atoi(e) == 1;
 }
 
+// Whether a solver forms its products from the cells: scalar Poisson operators
+// on the uniform mesh (lattice_operator), in FP64 and FP32_REFINED.  FP32_STRICT
+// and the FP32 integration are defined by their stored FP32 matrix.  Up to 4096
+// rows an iteration is launch latency whichever product it takes (32^2 Q1: 14.6
+// us stored, 11.1 us from the cells), and the stored matrix stays.
+constexpr int32_t kLatticeMinRows = 4097;
+bool wants_lattice(femhip_solver &s) {
+  return s.op->n >= kLatticeMinRows && !strict(s) && !(mixed(s) && fp32_integration()) && lattice_operator(*s.op);
+}
+
+void drop_graphs(femhip_solver &s) {
+  for (auto &row : s.graphs)
+    for (auto &g : row)
+      if (g) {
+        FH_HIP(hipGraphExecDestroy(g));
+        g = nullptr;
+      }
+}
+
+// host-side slots of the result and the pivot flag
+void prepare_host_slots(femhip_solver &s) {
+  for (int k = 0; k < 2; ++k) {   // written by the GPU, read by the host: mapped, coherent
+    if (!s.borrowed_host && !s.h_res[k])
+      FH_HIP(hipHostMalloc((void **)&s.h_res[k], sizeof(CgResult), hipHostMallocMapped | hipHostMallocCoherent));
+    std::memset(s.h_res[k], 0, sizeof(CgResult));
+    FH_HIP(hipHostGetDevicePointer((void **)&s.d_res_map[k], s.h_res[k], 0));
+  }
+  if (!s.borrowed_host && !s.h_flag)
+    FH_HIP(hipHostMalloc((void **)&s.h_flag, sizeof(int), hipHostMallocMapped | hipHostMallocCoherent));
+  *s.h_flag = 0;
+  FH_HIP(hipHostGetDevicePointer((void **)&s.d_flag, s.h_flag, 0));
+  if (!s.borrowed_host)
+    for (auto &e : s.ev)
+      if (!e) FH_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+}
+
+// One launch an iteration or two (cg_lattice.h).
+#ifndef FEMHIP_LAT_ONE
+#define FEMHIP_LAT_ONE 400000
+#endif
+bool lattice_one_pass(int32_t n) { return n < FEMHIP_LAT_ONE; }
+
+void prepare_lattice(femhip_solver &s) {
+  femhip_operator &op = *s.op;
+  hipStream_t st = s.ctx->stream;
+  const LatticeOp &L = *op.lat;
+  const bool jac = s.prm.preconditioner == FEMHIP_PREC_JACOBI;
+  const bool mx = mixed(s);
+  const int32_t n = op.n;
+  if (!s.prepared) {
+    s.n = n;
+    s.g_mat = L.grid;
+    // k_lat_b: 8 rows a thread, at most 4 workgroups per CU
+    s.g_vec = std::max(8, std::min(4 * std::max(1, s.ctx->num_cus), (n + 8 * kThreads - 1) / (8 * kThreads)));
+    s.x.alloc(n); s.b.alloc(n); s.q.alloc(n);
+    if (jac) s.invd.alloc(n);   // invD (FP64) or S (FP32_REFINED)
+    if (mx) {
+      for (auto *v : {&s.r32, &s.p32, &s.p32_alt, &s.q32, &s.d32}) v->alloc(n);
+      if (lattice_one_pass(n))
+        for (auto *v : {&s.r32_alt, &s.q32_alt}) v->alloc(n);
+    } else {
+      for (auto *v : {&s.r, &s.p, &s.p_alt}) v->alloc(n);
+      if (lattice_one_pass(n))
+        for (auto *v : {&s.r_alt, &s.q_alt}) v->alloc(n);
+    }
+    s.part_i.alloc((size_t)4 * s.g_mat);
+    s.part_s.alloc((size_t)kSums * s.g_mat);   // the passes' sums, alternating
+    s.part_u.alloc((size_t)kSums * std::max(s.g_mat, s.g_vec));
+    s.hist.alloc((size_t)std::max(1, s.prm.max_num_iterations));
+    s.st.alloc(2);
+    s.res.alloc(1);
+    prepare_host_slots(s);
+    s.q2tab = lattice_q2_tab();
+    s.prepared = true;
+  }
+  const CoefDev coef = lattice_coefficient(op);
+  const int kind = op.phys.k_kind == FEMHIP_K_SIN3 ? kCoefSin3
+                   : op.phys.k_kind == FEMHIP_K_QPOINT ? kCoefPoint : kCoefCell;
+  const LatticeKernels lk = lattice_kernels(L.dim, L.order, kind);
+  if (lk.cg != s.lk.cg || !(coef == s.coef)) drop_graphs(s);   // they hold both by value
+  s.coef = coef;
+  s.lk = lk;
+  if (jac && n > 0) {
+    *s.h_flag = 0;
+    hipLaunchKernelGGL(k_lat_jacobi, dim3((n + 255) / 256), dim3(256), 0, st, n, op.rowptr.p, op.col.p, op.val.p,
+                       L.identity ? nullptr : op.lat_perm.p, s.invd.p, mx ? 1 : 0, s.d_flag);
+    FH_HIP(hipGetLastError());
+  }
+}
+
 void prepare(femhip_solver &s) {
   femhip_operator &op = *s.op;
   FH_CHECK(op.computed, FEMHIP_ERR_STATE, "solve before fe_affine_operator%compute");
+  const bool lat = wants_lattice(s);
+  if (s.prepared && lat != s.lat) {   // the operator's mesh was moved since: other layout, other buffers
+    FH_HIP(hipStreamSynchronize(s.ctx->stream));
+    drop_graphs(s);
+    s.prepared = false;
+    s.have_solution = false;
+  }
+  s.lat = lat;
+  if (lat) {
+    prepare_lattice(s);
+    return;
+  }
   hipStream_t st = s.ctx->stream;
   const bool jac = s.prm.preconditioner == FEMHIP_PREC_JACOBI;
   const bool mx = mixed(s);
@@ -1496,18 +1637,7 @@ void prepare(femhip_solver &s) {
     if (mx) {
       s.r32.alloc(n); s.p32.alloc(n); s.q32.alloc(n); s.d32.alloc(n);
     }
-    for (int k = 0; k < 2; ++k) {   // written by the GPU, read by the host: mapped, coherent
-      if (!s.borrowed_host)
-        FH_HIP(hipHostMalloc((void **)&s.h_res[k], sizeof(CgResult), hipHostMallocMapped | hipHostMallocCoherent));
-      std::memset(s.h_res[k], 0, sizeof(CgResult));
-      FH_HIP(hipHostGetDevicePointer((void **)&s.d_res_map[k], s.h_res[k], 0));
-    }
-    if (!s.borrowed_host)
-      FH_HIP(hipHostMalloc((void **)&s.h_flag, sizeof(int), hipHostMallocMapped | hipHostMallocCoherent));
-    *s.h_flag = 0;
-    FH_HIP(hipHostGetDevicePointer((void **)&s.d_flag, s.h_flag, 0));
-    if (!s.borrowed_host)
-      for (auto &e : s.ev) FH_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    prepare_host_slots(s);
     s.prepared = true;
   }
   // matrix-dependent work, redone whenever the operator was recomputed
@@ -1577,20 +1707,21 @@ struct Launcher {
   hipStream_t stream = nullptr;
   hipGraph_t graph = nullptr;
   hipGraphNode_t last = nullptr;
+  size_t lds = 0;   // dynamic LDS of the next launches, bytes
 
   template <typename... P, typename... A>
   void operator()(void (*k)(P...), dim3 grid, dim3 block, A... a) {
     std::tuple<std::decay_t<P>...> vals(static_cast<std::decay_t<P>>(a)...);
     auto args = std::apply([](auto &...v) { return std::array<void *, sizeof...(P)>{(void *)&v...}; }, vals);
     if (!graph) {
-      FH_HIP(hipLaunchKernel((const void *)k, grid, block, args.data(), 0, stream));
+      FH_HIP(hipLaunchKernel((const void *)k, grid, block, args.data(), lds, stream));
       return;
     }
     hipKernelNodeParams prm{};
     prm.func = (void *)k;
     prm.gridDim = grid;
     prm.blockDim = block;
-    prm.sharedMemBytes = 0;
+    prm.sharedMemBytes = (unsigned)lds;
     prm.kernelParams = args.data();
     prm.extra = nullptr;
     hipGraphNode_t node;
@@ -1616,11 +1747,49 @@ bool three_kernel_refined(const femhip_solver &s) {
 // `rh`, the direction kernel also writes the result block there.
 void enqueue_one(femhip_solver &s, int par, Launcher &L, const hipEvent_t *ev = nullptr, CgResult *rh = nullptr) {
   femhip_operator &op = *s.op;
-  const SlicedDev m = sliced_dev(op);
   const int32_t n = s.n;
   const bool jac = s.prm.preconditioner == FEMHIP_PREC_JACOBI;
   const dim3 B(kThreads), GM(s.g_mat), GV(s.g_vec);
   if (ev) FH_HIP(hipEventRecord(ev[0], L.stream));
+  if (s.lat) {
+    const LatticeOp &lo = *op.lat;
+    const dim3 BL((unsigned)lo.threads);
+    const double *sc = jac ? s.invd.p : nullptr;   // invD, or S of the FP32 iterations
+    const double *in = par ? s.part_u.p : s.part_s.p;
+    double *out = par ? s.part_s.p : s.part_u.p;
+    L.lds = lo.lds;
+    const PairOf<double> p{{s.p.p, s.p_alt.p}};
+    const PairOf<float> p32{{s.p32.p, s.p32_alt.p}};
+    const bool one = lattice_one_pass(n);
+    if (one && !mixed(s))
+      L(s.lk.cg, GM, BL, lo.g, s.coef, s.q2tab, n, PairOf<double>{{s.r.p, s.r_alt.p}},
+        PairOf<double>{{s.q.p, s.q_alt.p}}, p, s.x.p, sc, s.st.p, par, in, out, s.hist.p, s.res.p, rh);
+    else if (one)
+      L(s.lk.rf, GM, BL, lo.g, s.coef, s.q2tab, n, PairOf<float>{{s.r32.p, s.r32_alt.p}},
+        PairOf<float>{{s.q32.p, s.q32_alt.p}}, p32, s.d32.p, s.x.p, s.b.p, sc, s.st.p, par, in, out, s.res.p, rh);
+    else if (!mixed(s))
+      L(s.lk.a, GM, BL, lo.g, s.coef, s.q2tab, n, s.r.p, sc, p, s.x.p, s.q.p, s.st.p, par, s.part_u.p, s.g_vec,
+        s.part_s.p, s.hist.p, s.res.p, rh);
+    else
+      L(s.lk.rf_a, GM, BL, lo.g, s.coef, s.q2tab, n, s.r32.p, sc, p32, s.d32.p, s.q32.p, s.x.p, s.st.p, par,
+        s.part_u.p, s.g_mat, s.part_s.p, s.res.p, rh);
+    if (!one) {
+      if (ev) FH_HIP(hipEventRecord(ev[1], L.stream));
+      if (!mixed(s)) {
+        L.lds = 0;
+        L(k_lat_b, GV, B, n, s.r.p, s.q.p, sc, s.st.p, par ^ 1, s.part_s.p, s.g_mat, s.part_u.p);
+      } else {
+        L(s.lk.rf_b, GM, BL, lo.g, s.coef, s.q2tab, n, s.r32.p, s.q32.p, sc, s.b.p, s.x.p, s.st.p, par ^ 1,
+          s.part_s.p, s.g_mat, s.part_u.p);
+        L.lds = 0;
+      }
+      return;
+    }
+    L.lds = 0;
+    if (ev) FH_HIP(hipEventRecord(ev[1], L.stream));
+    return;
+  }
+  const SlicedDev m = sliced_dev(op);
   if (!mixed(s)) {
     const double *invd = jac ? s.invd.p : nullptr;
     // reversed odd sweeps: CG 21.35 -> 21.13 ms at 128^3 Q1 and 270.3 -> 268.0 ms at
@@ -1690,12 +1859,7 @@ void ensure_graph(femhip_solver &s, int size_idx, int slot) {
   const int kind = mixed(s) ? 1 : 0;
   if (!use_graph(s)) return;
   if (s.graph_kind != kind) {
-    for (auto &row : s.graphs)
-      for (auto &g : row)
-        if (g) {
-          FH_HIP(hipGraphExecDestroy(g));
-          g = nullptr;
-        }
+    drop_graphs(s);
     s.graph_kind = kind;
   }
   hipGraphExec_t &g = s.graphs[size_idx][slot];
@@ -1757,7 +1921,11 @@ void iterate(femhip_solver &s, int maxit) {
     FH_HIP(hipEventSynchronize(s.ev[c.slot]));
     const CgResult r = *s.h_res[c.slot];
     if (r.done) break;
-    if (queued >= maxit) continue;   // budget queued: wait for the rest
+    // budget queued: wait for the rest.  The lattice passes take each decision
+    // one pass later, and an update of their refined form (at most one an
+    // iteration) spends three: there the device ends the solve, and chunks go
+    // on until it has.
+    if (queued >= (s.lat ? 4 * (int64_t)maxit + 8 : (int64_t)maxit)) continue;
     double need = 1e30;              // iterations still needed
     if (prev_it >= 0 && r.prog_it > prev_it && r.prog > 0.0 && prev > r.prog && r.rhs_test > 0.0) {
       const double rate = std::log(r.prog / prev) / (r.prog_it - prev_it);
@@ -1769,7 +1937,8 @@ void iterate(femhip_solver &s, int maxit) {
     }
     static const char *plan_env = getenv("FEMHIP_TAIL_CHUNKS");   // 0: always full chunks
     if (plan_env && atoi(plan_env) == 0) need = 1e30;
-    const double rest = need - (double)(queued - r.prog_it);   // beyond what is queued
+    const double rest = std::min(need, s.lat ? (double)maxit - r.prog_it + 4.0 : 1e30) -
+                        (double)(queued - r.prog_it);   // beyond what is queued
     if (nq > 0 && rest <= 0.0) continue;
     push(rest > kChunk ? 0 : 1);
   }
@@ -1786,20 +1955,30 @@ void upload_state(femhip_solver &s) {
   FH_HIP(hipMemcpyAsync(s.st.p, &h, sizeof(h), hipMemcpyHostToDevice, s.ctx->stream));
 }
 
-// initial residual, direction and device state (x and b already in place)
+// solver row of each operator row, null where they are the same
+const int32_t *solver_perm(const femhip_solver &s) {
+  const femhip_operator &op = *s.op;
+  if (s.lat) return op.lat->identity ? nullptr : op.lat_perm.p;
+  return op.sl.permuted ? op.sl.perm.p : nullptr;
+}
+
 // A vector in operator order (the RHS or x0; device or host) into solver
 // vector dst: copied, or for a permuted layout staged in q (free before a
 // solve) and scattered to the solver rows, padding rows cleared.
 void load_vector(femhip_solver &s, double *dst, const double *src, hipMemcpyKind kind) {
   hipStream_t st = s.ctx->stream;
   femhip_operator &op = *s.op;
-  if (!op.sl.permuted) {
+  const int32_t *perm = solver_perm(s);
+  if (!perm) {
     FH_HIP(hipMemcpyAsync(dst, src, sizeof(double) * (size_t)s.n, kind, st));
     return;
   }
-  FH_HIP(hipMemcpyAsync(s.q.p, src, sizeof(double) * (size_t)op.n, kind, st));
-  hipLaunchKernelGGL(k_fill0, dim3(1024), dim3(256), 0, st, (int64_t)s.n, dst);
-  hipLaunchKernelGGL(k_permute_in, dim3(1024), dim3(256), 0, st, op.n, op.sl.perm.p, s.q.p, dst);
+  if (kind != hipMemcpyDeviceToDevice) {
+    FH_HIP(hipMemcpyAsync(s.q.p, src, sizeof(double) * (size_t)op.n, kind, st));
+    src = s.q.p;
+  }
+  if (!s.lat) hipLaunchKernelGGL(k_fill0, dim3(1024), dim3(256), 0, st, (int64_t)s.n, dst);   // padding rows
+  hipLaunchKernelGGL(k_permute_in, dim3(1024), dim3(256), 0, st, op.n, perm, src, dst);
   FH_HIP(hipGetLastError());
 }
 
@@ -1810,12 +1989,13 @@ void load_vector(femhip_solver &s, double *dst, const double *src, hipMemcpyKind
 const double *solution_operator_order(const femhip_solver &s) {
   hipStream_t st = s.ctx->stream;
   const femhip_operator &op = *s.op;
-  if (op.sl.permuted && op.n > 0) {
-    hipLaunchKernelGGL(k_permute_out, dim3(1024), dim3(256), 0, st, op.n, op.sl.perm.p, s.x.p, s.q.p);
+  const int32_t *perm = solver_perm(s);
+  if (perm && op.n > 0) {
+    hipLaunchKernelGGL(k_permute_out, dim3(1024), dim3(256), 0, st, op.n, perm, s.x.p, s.q.p);
     FH_HIP(hipGetLastError());
   }
   FH_HIP(hipStreamSynchronize(st));
-  return op.sl.permuted ? s.q.p : s.x.p;
+  return perm ? s.q.p : s.x.p;
 }
 
 namespace {
@@ -1826,7 +2006,15 @@ void begin(femhip_solver &s, bool x_zero) {
   const SlicedDev m = sliced_dev(op);
   const bool jac = s.prm.preconditioner == FEMHIP_PREC_JACOBI;
   upload_state(s);
-  if (!mixed(s)) {
+  if (s.lat) {   // initial residual (the direction is formed by the first slot)
+    const LatticeOp &lo = *op.lat;
+    Launcher L;
+    L.stream = st;
+    L.lds = lo.lds;
+    L(s.lk.res, dim3(s.g_mat), dim3((unsigned)lo.threads), lo.g, s.coef, s.q2tab, s.n,
+      (int)(mixed(s) ? kLatInit32 : kLatInit64), x_zero ? 1 : 0, s.x.p, s.b.p, jac ? s.invd.p : nullptr,
+      jac ? s.invd.p : nullptr, s.r.p, s.r32.p, s.d32.p, s.part_i.p);
+  } else if (!mixed(s)) {
     hipLaunchKernelGGL((k_init<double>), dim3(s.g_mat), dim3(kThreads), 0, st, m, op.sl.v64.p, s.b.p, s.x.p,
                        x_zero ? 1 : 0, s.r.p, s.p.p, jac ? s.invd.p : nullptr, s.part_i.p);
   } else {
@@ -1903,11 +2091,69 @@ void profiled_solve(femhip_solver &s, double *spmv_ms, int32_t *iterations) {
   for (auto e : ev) (void)hipEventDestroy(e);
 }
 
+// Times `reps` CG iterations (vector updates and product) in a state that never
+// converges, with zero vectors and sums, so x stays; bytes: every vector read
+// and written as in cg_lattice.h, and the coefficient values.
+void profile_lattice(femhip_solver &s, int32_t reps, double *ms_per_launch, double *bytes) {
+  hipStream_t st = s.ctx->stream;
+  const femhip_operator &op = *s.op;
+  CgState h{};
+  h.rz = 1.0;
+  h.rhs_test = -1.0;
+  h.rscale = 1.0;
+  h.delta = -1.0;
+  h.maxit = INT32_MAX;
+  h.crit = FEMHIP_RES_RES;
+  FH_HIP(hipMemcpyAsync(s.st.p, &h, sizeof(h), hipMemcpyHostToDevice, st));
+  FH_HIP(hipStreamSynchronize(st));
+  const bool mx = mixed(s);
+  auto zero = [&](DevBuf<double> &v, size_t count) {
+    hipLaunchKernelGGL(k_fill0, dim3(1024), dim3(256), 0, st, (int64_t)count, v.p);
+  };
+  for (auto *v : {&s.part_s, &s.part_u}) zero(*v, v->n);
+  zero(s.q, (size_t)s.n);
+  for (auto *v : {&s.r32, &s.r32_alt, &s.p32, &s.p32_alt, &s.q32, &s.q32_alt, &s.d32})
+    if (v->p) hipLaunchKernelGGL(k_to_f32, dim3(1024), dim3(256), 0, st, (int64_t)s.n, s.q.p, v->p);
+  for (auto *v : {&s.r, &s.r_alt, &s.p, &s.p_alt, &s.q_alt})
+    if (v->p) zero(*v, (size_t)s.n);
+  Launcher L;
+  L.stream = st;
+  const double *sc = s.prm.preconditioner == FEMHIP_PREC_JACOBI ? s.invd.p : nullptr;
+  // every iteration as an even one: the sums it reads stay zero
+  auto launch = [&] { enqueue_one(s, 0, L); };
+  for (int w = 0; w < 3; ++w) launch();
+  hipEvent_t e0, e1;
+  FH_HIP(hipEventCreate(&e0));
+  FH_HIP(hipEventCreate(&e1));
+  FH_HIP(hipEventRecord(e0, st));
+  for (int k = 0; k < reps; ++k) launch();
+  FH_HIP(hipEventRecord(e1, st));
+  FH_HIP(hipEventSynchronize(e1));
+  float ms = 0.f;
+  FH_HIP(hipEventElapsedTime(&ms, e0, e1));
+  (void)hipEventDestroy(e0);
+  (void)hipEventDestroy(e1);
+  if (ms_per_launch) *ms_per_launch = ms / reps;
+  const bool one = lattice_one_pass(s.n);
+  const double values = s.coef.kq ? (double)op.space->fe.nq : s.coef.kc ? 1.0 : 0.0;
+  if (bytes)
+    *bytes = (double)s.n * (one ? (mx ? 32.0 : 64.0) + (sc ? 8.0 : 0.0) : (mx ? 36.0 : 72.0) + (sc ? mx ? 8.0 : 16.0 : 0.0)) +
+             8.0 * values * (double)s.coef.cells;
+}
+
 double true_residual(femhip_solver &s) {
   hipStream_t st = s.ctx->stream;
   femhip_operator &op = *s.op;
-  hipLaunchKernelGGL(k_true_res, dim3(s.g_mat), dim3(kThreads), 0, st, sliced_dev(op), op.sl.v64.p, s.b.p, s.x.p,
-                     s.part_i.p);
+  if (s.lat) {
+    Launcher L;
+    L.stream = st;
+    L.lds = op.lat->lds;
+    L(s.lk.res, dim3(s.g_mat), dim3((unsigned)op.lat->threads), op.lat->g, s.coef, s.q2tab, s.n, (int)kLatTrue, 0,
+      s.x.p, s.b.p, nullptr, nullptr, nullptr, nullptr, nullptr, s.part_i.p);
+  } else {
+    hipLaunchKernelGGL(k_true_res, dim3(s.g_mat), dim3(kThreads), 0, st, sliced_dev(op), op.sl.v64.p, s.b.p, s.x.p,
+                       s.part_i.p);
+  }
   FH_HIP(hipGetLastError());
   std::vector<double> h((size_t)s.g_mat);
   FH_HIP(hipMemcpyAsync(h.data(), s.part_i.p, sizeof(double) * h.size(), hipMemcpyDeviceToHost, st));
@@ -1971,9 +2217,9 @@ void solver_copy_solution(const femhip_solver &s, double *x) {
 
 size_t solver_device_bytes(const femhip_solver &s) {
   size_t b = s.st.bytes() + s.res.bytes();
-  for (auto *v : {&s.x, &s.b, &s.r, &s.p, &s.q, &s.invd, &s.part_i, &s.part_s, &s.part_u, &s.part_r, &s.hist})
+  for (auto *v : {&s.x, &s.b, &s.r, &s.r_alt, &s.p, &s.p_alt, &s.q, &s.q_alt, &s.invd, &s.part_i, &s.part_s, &s.part_u, &s.part_r, &s.hist})
     b += v->bytes();
-  for (auto *v : {&s.r32, &s.p32, &s.q32, &s.d32}) b += v->bytes();
+  for (auto *v : {&s.r32, &s.r32_alt, &s.p32, &s.p32_alt, &s.q32, &s.q32_alt, &s.d32}) b += v->bytes();
   return b;
 }
 
@@ -2063,6 +2309,10 @@ int femhip_solver_profile_spmv(femhip_solver_t *s, int32_t reps, double *ms_per_
     hipStream_t st = s->ctx->stream;
     const bool mx = mixed(*s);
     upload_state(*s);   // done = 0
+    if (s->lat) {
+      profile_lattice(*s, reps, ms_per_launch, bytes);
+      return FEMHIP_OK;
+    }
     hipLaunchKernelGGL(k_fill0, dim3(1024), dim3(256), 0, st, (int64_t)s->n, s->p.p);
     if (mx) hipLaunchKernelGGL(k_to_f32, dim3(1024), dim3(256), 0, st, (int64_t)s->n, s->p.p, s->p32.p);
     const SlicedDev m = sliced_dev(op);

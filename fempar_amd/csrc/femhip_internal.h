@@ -5,6 +5,7 @@
 
 #include <atomic>
 #include <cstdint>
+#include <memory>
 #include <string>
 #include <vector>
 
@@ -145,6 +146,10 @@ inline void ctx_release(femhip_ctx *c) {
 }
 }  // namespace femhip
 
+namespace femhip {
+struct LatticeOp;   // lattice.h
+}
+
 struct femhip_space {
   femhip_ctx *ctx = nullptr;
   std::atomic<int> refs{1};           // the handle + every operator built on it
@@ -267,6 +272,15 @@ struct femhip_operator {
   int sym_gather = 0;                       // 0 not checked, 1 in use, -1 not applicable
   int8_t sym_kidx[32];
   int sym_written = 0;
+  // products from the cells instead of a stored matrix (lattice.hip): 0 not
+  // checked, 1 the lattice is set up, -1 not applicable; the map of operator
+  // rows to lattice rows (none: the same), and the caller's point values of k
+  // as [point][cell] for the physics of version lat_kq_version
+  int lat_state = 0;
+  std::shared_ptr<femhip::LatticeOp> lat;
+  femhip::DevBuf<int32_t> lat_perm;
+  femhip::DevBuf<double> lat_kq;
+  int64_t lat_kq_version = -1, phys_version = 0;   // phys_version: bumped by every set_physics
   // structured stencil operator (no CSR, no space): rows are component-major
   // blocks of `blk` rows (the `nodes` free nodes, padded to a multiple of 64),
   // values assembled in place into the sliced layout
@@ -332,6 +346,8 @@ void setup_sym_gather(femhip_operator &op);
 // FP32 on the matrix cores (scalar Q1); false where that does not apply
 bool assemble_sym32(femhip_operator &op, const double *sc, float *v32);
 void upload_physics(femhip_operator &op);
+// the per-direction sine tables of the closed-form coefficients (op.trig), built once
+void ensure_trig(femhip_operator &op);
 void spmv_full(femhip_operator &op, const double *d_x, double *d_y);
 // address of the no-allocation staging array on `device` (noalloc.hip); called
 // by femhip_ctx_create with that device current
@@ -404,6 +420,7 @@ inline size_t operator_device_bytes(const femhip_operator &op) {
   b += s.perm.bytes() + s.soffs.bytes() + s.base.bytes() + s.meta.bytes() + s.srow.bytes() + s.aux.bytes() + s.offs.bytes() +
        s.ecol.bytes() +
        s.map.bytes() + s.v64.bytes() + s.v32.bytes();
+  b += op.lat_perm.bytes() + op.lat_kq.bytes();
   if (op.space) b += op.space->d_dofs.bytes() + op.space->d_rep.bytes() + op.space->vcoords.bytes();
   return b;
 }

@@ -1,0 +1,696 @@
+// lattice.h -- products with the operator of a uniform structured mesh formed
+// from its cells, without a stored matrix (device templates).
+//
+// On the structured generator's mesh every cell is a translate of the first,
+// so the assembled operator is A = sum_c P_c^T K_c P_c with K_c fixed by the
+// cell's coefficient alone: one value (or one per quadrature point, or a closed
+// form of the position) instead of the 14 to 125 stored values a row of the
+// assembled matrix.  The free nodes form a box of the fine grid (p n_k + 1
+// nodes per direction, less the fixed faces), the vectors are kept in that
+// lexicographic box order, and nodes outside the box are zeros that are never
+// loaded.
+//
+// A workgroup owns a tile of cell columns, one cell per lane, and marches along
+// the last direction: the new planes of nodes go through LDS to the lanes of
+// the cells around them, each lane applies its cell in registers (sums
+// factorised over the directions), the plane below passes its partial sums
+// on in registers and the sums of nodes shared within the tile go through LDS.
+// The first row and column of a tile (other than at the mesh's start) and the
+// layer before a chunk are computed by both neighbours, so no sum crosses
+// workgroups: no atomics, a fixed order of summation, every result written
+// once.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <cstdint>
+
+#include "femhip_internal.h"
+
+namespace femhip {
+
+// Box lattice of the free nodes and its split into workgroups.  Lane (tx, ty)
+// of tile (i, j) is cell (i (TX - 1) + tx, j (TY - 1) + ty); E_k counts the
+// cells along k plus one where the last node plane is free (its owner is a
+// cell past the mesh that only receives sums).
+struct Lattice {
+  int nc[3] = {1, 1, 1};   // cells
+  int m[3] = {1, 1, 1};    // free nodes
+  int o[3] = {0, 0, 0};    // grid index of free node 0
+  int E[3] = {1, 1, 1};
+  int TX = 1, TY = 1, xt = 1, tiles = 1, nch = 1;   // tile, tiles along x, all tiles, chunks of the march
+  int stride = 0;          // rows between the components of a vector field
+};
+
+// Logical workgroup: each XCD (workgroups are dispatched round-robin over 8)
+// takes a contiguous range, so tiles that share halos share an L2.
+__device__ __forceinline__ int lattice_block(const Lattice &g) {
+  const int per = (gridDim.x + 7) / 8;
+  const int b = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
+  return gridDim.x % 8 == 0 ? b : (int)blockIdx.x;
+}
+
+// Vectors are read and written through buffer resources whose range check
+// gives 0 outside the vector and drops the store: nodes outside the box and
+// lanes that own nothing need no branch.  Offsets are bytes of an 8-byte
+// element; a vector has at most 2^30 bytes, kOutside plus any of them stays out
+// of range, and so does kNoPlane plus an offset inside a plane.
+constexpr uint32_t kOutside = 0x80000000u, kNoPlane = 0x40000000u;
+constexpr int64_t kLatticeMaxRows = (int64_t)1 << 27;
+using BufRsrc = __amdgpu_buffer_rsrc_t;
+__device__ __forceinline__ BufRsrc buf_of(const void *p, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, (int)bytes, 0x00027000);
+}
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ double buf_ld64(BufRsrc r, uint32_t o8) {
+  return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, (int)o8, 0, 0));
+}
+__device__ __forceinline__ float buf_ld32(BufRsrc r, uint32_t o8) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, (int)(o8 >> 1), 0, 0));
+}
+__device__ __forceinline__ void buf_st64(BufRsrc r, uint32_t o8, double v) {
+  __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), r, (int)o8, 0, 0);
+}
+__device__ __forceinline__ void buf_st32(BufRsrc r, uint32_t o8, float v) {
+  __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), r, (int)(o8 >> 1), 0, 0);
+}
+
+template <int DIM, int P>
+struct LatticeShape {
+  static constexpr int N1 = P + 1;
+  static constexpr int NPL = DIM == 3 ? N1 * N1 : N1;   // a cell's nodes in one plane of the march
+  static constexpr int OWN = DIM == 3 ? P * P : P;      // those the cell owns
+  static constexpr int NX = NPL - OWN;                  // those it shares with the next cells
+  // Q1: two sets of the LDS buffers and one barrier a layer, the loads of the
+  // next plane in flight while a layer is computed.  Q2 holds too much in
+  // registers for that: one set, two barriers.
+  static constexpr bool PIPE = P == 1;
+};
+
+// Largest workgroup and wanted waves a SIMD (registers 512 / waves) of the marches.
+#ifndef FEMHIP_LAT_T31
+#define FEMHIP_LAT_T31 512
+#define FEMHIP_LAT_W31 4
+#endif
+__host__ __device__ constexpr int lattice_threads(int dim, int p) { return dim == 3 && p == 1 ? FEMHIP_LAT_T31 : 256; }
+__host__ __device__ constexpr int lattice_waves(int dim, int p) { return dim == 3 && p == 1 ? FEMHIP_LAT_W31 : p == 1 ? 4 : 2; }
+
+// What an Io keeps of a node from value() to out(), in doubles (kKeep, at most).
+constexpr int kLatticeKeep = 3;
+// doubles of LDS a workgroup needs (new node planes, shared sums; PIPE: what
+// the lanes keep of their own nodes in the last three planes)
+template <int DIM, int P>
+inline size_t lattice_lds(int TX, int TY) {
+  using S = LatticeShape<DIM, P>;
+  const size_t cells = (size_t)TX * TY, plane = (size_t)(P * TX + 1) * (DIM == 3 ? P * TY + 1 : 1);
+  return (S::PIPE ? 2 : 1) * (size_t)P * (plane + S::NX * cells) + (S::PIPE ? 3 * kLatticeKeep * cells : 0);
+}
+// nodes of the row and column after a tile, one a thread
+template <int DIM, int P>
+inline int lattice_halo(int TX, int TY) {
+  return DIM == 3 ? P * (TX + TY) + 1 : 1;
+}
+
+// March of one workgroup; false: it has no cells, and ready() was not called.
+// Cell: begin(cx, cy, in the mesh), prefetch(cz) and
+// advance() for its coefficient, bottom(u) with the nodes of the first plane,
+// step(active, u, s): the P next planes in, the finished sums of the P planes
+// before the last of them out (this cell's share).
+// Io: Raw fetch(o) loads what the node at offset o needs; ready() then forms
+// what the pass needs first (false: nothing to do); value(raw, o, keep) gives
+// the node's value and stores what the pass updates there (o = kOutside: not
+// this workgroup's); out<FULL>(o, keep, y) takes the finished sum y of the
+// node, with all of what value() kept (FULL) or only its value, keep[0].
+// halo(o) and halo_value(raw): the value alone, of a node past the tile.
+template <int DIM, int P, class Cell, class Io>
+__device__ __forceinline__ bool lattice_march(const Lattice &g, Cell &cell, Io &io, double *lds) {
+  using S = LatticeShape<DIM, P>;
+  constexpr int N1 = S::N1, NPL = S::NPL, OWN = S::OWN, NX = S::NX;
+  constexpr bool PIPE = S::PIPE;
+  constexpr int AX = DIM - 1;
+  const int lb = lattice_block(g);
+  if (lb >= g.tiles * g.nch) return false;   // the same for the whole workgroup
+  const int tile = lb % g.tiles, chunk = lb / g.tiles;
+  const int ti = tile % g.xt, tj = tile / g.xt;
+  const int TX = g.TX, TY = DIM == 3 ? g.TY : 1;
+  const int X0 = ti * (TX - 1), Y0 = DIM == 3 ? tj * (TY - 1) : 0;
+  const int tid = threadIdx.x, cells = TX * TY;
+  const int tx = DIM == 3 ? tid % TX : tid, ty = DIM == 3 ? tid / TX : 0;
+  const bool lane = tid < cells;
+  const int cx = X0 + tx, cy = Y0 + ty;
+  const bool own_xy = lane && (tx > 0 || ti == 0) && (DIM == 2 || ty > 0 || tj == 0);
+  const bool in_xy = lane && cx < g.nc[0] && (DIM == 2 || cy < g.nc[1]);
+  const int z0 = (int)((int64_t)g.E[AX] * chunk / g.nch), z1 = (int)((int64_t)g.E[AX] * (chunk + 1) / g.nch);
+  if (z0 >= z1) return false;
+  const int zs = z0 > 0 ? z0 - 1 : 0;
+  const int LX = P * TX + 1, LY = DIM == 3 ? P * TY + 1 : 1, LP = LX * LY;
+  const uint32_t plane_bytes = 8u * (uint32_t)(DIM == 3 ? g.m[0] * g.m[1] : g.m[0]);
+  const int half = P * (LP + NX * cells);   // doubles of one set of buffers: U [P][LY][LX], C [P][NX][cells]
+
+  auto row_offset = [&](int px, int py, bool ok) {
+    const int gx = px - g.o[0], gy = DIM == 3 ? py - g.o[1] : 0;
+    ok = ok && gx >= 0 && gx < g.m[0] && (DIM == 2 || (gy >= 0 && gy < g.m[1]));
+    return ok ? 8u * (uint32_t)(gx + g.m[0] * gy) : kOutside;
+  };
+  uint32_t off[OWN];   // this lane's own nodes in a plane
+#pragma unroll
+  for (int j = 0; j < OWN; ++j) off[j] = row_offset(P * cx + j % P, P * cy + j / P, lane);
+  // one node of the row and column after the tile
+  const int nhalo = DIM == 3 ? LX + P * TY : 1;
+  const int hrow = DIM == 2 ? 0 : tid < LX ? P * TY : tid - LX;
+  const int hcol = DIM == 2 || tid >= LX ? P * TX : tid;
+  const bool halo = tid < nhalo;
+  const uint32_t hoff = row_offset(P * X0 + hcol, P * Y0 + hrow, halo);
+  const int hat = hrow * LX + hcol;
+  const int uat = P * ty * LX + P * tx;
+
+  auto plane_base = [&](int z) {
+    const int gz = z - g.o[AX];
+    return gz >= 0 && gz < g.m[AX] ? (uint32_t)gz * plane_bytes : kNoPlane;
+  };
+  typename Io::Raw raw[P][OWN];
+  typename Io::Halo hraw[P];
+  constexpr int KEEP = Io::kKeep;
+  double *ring = lds + (PIPE ? 2 : 1) * half + (lane ? tid : 0);   // PIPE: [3][KEEP][cells], plane z in part z mod 3
+  auto fetch = [&](int z, int count) {   // planes z .. z + count - 1
+#pragma unroll
+    for (int c = 0; c < P; ++c)
+      if (c < count) {
+        const uint32_t base = plane_base(z + c);
+#pragma unroll
+        for (int j = 0; j < OWN; ++j) raw[c][j] = io.fetch(base + off[j]);
+        hraw[c] = io.halo(base + hoff);
+      }
+  };
+  auto store = [&](double *U, int z, int count, int part) {
+#pragma unroll
+    for (int c = 0; c < P; ++c)
+      if (c < count) {
+        const uint32_t base = plane_base(z + c);
+        const bool own = own_xy && (z + c) / P >= z0 && (z + c) / P < z1;   // the layer that owns the plane
+#pragma unroll
+        for (int j = 0; j < OWN; ++j) {
+          double keep[KEEP];
+          const double v = io.value(raw[c][j], own ? base + off[j] : kOutside, keep);
+          if (lane) {
+            U[c * LP + uat + (j / P) * LX + j % P] = v;
+            if (PIPE)
+#pragma unroll
+              for (int k = 0; k < KEEP; ++k) ring[(part * KEEP + k) * cells] = keep[k];
+          }
+        }
+        const double h = io.halo_value(hraw[c]);
+        if (halo) U[c * LP + hat] = h;
+      }
+  };
+  auto read_plane = [&](const double *U, int c, double (&u)[NPL]) {
+    const double *Up = U + c * LP + (lane ? uat : 0);
+#pragma unroll
+    for (int b = 0; b < (DIM == 3 ? N1 : 1); ++b)
+#pragma unroll
+      for (int a = 0; a < N1; ++a) u[b * N1 + a] = Up[b * LX + a];
+  };
+  // sums of shared nodes to their owners: slots (a = P, b < P), (b = P, a < P), (P, P)
+  auto share = [&](double *C, const double (&s)[P][NPL]) {
+    if (lane) {
+#pragma unroll
+      for (int c = 0; c < P; ++c) {
+        double *Cp = C + c * NX * cells + tid;
+        if (DIM == 2) {
+          Cp[0] = s[c][P];
+        } else {
+#pragma unroll
+          for (int j = 0; j < P; ++j) {
+            Cp[j * cells] = s[c][j * N1 + P];
+            Cp[(P + j) * cells] = s[c][P * N1 + j];
+          }
+          Cp[2 * P * cells] = s[c][P * N1 + P];
+        }
+      }
+    }
+  };
+  const bool left = tx > 0, below = DIM == 3 && ty > 0, corner = left && below;
+  // kept(c, j, keep): what is kept of own node j of plane c; so(c, j): this cell's sum there
+  auto finish = [&](const double *C, int cz, auto &&so, auto &&kept) {
+    if (cz < z0) return;
+#pragma unroll
+    for (int c = 0; c < P; ++c) {
+      const uint32_t base = plane_base(P * cz + c);
+      const double *Cp = C + c * NX * cells + (lane ? tid : 0);
+#pragma unroll
+      for (int j = 0; j < OWN; ++j) {
+        const int a = j % P, b = j / P;
+        double y = so(c, j);
+        if (DIM == 2) {
+          if (a == 0) y += left ? Cp[-1] : 0.0;
+        } else {
+          if (a == 0) y += left ? Cp[b * cells - 1] : 0.0;
+          if (b == 0) y += below ? Cp[(P + a) * cells - TX] : 0.0;
+          if (a == 0 && b == 0) y += corner ? Cp[2 * P * cells - TX - 1] : 0.0;
+        }
+        double keep[KEEP];
+        kept(c, j, keep);
+        io.template out<PIPE>(own_xy ? base + off[j] : kOutside, keep, y);
+      }
+    }
+  };
+
+  fetch(P * zs, 1);
+  cell.begin(g, cx, cy, in_xy);
+  if (!io.ready()) return true;   // the same for every workgroup
+  store(lds, P * zs, 1, 0);
+  double ub[OWN];   // !PIPE: own nodes of the plane below the layer
+  if (PIPE) {
+    fetch(P * zs + 1, P);
+    cell.prefetch(g, zs, in_xy);
+  }
+  __syncthreads();
+  {
+    double u[NPL];
+    read_plane(lds, 0, u);
+#pragma unroll
+    for (int j = 0; j < OWN; ++j) ub[j] = u[(j / P) * N1 + j % P];
+    cell.bottom(u);
+  }
+
+  if (PIPE) {
+    double so[OWN];
+    int part = 0;   // of the plane below the layer finished next
+    auto so_at = [&](int, int j) { return so[j]; };
+    auto kept = [&](int, int, double (&keep)[KEEP]) {
+#pragma unroll
+      for (int k = 0; k < KEEP; ++k) keep[k] = ring[(part * KEEP + k) * cells];
+    };
+    int set = 1, next = 1;   // buffers; ring part of the plane stored next
+    for (int cz = zs; cz < z1; ++cz) {
+      double *U = lds + set * half, *C = U + P * LP;
+      store(U, P * cz + 1, P, next);
+      next = next == 2 ? 0 : next + 1;
+      cell.advance();
+      __syncthreads();
+      if (cz > zs) {
+        finish(lds + (set ^ 1) * half + P * LP, cz - 1, so_at, kept);
+        part = part == 2 ? 0 : part + 1;
+      }
+      if (cz + 1 < z1) {
+        fetch(P * (cz + 1) + 1, P);
+        cell.prefetch(g, cz + 1, in_xy);
+      }
+      double u[P][NPL], s[P][NPL];
+#pragma unroll
+      for (int c = 0; c < P; ++c) read_plane(U, c, u[c]);
+      cell.step(in_xy && cz < g.nc[AX], u, s);
+      share(C, s);
+#pragma unroll
+      for (int j = 0; j < OWN; ++j) so[j] = s[0][(j / P) * N1 + j % P];
+      set ^= 1;
+    }
+    __syncthreads();
+    finish(lds + (set ^ 1) * half + P * LP, z1 - 1, so_at, kept);
+  } else {
+    double *U = lds, *C = U + P * LP;
+    const double *Uo = U + (lane ? uat : 0);
+    for (int cz = zs; cz < z1; ++cz) {
+      fetch(P * cz + 1, P);
+      cell.prefetch(g, cz, in_xy);
+      cell.advance();
+      __syncthreads();   // the layer before has read U and C
+      store(U, P * cz + 1, P, 0);
+      __syncthreads();
+      double u[P][NPL], s[P][NPL];
+#pragma unroll
+      for (int c = 0; c < P; ++c) read_plane(U, c, u[c]);
+      cell.step(in_xy && cz < g.nc[AX], u, s);
+      share(C, s);
+      __syncthreads();
+      auto u_at = [&](int c, int j) { return Uo[c * LP + (j / P) * LX + j % P]; };
+      finish(C, cz, [&](int c, int j) { return s[c][(j / P) * N1 + j % P]; },
+             [&](int c, int j, double (&keep)[KEEP]) { keep[0] = c == 0 ? ub[j] : u_at(c - 1, j); });
+#pragma unroll
+      for (int j = 0; j < OWN; ++j) ub[j] = u_at(P - 1, j);
+    }
+  }
+  return true;
+}
+
+// ----------------------------------------------------------------- cells ---
+
+// Where the coefficient of a Poisson cell comes from.
+enum { kCoefCell = 0,    // one value: k0, or kc[cell]
+       kCoefSin3 = 1,    // 1 + 1/2 prod sin(2 pi x_d), from the sines at the 1-D Gauss points of each layer
+       kCoefPoint = 2 }; // kq[q cells + cell]
+
+struct CoefDev {
+  double k0 = 1.0;
+  const double *kc = nullptr, *kq = nullptr;
+  const double4 *trig = nullptr;   // {., ., sin 2 pi x, .} per (layer, point), offsets per direction
+  int toff[3] = {0, 0, 0};
+  int64_t cells = 0;
+  double c[3] = {0, 0, 0};         // weight of the squared derivative along each direction
+  bool operator==(const CoefDev &o) const {
+    bool same = k0 == o.k0 && kc == o.kc && kq == o.kq && trig == o.trig && cells == o.cells;
+    for (int d = 0; d < 3; ++d) same = same && toff[d] == o.toff[d] && c[d] == o.c[d];
+    return same;
+  }
+};
+
+// Q1: in each direction the two end values become their sum and difference,
+// in which the 1-D interpolation to the Gauss points +-1/sqrt(3) is
+// (s +- d / sqrt(3)) / 2 and the derivative d / h.  A derivative along x is
+// constant along x, so it has 4 (2) values in a cell, each weighted by the
+// coefficient summed over the two points along x; the factors 1/2 and 1/h are
+// in CoefDev::c.  One value a cell: the weights pull out and the form is
+// diagonal in these modes.  About 55 (one value) to 140 FP64 operations a cell
+// in 3-D against 2 x 27 a row of the assembled matrix, but no stored value.
+constexpr double kGauss2 = 0.57735026918962576451;   // 1 / sqrt(3)
+
+template <int DIM, int KIND>
+struct CellQ1 {
+  static constexpr int NPL = DIM == 3 ? 4 : 2, NV = 1 << DIM, NK = KIND == kCoefPoint ? NV : 1;
+  CoefDev k;
+  double kv[NK], kn[NK];          // this layer's values, the next one's
+  double sz[2], sn[2];            // sines at the march's points
+  double ka[2], kb[2], kc4[4];    // in-plane factors of the coefficient summed along x, y and the march
+  double below[NPL], carry[NPL];  // modes of the plane below, unfinished sums of its modes
+  int64_t col, plane;
+
+  __device__ __forceinline__ void begin(const Lattice &g, int cx, int cy, bool in) {
+    col = in ? cx + (int64_t)g.nc[0] * (DIM == 3 ? cy : 0) : 0;
+    plane = (int64_t)g.nc[0] * (DIM == 3 ? g.nc[1] : 1);
+    if (KIND == kCoefSin3) {
+      const int x = in ? cx : 0, y = in ? cy : 0;
+      const double x0 = k.trig[k.toff[0] + 2 * x].z, x1 = k.trig[k.toff[0] + 2 * x + 1].z;
+      if (DIM == 3) {
+        const double y0 = k.trig[k.toff[1] + 2 * y].z, y1 = k.trig[k.toff[1] + 2 * y + 1].z;
+        ka[0] = 0.5 * (x0 + x1) * y0;
+        ka[1] = 0.5 * (x0 + x1) * y1;
+        kb[0] = 0.5 * (y0 + y1) * x0;
+        kb[1] = 0.5 * (y0 + y1) * x1;
+        kc4[0] = x0 * y0;
+        kc4[1] = x1 * y0;
+        kc4[2] = x0 * y1;
+        kc4[3] = x1 * y1;
+      } else {
+        ka[0] = 0.5 * (x0 + x1);
+        kb[0] = x0;
+        kb[1] = x1;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < NPL; ++i) carry[i] = 0.0;
+  }
+  __device__ __forceinline__ void prefetch(const Lattice &g, int cz, bool in) {
+    const int z = min(cz, g.nc[DIM - 1] - 1);
+    const int64_t at = col + plane * z;
+    if (KIND == kCoefCell) {
+      kn[0] = k.kc ? k.kc[at] : k.k0;
+    } else if (KIND == kCoefPoint) {
+#pragma unroll
+      for (int q = 0; q < NV; ++q) kn[q] = k.kq[q * k.cells + at];
+    } else {
+      sn[0] = k.trig[k.toff[DIM - 1] + 2 * z].z;
+      sn[1] = k.trig[k.toff[DIM - 1] + 2 * z + 1].z;
+    }
+  }
+  __device__ __forceinline__ void advance() {
+    if (KIND == kCoefSin3) {
+      sz[0] = sn[0];
+      sz[1] = sn[1];
+    } else {
+#pragma unroll
+      for (int q = 0; q < NK; ++q) kv[q] = kn[q];
+    }
+  }
+  // coefficient summed over the two points along direction d, at point (qe, qf)
+  // of the other directions (ascending)
+  __device__ __forceinline__ double ksum(int d, int qe, int qf) const {
+    if (KIND == kCoefPoint) {
+      const int e = d == 0 ? 1 : 0, f = 3 - d - e;
+      const int q = (qe << e) | (DIM == 3 ? qf << f : 0);
+      return kv[q] + kv[q | (1 << d)];
+    }
+    if (DIM == 2) return d == 0 ? __builtin_fma(ka[0], sz[qe], 2.0) : __builtin_fma(kb[qe], 0.5 * (sz[0] + sz[1]), 2.0);
+    if (d == 0) return __builtin_fma(ka[qe], sz[qf], 2.0);
+    if (d == 1) return __builtin_fma(kb[qe], sz[qf], 2.0);
+    return __builtin_fma(kc4[qe + 2 * qf], 0.5 * (sz[0] + sz[1]), 2.0);
+  }
+  // nodes of a plane -> sums and differences in the plane (bit set = difference)
+  static __device__ __forceinline__ void modes(const double (&u)[NPL], double (&m)[NPL]) {
+    if (DIM == 2) {
+      m[0] = u[0] + u[1];
+      m[1] = u[1] - u[0];
+    } else {
+      const double a = u[0] + u[1], b = u[1] - u[0], c = u[2] + u[3], d = u[3] - u[2];
+      m[0] = a + c;
+      m[1] = b + d;
+      m[2 % NPL] = c - a;
+      m[3 % NPL] = d - b;
+    }
+  }
+  // and the transpose
+  static __device__ __forceinline__ void nodes(const double (&m)[NPL], double (&u)[NPL]) {
+    if (DIM == 2) {
+      u[0] = m[0] - m[1];
+      u[1] = m[0] + m[1];
+    } else {
+      const double a = m[0] - m[2 % NPL], b = m[1] - m[3 % NPL], c = m[0] + m[2 % NPL], d = m[1] + m[3 % NPL];
+      u[0] = a - b;
+      u[1] = a + b;
+      u[2 % NPL] = c - d;
+      u[3 % NPL] = c + d;
+    }
+  }
+  __device__ __forceinline__ void bottom(const double (&u)[NPL]) { modes(u, below); }
+  __device__ __forceinline__ void step(bool active, const double (&u)[1][NPL], double (&s)[1][NPL]) {
+    double h[NV], r[NV], top[NPL], sum[NPL];
+    modes(u[0], top);
+#pragma unroll
+    for (int i = 0; i < NPL; ++i) {
+      h[i] = below[i] + top[i];
+      h[NPL + i] = top[i] - below[i];
+      below[i] = top[i];
+    }
+    constexpr double al = kGauss2, t = 1.0 / 3.0;   // interpolation's difference factor and its square
+    if (KIND == kCoefCell) {
+      const double kc = active ? kv[0] : 0.0;
+      r[0] = 0.0;
+#pragma unroll
+      for (int i = 1; i < NV; ++i) {
+        const int others = __builtin_popcount(i) - 1;
+        const double f = (others == 0 ? 1.0 : others == 1 ? t : t * t) * (double)NV;
+        double w = 0.0;
+#pragma unroll
+        for (int d = 0; d < DIM; ++d)
+          if ((i >> d) & 1) w += k.c[d];
+        r[i] = (w * f) * h[i];
+      }
+#pragma unroll
+      for (int i = 0; i < NPL; ++i) {
+        sum[i] = __builtin_fma(kc, r[i] - r[NPL + i], carry[i]);
+        carry[i] = kc * (r[i] + r[NPL + i]);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < NV; ++i) r[i] = 0.0;
+      if (active) {   // lanes past the mesh only pass sums on
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) {
+          const int D = 1 << d, e = d == 0 ? 1 : 0, E = 1 << e;
+          if (DIM == 2) {
+            const double g0 = __builtin_fma(-al, h[D | E], h[D]), g1 = __builtin_fma(al, h[D | E], h[D]);
+            const double w0 = g0 * ksum(d, 0, 0), w1 = g1 * ksum(d, 1, 0);
+            r[D] = __builtin_fma(k.c[d], w0 + w1, r[D]);
+            r[D | E] = __builtin_fma(k.c[d] * al, w1 - w0, r[D | E]);
+          } else {
+            const int f = 3 - d - e, F = 1 << f;
+            const double a0 = __builtin_fma(-al, h[D | E], h[D]), a1 = __builtin_fma(al, h[D | E], h[D]);
+            const double b0 = __builtin_fma(-al, h[D | E | F], h[D | F]), b1 = __builtin_fma(al, h[D | E | F], h[D | F]);
+            const double w00 = __builtin_fma(-al, b0, a0) * ksum(d, 0, 0);
+            const double w10 = __builtin_fma(-al, b1, a1) * ksum(d, 1, 0);
+            const double w01 = __builtin_fma(al, b0, a0) * ksum(d, 0, 1);
+            const double w11 = __builtin_fma(al, b1, a1) * ksum(d, 1, 1);
+            const double s0 = w00 + w10, d0 = w10 - w00, s1 = w01 + w11, d1 = w11 - w01;
+            r[D] = __builtin_fma(k.c[d], s0 + s1, r[D]);
+            r[D | E] = __builtin_fma(k.c[d] * al, d0 + d1, r[D | E]);
+            r[D | F] = __builtin_fma(k.c[d] * al, s1 - s0, r[D | F]);
+            r[D | E | F] = __builtin_fma(k.c[d] * al * al, d1 - d0, r[D | E | F]);
+          }
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < NPL; ++i) {
+        sum[i] = carry[i] + (r[i] - r[NPL + i]);
+        carry[i] = r[i] + r[NPL + i];
+      }
+    }
+    nodes(sum, s[0]);
+  }
+};
+
+// Q2: interpolation to the 3 Gauss points in every direction (values scaled by
+// the square roots of the weights, so no weight is left), then along each
+// direction the derivative at the points, the coefficient, and the transposes.
+// Both 3 x 3 factors split into the even and odd parts of the three values.
+struct Q2Tab {
+  double b0, b1, c, beta;      // interpolation: E = b0 (u0 + u2) + b1 u1, +- c (u2 - u0); centre beta u1
+  double r, delta, ec, b;      // derivative: R = r (v2 - v0), Q = ec (v0 + v2) - b v1; R -+ Q; centre delta (v2 - v0)
+};
+
+template <int DIM, int KIND>
+struct CellQ2 {
+  static constexpr int NPL = DIM == 3 ? 9 : 3, N = DIM == 3 ? 27 : 9;
+  CoefDev k;
+  Q2Tab t;
+  double kv, kn;
+  double sz[3], sn[3], kxy[NPL];
+  double below[NPL], carry[NPL];   // the plane below interpolated in the plane, its unfinished sums
+  int64_t col, plane, at0, atn;
+
+  __device__ __forceinline__ void begin(const Lattice &g, int cx, int cy, bool in) {
+    col = in ? cx + (int64_t)g.nc[0] * (DIM == 3 ? cy : 0) : 0;
+    plane = (int64_t)g.nc[0] * (DIM == 3 ? g.nc[1] : 1);
+    if (KIND == kCoefSin3) {
+      const int x = in ? cx : 0, y = in ? cy : 0;
+#pragma unroll
+      for (int i = 0; i < NPL; ++i)
+        kxy[i] = k.trig[k.toff[0] + 3 * x + i % 3].z * (DIM == 3 ? k.trig[k.toff[1] + 3 * y + i / 3].z : 1.0);
+    }
+#pragma unroll
+    for (int i = 0; i < NPL; ++i) carry[i] = 0.0;
+  }
+  __device__ __forceinline__ void prefetch(const Lattice &g, int cz, bool in) {
+    const int z = min(cz, g.nc[DIM - 1] - 1);
+    atn = col + plane * z;
+    if (KIND == kCoefCell) {
+      kn = k.kc ? k.kc[atn] : k.k0;
+    } else if (KIND == kCoefSin3) {
+#pragma unroll
+      for (int a = 0; a < 3; ++a) sn[a] = 0.5 * k.trig[k.toff[DIM - 1] + 3 * z + a].z;
+    }
+  }
+  __device__ __forceinline__ void advance() {
+    at0 = atn;
+    kv = kn;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) sz[a] = sn[a];
+  }
+  __device__ __forceinline__ double at(int q) const {
+    if (KIND == kCoefPoint) return k.kq[q * k.cells + at0];
+    if (KIND == kCoefSin3) return __builtin_fma(kxy[q % NPL], sz[q / NPL], 1.0);
+    return 1.0;
+  }
+  // The coefficients of a cell's points are formed (or loaded) again for each
+  // direction: 27 of them kept would spill.
+  __device__ __forceinline__ void forget() {
+    if (KIND == kCoefSin3) {
+#pragma unroll
+      for (int a = 0; a < 3; ++a) asm volatile("" : "+v"(sz[a]));
+    } else if (KIND == kCoefPoint) {
+      asm volatile("" : "+v"(at0));
+    }
+  }
+  // interpolation along the direction of stride st of M values, and its transpose
+  template <int st, int M>
+  __device__ __forceinline__ void interp(double (&v)[M]) const {
+#pragma unroll
+    for (int i = 0; i < M; ++i)
+      if ((i / st) % 3 == 0) {
+        const double u0 = v[i], u1 = v[i + st], u2 = v[i + 2 * st];
+        const double o = u2 - u0, e = __builtin_fma(t.b1, u1, t.b0 * (u0 + u2));
+        v[i] = __builtin_fma(-t.c, o, e);
+        v[i + st] = t.beta * u1;
+        v[i + 2 * st] = __builtin_fma(t.c, o, e);
+      }
+  }
+  template <int st, int M>
+  __device__ __forceinline__ void interp_t(double (&v)[M]) const {
+#pragma unroll
+    for (int i = 0; i < M; ++i)
+      if ((i / st) % 3 == 0) {
+        const double y0 = v[i], y1 = v[i + st], y2 = v[i + 2 * st];
+        const double e = y0 + y2, o = y2 - y0, E = t.b0 * e;
+        v[i] = __builtin_fma(-t.c, o, E);
+        v[i + st] = __builtin_fma(t.b1, e, t.beta * y1);
+        v[i + 2 * st] = __builtin_fma(t.c, o, E);
+      }
+  }
+  template <int st>
+  __device__ __forceinline__ void derive(double cd, const double (&v)[N], double (&w)[N]) const {
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+      if ((i / st) % 3 == 0) {
+        const double v0 = v[i], v1 = v[i + st], v2 = v[i + 2 * st];
+        const double o = v2 - v0, Q = __builtin_fma(t.ec, v0 + v2, -t.b * v1);
+        double g0 = __builtin_fma(t.r, o, -Q), g1 = t.delta * o, g2 = __builtin_fma(t.r, o, Q);
+        if (KIND != kCoefCell) {
+          g0 *= at(i);
+          g1 *= at(i + st);
+          g2 *= at(i + 2 * st);
+        }
+        const double R = g0 + g2, D = g2 - g0;
+        const double oc = __builtin_fma(t.r, R, t.delta * g1), e = t.ec * D;
+        w[i] = __builtin_fma(cd, e - oc, w[i]);
+        w[i + st] = __builtin_fma(-cd * t.b, D, w[i + st]);
+        w[i + 2 * st] = __builtin_fma(cd, e + oc, w[i + 2 * st]);
+      }
+  }
+  __device__ __forceinline__ void in_plane(double (&v)[NPL]) const {
+    interp<1, NPL>(v);
+    if (DIM == 3) interp<DIM == 3 ? 3 : 1, NPL>(v);
+  }
+  __device__ __forceinline__ void bottom(const double (&u)[NPL]) {
+#pragma unroll
+    for (int i = 0; i < NPL; ++i) below[i] = u[i];
+    in_plane(below);
+  }
+  __device__ __forceinline__ void step(bool active, double (&u)[2][NPL], double (&s)[2][NPL]) {
+    double v[N], w[N];
+    in_plane(u[0]);
+    in_plane(u[1]);
+#pragma unroll
+    for (int i = 0; i < NPL; ++i) {
+      v[i] = below[i];
+      v[NPL + i] = u[0][i];
+      v[2 * NPL + i] = u[1][i];
+      below[i] = u[1][i];
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i) w[i] = 0.0;
+    if (active) {   // lanes past the mesh only pass sums on
+      interp<NPL, N>(v);
+      const double f = KIND == kCoefCell ? kv : 1.0;
+      derive<1>(f * k.c[0], v, w);
+      forget();
+      derive<3>(f * k.c[1], v, w);
+      forget();
+      if (DIM == 3) derive<DIM == 3 ? 9 : 1>(f * k.c[2], v, w);
+      interp_t<NPL, N>(w);
+    }
+#pragma unroll
+    for (int i = 0; i < NPL; ++i) {
+      s[0][i] = carry[i] + w[i];
+      s[1][i] = w[NPL + i];
+      carry[i] = w[2 * NPL + i];
+    }
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      if (DIM == 3) interp_t<DIM == 3 ? 3 : 1, NPL>(s[c]);
+      interp_t<1, NPL>(s[c]);
+    }
+  }
+};
+
+// A lattice operator on the host (lattice.hip).
+struct LatticeOp {
+  Lattice g;
+  int dim = 0, order = 0, ncomp = 1;
+  int threads = 64, grid = 8;       // workgroup size and count
+  size_t lds = 0;                   // bytes of LDS a workgroup
+  bool identity = false;            // lattice rows are the operator's rows
+};
+bool lattice_plan(const femhip_mesh_desc_t &mesh, int cus, LatticeOp &L);
+bool lattice_operator(femhip_operator &op);
+CoefDev lattice_coefficient(femhip_operator &op);
+Q2Tab lattice_q2_tab();
+
+}  // namespace femhip
