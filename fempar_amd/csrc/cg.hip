@@ -40,6 +40,7 @@
 
 #include "femhip_internal.h"
 #include "lattice.h"
+#include "cg_state.h"
 
 namespace femhip {
 namespace {
@@ -57,25 +58,6 @@ constexpr int kPrefetch = 4;
 // recurrence residual fell by this factor (measured at 128^3: 0.02 gives 263
 // inner + 7 updates, 0.1 gives 259 + 11, 0.005 gives 276 + 5).
 constexpr double kDefaultDelta = 0.02;
-
-struct CgState {
-  double rz, rnrm_m, alpha, beta;
-  double rhs_test, rhs_extra, est, pap, pp;
-  double bnorm, r0norm, rnorm;
-  double rtol, atol;
-  double rmax, delta;          // reliable updates
-  double ru_rz, ru_rmax, ru_rnorm, ru_beta;
-  double rscale, ru_rscale;    // ||S r|| / ||r|| at the last update (scaled inner residual)
-  int iter, done, converged, maxit, crit, ru, updates, ru_conv, ru_done, first;
-  int set, pad;                // lattice FP32 passes: which of the two vector sets holds r, p, s
-};
-
-struct CgResult {
-  double est, rhs_test, rnorm, bnorm;
-  int iter, done, converged, updates;
-  double prog;                 // latest quantity the stopping test compares with rhs_test ...
-  int prog_it, pad;            // ... and its iteration (for the host's chunk planning)
-};
 
 struct SlicedDev {
   int32_t ns, n;
@@ -99,13 +81,6 @@ struct SlicedDev {
 __device__ __forceinline__ int slice_row_index(const SlicedDev &m, int s, int lane) {
   if (m.sym || m.srow == nullptr) return s * kSlice + lane;
   return ((m.meta[s] >> 28) & 1) ? m.srow[s * kSlice + lane] : s * kSlice + lane;
-}
-
-__device__ __forceinline__ bool is_delta(int c) {
-  return c == FEMHIP_DELTA_RHS || c == FEMHIP_DELTA_DELTA || c >= FEMHIP_DELTA_RHS_AND_RES_RES;
-}
-__device__ __forceinline__ bool is_delta_delta(int c) {
-  return c == FEMHIP_DELTA_DELTA || c == FEMHIP_DELTA_DELTA_AND_RES_RES || c == FEMHIP_DELTA_DELTA_AND_RES_RHS;
 }
 
 // Sum NV values over the block; every thread gets the result.
@@ -208,9 +183,6 @@ __device__ __forceinline__ void st_nt(T *p, T v) {
   __builtin_nontemporal_store(v, p);
 }
 
-// The next FP32 CG direction p' = beta p + z, rounded once (fused multiply-add).
-__device__ __forceinline__ float dir_value(float beta, float p, float z) { return __builtin_fmaf(beta, p, z); }
-
 // Right-hand vectors of the slice kernels.  operator()(c) is element c;
 // off(o, rb) is element row + o where rb = row * sizeof(elem): a scalar base
 // pointer per diagonal plus a per-lane 32-bit byte offset, so a gather needs no
@@ -222,12 +194,6 @@ struct VecRef {   // x
   __device__ __forceinline__ X operator()(int c) const { return x[c]; }
   __device__ __forceinline__ X off(int o, uint32_t rb) const { return *(const X *)((const char *)(x + o) + rb); }
 };
-// FP64 solution plus FP32 increment (scaled by sc when set): the solution a
-// reliable update makes.
-__device__ __forceinline__ double new_x(double x, float d, const double *sc, int64_t i) {
-  return sc ? __builtin_fma(sc[i], (double)d, x) : x + (double)d;
-}
-
 // Row `lane` of slice s (s wave-uniform): returns (A g)_row.  Slices whose
 // columns may leave [0, n) (flag bit 29) clamp the column.
 // Symmetric-diagonal rows: y_r = sum_k V[k][r] g[r+o_k] + sum_{k>0} V[k][r-o_k] g[r-o_k]
@@ -534,56 +500,6 @@ __global__ __launch_bounds__(kThreads) void k_update(int32_t n, T *__restrict__ 
   for (int64_t i = i0 + kPrefetch * stride; i < n; i += stride) row(i, r[i], q[i], invd ? invd[i] : (T)1);
   double out[2] = {(double)rz, (double)rr};
   write_partials<2>(out, part);
-}
-
-// Stopping test (cg.f90:323-407) after the iteration whose <r,z>, ||r||^2 are
-// red[0], red[1]; `lead` (one thread of the launch) writes the next state, the
-// history and the result blocks.  Returns done, beta for the next direction.
-__device__ __forceinline__ bool cg_decide(const CgState &cur, const double (&red)[2], bool lead, CgState &next,
-                                          double *hist, CgResult *R, CgResult *Rh, double &beta_out) {
-  const int it = cur.iter + 1;
-  const int c = cur.crit;
-  const double rnorm = sqrt(red[1]);
-  double est = cur.est, rhs_test = cur.rhs_test;
-  if (it == 1 && is_delta(c)) {
-    est = cur.alpha * sqrt(cur.pp);
-    if (is_delta_delta(c)) rhs_test = cur.rtol * est + cur.atol;
-  }
-  if (c == FEMHIP_RES_RES || c == FEMHIP_RES_RHS) est = rnorm;
-  else if (is_delta(c)) {
-    if (it != 1) est = cur.alpha * sqrt(cur.pp);
-  } else est = cur.rnrm_m;
-  int conv = est <= rhs_test;
-  if (c >= FEMHIP_DELTA_RHS_AND_RES_RES && conv) conv = rnorm <= cur.rhs_extra;
-  const bool done = conv || it >= cur.maxit;
-  double beta = 1.0 / cur.rz;
-  beta = beta * red[0];
-  if (lead) {
-    CgState nx = cur;
-    nx.first = 0;
-    nx.iter = it;
-    nx.est = est;
-    nx.rhs_test = rhs_test;
-    nx.rnorm = rnorm;
-    nx.converged = conv;
-    nx.done = done;
-    nx.beta = beta;
-    nx.rz = red[0];
-    nx.rnrm_m = sqrt(red[0]);
-    next = nx;
-    if (hist) hist[it - 1] = est;
-    R->iter = it;
-    R->est = est;
-    R->rhs_test = rhs_test;
-    R->rnorm = rnorm;
-    R->converged = conv;
-    R->done = done;
-    R->prog = est;
-    R->prog_it = it;
-    if (Rh) *Rh = *R;
-  }
-  beta_out = beta;
-  return done;
 }
 
 // stopping test (cg.f90:323-407) ; beta ; x += alpha p ; p = z + beta p
@@ -955,77 +871,6 @@ __global__ __launch_bounds__(kThreads) void k_ru_dir(int32_t n, float *__restric
 // S[par ^ 1], its block 0 stores alpha there for the next slot A.
 
 constexpr int kRfbGroup = 8;   // slices of a wave whose r and q loads k_rf_b keeps in flight together
-
-// What a slot A does: the decision after the previous slot B, whose <r,r> (and
-// after a fold the FP64 ||b - A x||^2) are red; `lead` writes the next state.
-struct RfStep {
-  int fold, upd_d, done;
-  double beta;
-};
-__device__ __forceinline__ RfStep rf_decide(const CgState &cur, const double (&red)[2], bool lead, CgState &next,
-                                            CgResult *R) {
-  if (lead) {
-    next = cur;
-    next.first = 0;
-  }
-  int fold = 0, upd_d = 0, done = 0;
-  double beta = 0.0;
-  if (cur.first) {           // p = r, q = A r
-  } else if (!cur.ru) {      // an iteration's r update has been made
-    const int it = cur.iter + 1;
-    const double rnorm = sqrt(red[0]);   // of the scaled FP32 residual
-    // residual fell by delta since the last update, looks converged (threshold
-    // carried into the scaled norm by the last update's ratio), or budget spent
-    fold = rnorm < cur.delta * cur.rmax || rnorm <= cur.rhs_test * cur.rscale || it >= cur.maxit;
-    if (!fold) {
-      beta = 1.0 / cur.rz;
-      beta = beta * red[0];
-      upd_d = 1;
-    }
-    if (lead) {
-      CgState &w = next;
-      w.iter = it;
-      w.rnorm = rnorm;
-      w.ru = fold;
-      if (!fold) {
-        w.beta = beta;
-        w.rz = red[0];
-        w.rmax = fmax(cur.rmax, rnorm);
-      }
-      R->iter = it;
-      R->prog = cur.rscale > 0.0 ? rnorm / cur.rscale : rnorm;   // estimate in the stopping test's norm
-      R->prog_it = it;
-    }
-  } else {                   // slot B replaced r by the FP64 residual of the folded x
-    const double rn64 = sqrt(red[1]);
-    const int conv = rn64 <= cur.rhs_test;
-    beta = 1.0 / cur.rz;
-    beta = beta * red[0];
-    done = conv || cur.iter >= cur.maxit;
-    if (lead) {
-      CgState &w = next;
-      w.ru = 0;
-      w.rz = red[0];
-      w.beta = beta;
-      w.rmax = sqrt(red[0]);
-      w.rscale = rn64 > 0.0 ? sqrt(red[0]) / rn64 : cur.rscale;
-      w.updates = cur.updates + 1;
-      w.est = rn64;
-      w.rnorm = rn64;
-      w.converged = conv;
-      w.done = done;
-      R->iter = cur.iter;
-      R->est = rn64;
-      R->rnorm = rn64;
-      R->converged = conv;
-      R->done = done;
-      R->updates = cur.updates + 1;
-      R->prog = rn64;
-      R->prog_it = cur.iter;
-    }
-  }
-  return {fold, upd_d, done, beta};
-}
 
 template <typename A>
 __global__ __launch_bounds__(kThreads, 4) void k_rf_a(SlicedDev m, SlicedDev m32, const float *__restrict__ v32,
@@ -1492,13 +1337,14 @@ bool fp32_integration() {
   return e && atoi(e) == 1;
 }
 
-// Whether a solver forms its products from the cells: scalar Poisson operators
-// on the uniform mesh (lattice_operator), in FP64 and FP32_REFINED.  FP32_STRICT
+// Whether a solver forms its products from the cells: scalar Poisson and vector
+// Q1 elasticity on the uniform mesh (lattice_operator), in FP64 and FP32_REFINED.  FP32_STRICT
 // and the FP32 integration are defined by their stored FP32 matrix.  Up to 4096
 // rows an iteration is launch latency whichever product it takes (32^2 Q1: 14.6
 // us stored, 11.1 us from the cells), and the stored matrix stays.
 constexpr int32_t kLatticeMinRows = 4097;
 bool wants_lattice(femhip_solver &s) {
+  if (s.op->structured) return true;   // has no other form
   return s.op->n >= kLatticeMinRows && !strict(s) && !(mixed(s) && fp32_integration()) && lattice_operator(*s.op);
 }
 
@@ -1529,10 +1375,8 @@ void prepare_host_slots(femhip_solver &s) {
 }
 
 // One launch an iteration or two (cg_lattice.h).
-#ifndef FEMHIP_LAT_ONE
-#define FEMHIP_LAT_ONE 400000
-#endif
-bool lattice_one_pass(int32_t n) { return n < FEMHIP_LAT_ONE; }
+constexpr int32_t kOneLaunchRows = 400000;
+bool lattice_one_pass(int32_t n) { return n < kOneLaunchRows; }
 
 void prepare_lattice(femhip_solver &s) {
   femhip_operator &op = *s.op;
@@ -1557,6 +1401,12 @@ void prepare_lattice(femhip_solver &s) {
       if (lattice_one_pass(n))
         for (auto *v : {&s.r_alt, &s.q_alt}) v->alloc(n);
     }
+    if (L.ncomp > 1)   // rows between the components are no nodes: they stay zero
+      for (auto *v : {&s.r, &s.r_alt, &s.p, &s.p_alt, &s.q, &s.q_alt})
+        if (v->p) FH_HIP(hipMemsetAsync(v->p, 0, v->bytes(), st));
+    if (L.ncomp > 1)
+      for (auto *v : {&s.r32, &s.r32_alt, &s.p32, &s.p32_alt, &s.q32, &s.q32_alt, &s.d32})
+        if (v->p) FH_HIP(hipMemsetAsync(v->p, 0, v->bytes(), st));
     s.part_i.alloc((size_t)4 * s.g_mat);
     s.part_s.alloc((size_t)kSums * s.g_mat);   // the passes' sums, alternating
     s.part_u.alloc((size_t)kSums * std::max(s.g_mat, s.g_vec));
@@ -1568,7 +1418,8 @@ void prepare_lattice(femhip_solver &s) {
     s.prepared = true;
   }
   const CoefDev coef = lattice_coefficient(op);
-  const int kind = op.phys.k_kind == FEMHIP_K_SIN3 ? kCoefSin3
+  const int kind = op.phys.kind == FEMHIP_PHYS_ELASTICITY ? kElastic
+                   : op.phys.k_kind == FEMHIP_K_SIN3 ? kCoefSin3
                    : op.phys.k_kind == FEMHIP_K_QPOINT ? kCoefPoint : kCoefCell;
   const LatticeKernels lk = lattice_kernels(L.dim, L.order, kind);
   if (lk.cg != s.lk.cg || !(coef == s.coef)) drop_graphs(s);   // they hold both by value
@@ -1576,7 +1427,11 @@ void prepare_lattice(femhip_solver &s) {
   s.lk = lk;
   if (jac && n > 0) {
     *s.h_flag = 0;
-    hipLaunchKernelGGL(k_lat_jacobi, dim3((n + 255) / 256), dim3(256), 0, st, n, op.rowptr.p, op.col.p, op.val.p,
+    if (op.structured)
+      hipLaunchKernelGGL(k_jacobi_diag, dim3((n + 255) / 256), dim3(256), 0, st, n, op.diag.p, s.invd.p, mx ? 1 : 0,
+                         s.d_flag);
+    else
+      hipLaunchKernelGGL(k_lat_jacobi, dim3((n + 255) / 256), dim3(256), 0, st, n, op.rowptr.p, op.col.p, op.val.p,
                        L.identity ? nullptr : op.lat_perm.p, s.invd.p, mx ? 1 : 0, s.d_flag);
     FH_HIP(hipGetLastError());
   }
@@ -1665,7 +1520,7 @@ void prepare(femhip_solver &s) {
     if (op.sl.sym)
       hipLaunchKernelGGL(k_jacobi_sym, G, B, 0, st, n, op.sl.v64.p, op.sl.stride, op.sl.kplus, s.invd.p, root,
                          s.d_flag);
-    else if (op.structured || op.sl.permuted)   // no CSR in the solver's order: the diagonal of the sliced copy
+    else if (op.sl.permuted)   // no CSR in the solver's order: the diagonal of the sliced copy
       hipLaunchKernelGGL(k_jacobi_sliced, dim3((unsigned)(((int64_t)op.sl.ns * kSlice + 255) / 256)), B, 0, st,
                          sliced_dev(op), op.sl.v64.p, s.invd.p, root, s.d_flag);
     else
@@ -1891,6 +1746,15 @@ void push_chunk(femhip_solver &s, int slot, int size_idx = 0) {
   FH_HIP(hipEventRecord(s.ev[slot], st));
 }
 
+}  // namespace
+
+int64_t solver_pass_budget(const femhip_solver &s) {
+  const int64_t maxit = s.prm.max_num_iterations;
+  return s.lat ? 4 * maxit + 8 : maxit;
+}
+
+namespace {
+
 // Launch chunks until the device state says done, keeping one chunk of
 // look-ahead.  Near the end the remaining iteration count is extrapolated from
 // the stopping quantity at the last two chunk ends (a geometric rate): chunks
@@ -1925,7 +1789,7 @@ void iterate(femhip_solver &s, int maxit) {
     // one pass later, and an update of their refined form (at most one an
     // iteration) spends three: there the device ends the solve, and chunks go
     // on until it has.
-    if (queued >= (s.lat ? 4 * (int64_t)maxit + 8 : (int64_t)maxit)) continue;
+    if (queued >= solver_pass_budget(s)) continue;
     double need = 1e30;              // iterations still needed
     if (prev_it >= 0 && r.prog_it > prev_it && r.prog > 0.0 && prev > r.prog && r.rhs_test > 0.0) {
       const double rate = std::log(r.prog / prev) / (r.prog_it - prev_it);

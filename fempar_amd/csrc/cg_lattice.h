@@ -31,7 +31,7 @@
 // the vectors round.
 
 template <int DIM, int P, int KIND>
-using LatticeCell = std::conditional_t<P == 1, CellQ1<DIM, KIND>, CellQ2<DIM, KIND>>;
+using LatticeCell = std::conditional_t<KIND == kElastic, CellElastic, std::conditional_t<P == 1, CellQ1<DIM, KIND>, CellQ2<DIM, KIND>>>;
 
 template <int DIM, int P, int KIND>
 __device__ __forceinline__ LatticeCell<DIM, P, KIND> lattice_cell(const CoefDev &c, const Q2Tab &t) {
@@ -179,7 +179,8 @@ struct IoCg {
   }
 };
 
-#define FEMHIP_LATTICE_BOUNDS __launch_bounds__(lattice_threads(DIM, P), lattice_waves(DIM, P))
+#define FEMHIP_LATTICE_BOUNDS \
+  __launch_bounds__(lattice_threads(DIM, P, KIND == kElastic ? 3 : 1), lattice_waves(DIM, P, KIND == kElastic ? 3 : 1))
 
 // The vectors that alternate between two sets: pass `par` reads set par.
 template <typename T>
@@ -723,6 +724,13 @@ __global__ void k_lat_jacobi(int32_t n, const int32_t *__restrict__ rowptr, cons
   jacobi_store(d, root, out, perm ? perm[i] : i, flag);
 }
 
+// the same from a diagonal held as such (operators without a CSR)
+__global__ void k_jacobi_diag(int32_t n, const double *__restrict__ diag, double *__restrict__ out, int root,
+                              int *flag) {
+  const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) jacobi_store(diag[i], root, out, i, flag);
+}
+
 struct LatticeKernels {
   decltype(&k_lat_a<3, 1, 0>) a;
   decltype(&k_lat_rf_a<3, 1, 0>) rf_a;
@@ -741,6 +749,7 @@ LatticeKernels lattice_kernels_by_kind(int kind) {
          : kind == kCoefSin3 ? lattice_kernels_of<DIM, P, kCoefSin3>() : lattice_kernels_of<DIM, P, kCoefPoint>();
 }
 LatticeKernels lattice_kernels(int dim, int order, int kind) {
+  if (kind == kElastic) return lattice_kernels_of<3, 1, kElastic>();
   if (dim == 2) return order == 1 ? lattice_kernels_by_kind<2, 1>(kind) : lattice_kernels_by_kind<2, 2>(kind);
   return order == 1 ? lattice_kernels_by_kind<3, 1>(kind) : lattice_kernels_by_kind<3, 2>(kind);
 }

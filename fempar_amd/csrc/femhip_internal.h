@@ -281,9 +281,10 @@ struct femhip_operator {
   femhip::DevBuf<int32_t> lat_perm;
   femhip::DevBuf<double> lat_kq;
   int64_t lat_kq_version = -1, phys_version = 0;   // phys_version: bumped by every set_physics
-  // structured stencil operator (no CSR, no space): rows are component-major
-  // blocks of `blk` rows (the `nodes` free nodes, padded to a multiple of 64),
-  // values assembled in place into the sliced layout
+  // structured elasticity operator (no CSR, no space, no matrix: products from
+  // the cells): rows are component-major blocks of `blk` rows (the `nodes` free
+  // nodes, padded to a multiple of 64); its diagonal
+  femhip::DevBuf<double> diag;
   bool structured = false;
   int32_t blk = 0, nodes = 0;
 };
@@ -371,12 +372,11 @@ void error_norms_mapped(femhip_operator &op, const double *d_x, int exact, doubl
 void elasticity_element(const RefFE &fe, const femhip_physics_t &ph, double *Ke, double *Fe);
 
 // Structured elasticity operator on the unit cube with n cells per direction,
-// clamped on x = 0 (stencil.hip): numbering, solver format, values, RHS built
-// on the device of ctx; row (c, node) = c * blk + node, node lexicographic
+// clamped on x = 0 (stencil.hip): lattice, diagonal and RHS built on the device
+// of ctx; row (c, node) = c * blk + node, node lexicographic
 // over the free vertices (x index 1..n fastest, then y, then z).
 femhip_operator *create_structured_elasticity(femhip_ctx *ctx, int32_t n, const femhip_physics_t &ph);
-// whether create_structured_elasticity accepts n (its sliced format indexes
-// 243 x padded vertices entries with 32-bit integers)
+// whether create_structured_elasticity accepts n (1 to 206)
 bool structured_elasticity_fits(int32_t n);
 
 // error norms of the FE function with free values d_x (norms.hip):
@@ -392,6 +392,8 @@ void error_norms(femhip_operator &op, const double *d_x, int exact, double out[4
 // solver_stream_launches makes the solver enqueue its chunks as plain stream
 // launches instead of hipGraphs (set before solver_start).
 int solver_chunk();
+// iterations' worth of chunks a solve may take (updates take passes too)
+int64_t solver_pass_budget(const femhip_solver &s);
 void solver_stream_launches(femhip_solver &s);
 // Pinned, device-mapped result slots and completion events a solver may use
 // instead of allocating its own (the request server keeps one set per slot
@@ -420,7 +422,7 @@ inline size_t operator_device_bytes(const femhip_operator &op) {
   b += s.perm.bytes() + s.soffs.bytes() + s.base.bytes() + s.meta.bytes() + s.srow.bytes() + s.aux.bytes() + s.offs.bytes() +
        s.ecol.bytes() +
        s.map.bytes() + s.v64.bytes() + s.v32.bytes();
-  b += op.lat_perm.bytes() + op.lat_kq.bytes();
+  b += op.lat_perm.bytes() + op.lat_kq.bytes() + op.diag.bytes();
   if (op.space) b += op.space->d_dofs.bytes() + op.space->d_rep.bytes() + op.space->vcoords.bytes();
   return b;
 }

@@ -75,7 +75,7 @@ __device__ __forceinline__ void buf_st32(BufRsrc r, uint32_t o8, float v) {
   __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), r, (int)(o8 >> 1), 0, 0);
 }
 
-template <int DIM, int P>
+template <int DIM, int P, int NC = 1>
 struct LatticeShape {
   static constexpr int N1 = P + 1;
   static constexpr int NPL = DIM == 3 ? N1 * N1 : N1;   // a cell's nodes in one plane of the march
@@ -83,27 +83,24 @@ struct LatticeShape {
   static constexpr int NX = NPL - OWN;                  // those it shares with the next cells
   // Q1: two sets of the LDS buffers and one barrier a layer, the loads of the
   // next plane in flight while a layer is computed.  Q2 holds too much in
-  // registers for that: one set, two barriers.
-  static constexpr bool PIPE = P == 1;
+  // registers for that, and vector Q1 in registers and LDS: one set, three
+  // barriers.
+  static constexpr bool PIPE = P == 1 && NC == 1;
 };
 
 // Largest workgroup and wanted waves a SIMD (registers 512 / waves) of the marches.
-#ifndef FEMHIP_LAT_T31
-#define FEMHIP_LAT_T31 512
-#define FEMHIP_LAT_W31 4
-#endif
-__host__ __device__ constexpr int lattice_threads(int dim, int p) { return dim == 3 && p == 1 ? FEMHIP_LAT_T31 : 256; }
-__host__ __device__ constexpr int lattice_waves(int dim, int p) { return dim == 3 && p == 1 ? FEMHIP_LAT_W31 : p == 1 ? 4 : 2; }
+__host__ __device__ constexpr int lattice_threads(int dim, int p, int nc) { return dim == 3 && p == 1 && nc == 1 ? 512 : 256; }
+__host__ __device__ constexpr int lattice_waves(int, int p, int nc) { return p == 1 && nc == 1 ? 4 : 2; }
 
 // What an Io keeps of a node from value() to out(), in doubles (kKeep, at most).
 constexpr int kLatticeKeep = 3;
 // doubles of LDS a workgroup needs (new node planes, shared sums; PIPE: what
 // the lanes keep of their own nodes in the last three planes)
-template <int DIM, int P>
+template <int DIM, int P, int NC>
 inline size_t lattice_lds(int TX, int TY) {
-  using S = LatticeShape<DIM, P>;
+  using S = LatticeShape<DIM, P, NC>;
   const size_t cells = (size_t)TX * TY, plane = (size_t)(P * TX + 1) * (DIM == 3 ? P * TY + 1 : 1);
-  return (S::PIPE ? 2 : 1) * (size_t)P * (plane + S::NX * cells) + (S::PIPE ? 3 * kLatticeKeep * cells : 0);
+  return (S::PIPE ? 2 : 1) * (size_t)(NC * P) * (plane + S::NX * cells) + (S::PIPE ? 3 * kLatticeKeep * cells : 0);
 }
 // nodes of the row and column after a tile, one a thread
 template <int DIM, int P>
@@ -111,7 +108,7 @@ inline int lattice_halo(int TX, int TY) {
   return DIM == 3 ? P * (TX + TY) + 1 : 1;
 }
 
-// March of one workgroup; false: it has no cells, and ready() was not called.
+// March of logical workgroup lb; false: it has no cells, and ready() was not called.
 // Cell: begin(cx, cy, in the mesh), prefetch(cz) and
 // advance() for its coefficient, bottom(u) with the nodes of the first plane,
 // step(active, u, s): the P next planes in, the finished sums of the P planes
@@ -124,7 +121,8 @@ inline int lattice_halo(int TX, int TY) {
 // halo(o) and halo_value(raw): the value alone, of a node past the tile.
 template <int DIM, int P, class Cell, class Io>
 __device__ __forceinline__ bool lattice_march(const Lattice &g, Cell &cell, Io &io, double *lds) {
-  using S = LatticeShape<DIM, P>;
+  constexpr int NC = Cell::kComps;
+  using S = LatticeShape<DIM, P, NC>;
   constexpr int N1 = S::N1, NPL = S::NPL, OWN = S::OWN, NX = S::NX;
   constexpr bool PIPE = S::PIPE;
   constexpr int AX = DIM - 1;
@@ -145,7 +143,9 @@ __device__ __forceinline__ bool lattice_march(const Lattice &g, Cell &cell, Io &
   const int zs = z0 > 0 ? z0 - 1 : 0;
   const int LX = P * TX + 1, LY = DIM == 3 ? P * TY + 1 : 1, LP = LX * LY;
   const uint32_t plane_bytes = 8u * (uint32_t)(DIM == 3 ? g.m[0] * g.m[1] : g.m[0]);
-  const int half = P * (LP + NX * cells);   // doubles of one set of buffers: U [P][LY][LX], C [P][NX][cells]
+  // doubles of one set of buffers: U [NC][P][LY][LX], C [NC][P][NX][cells]
+  const int half = NC * P * (LP + NX * cells);
+  const uint32_t comp_bytes = 8u * (uint32_t)g.stride;
 
   auto row_offset = [&](int px, int py, bool ok) {
     const int gx = px - g.o[0], gy = DIM == 3 ? py - g.o[1] : 0;
@@ -168,118 +168,129 @@ __device__ __forceinline__ bool lattice_march(const Lattice &g, Cell &cell, Io &
     const int gz = z - g.o[AX];
     return gz >= 0 && gz < g.m[AX] ? (uint32_t)gz * plane_bytes : kNoPlane;
   };
-  typename Io::Raw raw[P][OWN];
-  typename Io::Halo hraw[P];
+  typename Io::Raw raw[NC][P][OWN];
+  typename Io::Halo hraw[NC][P];
   constexpr int KEEP = Io::kKeep;
   double *ring = lds + (PIPE ? 2 : 1) * half + (lane ? tid : 0);   // PIPE: [3][KEEP][cells], plane z in part z mod 3
   auto fetch = [&](int z, int count) {   // planes z .. z + count - 1
 #pragma unroll
-    for (int c = 0; c < P; ++c)
-      if (c < count) {
-        const uint32_t base = plane_base(z + c);
+    for (int k = 0; k < NC; ++k)
 #pragma unroll
-        for (int j = 0; j < OWN; ++j) raw[c][j] = io.fetch(base + off[j]);
-        hraw[c] = io.halo(base + hoff);
-      }
+      for (int c = 0; c < P; ++c)
+        if (c < count) {
+          const uint32_t base = plane_base(z + c) + k * comp_bytes;
+#pragma unroll
+          for (int j = 0; j < OWN; ++j) raw[k][c][j] = io.fetch(base + off[j]);
+          hraw[k][c] = io.halo(base + hoff);
+        }
   };
   auto store = [&](double *U, int z, int count, int part) {
 #pragma unroll
-    for (int c = 0; c < P; ++c)
-      if (c < count) {
-        const uint32_t base = plane_base(z + c);
-        const bool own = own_xy && (z + c) / P >= z0 && (z + c) / P < z1;   // the layer that owns the plane
+    for (int k = 0; k < NC; ++k)
 #pragma unroll
-        for (int j = 0; j < OWN; ++j) {
-          double keep[KEEP];
-          const double v = io.value(raw[c][j], own ? base + off[j] : kOutside, keep);
-          if (lane) {
-            U[c * LP + uat + (j / P) * LX + j % P] = v;
-            if (PIPE)
+      for (int c = 0; c < P; ++c)
+        if (c < count) {
+          const uint32_t base = plane_base(z + c) + k * comp_bytes;
+          const bool own = own_xy && (z + c) / P >= z0 && (z + c) / P < z1;   // the layer that owns the plane
+          double *Up = U + (k * P + c) * LP;
 #pragma unroll
-              for (int k = 0; k < KEEP; ++k) ring[(part * KEEP + k) * cells] = keep[k];
+          for (int j = 0; j < OWN; ++j) {
+            double keep[KEEP];
+            const double v = io.value(raw[k][c][j], own ? base + off[j] : kOutside, keep);
+            if (lane) {
+              Up[uat + (j / P) * LX + j % P] = v;
+              if (PIPE)
+#pragma unroll
+                for (int i = 0; i < KEEP; ++i) ring[(part * KEEP + i) * cells] = keep[i];
+            }
           }
+          const double h = io.halo_value(hraw[k][c]);
+          if (halo) Up[hat] = h;
         }
-        const double h = io.halo_value(hraw[c]);
-        if (halo) U[c * LP + hat] = h;
-      }
   };
-  auto read_plane = [&](const double *U, int c, double (&u)[NPL]) {
-    const double *Up = U + c * LP + (lane ? uat : 0);
+  auto read_plane = [&](const double *U, int kc, double (&u)[NPL]) {   // kc = component * P + plane
+    const double *Up = U + kc * LP + (lane ? uat : 0);
 #pragma unroll
     for (int b = 0; b < (DIM == 3 ? N1 : 1); ++b)
 #pragma unroll
       for (int a = 0; a < N1; ++a) u[b * N1 + a] = Up[b * LX + a];
   };
   // sums of shared nodes to their owners: slots (a = P, b < P), (b = P, a < P), (P, P)
-  auto share = [&](double *C, const double (&s)[P][NPL]) {
+  auto share = [&](double *C, const double (&s)[NC][P][NPL]) {
     if (lane) {
 #pragma unroll
-      for (int c = 0; c < P; ++c) {
-        double *Cp = C + c * NX * cells + tid;
+      for (int kc = 0; kc < NC * P; ++kc) {
+        const double(&sp)[NPL] = s[kc / P][kc % P];
+        double *Cp = C + kc * NX * cells + tid;
         if (DIM == 2) {
-          Cp[0] = s[c][P];
+          Cp[0] = sp[P];
         } else {
 #pragma unroll
           for (int j = 0; j < P; ++j) {
-            Cp[j * cells] = s[c][j * N1 + P];
-            Cp[(P + j) * cells] = s[c][P * N1 + j];
+            Cp[j * cells] = sp[j * N1 + P];
+            Cp[(P + j) * cells] = sp[P * N1 + j];
           }
-          Cp[2 * P * cells] = s[c][P * N1 + P];
+          Cp[2 * P * cells] = sp[P * N1 + P];
         }
       }
     }
   };
   const bool left = tx > 0, below = DIM == 3 && ty > 0, corner = left && below;
-  // kept(c, j, keep): what is kept of own node j of plane c; so(c, j): this cell's sum there
+  // kept(k, c, j, keep): what is kept of own node j of plane c; so(k, c, j): this cell's sum there
   auto finish = [&](const double *C, int cz, auto &&so, auto &&kept) {
     if (cz < z0) return;
 #pragma unroll
-    for (int c = 0; c < P; ++c) {
-      const uint32_t base = plane_base(P * cz + c);
-      const double *Cp = C + c * NX * cells + (lane ? tid : 0);
+    for (int k = 0; k < NC; ++k)
 #pragma unroll
-      for (int j = 0; j < OWN; ++j) {
-        const int a = j % P, b = j / P;
-        double y = so(c, j);
-        if (DIM == 2) {
-          if (a == 0) y += left ? Cp[-1] : 0.0;
-        } else {
-          if (a == 0) y += left ? Cp[b * cells - 1] : 0.0;
-          if (b == 0) y += below ? Cp[(P + a) * cells - TX] : 0.0;
-          if (a == 0 && b == 0) y += corner ? Cp[2 * P * cells - TX - 1] : 0.0;
+      for (int c = 0; c < P; ++c) {
+        const uint32_t base = plane_base(P * cz + c) + k * comp_bytes;
+        const double *Cp = C + (k * P + c) * NX * cells + (lane ? tid : 0);
+#pragma unroll
+        for (int j = 0; j < OWN; ++j) {
+          const int a = j % P, b = j / P;
+          double y = so(k, c, j);
+          if (DIM == 2) {
+            if (a == 0) y += left ? Cp[-1] : 0.0;
+          } else {
+            if (a == 0) y += left ? Cp[b * cells - 1] : 0.0;
+            if (b == 0) y += below ? Cp[(P + a) * cells - TX] : 0.0;
+            if (a == 0 && b == 0) y += corner ? Cp[2 * P * cells - TX - 1] : 0.0;
+          }
+          double keep[KEEP];
+          kept(k, c, j, keep);
+          io.template out<PIPE>(own_xy ? base + off[j] : kOutside, keep, y);
         }
-        double keep[KEEP];
-        kept(c, j, keep);
-        io.template out<PIPE>(own_xy ? base + off[j] : kOutside, keep, y);
       }
-    }
   };
 
   fetch(P * zs, 1);
   cell.begin(g, cx, cy, in_xy);
   if (!io.ready()) return true;   // the same for every workgroup
   store(lds, P * zs, 1, 0);
-  double ub[OWN];   // !PIPE: own nodes of the plane below the layer
+  double ub[NC][OWN];   // !PIPE: own nodes of the plane below the layer
   if (PIPE) {
     fetch(P * zs + 1, P);
     cell.prefetch(g, zs, in_xy);
   }
   __syncthreads();
   {
-    double u[NPL];
-    read_plane(lds, 0, u);
+    double u[NC][NPL];
 #pragma unroll
-    for (int j = 0; j < OWN; ++j) ub[j] = u[(j / P) * N1 + j % P];
+    for (int k = 0; k < NC; ++k) {
+      read_plane(lds, k * P, u[k]);
+#pragma unroll
+      for (int j = 0; j < OWN; ++j) ub[k][j] = u[k][(j / P) * N1 + j % P];
+    }
     cell.bottom(u);
   }
 
   if (PIPE) {
     double so[OWN];
     int part = 0;   // of the plane below the layer finished next
-    auto so_at = [&](int, int j) { return so[j]; };
-    auto kept = [&](int, int, double (&keep)[KEEP]) {
+    auto so_at = [&](int, int, int j) { return so[j]; };
+    auto kept = [&](int, int, int, double (&keep)[KEEP]) {
 #pragma unroll
-      for (int k = 0; k < KEEP; ++k) keep[k] = ring[(part * KEEP + k) * cells];
+      for (int i = 0; i < KEEP; ++i) keep[i] = ring[(part * KEEP + i) * cells];
     };
     int set = 1, next = 1;   // buffers; ring part of the plane stored next
     for (int cz = zs; cz < z1; ++cz) {
@@ -296,20 +307,21 @@ __device__ __forceinline__ bool lattice_march(const Lattice &g, Cell &cell, Io &
         fetch(P * (cz + 1) + 1, P);
         cell.prefetch(g, cz + 1, in_xy);
       }
-      double u[P][NPL], s[P][NPL];
+      double u[NC][P][NPL], s[NC][P][NPL];
 #pragma unroll
-      for (int c = 0; c < P; ++c) read_plane(U, c, u[c]);
+      for (int c = 0; c < P; ++c) read_plane(U, c, u[0][c]);
       cell.step(in_xy && cz < g.nc[AX], u, s);
       share(C, s);
 #pragma unroll
-      for (int j = 0; j < OWN; ++j) so[j] = s[0][(j / P) * N1 + j % P];
+      for (int j = 0; j < OWN; ++j) so[j] = s[0][0][(j / P) * N1 + j % P];
       set ^= 1;
     }
     __syncthreads();
     finish(lds + (set ^ 1) * half + P * LP, z1 - 1, so_at, kept);
   } else {
-    double *U = lds, *C = U + P * LP;
+    double *U = lds, *C = U + NC * P * LP;
     const double *Uo = U + (lane ? uat : 0);
+    auto u_at = [&](int k, int c, int j) { return Uo[(k * P + c) * LP + (j / P) * LX + j % P]; };
     for (int cz = zs; cz < z1; ++cz) {
       fetch(P * cz + 1, P);
       cell.prefetch(g, cz, in_xy);
@@ -317,17 +329,18 @@ __device__ __forceinline__ bool lattice_march(const Lattice &g, Cell &cell, Io &
       __syncthreads();   // the layer before has read U and C
       store(U, P * cz + 1, P, 0);
       __syncthreads();
-      double u[P][NPL], s[P][NPL];
+      double u[NC][P][NPL], s[NC][P][NPL];
 #pragma unroll
-      for (int c = 0; c < P; ++c) read_plane(U, c, u[c]);
+      for (int kc = 0; kc < NC * P; ++kc) read_plane(U, kc, u[kc / P][kc % P]);
       cell.step(in_xy && cz < g.nc[AX], u, s);
       share(C, s);
       __syncthreads();
-      auto u_at = [&](int c, int j) { return Uo[c * LP + (j / P) * LX + j % P]; };
-      finish(C, cz, [&](int c, int j) { return s[c][(j / P) * N1 + j % P]; },
-             [&](int c, int j, double (&keep)[KEEP]) { keep[0] = c == 0 ? ub[j] : u_at(c - 1, j); });
+      finish(C, cz, [&](int k, int c, int j) { return s[k][c][(j / P) * N1 + j % P]; },
+             [&](int k, int c, int j, double (&keep)[KEEP]) { keep[0] = c == 0 ? ub[k][j] : u_at(k, c - 1, j); });
 #pragma unroll
-      for (int j = 0; j < OWN; ++j) ub[j] = u_at(P - 1, j);
+      for (int k = 0; k < NC; ++k)
+#pragma unroll
+        for (int j = 0; j < OWN; ++j) ub[k][j] = u_at(k, P - 1, j);
     }
   }
   return true;
@@ -338,17 +351,18 @@ __device__ __forceinline__ bool lattice_march(const Lattice &g, Cell &cell, Io &
 // Where the coefficient of a Poisson cell comes from.
 enum { kCoefCell = 0,    // one value: k0, or kc[cell]
        kCoefSin3 = 1,    // 1 + 1/2 prod sin(2 pi x_d), from the sines at the 1-D Gauss points of each layer
-       kCoefPoint = 2 }; // kq[q cells + cell]
+       kCoefPoint = 2,   // kq[q cells + cell]
+       kElastic = 3 };   // vector Q1, constant Lame coefficients
 
 struct CoefDev {
-  double k0 = 1.0;
+  double k0 = 1.0, mu = 0.0;       // kElastic: lambda and mu, times the weights of the points
   const double *kc = nullptr, *kq = nullptr;
   const double4 *trig = nullptr;   // {., ., sin 2 pi x, .} per (layer, point), offsets per direction
   int toff[3] = {0, 0, 0};
   int64_t cells = 0;
   double c[3] = {0, 0, 0};         // weight of the squared derivative along each direction
   bool operator==(const CoefDev &o) const {
-    bool same = k0 == o.k0 && kc == o.kc && kq == o.kq && trig == o.trig && cells == o.cells;
+    bool same = k0 == o.k0 && mu == o.mu && kc == o.kc && kq == o.kq && trig == o.trig && cells == o.cells;
     for (int d = 0; d < 3; ++d) same = same && toff[d] == o.toff[d] && c[d] == o.c[d];
     return same;
   }
@@ -366,7 +380,7 @@ constexpr double kGauss2 = 0.57735026918962576451;   // 1 / sqrt(3)
 
 template <int DIM, int KIND>
 struct CellQ1 {
-  static constexpr int NPL = DIM == 3 ? 4 : 2, NV = 1 << DIM, NK = KIND == kCoefPoint ? NV : 1;
+  static constexpr int kComps = 1, NPL = DIM == 3 ? 4 : 2, NV = 1 << DIM, NK = KIND == kCoefPoint ? NV : 1;
   CoefDev k;
   double kv[NK], kn[NK];          // this layer's values, the next one's
   double sz[2], sn[2];            // sines at the march's points
@@ -460,10 +474,10 @@ struct CellQ1 {
       u[3 % NPL] = c + d;
     }
   }
-  __device__ __forceinline__ void bottom(const double (&u)[NPL]) { modes(u, below); }
-  __device__ __forceinline__ void step(bool active, const double (&u)[1][NPL], double (&s)[1][NPL]) {
+  __device__ __forceinline__ void bottom(const double (&u)[1][NPL]) { modes(u[0], below); }
+  __device__ __forceinline__ void step(bool active, const double (&u)[1][1][NPL], double (&s)[1][1][NPL]) {
     double h[NV], r[NV], top[NPL], sum[NPL];
-    modes(u[0], top);
+    modes(u[0][0], top);
 #pragma unroll
     for (int i = 0; i < NPL; ++i) {
       h[i] = below[i] + top[i];
@@ -523,7 +537,89 @@ struct CellQ1 {
         carry[i] = r[i] + r[NPL + i];
       }
     }
-    nodes(sum, s[0]);
+    nodes(sum, s[0][0]);
+  }
+};
+
+// Vector Q1, lambda div div + 2 mu eps : eps with constant lambda, mu.  In the
+// sums and differences of CellQ1 the derivative along i at the Gauss points is
+// a polynomial in the point's signs: one coefficient for each subset of the
+// other directions, and products of different subsets sum to zero over the
+// points.  So the form is a few 3 x 3 couplings, one for each subset.
+struct CellElastic {
+  static constexpr int kComps = 3, NPL = 4, NV = 8;
+  CoefDev k;   // c[i] = 1 / (4 h_i); k0, mu = lambda, mu times the eight points' weights
+  double below[3][NPL], carry[3][NPL];
+
+  __device__ __forceinline__ void begin(const Lattice &, int, int, bool) {
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+#pragma unroll
+      for (int i = 0; i < NPL; ++i) carry[c][i] = 0.0;
+  }
+  __device__ __forceinline__ void prefetch(const Lattice &, int, bool) {}
+  __device__ __forceinline__ void advance() {}
+  __device__ __forceinline__ void bottom(const double (&u)[3][NPL]) {
+#pragma unroll
+    for (int c = 0; c < 3; ++c) CellQ1<3, kCoefCell>::modes(u[c], below[c]);
+  }
+  __device__ __forceinline__ void step(bool active, const double (&u)[3][1][NPL], double (&s)[3][1][NPL]) {
+    double h[3][NV], r[3][NV];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      double top[NPL];
+      CellQ1<3, kCoefCell>::modes(u[c][0], top);
+#pragma unroll
+      for (int i = 0; i < NPL; ++i) {
+        h[c][i] = below[c][i] + top[i];
+        h[c][NPL + i] = top[i] - below[c][i];
+        below[c][i] = top[i];
+      }
+#pragma unroll
+      for (int i = 0; i < NV; ++i) r[c][i] = 0.0;
+    }
+    if (active) {   // lanes past the mesh only pass sums on
+      constexpr double al = kGauss2;
+      auto power = [](int S) { return S == 0 ? 1.0 : (S & (S - 1)) == 0 ? al : al * al; };
+#pragma unroll
+      for (int S = 0; S < 7; ++S) {   // subsets of the directions
+        const double f = power(S);
+        double div = 0.0;
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+          if (!((S >> c) & 1)) div = __builtin_fma(k.c[c] * f, h[c][(1 << c) | S], div);
+        div *= k.k0;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+          if ((S >> c) & 1) continue;
+          const double g = (k.c[c] * f) * h[c][(1 << c) | S];
+          r[c][(1 << c) | S] = __builtin_fma(k.c[c] * f, __builtin_fma(2.0 * k.mu, g, div), r[c][(1 << c) | S]);
+        }
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+#pragma unroll
+          for (int i = c + 1; i < 3; ++i) {   // shear: derivatives of component c along i and of i along c
+            const bool ci = !((S >> i) & 1), ic = !((S >> c) & 1);
+            if (!ci && !ic) continue;
+            double e = 0.0;
+            if (ci) e = (k.c[i] * f) * h[c][((1 << i) | S) & 7];
+            if (ic) e = __builtin_fma(k.c[c] * f, h[i][((1 << c) | S) & 7], e);
+            e *= k.mu;
+            if (ci) r[c][((1 << i) | S) & 7] = __builtin_fma(k.c[i] * f, e, r[c][((1 << i) | S) & 7]);
+            if (ic) r[i][((1 << c) | S) & 7] = __builtin_fma(k.c[c] * f, e, r[i][((1 << c) | S) & 7]);
+          }
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      double sum[NPL];
+#pragma unroll
+      for (int i = 0; i < NPL; ++i) {
+        sum[i] = carry[c][i] + (r[c][i] - r[c][NPL + i]);
+        carry[c][i] = r[c][i] + r[c][NPL + i];
+      }
+      CellQ1<3, kCoefCell>::nodes(sum, s[c][0]);
+    }
   }
 };
 
@@ -538,7 +634,7 @@ struct Q2Tab {
 
 template <int DIM, int KIND>
 struct CellQ2 {
-  static constexpr int NPL = DIM == 3 ? 9 : 3, N = DIM == 3 ? 27 : 9;
+  static constexpr int kComps = 1, NPL = DIM == 3 ? 9 : 3, N = DIM == 3 ? 27 : 9;
   CoefDev k;
   Q2Tab t;
   double kv, kn;
@@ -638,13 +734,15 @@ struct CellQ2 {
     interp<1, NPL>(v);
     if (DIM == 3) interp<DIM == 3 ? 3 : 1, NPL>(v);
   }
-  __device__ __forceinline__ void bottom(const double (&u)[NPL]) {
+  __device__ __forceinline__ void bottom(const double (&u)[1][NPL]) {
 #pragma unroll
-    for (int i = 0; i < NPL; ++i) below[i] = u[i];
+    for (int i = 0; i < NPL; ++i) below[i] = u[0][i];
     in_plane(below);
   }
-  __device__ __forceinline__ void step(bool active, double (&u)[2][NPL], double (&s)[2][NPL]) {
+  __device__ __forceinline__ void step(bool active, double (&uc)[1][2][NPL], double (&sc)[1][2][NPL]) {
     double v[N], w[N];
+    auto &u = uc[0];
+    auto &s = sc[0];
     in_plane(u[0]);
     in_plane(u[1]);
 #pragma unroll

@@ -63,9 +63,9 @@ __global__ void k_points_by_q(int64_t cells, int nq, const double *__restrict__ 
   if (i < cells * nq) out[(i % nq) * cells + i / nq] = in[i];
 }
 
-template <int DIM, int P>
+template <int DIM, int P, int NC = 1>
 void split(LatticeOp &L, int cus) {
-  constexpr int max_threads = lattice_threads(DIM, P);
+  constexpr int max_threads = lattice_threads(DIM, P, NC);
   Lattice &g = L.g;
   const int e0 = g.E[0], e1 = DIM == 3 ? g.E[1] : 1, ez = g.E[DIM - 1];
   // Tile: the least lanes over all tiles.  Neighbouring tiles both compute the
@@ -93,11 +93,11 @@ void split(LatticeOp &L, int cus) {
     }
     if (TX <= 2) break;
   }
-  L.lds = lattice_lds<DIM, P>(g.TX, g.TY) * sizeof(double);
+  L.lds = lattice_lds<DIM, P, NC>(g.TX, g.TY) * sizeof(double);
   // Chunks of the march: each repeats one layer, so few long ones repeat
   // little and many short ones fill the chip; the fewest layers in turn on one
-  // CU (16 waves of it resident) wins.
-  const int per_cu = std::max(1, std::min(256 * lattice_waves(DIM, P) / L.threads, (int)(160 * 1024 / std::max<size_t>(1, L.lds))));
+  // CU wins.
+  const int per_cu = std::max(1, std::min(256 * lattice_waves(DIM, P, NC) / L.threads, (int)(160 * 1024 / std::max<size_t>(1, L.lds))));
   const int64_t slots = (int64_t)per_cu * std::max(1, cus);
   double bestc = 1e300;
   for (int c = 1; c <= ez; ++c) {
@@ -138,26 +138,28 @@ bool lattice_plan(const femhip_mesh_desc_t &mesh, int cus, LatticeOp &L) {
     rows *= m;
     if (rows * L.ncomp > kLatticeMaxRows) return false;   // byte offsets of the vectors
   }
-  g.stride = L.ncomp > 1 ? (int)((rows + 63) / 64 * 64) : (int)rows;
+  g.stride = (int)rows;
   if (dim == 2 && p == 1) split<2, 1>(L, cus);
   else if (dim == 2) split<2, 2>(L, cus);
+  else if (p == 1 && L.ncomp == 3) split<3, 1, 3>(L, cus);
   else if (p == 1) split<3, 1>(L, cus);
   else split<3, 2>(L, cus);
   return true;
 }
 
-// The lattice form of a scalar Poisson operator on the uniform mesh (checked
-// once against the space's DOF lists, whoever numbered them): op.lat,
-// op.lat_perm.  Cells with their own map keep the stored matrix.
+// The lattice form of a scalar Poisson or a vector Q1 elasticity operator on the
+// uniform mesh (checked once against the space's DOF lists, whoever numbered
+// them): op.lat, op.lat_perm.  Cells with their own map keep the stored matrix.
 bool lattice_operator(femhip_operator &op) {
-  if (!op.space || op.structured || op.tab_kind != 0 || op.space->mapped || op.n <= 0) return false;
+  if (op.structured) return op.lat_state > 0;
+  if (!op.space || op.space->mapped || op.n <= 0) return false;
   if (op.lat_state != 0) return op.lat_state > 0;
   op.lat_state = -1;
   femhip_space &s = *op.space;
-  if (s.fe.ncomp != 1) return false;
+  if (op.tab_kind == 0 ? s.fe.ncomp != 1 : s.fe.ncomp != 3 || s.fe.dim != 3 || s.fe.order != 1) return false;
   auto L = std::make_shared<LatticeOp>();
   if (!lattice_plan(s.mesh, op.ctx->num_cus, *L)) return false;
-  int64_t rows = 1;
+  int64_t rows = L->ncomp;
   for (int d = 0; d < s.mesh.dim; ++d) rows *= L->g.m[d];
   if (rows != op.n) return false;
   hipStream_t st = op.ctx->stream;
@@ -194,17 +196,36 @@ bool lattice_operator(femhip_operator &op) {
   return true;
 }
 
+// Elasticity coefficients of cells of sides h.
+static CoefDev elastic_coefficient(const double h[3], const femhip_physics_t &ph) {
+  CoefDev c;
+  const double w = h[0] * h[1] * h[2];   // eight points of weight det J
+  c.k0 = w * (ph.nu * ph.E) / ((1 + ph.nu) * (1 - 2 * ph.nu));
+  c.mu = w * ph.E / (2 * (1 + ph.nu));
+  for (int d = 0; d < 3; ++d) c.c[d] = 1.0 / (4.0 * h[d]);
+  return c;
+}
+
 // The operator's coefficient as the cells read it (after set_physics).
 CoefDev lattice_coefficient(femhip_operator &op) {
+  if (op.structured) {
+    const double h[3] = {1.0 / op.lat->g.nc[0], 1.0 / op.lat->g.nc[1], 1.0 / op.lat->g.nc[2]};
+    return elastic_coefficient(h, op.phys);
+  }
   femhip_space &s = *op.space;
   const RefFE &fe = s.fe;
   CoefDev c;
   c.cells = s.ncells;
   c.k0 = op.phys.k0;
-  // Q1: Gauss weights one; Q2: the weights are in the 1-D tables
+  double hs[3] = {1.0, 1.0, 1.0};   // the first cell's sides
   for (int d = 0; d < fe.dim; ++d) {
     const double lo = s.mesh.limits[2 * d], hi = s.mesh.limits[2 * d + 1];
-    const double h = ((hi - lo) * (1.0 / (double)s.mesh.n[d]) + lo) - lo;   // the first cell's spacing
+    hs[d] = ((hi - lo) * (1.0 / (double)s.mesh.n[d]) + lo) - lo;
+  }
+  if (op.tab_kind == 1) return elastic_coefficient(hs, op.phys);
+  // Q1: Gauss weights one; Q2: the weights are in the 1-D tables
+  for (int d = 0; d < fe.dim; ++d) {
+    const double h = hs[d];
     c.c[d] = fe.order == 1 ? fe.detj[0] * (4.0 / (h * h)) / (double)(1 << (2 * fe.dim)) : fe.detj[0] * (4.0 / (h * h));
   }
   if (op.phys.k_kind == FEMHIP_K_CELL) c.kc = op.k_cell.p;

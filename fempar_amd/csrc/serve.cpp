@@ -100,10 +100,11 @@ struct femhip_server {
 
 namespace {
 
-// Device memory bound for a request on the structured stencil operator: 81
-// FP64 + FP32 values per row, RHS, per-slice data, FP64 and FP32 Krylov
-// vectors, block partials and the residual history (rows = 3 x the free
-// vertices padded to a multiple of 64).
+// Device memory bound for a request: what the operator held when its 81-point
+// stencil was stored (81 FP64 + FP32 values per row, RHS, per-slice data, FP64 and FP32 Krylov
+// vectors, block partials and the residual history; rows = 3 x the free
+// vertices padded to a multiple of 64).  The operator now holds a tenth of
+// that; admission keeps the bound, so a budget admits and refuses as before.
 double estimate_bytes(int32_t n, int32_t maxit) {
   const double nn = n, nodes = nn * (nn + 1) * (nn + 1);
   const double rows = 3.0 * std::ceil(nodes / 64.0) * 64.0;
@@ -303,7 +304,6 @@ std::multimap<std::pair<double, int64_t>, ReqP>::iterator next_admission(femhip_
 void scheduler_loop(femhip_server &S) {
   (void)hipSetDevice(S.ctx->device);
   const int chunk = solver_chunk();
-  const int64_t maxit = S.prm.cg.max_num_iterations;
   std::vector<ReqP> running;
   for (;;) {
     std::vector<ReqP> started;
@@ -353,7 +353,7 @@ void scheduler_loop(femhip_server &S) {
       try {
         solver_push(*r->solver, 0);
         r->queued_its = chunk;
-        if (r->queued_its < maxit) {
+        if (r->queued_its < solver_pass_budget(*r->solver)) {
           solver_push(*r->solver, 1);
           r->queued_its += chunk;
         }
@@ -391,7 +391,7 @@ void scheduler_loop(femhip_server &S) {
         continue;
       }
       progress = true;
-      if (st == 2 || r.queued_its >= maxit) {
+      if (st == 2 || r.queued_its >= solver_pass_budget(*r.solver)) {
         std::lock_guard<std::mutex> lk(S.mu);
         r.state = RETIRING;
         S.retire_q.push_back(running[i]);

@@ -102,6 +102,31 @@ def test_lattice_solves_match_oracle(env, n, order, k, bc, precond):
         assert s.did_converge() and np.linalg.norm(x - ref) <= tol * np.linalg.norm(ref), precision
 
 
+@pytest.mark.parametrize("n", [(9, 13, 11), (2, 30, 30), (33, 9, 8)])
+def test_lattice_elasticity_matches_oracle(env, n):
+    """Vector Q1 elasticity on the lattice: component-blocked rows inside, the
+    operator's first-touch order outside (right-hand side, guess and solution)."""
+    print(f"[lattice] elasticity {n}", flush=True)
+    lim = [0, 1, -0.5, 1, 0, 2]
+    osp = O.Space(O.make_problem(3, n, 1, 3, O.BC_X0, lim=lim))
+    irp, ja, val, rhs = osp.assemble(O.make_physics(kind=O.PHYS_ELASTICITY, E=20.0, nu=0.35, body=(0.5, 0.0, -1.0)), True)
+    tria = F.serial_triangulation_t().create(env, {
+        "STRUCT_HEX_MESH_GENERATOR_NUM_DIMS": 3, "STRUCT_HEX_MESH_GENERATOR_NUM_CELLS_X_DIM": list(n),
+        "STRUCT_HEX_MESH_GENERATOR_DOMAIN_LIMITS": lim})
+    fes = F.serial_fe_space_t().create(tria, order=1, num_components=3, dirichlet="x0")
+    op = F.fe_affine_operator_t()
+    op.create("CSR", [True], fes, F.linear_elasticity_discrete_integration_t(20.0, 0.35, (0.5, 0.0, -1.0)))
+    op.compute()
+    assert op.n == len(rhs) > 4096
+    rng = np.random.default_rng(5)
+    b, x0 = rng.standard_normal(op.n), rng.standard_normal(op.n)
+    for rh, guess in ((rhs, None), (b, x0)):
+        ref, info = O.cg(irp, ja, val, rh, True, precond="jacobi", rtol=1e-12, maxit=50000)
+        for precision, rtol, tol in (("FP64", 1e-12, 1e-9), ("FP32_REFINED", 1e-10, 1e-7)):
+            s, x = _solve(env, op, precision, "jacobi", rtol, None if rh is rhs else rh, guess)
+            assert s.did_converge() and np.linalg.norm(x - ref) <= tol * np.linalg.norm(ref), precision
+
+
 def test_lattice_both_forms_and_limits(env):
     """A system of more than 400,000 rows (two launches an iteration) and one of
     fewer give the same solution as their assembled rows; the iteration limit
