@@ -1,4 +1,4 @@
-// batch.hip -- many independent Poisson problems in one persistent launch.
+// batch.hip -- many independent Poisson problems advanced together.
 //
 // Problem = FEMPAR's test_poisson setting on its own structured mesh: Q1 on the
 // unit square/cube, strong Dirichlet on the whole boundary, constant k, source
@@ -9,8 +9,7 @@
 // so row r is interior node (a,b,c) = r in base m = n-1 and every row's columns
 // are r + dx + m dy + m^2 dz, (dx,dy,dz) in {-1,0,1}^d: the matrix is a
 // diagonal matrix with 3^d diagonals.  Each problem stores its diagonals
-// [k][row] (rows padded to 64) in FP64 and FP32 in shared pools at a
-// per-problem offset.
+// [k][row] (rows padded to 64) in a shared pool at a per-problem offset.
 //
 // Assembly: one launch over (problem, 256-row chunk) tasks; a thread owns a
 // row and sums, over the 2^d cells around its node, the element entries
@@ -18,11 +17,22 @@
 // thread (conflict-free, deterministic; the reference's COO duplicate sum in
 // owner order).
 //
-// Solve: one persistent launch; each workgroup takes the next problem from a
-// largest-first work queue (single-lane atomic), runs FP32 Jacobi-PCG with
-// FP64 reliable updates for it with workgroup-level reductions only, and
-// stamps its completion with the device wall clock.  The launch (queue reset +
-// solve) is captured once in a hipGraph and replayed.
+// Solve, problems up to about 16000 rows: a workgroup each (k_batch_small).
+//
+// Solve, the others: every problem advances by one CG iteration in each pass.  A
+// pass is one launch over the workgroups of all problems (a table gives each its
+// problem and its tile there, a problem's workgroups on one XCD), in which a
+// problem goes through the slots of the FP32-refined solver: FP32 CG in the
+// one-launch form with FP64 reliable updates, its products formed from the
+// cells, which with constant k are one stencil: 32 B a row and pass, nothing
+// stored but the vectors.  With the whole boundary fixed every diagonal entry
+// is the same, so Jacobi is a division by it: the passes run on A / diag.
+// Problems that are done return at entry; the host queues chunks of passes (a
+// hipGraph) until the device has counted every problem done.  Completion is
+// stamped with the device wall clock.
+// (One workgroup a problem whatever its size leaves the end of a batch to the
+// largest, each at the rate of one CU: 512 problems up to 256^2 and 48^3 took
+// 67 ms of solving, now 8.4 ms; one 40^3 24 ms, now 0.46 ms.)
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -32,6 +42,9 @@
 #include <numeric>
 
 #include "femhip_internal.h"
+#include "cg_state.h"
+#include "lattice.h"
+#include "lattice_io.h"
 
 namespace femhip {
 namespace {
@@ -70,8 +83,7 @@ __device__ __forceinline__ void diag_shift(int k, int dim, int &dx, int &dy, int
 __global__ __launch_bounds__(kChunk) void k_batch_assemble(const BProb *__restrict__ probs, int count,
                                                            const int64_t *__restrict__ task_ptr,
                                                            const BTables *__restrict__ tabs,
-                                                           double *__restrict__ v64, float *__restrict__ v32,
-                                                           double *__restrict__ bvec, float *__restrict__ invd) {
+                                                           double *__restrict__ v64, double *__restrict__ bvec) {
   // problem of this block: last p with task_ptr[p] <= blockIdx.x
   int lo = 0, hi = count - 1;
   const int64_t t = blockIdx.x;
@@ -85,20 +97,16 @@ __global__ __launch_bounds__(kChunk) void k_batch_assemble(const BProb *__restri
   const int r = (int)(t - task_ptr[lo]) * kChunk + threadIdx.x;
   if (r >= P.stride) return;
   double *V = v64 + P.voff;
-  float *V32 = v32 + P.voff;
   if (r >= P.nrows) {   // padding rows
     for (int k = 0; k < P.K; ++k) {
       V[(int64_t)k * P.stride + r] = 0.0;
-      V32[(int64_t)k * P.stride + r] = 0.0f;
     }
     bvec[P.xoff + r] = 0.0;
-    invd[P.xoff + r] = 0.0f;
     return;
   }
   const int dim = P.dim, m = P.m, nv = 1 << dim;
   int a[3] = {r % m, dim > 1 ? (r / m) % m : 0, dim > 2 ? r / (m * m) : 0};
   int node[3] = {a[0] + 1, a[1] + 1, a[2] + 1};   // vertex index in [1, n-1]
-  double diag = 0.0;
   for (int k = 0; k < P.K; ++k) {
     int dd[3];
     diag_shift(k, dim, dd[0], dd[1], dd[2]);
@@ -122,10 +130,6 @@ __global__ __launch_bounds__(kChunk) void k_batch_assemble(const BProb *__restri
       val *= P.k;
     }
     V[(int64_t)k * P.stride + r] = val;
-    V32[(int64_t)k * P.stride + r] = (float)val;
-    // the centre diagonal is k = K/2; with m = 1 other offsets are 0 as well
-    // (dx = -m dy), so the offset cannot identify it
-    if (k == (P.K >> 1)) diag = val;
   }
   // RHS: sum over the cells around the node of int f N_node
   const double h = 1.0 / P.n;
@@ -146,230 +150,404 @@ __global__ __launch_bounds__(kChunk) void k_batch_assemble(const BProb *__restri
     }
   }
   bvec[P.xoff + r] = bsum;
-  invd[P.xoff + r] = (float)(1.0 / diag);
 }
 
 // ------------------------------------------------------------------- solve ---
 
-template <int BS, int NV>
-__device__ __forceinline__ void bsum(double (&v)[NV], double *sm) {
-  for (int off = 32; off > 0; off >>= 1)
-    for (int j = 0; j < NV; ++j) v[j] += __shfl_down(v[j], off, 64);
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  __syncthreads();   // sm free (previous readers done)
-  if (lane == 0)
-    for (int j = 0; j < NV; ++j) sm[j * (BS / 64) + w] = v[j];
-  __syncthreads();
-  for (int j = 0; j < NV; ++j) {
-    double s = 0.0;
-#pragma unroll 4   // a full unroll at 16 waves holds 16 NV values and spills the 1024-thread solve
-    for (int i = 0; i < BS / 64; ++i) s += sm[j * (BS / 64) + i];
-    v[j] = s;
-  }
-}
+constexpr int kBatchThreads = 256;
 
-// Diagonal offsets of a d-dimensional Q1 stencil, k = (dx+1) + 3(dy+1) + 9(dz+1)
-template <int DIM>
-__device__ __forceinline__ int stencil_off(int k, int m) {
-  const int dx = k % 3 - 1;
-  const int dy = DIM > 1 ? (k / 3) % 3 - 1 : 0;
-  const int dz = DIM > 2 ? k / 9 - 1 : 0;
-  return dx + m * (dy + m * dz);
-}
-
-// q_i = sum_k V[k][i] p[i + o_k] for this thread's rows (FP32), returns <p, q> partial
-template <int DIM>
-__device__ __forceinline__ double dia_spmv32(const float *__restrict__ V, int S, int n, int m,
-                                             const float *__restrict__ p, float *__restrict__ q, int BS) {
-  constexpr int K = DIM == 2 ? 9 : 27;
-  int off[K];
-#pragma unroll
-  for (int k = 0; k < K; ++k) off[k] = stencil_off<DIM>(k, m);
-  const int hi = n - 1;
-  double pq = 0.0;
-  for (int i = threadIdx.x; i < n; i += BS) {
-    float acc = 0.f;
-#pragma unroll
-    for (int k = 0; k < K; ++k) acc += V[(int64_t)k * S + i] * p[min(max(i + off[k], 0), hi)];
-    q[i] = acc;
-    pq += (double)(p[i] * acc);
-  }
-  return pq;
-}
-
-// FP64 residual for a reliable update: r = b - A (x + d); writes r32, returns
-// ||r||^2, <r32, M r32>, ||r32||^2 partials
-template <int DIM>
-__device__ __forceinline__ void dia_residual64(const double *__restrict__ V, int S, int n, int m,
-                                               const double *__restrict__ b, const double *__restrict__ x,
-                                               const float *__restrict__ d, const float *__restrict__ iv,
-                                               float *__restrict__ r, double (&t3)[3], int BS) {
-  constexpr int K = DIM == 2 ? 9 : 27;
-  int off[K];
-#pragma unroll
-  for (int k = 0; k < K; ++k) off[k] = stencil_off<DIM>(k, m);
-  const int hi = n - 1;
-  for (int i = threadIdx.x; i < n; i += BS) {
-    double acc = 0.0;
-#pragma unroll
-    for (int k = 0; k < K; ++k) {
-      const int c = min(max(i + off[k], 0), hi);
-      acc += V[(int64_t)k * S + i] * (x[c] + (double)d[c]);
-    }
-    const double ri = b[i] - acc;
-    const float rf = (float)ri;
-    r[i] = rf;
-    t3[0] += ri * ri;
-    t3[1] += (double)(rf * (iv[i] * rf));
-    t3[2] += (double)(rf * rf);
-  }
-}
-
-struct BPools {
-  const double *v64;
-  const float *v32;
-  const double *b;
-  double *x;
-  float *r, *p, *q, *d;
-  const float *invd;
+// A problem in the passes.
+struct BSolve {
+  Lattice g;
+  int dim, nrows, blocks, id;
+  int64_t xoff, poff;        // offsets in the vector pools and in the partial sums
+  double c[3], cu[3];        // cell weights of A, and of A / diag
+  double inv_diag;
 };
 
-template <int BS>
-__device__ void solve_one(const BProb &P, const BPools &pl, double rtol, double delta, int maxit, BOut *out,
-                          double *sm) {
-  const int n = P.nrows, K = P.K, S = P.stride, hi = n - 1;
-  const double *V64 = pl.v64 + P.voff;
-  const float *V32 = pl.v32 + P.voff;
-  const double *b = pl.b + P.xoff;
-  double *x = pl.x + P.xoff;
-  float *r = pl.r + P.xoff, *p = pl.p + P.xoff, *q = pl.q + P.xoff, *d = pl.d + P.xoff;
-  const float *iv = pl.invd + P.xoff;
-  (void)K;
-  (void)hi;
-  // x0 = 0: r = b, z = M r, p = z, d = 0
-  double s3[3] = {0, 0, 0};
-  for (int i = threadIdx.x; i < n; i += BS) {
-    x[i] = 0.0;
-    d[i] = 0.0f;
-    const float rf = (float)b[i];
-    r[i] = rf;
-    const float z = iv[i] * rf;
-    p[i] = z;
-    s3[0] += (double)(rf * z);
-    s3[1] += b[i] * b[i];
-    s3[2] += (double)(rf * rf);
+struct BPools {
+  const double *b;
+  double *x;
+  PairOf<float> r, q, p;
+  float *d;
+  double *part[2];           // the passes' sums, alternating
+};
+
+struct BCount {
+  int done;
+  int pad;
+  long long t0;
+};
+
+// problem and logical workgroup of this block (problem -1: none)
+__device__ __forceinline__ int2 batch_block(const int2 *__restrict__ table) { return table[blockIdx.x]; }
+
+__global__ void k_batch_start(BCount *count) {
+  if (threadIdx.x == 0 && blockIdx.x == 0) {
+    count->done = 0;
+    count->t0 = (long long)wall_clock64();
   }
-  bsum<BS, 3>(s3, sm);
-  double rz = s3[0];
-  const double bnorm = sqrt(s3[1]);
-  const double rhs_test = rtol * bnorm;   // RES_RES with x0 = 0 (cg.f90:305-307)
-  double rmax = sqrt(s3[2]), rnorm64 = bnorm;
-  // every thread holds the same reduced values; readfirstlane makes the loop
-  // and branch conditions wave-uniform for the compiler as well
+}
+
+// x = 0, d = 0, r = b / diag; partials ||r32||^2, ||b||^2
+__global__ __launch_bounds__(kBatchThreads) void k_batch_init(const BSolve *__restrict__ probs,
+                                                              const int2 *__restrict__ table, BPools pl) {
+  const int2 at = batch_block(table);
+  if (at.x < 0) return;
+  const BSolve &P = probs[at.x];
+  double v[2] = {0.0, 0.0};
+  for (int64_t i = (int64_t)at.y * kBatchThreads + threadIdx.x; i < P.nrows; i += (int64_t)P.blocks * kBatchThreads) {
+    const double bi = pl.b[P.xoff + i];
+    const float rf = (float)(P.inv_diag * bi);
+    pl.x[P.xoff + i] = 0.0;
+    pl.d[P.xoff + i] = 0.0f;
+    pl.r.v[0][P.xoff + i] = rf;
+    v[0] += (double)rf * (double)rf;
+    v[1] += bi * bi;
+  }
+  group_partials<2>(v, pl.part[0] + P.poff, P.blocks, at.y);
+}
+
+// one wave a problem: its first state (RES_RES, x0 = 0: cg.f90:305-307)
+__global__ __launch_bounds__(64) void k_batch_begin(const BSolve *__restrict__ probs, int count, BPools pl, CgState *st,
+                                                    double rtol, double delta, int maxit, BOut *out, BCount *cnt) {
+  const int pi = blockIdx.x;
+  if (pi >= count) return;
+  const BSolve &P = probs[pi];
+  double v[2];
+  group_reduce<2>(pl.part[0] + P.poff, P.blocks, v);
+  if (threadIdx.x != 0) return;
+  CgState s{};
+  s.rtol = rtol;
+  s.delta = delta;
+  s.maxit = maxit;
+  s.crit = FEMHIP_RES_RES;
+  s.rz = v[0];
+  s.bnorm = s.r0norm = s.rnorm = sqrt(v[1]);
+  s.rhs_test = rtol * s.bnorm;
+  s.rmax = sqrt(v[0]);
+  s.rscale = s.bnorm > 0.0 ? s.rmax / s.bnorm : 1.0;
+  s.first = 1;
+  s.converged = s.bnorm <= s.rhs_test;
+  s.done = s.converged || maxit <= 0;
+  st[2 * pi] = st[2 * pi + 1] = s;
+  BOut o{0, 0, s.converged, 0, s.bnorm, s.bnorm, 0};
+  if (s.done) {
+    o.t_end = (long long)wall_clock64();
+    atomicAdd(&cnt->done, 1);
+  }
+  out[P.id] = o;
+}
+
+template <int DIM>
+__device__ __forceinline__ void batch_pass(const BSolve &P, int lb, const BPools &pl, CgState *S, int par, BOut *out,
+                                           BCount *cnt, double *lds) {
+  const CgState &cur = S[par];
+  CgState &next = S[par ^ 1];
+  const bool lead = lb == 0 && threadIdx.x == 0;
+  if (cur.done) {
+    if (lead) next.done = 1;
+    return;
+  }
+  const double *part_in = pl.part[par ^ 1] + P.poff;
+  double *part_out = pl.part[par] + P.poff;
+  const int set = cur.set;
+  int64_t row0, rows;
+  const Lattice w = lattice_window(P.g, DIM, 1, lb, row0, rows);
+  const int64_t off = P.xoff + row0;
+  const uint32_t b4 = 4u * (uint32_t)rows, b8 = 8u * (uint32_t)rows;
+  CellQ1<DIM, kCoefCell> cell;
+  cell.k = CoefDev{};
+  double alpha = 0.0, beta = 0.0;
+  if (cur.ru == 1) {
+    if (lead) {
+      next = cur;
+      next.ru = 2;
+    }
+    IoRes io{pl.x + off, pl.b + off, nullptr, nullptr, nullptr, pl.r.v[set] + off, nullptr, kLatUpdate,
+             {0.0, 0.0, 0.0, 0.0}, buf_of(pl.x + off, b8), P.inv_diag};
+    for (int d = 0; d < DIM; ++d) cell.k.c[d] = P.c[d];
+    lattice_march<DIM, 1>(w, lb, cell, io, lds);
+    double v[2] = {io.acc[0], io.acc[1]};
+    group_partials<2>(v, part_out, P.blocks, lb);
+    return;
+  }
+  CgResult unused;
+  if (cur.first == 1) {   // p = r
+    if (lead) {
+      next = cur;
+      next.first = 2;
+      next.set = set ^ 1;
+    }
+  } else if (cur.ru == 2) {
+    double rd[2];
+    group_reduce<2>(part_in, P.blocks, rd);
+    const RfStep step = rf_decide(cur, rd, lead, next, &unused);   // FP64 stopping test, beta
+    if (lead) {
+      next.first = 2;
+      next.set = set ^ 1;
+      if (step.done) {
+        out->iters = next.iter;
+        out->updates = next.updates;
+        out->conv = next.converged;
+        out->rnorm = next.rnorm;
+        out->t_end = (long long)wall_clock64();
+        atomicAdd(&cnt->done, 1);
+      }
+    }
+    if (step.done) return;
+    beta = step.beta;
+  } else {
+    double red[kSums];
+    group_reduce<kSums>(part_in, P.blocks, red);
+    const double rd[2] = {red[kSumNu], 0.0};
+    if (cur.first == 2) {   // no iteration made since the direction was set
+      if (lead) {
+        next = cur;
+        next.first = 0;
+        next.rz = red[kSumNu];
+      }
+    } else {
+      const RfStep step = rf_decide(cur, rd, lead, next, &unused);
+      if (step.fold) {   // back to the set of the direction before last
+        if (lead) {
+          next.ru = 1;
+          next.set = set ^ 1;
+        }
+        for (int64_t i = (int64_t)lb * kBatchThreads + threadIdx.x; i < P.nrows;
+             i += (int64_t)P.blocks * kBatchThreads) {
+          pl.x[P.xoff + i] += (double)pl.d[P.xoff + i];
+          pl.d[P.xoff + i] = 0.0f;
+        }
+        return;
+      }
+    }
+    pr_scalars(red, lead, next, alpha, beta);
+    if (lead) next.set = set ^ 1;
+  }
+  const uint32_t old = cur.first == 1 ? 0 : b4;
+  IoRf io{buf_of(pl.r.v[set] + off, b4), buf_of(pl.q.v[set] + off, cur.ru == 2 ? 0 : old), buf_of(nullptr, 0),
+          buf_of(pl.p.v[set] + off, old), buf_of(pl.r.v[set ^ 1] + off, b4), buf_of(pl.q.v[set ^ 1] + off, b4),
+          buf_of(pl.p.v[set ^ 1] + off, b4), buf_of(pl.d + off, b4), false, alpha, beta, (float)alpha, (float)beta,
+          {0.0, 0.0, 0.0, 0.0, 0.0, 0.0}};
+  for (int d = 0; d < DIM; ++d) cell.k.c[d] = P.cu[d];
+  lattice_march<DIM, 1>(w, lb, cell, io, lds);
+  group_partials<kSums>(io.sum, part_out, P.blocks, lb);
+}
+
+__global__ __launch_bounds__(kBatchThreads, 4) void k_batch_pass(const BSolve *__restrict__ probs,
+                                                                 const int2 *__restrict__ table, BPools pl, CgState *st,
+                                                                 int par, BOut *out, BCount *cnt) {
+  const int2 at = batch_block(table);
+  if (at.x < 0) return;
+  const BSolve &P = probs[at.x];
+  if (P.dim == 2) batch_pass<2>(P, at.y, pl, st + 2 * at.x, par, out + P.id, cnt, lattice_smem);
+  else batch_pass<3>(P, at.y, pl, st + 2 * at.x, par, out + P.id, cnt, lattice_smem);
+}
+
+// ------------------------------------------------------- small problems ---
+//
+// A problem that fits one workgroup's registers (at most RPT rows a thread) is
+// solved there from start to end: its direction lies in LDS inside a frame of
+// zeros, a thread owns a run of rows along the last direction, and the product
+// is the constant stencil by the number of directions two nodes differ in:
+// weights w0..w3.  Three LDS (9 in 3-D) reads a row, no memory traffic but the
+// reliable updates', three barriers an iteration.  64^2 cells take 5.5 us an
+// iteration (10 us with the matrix streamed from memory; 9 us a pass in the
+// passes), 500 problems of 58 rows 33 us in all (69 us; 333 us in the passes).
+
+struct BSmall {
+  double c[4], inv_diag;     // weights of A; 1 / its diagonal
+  float cu[4];               // weights of A / diag
+  int id, dim, m, nrows;
+  int cols, segs, len, plane;   // columns, runs a column, rows a run, frame entries a plane
+  int64_t xoff;
+};
+
+struct BParams {
+  double rtol, delta;
+  int maxit, pad;
+};
+
+// sums of v over the workgroup, the same in every thread; sm: NV rows
+template <int T, int NV>
+__device__ __forceinline__ void small_sum(double (&v)[NV], double *sm) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1)
+#pragma unroll
+    for (int k = 0; k < NV; ++k) v[k] += __shfl_xor(v[k], off, 64);
+  if constexpr (T > 64) {
+    const int w = threadIdx.x >> 6;
+    if ((threadIdx.x & 63) == 0)
+#pragma unroll
+      for (int k = 0; k < NV; ++k) sm[k * (T / 64) + w] = v[k];
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+      double s = 0.0;
+#pragma unroll
+      for (int i = 0; i < T / 64; ++i) s += sm[k * (T / 64) + i];
+      v[k] = s;
+    }
+  } else {
+    __syncthreads();
+  }
+}
+
+// The stencil along a run: f(j, centre, w0 u + ...) for rows j < len
+template <int DIM, int RPT, class Real, class F>
+__device__ __forceinline__ void run_stencil(const Real *u, int at, int L, int plane, int len, const Real (&w)[4], F &&f) {
+  Real a[3], b[3], c[3];   // in-plane sums: own node, the neighbours' share, centre
+#pragma unroll
+  for (int j = 0; j < RPT + 2; ++j) {
+    if (j < len + 2) {
+      if (j > 0) {
+        at += plane;
+        asm volatile("" : "+v"(at));   // formed here: addresses kept for every row would spill
+      }
+      const Real *q = u + at;
+      const Real p0 = q[0], p1 = q[-1] + q[1] + (DIM == 3 ? q[-L] + q[L] : Real(0));
+      Real own = w[0] * p0 + w[1] * p1, side = w[1] * p0 + w[2] * p1;
+      if (DIM == 3) {
+        const Real p2 = (q[-L - 1] + q[-L + 1]) + (q[L - 1] + q[L + 1]);
+        own += w[2] * p2;
+        side += w[3] * p2;
+      }
+      a[j % 3] = own;
+      b[j % 3] = side;
+      c[j % 3] = p0;
+      if (j >= 2) f(j - 2, c[(j - 1) % 3], a[(j - 1) % 3] + (b[j % 3] + b[(j - 2) % 3]));
+      if (RPT > 8 || sizeof(Real) > 4) __builtin_amdgcn_sched_barrier(0);   // a row's loads at a time: registers
+    }
+  }
+}
+
+template <int DIM, int T, int RPT>
+__device__ __forceinline__ void small_solve(const BSmall &P, const BPools &pl, const BParams &prm, BOut *out, double *lds) {
+  __shared__ double sums[6][T / 64];
+  const int tid = threadIdx.x, L = P.m + 2, plane = P.plane, len = P.len;
+  const int seg = tid / P.cols, col = tid % P.cols, z0 = seg * len;
+  const bool active = seg < P.segs;
+  const int rows = active ? min(len, P.m - z0) : 0;   // may be < 0: a run past the last row
+  // frame entry of the column's own node, in the plane before the run
+  const int at = active ? (DIM == 3 ? (col % P.m + 1) + L * (col / P.m + 1) : col + 1) + plane * z0 : L + 1 < plane ? L + 1 : 1;
+  const int entries = plane * (P.segs * len + 2);
+  const uint32_t row0 = (uint32_t)(col + P.cols * z0), cols = (uint32_t)P.cols;
+  double *x = pl.x + P.xoff;
+  const double *rhs = pl.b + P.xoff;
+  float *u32 = reinterpret_cast<float *>(lds);
+  const float w32[4] = {P.cu[0], P.cu[1], P.cu[2], P.cu[3]};
+  float r[RPT], p[RPT], d[RPT], q[RPT];
+  for (int i = tid; i < entries; i += T) u32[i] = 0.0f;
+  double s2[2] = {0.0, 0.0};
+#pragma unroll
+  for (int j = 0; j < RPT; ++j) {
+    r[j] = d[j] = q[j] = 0.0f;
+    if (j < rows) {
+      const uint32_t i = row0 + cols * (uint32_t)j;
+      const double b = rhs[i];
+      r[j] = (float)(P.inv_diag * b);
+      s2[0] += (double)r[j] * (double)r[j];
+      s2[1] += b * b;
+      x[i] = 0.0;
+    }
+    p[j] = r[j];
+  }
+  small_sum<T>(s2, sums[0]);   // also: the frame is cleared
+  auto put = [&]() {
+#pragma unroll
+    for (int j = 0, to = at; j < RPT; ++j) {
+      to += plane;
+      asm volatile("" : "+v"(to));
+      if (j < rows) u32[to] = p[j];
+    }
+  };
+  double rz = s2[0], rmax = sqrt(s2[0]), rnorm64 = sqrt(s2[1]);
+  const double bnorm = rnorm64, rhs_test = prm.rtol * bnorm, scale = fabs(P.inv_diag);
+  // readfirstlane: wave-uniform for the compiler as well
   int it = 0, upd = 0, conv = __builtin_amdgcn_readfirstlane(bnorm <= rhs_test ? 1 : 0);
-  while (!conv && it < maxit) {
-    __syncthreads();   // p complete before neighbours are gathered
-    double s1[1] = {P.dim == 2 ? dia_spmv32<2>(V32, S, n, P.m, p, q, BS) : dia_spmv32<3>(V32, S, n, P.m, p, q, BS)};
-    bsum<BS, 1>(s1, sm);
+  while (!conv && it < prm.maxit) {
+    put();
+    __syncthreads();
+    double s1[1] = {0.0};
+    run_stencil<DIM, RPT>(u32, at, L, plane, len, w32, [&](int j, float, float y) {
+      q[j] = j < rows ? y : 0.0f;
+      s1[0] += (double)p[j] * (double)q[j];
+    });
+    small_sum<T>(s1, sums[2]);
     const double alpha = s1[0] != 0.0 ? rz / s1[0] : 0.0;
     const float af = (float)alpha;
-    double s2[2] = {0, 0};
-    float rzl = 0.f, rrl = 0.f;
-    for (int i = threadIdx.x; i < n; i += BS) {
-      d[i] = d[i] + af * p[i];
-      const float ri = r[i] + (-af) * q[i];
-      r[i] = ri;
-      const float z = iv[i] * ri;
-      rzl += ri * z;
-      rrl += ri * ri;
+    double sr[1] = {0.0};
+#pragma unroll
+    for (int j = 0; j < RPT; ++j) {
+      d[j] = __builtin_fmaf(af, p[j], d[j]);
+      r[j] = __builtin_fmaf(-af, q[j], r[j]);
+      sr[0] += (double)r[j] * (double)r[j];
     }
-    s2[0] = rzl;
-    s2[1] = rrl;
-    bsum<BS, 2>(s2, sm);
+    small_sum<T>(sr, sums[3]);
     ++it;
-    double rz_new = s2[0];
-    const double rnorm = sqrt(s2[1]);
-    const int do_ru = __builtin_amdgcn_readfirstlane((rnorm < delta * rmax || rnorm <= rhs_test || it >= maxit) ? 1 : 0);
-    if (do_ru) {
-      // reliable update: r = b - A64 (x + d) in FP64 replaces the FP32 residual
-      __syncthreads();   // d complete before neighbours are gathered
-      double t3[3] = {0, 0, 0};
-      if (P.dim == 2) dia_residual64<2>(V64, S, n, P.m, b, x, d, iv, r, t3, BS);
-      else dia_residual64<3>(V64, S, n, P.m, b, x, d, iv, r, t3, BS);
-      bsum<BS, 3>(t3, sm);   // also orders the gathers above before x, d change
-      for (int i = threadIdx.x; i < n; i += BS) {
-        x[i] = x[i] + (double)d[i];
-        d[i] = 0.0f;
+    const double rnorm = sqrt(sr[0]);
+    double rz_new = sr[0];
+    rmax = fmax(rmax, rnorm);
+    const int update = __builtin_amdgcn_readfirstlane((rnorm < prm.delta * rmax || rnorm <= rhs_test * scale || it >= prm.maxit) ? 1 : 0);
+    if (update) {   // x += d; r = b - A x in FP64 replaces the FP32 residual
+      for (int e = tid; e < entries; e += T) lds[e] = 0.0;
+      __syncthreads();
+      uint32_t i = row0;
+#pragma unroll
+      for (int j = 0, to = at; j < RPT; ++j) {
+        to += plane;
+        asm volatile("" : "+v"(to), "+v"(i));
+        if (j < rows) lds[to] = x[i] + (double)d[j];
+        i += cols;
       }
+      i = row0;
+      __syncthreads();
+      double t2[2] = {0.0, 0.0};
+      run_stencil<DIM, RPT>(lds, at, L, plane, len, P.c, [&](int j, double xj, double y) {
+        asm volatile("" : "+v"(i));
+        if (j < rows) {
+          x[i] = xj;
+          const double ri = rhs[i] - y;
+          r[j] = (float)(P.inv_diag * ri);
+          t2[0] += (double)r[j] * (double)r[j];
+          t2[1] += ri * ri;
+        }
+        d[j] = 0.0f;
+        i += cols;
+      });
+      small_sum<T>(t2, sums[4]);
+      for (int i = tid; i < entries; i += T) u32[i] = 0.0f;   // the frame again
+      __syncthreads();
       ++upd;
-      rnorm64 = sqrt(t3[0]);
-      rz_new = t3[1];
-      rmax = sqrt(t3[2]);
-      if (__builtin_amdgcn_readfirstlane(rnorm64 <= rhs_test ? 1 : 0)) {
-        conv = 1;
-        break;
-      }
-      if (it >= maxit) break;
-    } else {
-      rmax = fmax(rmax, rnorm);
+      rz_new = t2[0];
+      rmax = sqrt(t2[0]);
+      rnorm64 = sqrt(t2[1]);
+      conv = __builtin_amdgcn_readfirstlane(rnorm64 <= rhs_test ? 1 : 0);
     }
-    double beta = 1.0 / rz;
-    beta = beta * rz_new;
+    const float beta = (float)(rz_new / rz);
     rz = rz_new;
-    const float bt = (float)beta;
-    for (int i = threadIdx.x; i < n; i += BS) {
-      const float z = iv[i] * r[i];
-      const float t = bt * p[i];
-      p[i] = t + z;
-    }
+#pragma unroll
+    for (int j = 0; j < RPT; ++j) p[j] = dir_value(beta, p[j], r[j]);
   }
-  // Wave 0 stores the record (all its lanes store the same values): a branch
-  // on threadIdx.x == 0 here, next to the queue fetch of the caller's loop,
-  // lets the compiler thread the two lane-0 branches across the loop's back
-  // edge and park lane 0 while the other lanes loop on a stale index.
-  if (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) == 0) {
-    out->iters = it;
-    out->updates = upd;
-    out->conv = conv;
-    out->rnorm = rnorm64;
-    out->bnorm = bnorm;
-    out->t_end = (long long)wall_clock64();
+  if (tid == 0) {
+    BOut o{it, upd, conv, 0, rnorm64, bnorm, (long long)wall_clock64()};
+    out[P.id] = o;
   }
 }
 
-__global__ void k_batch_start(int *counter, long long *t0) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) {
-    *counter = 0;
-    *t0 = (long long)wall_clock64();
-  }
+template <int T, int RPT>
+__global__ __launch_bounds__(T) void k_batch_small(const BSmall *__restrict__ probs, int count, BPools pl, BParams prm,
+                                                   BOut *out) {
+  if ((int)blockIdx.x >= count) return;
+  const BSmall P = probs[blockIdx.x];
+  if (P.dim == 2) small_solve<2, T, RPT>(P, pl, prm, out, lattice_smem);
+  else small_solve<3, T, RPT>(P, pl, prm, out, lattice_smem);
 }
 
-// Persistent solve: workgroups take problems from the queue until it is empty
-// (every workgroup reaches the exit once the counter passes `count`).  Every
-// branch that encloses or follows a barrier is wave-uniform: the queue fetch is
-// made by the whole of wave 0 (lane 0 adds 1, the others 0) and the fetched
-// index is read back through readfirstlane.
-// BS threads (BS / 64 waves) per problem; 1024 / BS workgroups per CU, each
-// held to 128 VGPRs (four waves per SIMD)
-template <int BS>
-__global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(4))) void k_batch_solve(const BProb *__restrict__ probs, const int *__restrict__ order,
-                                                    int count, int *counter, BPools pl, double rtol, double delta,
-                                                    int maxit, BOut *out) {
-  __shared__ double sm[3 * (BS / 64)];
-  __shared__ int s_idx;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  for (;;) {
-    __syncthreads();   // readers of s_idx and sm from the previous problem are done
-    if (wave == 0) {
-      const int v = atomicAdd(counter, (threadIdx.x & 63) == 0 ? 1 : 0);
-      s_idx = __builtin_amdgcn_readfirstlane(v);   // lane 0's fetch
-    }
-    __syncthreads();
-    const int idx = __builtin_amdgcn_readfirstlane(s_idx);
-    if (idx >= count) break;
-    const int pi = order[idx];
-    solve_one<BS>(probs[pi], pl, rtol, delta, maxit, out + pi, sm);
-  }
+// the count of finished problems, for the host
+__global__ void k_batch_poll(const BCount *cnt, int *host) {
+  if (threadIdx.x == 0) *host = cnt->done;
 }
 
 }  // namespace
@@ -377,82 +555,288 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(4))) void k_
 
 using namespace femhip;
 
+// workgroups of the small problems: threads, rows a thread
+constexpr int kSmallClasses = 3;
+constexpr int kSmallT[kSmallClasses] = {64, 256, 1024}, kSmallRows[kSmallClasses] = {8, 8, 16};
+constexpr size_t kSmallLds = 144 * 1024;
+
 struct femhip_batch {
   femhip_ctx *ctx = nullptr;
   femhip_cg_params_t prm{};
   std::vector<BProb> probs;
-  std::vector<int> order;            // largest first
   std::vector<int64_t> task_ptr;
   int64_t entries = 0, vec = 0;
   DevBuf<BProb> d_probs;
-  DevBuf<int> d_order, d_sample, counter;
   DevBuf<int64_t> d_task;
   DevBuf<BTables> d_tabs;
   DevBuf<double> v64, b, x;
-  DevBuf<float> v32, r, p, q, d, invd;
+  // passes
+  DevBuf<BSmall> d_small;            // by class
+  int small_at[kSmallClasses + 1] = {};
+  size_t small_lds[kSmallClasses] = {};
+  DevBuf<BSolve> d_solve;
+  int passes = 0;                    // problems in the passes
+  DevBuf<int2> table;
+  int blocks = 0;                    // entries of the table
+  size_t lds = 0;
+  DevBuf<float> r[2], p[2], q[2], d;
+  DevBuf<double> part[2];
+  DevBuf<CgState> st;
   DevBuf<BOut> out;
-  DevBuf<long long> t0;
-  int threads = 512;
-  int wg_per_cu = 2;
-  hipGraphExec_t graph = nullptr;
-  int graph_threads = 0;
+  DevBuf<BCount> cnt;
+  int *h_done[2] = {nullptr, nullptr}, *d_done[2] = {nullptr, nullptr};   // pinned, mapped
+  hipEvent_t ev[2] = {nullptr, nullptr};
+  hipGraphExec_t graph[2] = {nullptr, nullptr};
   bool assembled = false;
   ~femhip_batch() {
-    if (graph) (void)hipGraphExecDestroy(graph);
+    for (auto g : graph)
+      if (g) (void)hipGraphExecDestroy(g);
+    for (auto *h : h_done)
+      if (h) (void)hipHostFree(h);
+    for (auto e : ev)
+      if (e) (void)hipEventDestroy(e);
   }
 };
 
 namespace femhip {
 namespace {
 
-BPools pools(femhip_batch &B) {
-  return BPools{B.v64.p, B.v32.p, B.b.p, B.x.p, B.r.p, B.p.p, B.q.p, B.d.p, B.invd.p};
+BPools pools(femhip_batch &B);
+
+template <int K>
+constexpr auto small_kernel = k_batch_small<kSmallT[K], kSmallRows[K]>;
+
+template <int K>
+void launch_small(femhip_batch &B, const BParams &prm) {
+  const int count = B.small_at[K + 1] - B.small_at[K];
+  if (!count) return;
+  hipLaunchKernelGGL(small_kernel<K>, dim3((unsigned)count), dim3(kSmallT[K]), B.small_lds[K], B.ctx->stream,
+                     B.d_small.p + B.small_at[K], count, pools(B), prm, B.out.p);
 }
 
-void launch_solve(femhip_batch &B, const int *order, int count, int threads) {
-  hipStream_t st = B.ctx->stream;
-  const int grid = std::max(1, B.ctx->num_cus * std::max(1, 1024 / threads));   // 16 waves a CU
-  const double delta = B.prm.inner_rtol > 0 ? B.prm.inner_rtol : 0.1;
-  hipLaunchKernelGGL(k_batch_start, dim3(1), dim3(64), 0, st, B.counter.p, B.t0.p);
-  BPools pl = pools(B);
-  switch (threads) {
-    case 64:
-      hipLaunchKernelGGL(k_batch_solve<64>, dim3(grid), dim3(64), 0, st, B.d_probs.p, order, count, B.counter.p, pl,
-                         B.prm.rtol, delta, B.prm.max_num_iterations, B.out.p);
-      break;
-    case 128:
-      hipLaunchKernelGGL(k_batch_solve<128>, dim3(grid), dim3(128), 0, st, B.d_probs.p, order, count, B.counter.p,
-                         pl, B.prm.rtol, delta, B.prm.max_num_iterations, B.out.p);
-      break;
-    case 256:
-      hipLaunchKernelGGL(k_batch_solve<256>, dim3(grid), dim3(256), 0, st, B.d_probs.p, order, count, B.counter.p,
-                         pl, B.prm.rtol, delta, B.prm.max_num_iterations, B.out.p);
-      break;
-    case 1024:
-      hipLaunchKernelGGL(k_batch_solve<1024>, dim3(grid), dim3(1024), 0, st, B.d_probs.p, order, count,
-                         B.counter.p, pl, B.prm.rtol, delta, B.prm.max_num_iterations, B.out.p);
-      break;
-    default:
-      hipLaunchKernelGGL(k_batch_solve<512>, dim3(grid), dim3(512), 0, st, B.d_probs.p, order, count, B.counter.p,
-                         pl, B.prm.rtol, delta, B.prm.max_num_iterations, B.out.p);
+BPools pools(femhip_batch &B) {
+  return BPools{B.b.p, B.x.p, {{B.r[0].p, B.r[1].p}}, {{B.q[0].p, B.q[1].p}}, {{B.p[0].p, B.p[1].p}}, B.d.p,
+                {B.part[0].p, B.part[1].p}};
+}
+
+// The class a problem is solved in by one workgroup, -1: in the passes.
+int small_class(const BProb &P, BSmall &S) {
+  for (int k = 0; k < kSmallClasses; ++k) {
+    const int64_t cols = P.dim == 3 ? (int64_t)P.m * P.m : P.m;
+    if (cols > kSmallT[k]) continue;
+    S.dim = P.dim;
+    S.m = P.m;
+    S.nrows = P.nrows;
+    S.xoff = P.xoff;
+    S.cols = (int)cols;
+    S.segs = std::min(P.m, kSmallT[k] / S.cols);
+    S.len = (P.m + S.segs - 1) / S.segs;
+    S.segs = (P.m + S.len - 1) / S.len;
+    S.plane = P.dim == 3 ? (P.m + 2) * (P.m + 2) : P.m + 2;
+    if (S.len <= kSmallRows[k] && sizeof(double) * S.plane * (S.segs * S.len + 2) <= kSmallLds) return k;
+  }
+  return -1;
+}
+
+// Each problem's path; tiles of the problems in the passes and the table of
+// their workgroups.  A workgroup takes about an eighth of what would fill every
+// CU once, within bounds: long marches repeat little, short ones leave no CU
+// waiting for the last problem.
+void plan_passes(femhip_batch &B, const std::vector<BTables> &tabs) {
+  const int count = (int)B.probs.size();
+  std::vector<BSmall> small[kSmallClasses];
+  std::vector<BSolve> sv;
+  std::vector<int> large;
+  int64_t total = 0;
+  for (int i = 0; i < count; ++i) {
+    const BProb &P = B.probs[(size_t)i];
+    BSmall S{};
+    const int cls = small_class(P, S);
+    if (cls < 0) {
+      large.push_back(i);
+      total += P.nrows;
+      continue;
+    }
+    const BTables &T = tabs[(size_t)P.cls];
+    double w[4] = {0.0, 0.0, 0.0, 0.0};   // the entries of a class are the same but for rounding
+    for (int a = 0; a < T.nd; ++a)
+      for (int b2 = 0; b2 < T.nd; ++b2) w[__builtin_popcount((unsigned)(a ^ b2))] += T.E[a * T.nd + b2];
+    // 2^d C(d, t) pairs differ in t directions; 2^(d-t) cells hold such a pair
+    const double pairs[2][4] = {{1, 2, 1, 1}, {1, 3, 3, 1}};
+    for (int t = 0; t <= P.dim; ++t) w[t] /= pairs[P.dim - 2][t] * (double)(1 << t);
+    for (int t = 0; t < 4; ++t) {
+      S.c[t] = P.k * w[t];
+      S.cu[t] = (float)(w[t] / w[0]);
+    }
+    S.inv_diag = 1.0 / (P.k * w[0]);
+    S.id = i;
+    small[cls].push_back(S);
+    B.small_lds[cls] = std::max(B.small_lds[cls], sizeof(double) * (size_t)S.plane * (size_t)(S.segs * S.len + 2));
+  }
+  size_t nsmall = 0;
+  for (int k = 0; k < kSmallClasses; ++k) {
+    std::stable_sort(small[k].begin(), small[k].end(), [](const BSmall &a, const BSmall &b2) { return a.nrows > b2.nrows; });
+    B.small_at[k] = (int)nsmall;
+    nsmall += small[k].size();
+  }
+  B.small_at[kSmallClasses] = (int)nsmall;
+  if (nsmall) {
+    B.d_small.alloc(nsmall);
+    for (int k = 0; k < kSmallClasses; ++k)
+      if (!small[k].empty())
+        FH_HIP(hipMemcpy(B.d_small.p + B.small_at[k], small[k].data(), sizeof(BSmall) * small[k].size(), hipMemcpyHostToDevice));
+    const void *fn[kSmallClasses] = {(const void *)small_kernel<0>, (const void *)small_kernel<1>, (const void *)small_kernel<2>};
+    for (int k = 0; k < kSmallClasses; ++k)
+      FH_HIP(hipFuncSetAttribute(fn[k], hipFuncAttributeMaxDynamicSharedMemorySize, (int)kSmallLds));
+  }
+  B.cnt.alloc(1);
+  B.passes = (int)large.size();
+  if (large.empty()) return;
+  const int per = (int)std::min<int64_t>(16384, std::max<int64_t>(1024, total / (8 * std::max(1, B.ctx->num_cus))));
+  std::vector<std::vector<int2>> lists(8);   // one an XCD: a problem's workgroups share an L2
+  int64_t poff = 0;
+  for (int i : large) {
+    const BProb &P = B.probs[(size_t)i];
+    femhip_mesh_desc_t mesh{};
+    mesh.dim = P.dim;
+    mesh.order = 1;
+    mesh.num_components = 1;
+    mesh.dirichlet = FEMHIP_BC_ALL_BOUNDARY;
+    for (int d = 0; d < 3; ++d) {
+      mesh.n[d] = d < P.dim ? P.n : 1;
+      mesh.limits[2 * d + 1] = 1.0;
+    }
+    LatticeOp L;
+    FH_CHECK(lattice_plan(mesh, 0, L, kBatchThreads, per), FEMHIP_ERR_INVALID, "batch problem too large");
+    BSolve S{};
+    S.g = L.g;
+    S.dim = P.dim;
+    S.nrows = P.nrows;
+    S.blocks = L.grid;
+    S.id = i;
+    S.xoff = P.xoff;
+    S.poff = poff;
+    poff += (int64_t)kSums * L.grid;
+    const BTables &T = tabs[(size_t)P.cls];
+    double diag = 0.0;   // every row's: the 2^d cells around its node
+    for (int a = 0; a < T.nd; ++a) diag += T.E[a * T.nd + a];
+    const double h = 1.0 / P.n, w = std::pow(0.5 * h, P.dim) * 4.0 / (h * h) / (double)(1 << (2 * P.dim));
+    for (int d = 0; d < 3; ++d) {
+      S.c[d] = d < P.dim ? P.k * w : 0.0;
+      S.cu[d] = d < P.dim ? w / diag : 0.0;
+    }
+    S.inv_diag = 1.0 / (P.k * diag);
+    B.lds = std::max(B.lds, L.lds);
+    sv.push_back(S);
+  }
+  std::stable_sort(sv.begin(), sv.end(), [](const BSolve &a, const BSolve &b2) { return a.blocks > b2.blocks; });
+  for (size_t i = 0; i < sv.size(); ++i) {   // largest first to the shortest list
+    auto &l = *std::min_element(lists.begin(), lists.end(), [](const auto &a, const auto &b2) { return a.size() < b2.size(); });
+    for (int k = 0; k < sv[i].blocks; ++k) l.push_back(int2{(int)i, k});
+  }
+  size_t rows = 0;
+  for (auto &l : lists) rows = std::max(rows, l.size());
+  FH_CHECK(rows * 8 < (size_t)INT32_MAX, FEMHIP_ERR_INVALID, "batch too large");
+  std::vector<int2> table(rows * 8, int2{-1, 0});
+  for (int x = 0; x < 8; ++x)
+    for (size_t j = 0; j < lists[(size_t)x].size(); ++j) table[j * 8 + (size_t)x] = lists[(size_t)x][j];
+  B.blocks = (int)table.size();
+  B.table.alloc(table.size());
+  B.d_solve.alloc(sv.size());
+  FH_HIP(hipMemcpy(B.table.p, table.data(), sizeof(int2) * table.size(), hipMemcpyHostToDevice));
+  FH_HIP(hipMemcpy(B.d_solve.p, sv.data(), sizeof(BSolve) * sv.size(), hipMemcpyHostToDevice));
+  for (auto *v : {&B.r[0], &B.r[1], &B.p[0], &B.p[1], &B.q[0], &B.q[1], &B.d}) v->alloc((size_t)B.vec);
+  for (auto &v : B.part) v.alloc((size_t)poff);
+  B.st.alloc(2 * sv.size());
+  for (int k = 0; k < 2; ++k) {   // written by the GPU, read by the host: mapped, coherent
+    FH_HIP(hipHostMalloc((void **)&B.h_done[k], sizeof(int), hipHostMallocMapped | hipHostMallocCoherent));
+    FH_HIP(hipHostGetDevicePointer((void **)&B.d_done[k], B.h_done[k], 0));
+    FH_HIP(hipEventCreateWithFlags(&B.ev[k], hipEventDisableTiming));
   }
 }
 
-float timed_solve(femhip_batch &B, const int *order, int count, int threads) {
+constexpr int kBatchChunk = 16;   // passes a graph (even: the parity restarts at 0)
+
+// the chunk's graph for result slot k, node by node (a stream capture would
+// make other threads' synchronous calls fail)
+void ensure_chunk(femhip_batch &B, int k) {
+  if (B.graph[k]) return;
+  hipGraph_t g;
+  FH_HIP(hipGraphCreate(&g, 0));
+  try {
+    hipGraphNode_t last = nullptr;
+    auto add = [&](void *fn, dim3 grid, dim3 block, size_t lds, void **args) {
+      hipKernelNodeParams prm{};
+      prm.func = fn;
+      prm.gridDim = grid;
+      prm.blockDim = block;
+      prm.sharedMemBytes = (unsigned)lds;
+      prm.kernelParams = args;
+      hipGraphNode_t node;
+      FH_HIP(hipGraphAddKernelNode(&node, g, last ? &last : nullptr, last ? 1 : 0, &prm));
+      last = node;
+    };
+    const BSolve *probs = B.d_solve.p;
+    const int2 *table = B.table.p;
+    BPools pl = pools(B);
+    CgState *st = B.st.p;
+    BOut *out = B.out.p;
+    BCount *cnt = B.cnt.p;
+    for (int i = 0; i < kBatchChunk; ++i) {
+      int par = i & 1;
+      void *args[] = {&probs, &table, &pl, &st, &par, &out, &cnt};
+      add((void *)k_batch_pass, dim3((unsigned)B.blocks), dim3(kBatchThreads), B.lds, args);
+    }
+    const BCount *cc = cnt;
+    int *host = B.d_done[k];
+    void *args[] = {&cc, &host};
+    add((void *)k_batch_poll, dim3(1), dim3(64), 0, args);
+    FH_HIP(hipGraphInstantiate(&B.graph[k], g, nullptr, nullptr, 0));
+  } catch (...) {
+    (void)hipGraphDestroy(g);
+    throw;
+  }
+  FH_HIP(hipGraphDestroy(g));
+}
+
+// The small problems (the quickest class first, its largest first), then the passes: enqueue chunks, one
+// ahead, until every problem is done.  A problem takes at most 4 maxit + 8
+// passes (an update takes three, at most one an iteration).
+void run_passes(femhip_batch &B) {
   hipStream_t st = B.ctx->stream;
-  hipEvent_t e0, e1;
-  FH_HIP(hipEventCreate(&e0));
-  FH_HIP(hipEventCreate(&e1));
-  FH_HIP(hipEventRecord(e0, st));
-  launch_solve(B, order, count, threads);
+  const BParams prm{B.prm.rtol, B.prm.inner_rtol > 0 ? B.prm.inner_rtol : 0.1, B.prm.max_num_iterations, 0};
+  hipLaunchKernelGGL(k_batch_start, dim3(1), dim3(64), 0, st, B.cnt.p);
+  launch_small<0>(B, prm);
+  launch_small<1>(B, prm);
+  launch_small<2>(B, prm);
   FH_HIP(hipGetLastError());
-  FH_HIP(hipEventRecord(e1, st));
-  FH_HIP(hipEventSynchronize(e1));
-  float ms = 0.f;
-  FH_HIP(hipEventElapsedTime(&ms, e0, e1));
-  (void)hipEventDestroy(e0);
-  (void)hipEventDestroy(e1);
-  return ms;
+  const int count = B.passes;
+  if (!count) {
+    FH_HIP(hipStreamSynchronize(st));
+    return;
+  }
+  for (int k = 0; k < 2; ++k) ensure_chunk(B, k);
+  BPools pl = pools(B);
+  hipLaunchKernelGGL(k_batch_init, dim3((unsigned)B.blocks), dim3(kBatchThreads), 0, st, B.d_solve.p, B.table.p, pl);
+  hipLaunchKernelGGL(k_batch_begin, dim3((unsigned)count), dim3(64), 0, st, B.d_solve.p, count, pl, B.st.p, prm.rtol,
+                     prm.delta, prm.maxit, B.out.p, B.cnt.p);
+  FH_HIP(hipGetLastError());
+  const int64_t most = 4 * (int64_t)B.prm.max_num_iterations + 8;
+  int64_t queued = 0;
+  auto push = [&](int k) {
+    *B.h_done[k] = 0;
+    FH_HIP(hipGraphLaunch(B.graph[k], st));
+    FH_HIP(hipEventRecord(B.ev[k], st));
+    queued += kBatchChunk;
+  };
+  push(0);
+  push(1);
+  for (int k = 0;; k ^= 1) {
+    FH_HIP(hipEventSynchronize(B.ev[k]));
+    if (*B.h_done[k] >= count || queued >= most + 2 * kBatchChunk) break;
+    push(k);
+  }
+  FH_HIP(hipStreamSynchronize(st));
 }
 
 }  // namespace
@@ -526,39 +910,21 @@ int femhip_batch_create(femhip_ctx_t *ctx, int32_t count, const femhip_batch_pro
       }
       B->entries = voff;
       B->vec = xoff;
-      // largest estimated work first: rows x diagonals x n (CG iterations grow ~ n)
-      B->order.resize((size_t)count);
-      std::iota(B->order.begin(), B->order.end(), 0);
-      std::stable_sort(B->order.begin(), B->order.end(), [&](int a, int b2) {
-        const BProb &A = B->probs[(size_t)a], &C = B->probs[(size_t)b2];
-        return (double)A.nrows * A.K * A.n > (double)C.nrows * C.K * C.n;
-      });
       B->task_ptr.resize((size_t)count + 1);
       B->task_ptr[0] = 0;
       for (int i = 0; i < count; ++i)
         B->task_ptr[(size_t)i + 1] = B->task_ptr[(size_t)i] + (B->probs[(size_t)i].stride + kChunk - 1) / kChunk;
       B->d_probs.alloc((size_t)count);
-      B->d_order.alloc((size_t)count);
       B->d_task.alloc((size_t)count + 1);
       B->d_tabs.alloc(tabs.size());
-      B->counter.alloc(1);
-      B->t0.alloc(1);
       B->out.alloc((size_t)count);
       FH_HIP(hipMemcpy(B->d_probs.p, B->probs.data(), sizeof(BProb) * count, hipMemcpyHostToDevice));
-      FH_HIP(hipMemcpy(B->d_order.p, B->order.data(), sizeof(int) * count, hipMemcpyHostToDevice));
       FH_HIP(hipMemcpy(B->d_task.p, B->task_ptr.data(), sizeof(int64_t) * (count + 1), hipMemcpyHostToDevice));
       FH_HIP(hipMemcpy(B->d_tabs.p, tabs.data(), sizeof(BTables) * tabs.size(), hipMemcpyHostToDevice));
       B->v64.alloc((size_t)B->entries);
-      B->v32.alloc((size_t)B->entries);
-      for (auto *buf : {&B->r, &B->p, &B->q, &B->d, &B->invd}) buf->alloc((size_t)B->vec);
       B->b.alloc((size_t)B->vec);
       B->x.alloc((size_t)B->vec);
-      if (const char *t = getenv("FEMHIP_BATCH_THREADS")) {
-        const int v = atoi(t);
-        FH_CHECK(v == 64 || v == 128 || v == 256 || v == 512 || v == 1024, FEMHIP_ERR_INVALID,
-                 "FEMHIP_BATCH_THREADS must be 64, 128, 256, 512 or 1024");
-        B->threads = v;
-      }
+      plan_passes(*B, tabs);
     } catch (...) {
       femhip_batch_destroy(B);
       throw;
@@ -583,7 +949,7 @@ int femhip_batch_assemble(femhip_batch_t *B, double *ms) {
     const int64_t tasks = B->task_ptr.back();
     FH_CHECK(tasks < (int64_t)INT32_MAX, FEMHIP_ERR_INVALID, "batch too large");
     hipLaunchKernelGGL(k_batch_assemble, dim3((unsigned)tasks), dim3(kChunk), 0, st, B->d_probs.p,
-                       (int)B->probs.size(), B->d_task.p, B->d_tabs.p, B->v64.p, B->v32.p, B->b.p, B->invd.p);
+                       (int)B->probs.size(), B->d_task.p, B->d_tabs.p, B->v64.p, B->b.p);
     FH_HIP(hipGetLastError());
     FH_HIP(hipEventRecord(e1, st));
     FH_HIP(hipEventSynchronize(e1));
@@ -605,25 +971,7 @@ int femhip_batch_autotune(femhip_batch_t *B, int32_t *threads) {
     FH_CHECK(B, FEMHIP_ERR_INVALID, "null batch");
     FH_CHECK(B->assembled, FEMHIP_ERR_STATE, "assemble the batch first");
     FH_HIP(hipSetDevice(B->ctx->device));
-    // sample: every k-th problem of the largest-first order, up to 4 per CU
-    const int count = (int)B->order.size();
-    const int want = std::min(count, 4 * std::max(1, B->ctx->num_cus));
-    std::vector<int> sample;
-    for (int i = 0; i < want; ++i) sample.push_back(B->order[(size_t)((int64_t)i * count / want)]);
-    B->d_sample.alloc(sample.size());
-    FH_HIP(hipMemcpy(B->d_sample.p, sample.data(), sizeof(int) * sample.size(), hipMemcpyHostToDevice));
-    float best = 1e30f;
-    int best_t = B->threads;
-    for (int t : {64, 128, 256, 512, 1024}) {   // waves per problem: 1 to 16
-      timed_solve(*B, B->d_sample.p, (int)sample.size(), t);   // warm-up
-      const float ms = timed_solve(*B, B->d_sample.p, (int)sample.size(), t);
-      if (ms < best) {
-        best = ms;
-        best_t = t;
-      }
-    }
-    B->threads = best_t;
-    if (threads) *threads = best_t;
+    if (threads) *threads = kBatchThreads;   // the passes have one workgroup size
     return FEMHIP_OK;
   } catch (const Error &e) {
     set_error(e.msg);
@@ -637,23 +985,11 @@ int femhip_batch_solve(femhip_batch_t *B, femhip_batch_result_t *results, double
     FH_CHECK(B->assembled, FEMHIP_ERR_STATE, "assemble the batch first");
     FH_HIP(hipSetDevice(B->ctx->device));
     hipStream_t st = B->ctx->stream;
-    if (getenv("FEMHIP_AUTOTUNE") && !B->graph) femhip_batch_autotune(B, nullptr);
-    if (!B->graph || B->graph_threads != B->threads) {
-      if (B->graph) FH_HIP(hipGraphExecDestroy(B->graph));
-      B->graph = nullptr;
-      hipGraph_t g;
-      FH_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-      launch_solve(*B, B->d_order.p, (int)B->order.size(), B->threads);
-      FH_HIP(hipStreamEndCapture(st, &g));
-      FH_HIP(hipGraphInstantiate(&B->graph, g, nullptr, nullptr, 0));
-      FH_HIP(hipGraphDestroy(g));
-      B->graph_threads = B->threads;
-    }
     hipEvent_t e0, e1;
     FH_HIP(hipEventCreate(&e0));
     FH_HIP(hipEventCreate(&e1));
     FH_HIP(hipEventRecord(e0, st));
-    FH_HIP(hipGraphLaunch(B->graph, st));
+    run_passes(*B);
     FH_HIP(hipEventRecord(e1, st));
     FH_HIP(hipEventSynchronize(e1));
     float t = 0.f;
@@ -664,9 +1000,9 @@ int femhip_batch_solve(femhip_batch_t *B, femhip_batch_result_t *results, double
     if (results) {
       const size_t count = B->probs.size();
       std::vector<BOut> out(count);
-      long long t0 = 0;
+      BCount cnt{};
       FH_HIP(hipMemcpy(out.data(), B->out.p, sizeof(BOut) * count, hipMemcpyDeviceToHost));
-      FH_HIP(hipMemcpy(&t0, B->t0.p, sizeof(t0), hipMemcpyDeviceToHost));
+      FH_HIP(hipMemcpy(&cnt, B->cnt.p, sizeof(cnt), hipMemcpyDeviceToHost));
       int rate_khz = 0;
       FH_HIP(hipDeviceGetAttribute(&rate_khz, hipDeviceAttributeWallClockRate, B->ctx->device));
       const double us_per_tick = rate_khz > 0 ? 1e3 / rate_khz : 0.01;
@@ -678,7 +1014,7 @@ int femhip_batch_solve(femhip_batch_t *B, femhip_batch_result_t *results, double
         R.num_dofs = B->probs[i].nrows;
         R.true_residual = out[i].rnorm;
         R.rhs_norm = out[i].bnorm;
-        R.latency_us = (double)(out[i].t_end - t0) * us_per_tick;
+        R.latency_us = (double)(out[i].t_end - cnt.t0) * us_per_tick;
       }
     }
     return FEMHIP_OK;

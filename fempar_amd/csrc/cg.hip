@@ -41,6 +41,7 @@
 #include "femhip_internal.h"
 #include "lattice.h"
 #include "cg_state.h"
+#include "lattice_io.h"
 
 namespace femhip {
 namespace {

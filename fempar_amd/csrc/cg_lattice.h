@@ -41,62 +41,6 @@ __device__ __forceinline__ LatticeCell<DIM, P, KIND> lattice_cell(const CoefDev 
   return cell;
 }
 
-// Workgroup's partial sums: part[k * gridDim.x + blockIdx.x].
-template <int NV>
-__device__ __forceinline__ void group_partials(double (&v)[NV], double *part) {
-  __shared__ double sm[NV][16];
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1)
-#pragma unroll
-    for (int k = 0; k < NV; ++k) v[k] += __shfl_down(v[k], off, 64);
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
-  if (lane == 0)
-#pragma unroll
-    for (int k = 0; k < NV; ++k) sm[k][w] = v[k];
-  __syncthreads();
-  if (threadIdx.x < NV) {
-    double s = 0.0;
-    for (int i = 0; i < nw; ++i) s += sm[threadIdx.x][i];
-    part[threadIdx.x * gridDim.x + blockIdx.x] = s;
-  }
-}
-// Sums of a launch's partials, in the same order in every workgroup: a wave
-// takes a whole sum.
-template <int NV>
-__device__ __forceinline__ void group_reduce(const double *part, int g, double (&v)[NV]) {
-  __shared__ double sm[NV];
-  const int lane = threadIdx.x & 63, nw = blockDim.x >> 6;
-  for (int k = threadIdx.x >> 6; k < NV; k += nw) {
-    double a = 0.0;
-    for (int b = lane; b < g; b += 64) a += part[k * g + b];
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) a += __shfl_down(a, off, 64);
-    if (lane == 0) sm[k] = a;
-  }
-  __syncthreads();
-#pragma unroll
-  for (int k = 0; k < NV; ++k) v[k] = sm[k];
-}
-
-extern __shared__ double lattice_smem[];
-
-// Sums of a pass.
-enum { kSumMu = 0, kSumDelta = 1, kSumGamma = 2, kSumNu = 3, kSumRr = 4, kSumPp = 5, kSums = 6 };
-
-// alpha and beta from the sums of the pass before; `lead` notes them in the next state
-__device__ __forceinline__ void pr_scalars(const double (&red)[kSums], bool lead, CgState &next, double &alpha,
-                                           double &beta) {
-  const double nu = red[kSumNu];
-  alpha = red[kSumMu] != 0.0 ? nu / red[kSumMu] : 0.0;   // cg.f90:195-199
-  const double pred = __builtin_fma(alpha, __builtin_fma(alpha, red[kSumGamma], -2.0 * red[kSumDelta]), nu);
-  beta = nu != 0.0 ? pred / nu : 0.0;
-  if (lead) {
-    next.alpha = alpha;
-    next.pap = red[kSumMu];
-    next.pp = red[kSumPp];
-  }
-}
-
 struct IoCg {
   static constexpr int kKeep = 3;
   struct Halo {
@@ -182,12 +126,6 @@ struct IoCg {
 #define FEMHIP_LATTICE_BOUNDS \
   __launch_bounds__(lattice_threads(DIM, P, KIND == kElastic ? 3 : 1), lattice_waves(DIM, P, KIND == kElastic ? 3 : 1))
 
-// The vectors that alternate between two sets: pass `par` reads set par.
-template <typename T>
-struct PairOf {
-  T *v[2];
-};
-
 template <int DIM, int P, int KIND>
 __global__ FEMHIP_LATTICE_BOUNDS void k_lat_cg(Lattice g, CoefDev c, Q2Tab t, int32_t n, PairOf<double> r,
                                                PairOf<double> s, PairOf<double> p, double *x, const double *invd,
@@ -207,65 +145,9 @@ __global__ FEMHIP_LATTICE_BOUNDS void k_lat_cg(Lattice g, CoefDev c, Q2Tab t, in
           buf_of(s.v[par ^ 1], bytes), buf_of(p.v[par ^ 1], bytes), buf_of(x, bytes), invd != nullptr,
           (int)gridDim.x, 0.0, 0.0, {0.0, 0.0, 0.0, 0.0, 0.0, 0.0}};
   auto cell = lattice_cell<DIM, P, KIND>(c, t);
-  lattice_march<DIM, P>(g, cell, io, lattice_smem);
+  lattice_march<DIM, P>(g, lattice_block(g), cell, io, lattice_smem);
   group_partials<kSums>(io.sum, part_out);
 }
-
-// Residuals of x in FP64, r = b - A x, for what mode asks.
-enum { kLatInit64 = 0,   // r64; partials <r,z>, ||r||^2, ||b||^2, <b,Mb>
-       kLatInit32 = 1,   // r32 = S r, d = 0; partials <r32,r32>, ||r||^2, ||b||^2, <r32,r32>
-       kLatTrue = 2,     // partial ||r||^2 (reporting only)
-       kLatUpdate = 3 }; // r32 = S r; partials <r32,r32>, ||r||^2
-
-struct IoRes {
-  static constexpr int kKeep = 1;
-  struct Raw {
-    double x;
-  };
-  using Halo = Raw;
-  const double *__restrict__ x, *__restrict__ b, *__restrict__ invd;
-  const double *__restrict__ sc;
-  double *__restrict__ r64;
-  float *__restrict__ r32, *__restrict__ d32;
-  int mode;
-  double acc[4];
-  BufRsrc xb;
-  __device__ __forceinline__ bool ready() const { return true; }
-  __device__ __forceinline__ Raw fetch(uint32_t o) const { return Raw{buf_ld64(xb, o)}; }
-  __device__ __forceinline__ Halo halo(uint32_t o) const { return fetch(o); }
-  __device__ __forceinline__ double halo_value(const Halo &w) const { return w.x; }
-  __device__ __forceinline__ double value(const Raw &w, uint32_t, double (&)[kKeep]) const {
-    return w.x;
-  }
-  template <bool FULL>
-  __device__ __forceinline__ void out(uint32_t o, const double (&)[kKeep], double y) {
-    if (o < kNoPlane) row((int)(o >> 3), y);
-  }
-  __device__ __forceinline__ void row(int i, double y) {
-    const double bi = b[i], ri = bi - y;
-    if (mode == kLatTrue) {
-      acc[0] += ri * ri;
-    } else if (mode == kLatInit64) {
-      const double di = invd ? invd[i] : 1.0;
-      r64[i] = ri;
-      acc[0] += ri * (di * ri);
-      acc[1] += ri * ri;
-      acc[2] += bi * bi;
-      acc[3] += bi * (di * bi);
-    } else {
-      const float rf = (float)(sc ? sc[i] * ri : ri);
-      r32[i] = rf;
-      const double rr = (double)rf * (double)rf;
-      acc[0] += rr;
-      acc[1] += ri * ri;
-      if (mode == kLatInit32) {
-        d32[i] = 0.0f;
-        acc[2] += bi * bi;
-        acc[3] += rr;
-      }
-    }
-  }
-};
 
 template <int DIM, int P, int KIND>
 __global__ FEMHIP_LATTICE_BOUNDS void k_lat_res(Lattice g, CoefDev c, Q2Tab t, int32_t n, int mode, int x_zero,
@@ -279,7 +161,7 @@ __global__ FEMHIP_LATTICE_BOUNDS void k_lat_res(Lattice g, CoefDev c, Q2Tab t, i
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) io.row((int)i, 0.0);
   } else {
     auto cell = lattice_cell<DIM, P, KIND>(c, t);
-    lattice_march<DIM, P>(g, cell, io, lattice_smem);
+    lattice_march<DIM, P>(g, lattice_block(g), cell, io, lattice_smem);
   }
   if (mode == kLatTrue) {
     double out[1] = {io.acc[0]};
@@ -288,58 +170,6 @@ __global__ FEMHIP_LATTICE_BOUNDS void k_lat_res(Lattice g, CoefDev c, Q2Tab t, i
     group_partials<4>(io.acc, part);
   }
 }
-
-// FP32 passes of the one-launch form: p, r, s are those of the scaled system S A S (sc = S in FP64,
-// null: S = I), d the increment in its variables.
-struct IoRf {
-  static constexpr int kKeep = 3;
-  struct Halo {
-    double s;
-    float r, q, p;
-  };
-  struct Raw : Halo {
-    float d;
-  };
-  BufRsrc r, q, sc, p, rn, qn, pn, d;   // q = S A S p; q and p have no bytes in the first pass: read as 0
-  bool jac;
-  double alpha64, beta64;
-  float alpha, beta;
-  double sum[kSums];
-  __device__ __forceinline__ bool ready() const { return true; }
-  __device__ __forceinline__ Raw fetch(uint32_t o) const {
-    return Raw{halo(o), buf_ld32(d, o)};
-  }
-  __device__ __forceinline__ Halo halo(uint32_t o) const {
-    return Halo{jac ? buf_ld64(sc, o) : 1.0, buf_ld32(r, o), buf_ld32(q, o), buf_ld32(p, o)};
-  }
-  __device__ __forceinline__ double halo_value(const Halo &w) const {
-    return w.s * (double)dir_value(beta, w.p, __builtin_fmaf(-alpha, w.q, w.r));
-  }
-  __device__ __forceinline__ double value(const Raw &w, uint32_t o, double (&keep)[kKeep]) {
-    const float ri = __builtin_fmaf(-alpha, w.q, w.r), pi = dir_value(beta, w.p, ri);
-    buf_st32(rn, o, ri);
-    buf_st32(pn, o, pi);
-    buf_st32(d, o, __builtin_fmaf(alpha, w.p, w.d));
-    const double rm = o < kNoPlane ? (double)ri : 0.0;   // 0 where a neighbour owns the node
-    sum[kSumNu] += rm * rm;
-    const double u = w.s * (double)pi;
-    keep[0] = u;
-    keep[1] = (double)ri;
-    keep[2] = w.s;
-    return u;
-  }
-  template <bool FULL>
-  __device__ __forceinline__ void out(uint32_t o, const double (&keep)[kKeep], double y) {
-    const double si = FULL ? keep[2] : jac ? buf_ld64(sc, o) : 1.0;
-    const double ri = FULL ? keep[1] : (double)buf_ld32(rn, o);
-    const float qi = (float)(si * y);
-    buf_st32(qn, o, qi);
-    const double ym = o < kNoPlane ? y : 0.0, qm = o < kNoPlane ? (double)qi : 0.0;
-    sum[kSumMu] += keep[0] * ym;
-    sum[kSumDelta] += ri * qm;
-    sum[kSumGamma] += qm * qm;
-  }
-};
 
 // A slot of the FP32 path: a CG pass, or one of a reliable update's two (state
 // ru): the slot that finds an update due folds the increment into the FP64
@@ -373,7 +203,7 @@ __global__ FEMHIP_LATTICE_BOUNDS void k_lat_rf(Lattice g, CoefDev c, Q2Tab t, in
     }
     IoRes io{x, b, nullptr, sc, nullptr, r.v[set], nullptr, kLatUpdate, {0.0, 0.0, 0.0, 0.0}, buf_of(x, b8)};
     auto cell = lattice_cell<DIM, P, KIND>(c, t);
-    lattice_march<DIM, P>(g, cell, io, lattice_smem);
+    lattice_march<DIM, P>(g, lattice_block(g), cell, io, lattice_smem);
     double out[2] = {io.acc[0], io.acc[1]};
     group_partials<2>(out, part_out);
     return;
@@ -430,7 +260,7 @@ __global__ FEMHIP_LATTICE_BOUNDS void k_lat_rf(Lattice g, CoefDev c, Q2Tab t, in
           buf_of(r.v[set ^ 1], b4), buf_of(q.v[set ^ 1], b4), buf_of(p.v[set ^ 1], b4), buf_of(d, b4), sc != nullptr,
           alpha, beta, (float)alpha, (float)beta, {0.0, 0.0, 0.0, 0.0, 0.0, 0.0}};
   auto cell = lattice_cell<DIM, P, KIND>(c, t);
-  lattice_march<DIM, P>(g, cell, io, lattice_smem);
+  lattice_march<DIM, P>(g, lattice_block(g), cell, io, lattice_smem);
   group_partials<kSums>(io.sum, part_out);
 }
 
@@ -509,7 +339,7 @@ __global__ FEMHIP_LATTICE_BOUNDS void k_lat_a(Lattice g, CoefDev c, Q2Tab t, int
            buf_of(p.v[par], cur.first ? 0 : bytes), buf_of(p.v[par ^ 1], bytes), buf_of(x, bytes), buf_of(q, bytes),
            invd != nullptr, false, gb, 0.0, 0.0, 0.0, 0.0};
   auto cell = lattice_cell<DIM, P, KIND>(c, t);
-  if (!lattice_march<DIM, P>(g, cell, io, lattice_smem)) io.ready();   // no cells: the decision all the same
+  if (!lattice_march<DIM, P>(g, lattice_block(g), cell, io, lattice_smem)) io.ready();   // no cells: the decision all the same
   if (io.done) {   // the last iteration: x += alpha p
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     const double *pold = p.v[par];
@@ -643,7 +473,7 @@ __global__ FEMHIP_LATTICE_BOUNDS void k_lat_rf_a(Lattice g, CoefDev c, Q2Tab t, 
   IoRfA io{buf_of(r, b4), buf_of(sc, sc ? 2 * b4 : 0), buf_of(pold, cur.first ? 0 : b4), buf_of(p.v[par ^ 1], b4),
            buf_of(d, b4), buf_of(q, b4), step.upd_d ? a : 0.0f, (float)step.beta, sc != nullptr, 0.0};
   auto cell = lattice_cell<DIM, P, KIND>(c, t);
-  lattice_march<DIM, P>(g, cell, io, lattice_smem);
+  lattice_march<DIM, P>(g, lattice_block(g), cell, io, lattice_smem);
   double out[1] = {io.pq};
   group_partials<1>(out, part);
 }
@@ -659,7 +489,7 @@ __global__ FEMHIP_LATTICE_BOUNDS void k_lat_rf_b(Lattice g, CoefDev c, Q2Tab t, 
   if (st.ru) {
     IoRes io{x, b, nullptr, sc, nullptr, r, nullptr, kLatUpdate, {0.0, 0.0, 0.0, 0.0}, buf_of(x, 8u * (uint32_t)n)};
     auto cell = lattice_cell<DIM, P, KIND>(c, t);
-    lattice_march<DIM, P>(g, cell, io, lattice_smem);
+    lattice_march<DIM, P>(g, lattice_block(g), cell, io, lattice_smem);
     double out[2] = {io.acc[0], io.acc[1]};
     group_partials<2>(out, part);
     return;

@@ -75,6 +75,22 @@ __device__ __forceinline__ void buf_st32(BufRsrc r, uint32_t o8, float v) {
   __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), r, (int)(o8 >> 1), 0, 0);
 }
 
+// The part of a lattice that logical workgroup lb reads, as a lattice of its
+// own planes: row0 is its first row (vectors of any length then keep 30-bit
+// byte offsets, as long as a chunk's planes do).
+__device__ __forceinline__ Lattice lattice_window(const Lattice &g, int dim, int p, int lb, int64_t &row0, int64_t &rows) {
+  Lattice w = g;
+  const int a = dim - 1, chunk = lb / g.tiles;
+  const int z0 = (int)((int64_t)g.E[a] * chunk / g.nch), z1 = (int)((int64_t)g.E[a] * (chunk + 1) / g.nch);
+  const int first = max(p * max(z0 - 1, 0) - g.o[a], 0), last = min(p * z1 - g.o[a], g.m[a] - 1);   // planes of the box
+  const int64_t plane = dim == 3 ? (int64_t)g.m[0] * g.m[1] : g.m[0];
+  w.o[a] = g.o[a] + first;
+  w.m[a] = max(last - first + 1, 0);
+  row0 = first * plane;
+  rows = w.m[a] * plane;
+  return w;
+}
+
 template <int DIM, int P, int NC = 1>
 struct LatticeShape {
   static constexpr int N1 = P + 1;
@@ -120,13 +136,12 @@ inline int lattice_halo(int TX, int TY) {
 // node, with all of what value() kept (FULL) or only its value, keep[0].
 // halo(o) and halo_value(raw): the value alone, of a node past the tile.
 template <int DIM, int P, class Cell, class Io>
-__device__ __forceinline__ bool lattice_march(const Lattice &g, Cell &cell, Io &io, double *lds) {
+__device__ __forceinline__ bool lattice_march(const Lattice &g, int lb, Cell &cell, Io &io, double *lds) {
   constexpr int NC = Cell::kComps;
   using S = LatticeShape<DIM, P, NC>;
   constexpr int N1 = S::N1, NPL = S::NPL, OWN = S::OWN, NX = S::NX;
   constexpr bool PIPE = S::PIPE;
   constexpr int AX = DIM - 1;
-  const int lb = lattice_block(g);
   if (lb >= g.tiles * g.nch) return false;   // the same for the whole workgroup
   const int tile = lb % g.tiles, chunk = lb / g.tiles;
   const int ti = tile % g.xt, tj = tile / g.xt;
@@ -786,7 +801,8 @@ struct LatticeOp {
   size_t lds = 0;                   // bytes of LDS a workgroup
   bool identity = false;            // lattice rows are the operator's rows
 };
-bool lattice_plan(const femhip_mesh_desc_t &mesh, int cus, LatticeOp &L);
+// cus > 0: chunks that fill that many CUs; otherwise of about `cells` cells a workgroup
+bool lattice_plan(const femhip_mesh_desc_t &mesh, int cus, LatticeOp &L, int max_threads = 0, int cells = 0);
 bool lattice_operator(femhip_operator &op);
 CoefDev lattice_coefficient(femhip_operator &op);
 Q2Tab lattice_q2_tab();

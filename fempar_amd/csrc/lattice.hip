@@ -64,8 +64,8 @@ __global__ void k_points_by_q(int64_t cells, int nq, const double *__restrict__ 
 }
 
 template <int DIM, int P, int NC = 1>
-void split(LatticeOp &L, int cus) {
-  constexpr int max_threads = lattice_threads(DIM, P, NC);
+void split(LatticeOp &L, int cus, int max_threads, int cells) {
+  if (max_threads <= 0) max_threads = lattice_threads(DIM, P, NC);
   Lattice &g = L.g;
   const int e0 = g.E[0], e1 = DIM == 3 ? g.E[1] : 1, ez = g.E[DIM - 1];
   // Tile: the least lanes over all tiles.  Neighbouring tiles both compute the
@@ -97,6 +97,12 @@ void split(LatticeOp &L, int cus) {
   // Chunks of the march: each repeats one layer, so few long ones repeat
   // little and many short ones fill the chip; the fewest layers in turn on one
   // CU wins.
+  if (cus <= 0) {
+    const int layers = std::max(2, std::min(ez, cells / std::max(1, g.TX * g.TY)));
+    g.nch = (ez + layers - 1) / layers;
+    L.grid = g.tiles * g.nch;
+    return;
+  }
   const int per_cu = std::max(1, std::min(256 * lattice_waves(DIM, P, NC) / L.threads, (int)(160 * 1024 / std::max<size_t>(1, L.lds))));
   const int64_t slots = (int64_t)per_cu * std::max(1, cus);
   double bestc = 1e300;
@@ -118,7 +124,7 @@ void split(LatticeOp &L, int cus) {
 
 // Box of the free nodes of a structured mesh and its split.  False where the
 // free nodes are no box or an index would not fit.
-bool lattice_plan(const femhip_mesh_desc_t &mesh, int cus, LatticeOp &L) {
+bool lattice_plan(const femhip_mesh_desc_t &mesh, int cus, LatticeOp &L, int max_threads, int cells) {
   const int dim = mesh.dim, p = mesh.order;
   L = LatticeOp{};
   L.dim = dim;
@@ -132,18 +138,18 @@ bool lattice_plan(const femhip_mesh_desc_t &mesh, int cus, LatticeOp &L) {
     const bool hi = mesh.dirichlet == FEMHIP_BC_ALL_BOUNDARY;
     g.o[d] = lo ? 1 : 0;
     const int64_t m = (int64_t)p * mesh.n[d] + 1 - (lo ? 1 : 0) - (hi ? 1 : 0);
-    if (m < 1 || m > kLatticeMaxRows) return false;
+    if (m < 1 || m > INT32_MAX) return false;
     g.m[d] = (int)m;
     g.E[d] = mesh.n[d] + (hi ? 0 : 1);
     rows *= m;
-    if (rows * L.ncomp > kLatticeMaxRows) return false;   // byte offsets of the vectors
+    if (rows * L.ncomp > INT32_MAX) return false;
   }
   g.stride = (int)rows;
-  if (dim == 2 && p == 1) split<2, 1>(L, cus);
-  else if (dim == 2) split<2, 2>(L, cus);
-  else if (p == 1 && L.ncomp == 3) split<3, 1, 3>(L, cus);
-  else if (p == 1) split<3, 1>(L, cus);
-  else split<3, 2>(L, cus);
+  if (dim == 2 && p == 1) split<2, 1>(L, cus, max_threads, cells);
+  else if (dim == 2) split<2, 2>(L, cus, max_threads, cells);
+  else if (p == 1 && L.ncomp == 3) split<3, 1, 3>(L, cus, max_threads, cells);
+  else if (p == 1) split<3, 1>(L, cus, max_threads, cells);
+  else split<3, 2>(L, cus, max_threads, cells);
   return true;
 }
 
@@ -158,7 +164,7 @@ bool lattice_operator(femhip_operator &op) {
   femhip_space &s = *op.space;
   if (op.tab_kind == 0 ? s.fe.ncomp != 1 : s.fe.ncomp != 3 || s.fe.dim != 3 || s.fe.order != 1) return false;
   auto L = std::make_shared<LatticeOp>();
-  if (!lattice_plan(s.mesh, op.ctx->num_cus, *L)) return false;
+  if (op.n > kLatticeMaxRows || !lattice_plan(s.mesh, op.ctx->num_cus, *L)) return false;   // byte offsets of the vectors
   int64_t rows = L->ncomp;
   for (int d = 0; d < s.mesh.dim; ++d) rows *= L->g.m[d];
   if (rows != op.n) return false;

@@ -1,0 +1,190 @@
+// lattice_io.h -- what a lattice march (lattice.h) reads and writes at the nodes
+// in the FP32-refined CG passes and in FP64 residuals, and the sums of a pass
+// (device code shared by cg.hip and batch.hip).
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include "cg_state.h"
+#include "lattice.h"
+
+namespace femhip {
+namespace {
+
+extern __shared__ double lattice_smem[];
+
+// Partial sums of workgroup lb of g: part[k * g + lb].
+template <int NV>
+__device__ __forceinline__ void group_partials(double (&v)[NV], double *part, int g, int lb) {
+  __shared__ double sm[NV][16];
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1)
+#pragma unroll
+    for (int k = 0; k < NV; ++k) v[k] += __shfl_down(v[k], off, 64);
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  if (lane == 0)
+#pragma unroll
+    for (int k = 0; k < NV; ++k) sm[k][w] = v[k];
+  __syncthreads();
+  if (threadIdx.x < NV) {
+    double s = 0.0;
+    for (int i = 0; i < nw; ++i) s += sm[threadIdx.x][i];
+    part[threadIdx.x * g + lb] = s;
+  }
+}
+// Sums of a launch's partials, in the same order in every workgroup: a wave
+// takes a whole sum.
+template <int NV>
+__device__ __forceinline__ void group_reduce(const double *part, int g, double (&v)[NV]) {
+  __shared__ double sm[NV];
+  const int lane = threadIdx.x & 63, nw = blockDim.x >> 6;
+  for (int k = threadIdx.x >> 6; k < NV; k += nw) {
+    double a = 0.0;
+    for (int b = lane; b < g; b += 64) a += part[k * g + b];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) a += __shfl_down(a, off, 64);
+    if (lane == 0) sm[k] = a;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < NV; ++k) v[k] = sm[k];
+}
+template <int NV>
+__device__ __forceinline__ void group_partials(double (&v)[NV], double *part) {
+  group_partials<NV>(v, part, (int)gridDim.x, (int)blockIdx.x);
+}
+
+// Sums of a pass.
+enum { kSumMu = 0, kSumDelta = 1, kSumGamma = 2, kSumNu = 3, kSumRr = 4, kSumPp = 5, kSums = 6 };
+
+// alpha and beta from the sums of the pass before; `lead` notes them in the next state
+__device__ __forceinline__ void pr_scalars(const double (&red)[kSums], bool lead, CgState &next, double &alpha,
+                                           double &beta) {
+  const double nu = red[kSumNu];
+  alpha = red[kSumMu] != 0.0 ? nu / red[kSumMu] : 0.0;   // cg.f90:195-199
+  const double pred = __builtin_fma(alpha, __builtin_fma(alpha, red[kSumGamma], -2.0 * red[kSumDelta]), nu);
+  beta = nu != 0.0 ? pred / nu : 0.0;
+  if (lead) {
+    next.alpha = alpha;
+    next.pap = red[kSumMu];
+    next.pp = red[kSumPp];
+  }
+}
+
+// The vectors that alternate between two sets: pass `par` reads set par.
+template <typename T>
+struct PairOf {
+  T *v[2];
+};
+
+// Residuals of x in FP64, r = b - A x, for what mode asks.
+enum { kLatInit64 = 0,   // r64; partials <r,z>, ||r||^2, ||b||^2, <b,Mb>
+       kLatInit32 = 1,   // r32 = S r, d = 0; partials <r32,r32>, ||r||^2, ||b||^2, <r32,r32>
+       kLatTrue = 2,     // partial ||r||^2 (reporting only)
+       kLatUpdate = 3 }; // r32 = S r; partials <r32,r32>, ||r||^2
+
+struct IoRes {
+  static constexpr int kKeep = 1;
+  struct Raw {
+    double x;
+  };
+  using Halo = Raw;
+  const double *__restrict__ x, *__restrict__ b, *__restrict__ invd;
+  const double *__restrict__ sc;
+  double *__restrict__ r64;
+  float *__restrict__ r32, *__restrict__ d32;
+  int mode;
+  double acc[4];
+  BufRsrc xb;
+  double scale = 1.0;        // S r = sc r, or scale r without sc
+  __device__ __forceinline__ bool ready() const { return true; }
+  __device__ __forceinline__ Raw fetch(uint32_t o) const { return Raw{buf_ld64(xb, o)}; }
+  __device__ __forceinline__ Halo halo(uint32_t o) const { return fetch(o); }
+  __device__ __forceinline__ double halo_value(const Halo &w) const { return w.x; }
+  __device__ __forceinline__ double value(const Raw &w, uint32_t, double (&)[kKeep]) const {
+    return w.x;
+  }
+  template <bool FULL>
+  __device__ __forceinline__ void out(uint32_t o, const double (&)[kKeep], double y) {
+    if (o < kNoPlane) row((int)(o >> 3), y);
+  }
+  __device__ __forceinline__ void row(int i, double y) {
+    const double bi = b[i], ri = bi - y;
+    if (mode == kLatTrue) {
+      acc[0] += ri * ri;
+    } else if (mode == kLatInit64) {
+      const double di = invd ? invd[i] : 1.0;
+      r64[i] = ri;
+      acc[0] += ri * (di * ri);
+      acc[1] += ri * ri;
+      acc[2] += bi * bi;
+      acc[3] += bi * (di * bi);
+    } else {
+      const float rf = (float)(sc ? sc[i] * ri : scale * ri);
+      r32[i] = rf;
+      const double rr = (double)rf * (double)rf;
+      acc[0] += rr;
+      acc[1] += ri * ri;
+      if (mode == kLatInit32) {
+        d32[i] = 0.0f;
+        acc[2] += bi * bi;
+        acc[3] += rr;
+      }
+    }
+  }
+};
+
+// FP32 passes of the one-launch form: p, r, s are those of the scaled system S A S (sc = S in FP64,
+// null: S = I), d the increment in its variables.
+struct IoRf {
+  static constexpr int kKeep = 3;
+  struct Halo {
+    double s;
+    float r, q, p;
+  };
+  struct Raw : Halo {
+    float d;
+  };
+  BufRsrc r, q, sc, p, rn, qn, pn, d;   // q = S A S p; q and p have no bytes in the first pass: read as 0
+  bool jac;
+  double alpha64, beta64;
+  float alpha, beta;
+  double sum[kSums];
+  __device__ __forceinline__ bool ready() const { return true; }
+  __device__ __forceinline__ Raw fetch(uint32_t o) const {
+    return Raw{halo(o), buf_ld32(d, o)};
+  }
+  __device__ __forceinline__ Halo halo(uint32_t o) const {
+    return Halo{jac ? buf_ld64(sc, o) : 1.0, buf_ld32(r, o), buf_ld32(q, o), buf_ld32(p, o)};
+  }
+  __device__ __forceinline__ double halo_value(const Halo &w) const {
+    return w.s * (double)dir_value(beta, w.p, __builtin_fmaf(-alpha, w.q, w.r));
+  }
+  __device__ __forceinline__ double value(const Raw &w, uint32_t o, double (&keep)[kKeep]) {
+    const float ri = __builtin_fmaf(-alpha, w.q, w.r), pi = dir_value(beta, w.p, ri);
+    buf_st32(rn, o, ri);
+    buf_st32(pn, o, pi);
+    buf_st32(d, o, __builtin_fmaf(alpha, w.p, w.d));
+    const double rm = o < kNoPlane ? (double)ri : 0.0;   // 0 where a neighbour owns the node
+    sum[kSumNu] += rm * rm;
+    const double u = w.s * (double)pi;
+    keep[0] = u;
+    keep[1] = (double)ri;
+    keep[2] = w.s;
+    return u;
+  }
+  template <bool FULL>
+  __device__ __forceinline__ void out(uint32_t o, const double (&keep)[kKeep], double y) {
+    const double si = FULL ? keep[2] : jac ? buf_ld64(sc, o) : 1.0;
+    const double ri = FULL ? keep[1] : (double)buf_ld32(rn, o);
+    const float qi = (float)(si * y);
+    buf_st32(qn, o, qi);
+    const double ym = o < kNoPlane ? y : 0.0, qm = o < kNoPlane ? (double)qi : 0.0;
+    sum[kSumMu] += keep[0] * ym;
+    sum[kSumDelta] += ri * qm;
+    sum[kSumGamma] += qm * qm;
+  }
+};
+
+}  // namespace
+}  // namespace femhip

@@ -71,3 +71,27 @@ def test_batch_autotune(batch):
     assert t in (256, 512, 1024)
     res = batch.solve()
     assert np.all(res["did_converge"] == 1)
+
+
+# the sizes on both sides of each step between the ways a problem is solved
+# (one wave, one workgroup of 256 or 1024 threads, passes over all problems),
+# one batch for the small ones alone and one for the passes alone
+@pytest.mark.parametrize("problems", [
+    [(2, n, 0.3 + 0.1 * n, 1.0) for n in (3, 22, 23, 43, 44, 129, 130, 257)] +
+    [(3, n, 5.0 - 0.1 * n, 2.0) for n in (4, 9, 10, 12, 13, 23, 24, 33)],
+    [(2, 5, 1.0, 1.0), (3, 5, 2.0, 1.0)],
+    [(3, 25, 2.0, 1.0), (2, 140, 0.5, 1.0)]], ids=["edges", "small", "passes"])
+def test_batch_paths_match_oracle(env, problems):
+    b = F.batch_t(env, problems, rtol=1e-8)
+    b.assemble()
+    res = b.solve()
+    assert np.all(res["did_converge"] == 1) and np.all(res["latency_us"] > 0)
+    for i, (dim, n, k, f0) in enumerate(problems):
+        irp, ja, val, rhs = _oracle(dim, n, k, f0)
+        x = b.get_solution(i)
+        r = rhs - O.spmv(irp, ja, val, x, False)
+        assert np.linalg.norm(r) <= 1.0001e-8 * np.linalg.norm(rhs), (dim, n)
+        assert abs(res["true_residual"][i] - np.linalg.norm(r)) <= 1e-6 * np.linalg.norm(rhs), (dim, n)
+        x_ref, _ = O.cg(irp, ja, val, rhs, False, precond="jacobi", rtol=1e-12, maxit=20000)
+        assert np.linalg.norm(x - x_ref) <= 1e-5 * np.linalg.norm(x_ref), (dim, n)
+    b.free()
