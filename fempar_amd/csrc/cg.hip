@@ -1214,6 +1214,7 @@ __global__ __launch_bounds__(kThreads) void k_true_res(SlicedDev m, const double
 }
 
 #include "cg_lattice.h"
+#include "cg_small.h"
 
 }  // namespace
 }  // namespace femhip
@@ -1236,6 +1237,7 @@ struct femhip_solver {
   CoefDev coef;
   Q2Tab q2tab{};
   LatticeKernels lk{};
+  SmallCg small;                 // one workgroup's iterations (cg_small.h)
   DevBuf<CgState> st;            // S[2]
   DevBuf<CgResult> res;
   int *h_flag = nullptr, *d_flag = nullptr;    // zero-pivot flag of the Jacobi setup (pinned, mapped)
@@ -1338,15 +1340,29 @@ bool fp32_integration() {
   return e && atoi(e) == 1;
 }
 
+// Fewest rows of an operator whose products are formed from the cells.  In FP64
+// the stored matrix is faster up to what one workgroup holds or streams in an
+// iteration (cg_small.h), us an iteration stored / from the cells: 2-D Q1 4.0 at
+// 3969 rows / 11; 2-D Q2 6.0 / 11.3 at 961, 13.2 / 11.1 at 3969; 3-D Q1 7.8 / 8.9
+// at 1728, 15 / 9.7 at 3375 (too large for one workgroup); 3-D Q2 15 / 23 at 729,
+// 26 / 22 at 1331; 3-D elasticity 8.0 / 12 at 300, 13.3 / 11.8 at 882.
+// FP32_REFINED: 15.3 / 15.9 at 225 rows, 13.7 / 13.2 at 961 (2-D Q1), and the
+// cells gain with size and order (36 / 27 at 1331 rows of 3-D Q2).
+int32_t lattice_min_rows(const femhip_solver &s) {
+  if (mixed(s)) return 257;
+  const RefFE &fe = s.op->space->fe;
+  if (fe.ncomp > 1) return 641;
+  if (fe.dim == 2) return fe.order == 1 ? 4097 : 3001;
+  return fe.order == 1 ? 2049 : 1025;
+}
+
 // Whether a solver forms its products from the cells: scalar Poisson and vector
-// Q1 elasticity on the uniform mesh (lattice_operator), in FP64 and FP32_REFINED.  FP32_STRICT
-// and the FP32 integration are defined by their stored FP32 matrix.  Up to 4096
-// rows an iteration is launch latency whichever product it takes (32^2 Q1: 14.6
-// us stored, 11.1 us from the cells), and the stored matrix stays.
-constexpr int32_t kLatticeMinRows = 4097;
+// Q1 elasticity on the uniform mesh (lattice_operator), in FP64 and FP32_REFINED.
+// FP32_STRICT and the FP32 integration are defined by their stored FP32 matrix.
 bool wants_lattice(femhip_solver &s) {
   if (s.op->structured) return true;   // has no other form
-  return s.op->n >= kLatticeMinRows && !strict(s) && !(mixed(s) && fp32_integration()) && lattice_operator(*s.op);
+  if (!s.op->space || strict(s) || (mixed(s) && fp32_integration())) return false;
+  return s.op->n >= lattice_min_rows(s) && lattice_operator(*s.op);
 }
 
 void drop_graphs(femhip_solver &s) {
@@ -1450,6 +1466,7 @@ void prepare(femhip_solver &s) {
   }
   s.lat = lat;
   if (lat) {
+    s.small = SmallCg{};
     prepare_lattice(s);
     return;
   }
@@ -1493,6 +1510,9 @@ void prepare(femhip_solver &s) {
     if (mx) {
       s.r32.alloc(n); s.p32.alloc(n); s.q32.alloc(n); s.d32.alloc(n);
     }
+    s.small = mx ? SmallCg{} : small_cg(op.sl, n);
+    if (s.small.fn)   // above the default of 64 KiB
+      FH_HIP(hipFuncSetAttribute((const void *)s.small.fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)s.small.lds));
     prepare_host_slots(s);
     s.prepared = true;
   }
@@ -1736,7 +1756,14 @@ void ensure_graph(femhip_solver &s, int size_idx, int slot) {
 // (mapped host memory), and the slot's event marks the chunk's completion
 void push_chunk(femhip_solver &s, int slot, int size_idx = 0) {
   hipStream_t st = s.ctx->stream;
-  if (!use_graph(s)) {
+  if (s.small.fn) {
+    Launcher L;
+    L.stream = st;
+    L.lds = s.small.lds;
+    L(s.small.fn, dim3(1), dim3((unsigned)s.small.threads), sliced_dev(*s.op), s.op->sl.v64.p, s.r.p, s.x.p, s.p.p,
+      s.prm.preconditioner == FEMHIP_PREC_JACOBI ? s.invd.p : nullptr, s.st.p, s.small.margin, kSmallChunk, s.hist.p,
+      s.res.p, s.d_res_map[slot]);
+  } else if (!use_graph(s)) {
     Launcher L;
     L.stream = st;
     enqueue_iterations(s, kChunkSizes[size_idx], L, s.d_res_map[slot]);
@@ -1770,13 +1797,14 @@ void iterate(femhip_solver &s, int maxit) {
   int64_t queued = 0;
   auto push = [&](int size_idx) {
     push_chunk(s, next_slot, size_idx);
-    q[(head + nq) & 1] = {next_slot, kChunkSizes[size_idx]};
+    const int size = s.small.fn ? kSmallChunk : kChunkSizes[size_idx];
+    q[(head + nq) & 1] = {next_slot, size};
     ++nq;
     next_slot ^= 1;
-    queued += kChunkSizes[size_idx];
+    queued += size;
   };
   push(0);
-  if (queued < maxit) push(0);
+  if (queued < maxit && !s.small.fn) push(0);
   double prev = 0.0;
   int prev_it = -1;
   while (nq > 0) {

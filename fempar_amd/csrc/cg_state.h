@@ -44,15 +44,14 @@ __device__ __forceinline__ double new_x(double x, float d, const double *sc, int
   return sc ? __builtin_fma(sc[i], (double)d, x) : x + (double)d;
 }
 
-// Stopping test (cg.f90:323-407) after the iteration whose <r,z>, ||r||^2 are
-// red[0], red[1]; `lead` (one thread of the launch) writes the next state, the
-// history and the result blocks.  Returns done, beta for the next direction.
-__device__ __forceinline__ bool cg_decide(const CgState &cur, const double (&red)[2], bool lead, CgState &next,
-                                          double *hist, CgResult *R, CgResult *Rh, double &beta_out) {
-  const int it = cur.iter + 1;
+// Stopping test (cg.f90:323-407) of iteration `it`, whose <r,z>, ||r||^2 are
+// red[0], red[1] and whose alpha and ||p||^2 are in cur: its estimate and
+// threshold; returns whether it converged.
+__device__ __forceinline__ bool cg_test(const CgState &cur, int it, const double (&red)[2], double rnorm, double &est,
+                                        double &rhs_test) {
   const int c = cur.crit;
-  const double rnorm = sqrt(red[1]);
-  double est = cur.est, rhs_test = cur.rhs_test;
+  est = cur.est;
+  rhs_test = cur.rhs_test;
   if (it == 1 && is_delta(c)) {
     est = cur.alpha * sqrt(cur.pp);
     if (is_delta_delta(c)) rhs_test = cur.rtol * est + cur.atol;
@@ -61,8 +60,20 @@ __device__ __forceinline__ bool cg_decide(const CgState &cur, const double (&red
   else if (is_delta(c)) {
     if (it != 1) est = cur.alpha * sqrt(cur.pp);
   } else est = cur.rnrm_m;
-  int conv = est <= rhs_test;
+  bool conv = est <= rhs_test;
   if (c >= FEMHIP_DELTA_RHS_AND_RES_RES && conv) conv = rnorm <= cur.rhs_extra;
+  return conv;
+}
+
+// The test after an iteration; `lead` (one thread of the launch) writes the
+// next state, the history and the result blocks.  Returns done, beta for the
+// next direction.
+__device__ __forceinline__ bool cg_decide(const CgState &cur, const double (&red)[2], bool lead, CgState &next,
+                                          double *hist, CgResult *R, CgResult *Rh, double &beta_out) {
+  const int it = cur.iter + 1;
+  const double rnorm = sqrt(red[1]);
+  double est, rhs_test;
+  const int conv = cg_test(cur, it, red, rnorm, est, rhs_test);
   const bool done = conv || it >= cur.maxit;
   double beta = 1.0 / cur.rz;
   beta = beta * red[0];
