@@ -803,6 +803,7 @@ struct LatticeOp {
 };
 // cus > 0: chunks that fill that many CUs; otherwise of about `cells` cells a workgroup
 bool lattice_plan(const femhip_mesh_desc_t &mesh, int cus, LatticeOp &L, int max_threads = 0, int cells = 0);
+bool lattice_rows(const femhip_space &s, LatticeOp &L, DevBuf<int32_t> &perm);
 bool lattice_operator(femhip_operator &op);
 CoefDev lattice_coefficient(femhip_operator &op);
 Q2Tab lattice_q2_tab();

@@ -153,6 +153,37 @@ bool lattice_plan(const femhip_mesh_desc_t &mesh, int cus, LatticeOp &L, int max
   return true;
 }
 
+// The lattice row of every row of a space, perm, if each (cell, local DOF) of
+// its lists is the row its node has in the box (whoever numbered them).
+bool lattice_rows(const femhip_space &s, LatticeOp &L, DevBuf<int32_t> &perm) {
+  const int32_t n = s.n_free;
+  int64_t rows = L.ncomp;
+  for (int d = 0; d < s.mesh.dim; ++d) rows *= L.g.m[d];
+  if (rows != n) return false;
+  hipStream_t st = s.ctx->stream;
+  const FaceTab t = face_tab(s);
+  DevBuf<int> bad;
+  bad.alloc(1);
+  perm.alloc((size_t)n);
+  FH_HIP(hipMemsetAsync(bad.p, 0, sizeof(int), st));
+  hipLaunchKernelGGL(k_lattice_perm, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, L.g, t, n, s.d_rep.p, perm.p,
+                     bad.p);
+  FH_HIP(hipGetLastError());
+  int f = 1;
+  FH_HIP(hipMemcpyAsync(&f, bad.p, sizeof(int), hipMemcpyDeviceToHost, st));
+  FH_HIP(hipStreamSynchronize(st));
+  if (f & 1) return false;
+  L.identity = !(f & 2);
+  FH_HIP(hipMemsetAsync(bad.p, 0, sizeof(int), st));
+  const int64_t cnt = s.ncells * s.fe.nd;
+  hipLaunchKernelGGL(k_lattice_check, dim3((unsigned)((cnt + 255) / 256)), dim3(256), 0, st, L.g, t, s.ncells, n,
+                     s.d_dofs.p, perm.p, bad.p);
+  FH_HIP(hipGetLastError());
+  FH_HIP(hipMemcpyAsync(&f, bad.p, sizeof(int), hipMemcpyDeviceToHost, st));
+  FH_HIP(hipStreamSynchronize(st));
+  return !f;
+}
+
 // The lattice form of a scalar Poisson or a vector Q1 elasticity operator on the
 // uniform mesh (checked once against the space's DOF lists, whoever numbered
 // them): op.lat, op.lat_perm.  Cells with their own map keep the stored matrix.
@@ -165,38 +196,9 @@ bool lattice_operator(femhip_operator &op) {
   if (op.tab_kind == 0 ? s.fe.ncomp != 1 : s.fe.ncomp != 3 || s.fe.dim != 3 || s.fe.order != 1) return false;
   auto L = std::make_shared<LatticeOp>();
   if (op.n > kLatticeMaxRows || !lattice_plan(s.mesh, op.ctx->num_cus, *L)) return false;   // byte offsets of the vectors
-  int64_t rows = L->ncomp;
-  for (int d = 0; d < s.mesh.dim; ++d) rows *= L->g.m[d];
-  if (rows != op.n) return false;
-  hipStream_t st = op.ctx->stream;
-  const FaceTab t = face_tab(s);
-  DevBuf<int> bad;
-  bad.alloc(1);
-  DevBuf<int32_t> perm;
-  perm.alloc((size_t)op.n);
-  FH_HIP(hipMemsetAsync(bad.p, 0, sizeof(int), st));
-  hipLaunchKernelGGL(k_lattice_perm, dim3((unsigned)((op.n + 255) / 256)), dim3(256), 0, st, L->g, t, op.n, s.d_rep.p,
-                     perm.p, bad.p);
-  FH_HIP(hipGetLastError());
-  int f = 1;
-  FH_HIP(hipMemcpyAsync(&f, bad.p, sizeof(int), hipMemcpyDeviceToHost, st));
-  FH_HIP(hipStreamSynchronize(st));
-  if (f & 1) return false;
-  L->identity = !(f & 2);
-  FH_HIP(hipMemsetAsync(bad.p, 0, sizeof(int), st));
-  const int64_t cnt = s.ncells * s.fe.nd;
-  hipLaunchKernelGGL(k_lattice_check, dim3((unsigned)((cnt + 255) / 256)), dim3(256), 0, st, L->g, t, s.ncells, op.n,
-                     s.d_dofs.p, perm.p, bad.p);
-  FH_HIP(hipGetLastError());
-  FH_HIP(hipMemcpyAsync(&f, bad.p, sizeof(int), hipMemcpyDeviceToHost, st));
-  FH_HIP(hipStreamSynchronize(st));
-  if (f) return false;
-  if (!L->identity) {   // the check's buffer is the map
-    op.lat_perm.p = perm.p;
-    op.lat_perm.n = perm.n;
-    op.lat_perm.owned = perm.owned;
-    perm.p = nullptr;
-  }
+  const bool rows = lattice_rows(s, *L, op.lat_perm);
+  if (!rows || L->identity) op.lat_perm.release();
+  if (!rows) return false;
   op.lat = L;
   op.lat_state = 1;
   return true;

@@ -20,11 +20,18 @@
 // val; a diagonal block's symmetric-storage view is taken row by row when the
 // host asks), rows of a block ordered field by field; one vector of all
 // blocks' rows concatenated in block order for the RHS and the solver.
-// Kernels (one wavefront per block row): the pattern (the columns of the
-// coupled fields in the cells around the row's vef, sorted in LDS), the
-// assembly (the row's entries summed over those cells in ascending order from
-// element tables, no atomics), and a CSR SpMV that adds the blocks of a block
-// row in block order.
+// Kernels: the pattern, one wavefront per block row (the columns of the coupled
+// fields in the cells around the row's vef, sorted in LDS); the assembly (every
+// entry summed over the cells it lies in, in ascending order, from element
+// tables, no atomics); a CSR SpMV that adds the blocks of a block row in block
+// order.
+//
+// The coefficients are constants and the mesh is uniform, so every cell has the
+// same element tables: where the fields' free nodes are boxes of the grid
+// (every numbering of the structured generator; checked on the device), the CG
+// forms its products from those tables in the boxes' order, and the assembly
+// finds an entry's cells from the two nodes' grid positions.  Numberings that
+// are no box lattice keep the row-wise assembly and the CSR product.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -34,6 +41,9 @@
 #include <vector>
 
 #include "femhip_internal.h"
+#include "cg_state.h"
+#include "lattice.h"
+#include "lattice_io.h"
 
 using namespace femhip;
 
@@ -51,6 +61,7 @@ struct ColSet {
   int32_t nd[kMaxFields];
   int32_t off[kMaxFields];
   int32_t tab[kMaxFields];
+  int32_t fld[kMaxFields], rows[kMaxFields];   // which field, its free rows
 };
 
 __device__ __forceinline__ int col_candidate(const ColSet &cs, int tot, int i, int &b, int &g, int &j) {
@@ -259,8 +270,8 @@ __global__ __launch_bounds__(kSpmvThreads) void k_block_spmv(int32_t n, const in
                                                              const int32_t *__restrict__ col,
                                                              const double *__restrict__ val,
                                                              const double *__restrict__ x, double *__restrict__ y,
-                                                             int add, const double *__restrict__ stop) {
-  if (stop && *stop != 0.0) return;   // the solve has ended (see k_cg_test)
+                                                             int add, const CgState *stop) {
+  if (stop && stop->done) return;   // the solve has ended
   const int sub = threadIdx.x % LANES;
   const int64_t r = ((int64_t)blockIdx.x * kSpmvThreads + threadIdx.x) / LANES;
   double acc = 0.0;
@@ -290,98 +301,439 @@ __global__ __launch_bounds__(kSpmvThreads) void k_block_spmv(int32_t n, const in
 // 16 lanes a row: 8 take the same time, 32 are 20 % slower (48^3 Q2 + Q1 block CG)
 constexpr int kSpmvLanes = 16;
 
-// dot products in a fixed order: kDotBlocks partial sums (grid-strided rows,
-// block tree), then one block sums them in order
-constexpr int kDotBlocks = 256, kDotThreads = 256;
-__device__ __forceinline__ double block_sum(double v) {
-  __shared__ double red[kDotThreads];
-  red[threadIdx.x] = v;
-  __syncthreads();
-  for (int s = kDotThreads / 2; s > 0; s >>= 1) {
-    if ((int)threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
-    __syncthreads();
+// ------------------------------------------------- boxes of the fields ---
+
+// A field's free nodes: the box [o, o + m) of the grid of its order, its rows
+// in the block vectors (base) and in its block (off), and the box position of
+// each of its rows.
+struct MfField {
+  int p, nd, rows, off;
+  int o[3], m[3];
+  int64_t base;
+  const int32_t *perm;
+};
+
+// The nodes of one field whose positions along y and z have the same parities:
+// the cells around them and their local nodes there are the same, so the
+// element tables are read by scalar loads.  A thread takes the p nodes from one
+// vertex of the cells to the next along x.
+struct MfSeg {
+  int f, rows, blocks, pad;      // rows: threads; blocks: workgroups on each XCD
+  int aligned[3], first[3], cnt[3];
+};
+
+struct MfPlan {
+  int nf, dim, nseg, items;      // items: workgroups in all
+  int n[3], pad;
+  MfField fld[kMaxFields];
+  MfSeg seg[kMaxFields * 4];
+  int tab[kMaxFields][kMaxFields];   // element table of (row, column) fields, -1: not coupled
+};
+
+constexpr int kMfThreads = 256;
+
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef double f64x2 __attribute__((ext_vector_type(2)));
+
+// A thread's nodes: cell i along x (its first node is the cell's vertex), grid
+// positions gy, gz.
+struct MfAt {
+  int i, g[3];
+};
+
+// y[a] += sum over the cells around node a of the element rows times field g's
+// values.  The values of 2 PG + 1 nodes along x serve both nodes of a thread
+// and both cells of the vertex, in pairs (16 B a lane, so a wave reads whole
+// lines); O: field g's box begins at node O, which decides the pairs that never
+// begin before it.  Nodes outside the box and cells outside the mesh count 0:
+// along y and z by an offset out of the vector's range, along x by selects.
+template <int DIM, int PF, int PG, int O>
+__device__ __forceinline__ void mf_rows(const MfPlan &P, const MfField &G, const MfSeg &s, const MfAt &at,
+                                        const double *__restrict__ tab, BufRsrc x, double (&y)[PF]) {
+  constexpr int N1 = PG + 1, NZ = DIM == 3 ? N1 : 1, ND = N1 * N1 * NZ, F1 = PF + 1, NX = 2 * PG + 1;
+  const uint32_t sy = 8u * (uint32_t)G.m[0], sz = sy * (uint32_t)G.m[1];
+  const bool lower = at.i >= 1, upper = at.i < P.n[0];   // the cells before and after the vertex
+  bool in[NX];
+#pragma unroll
+  for (int j = 0; j < NX; ++j) {
+    const int v = PG * at.i - PG + j - G.o[0];
+    in[j] = v >= 0 && v < G.m[0];
   }
-  return red[0];
+  auto xoff = [&](int j) { return 8u * (uint32_t)max(PG * at.i - PG + j - G.o[0], 0); };
+  auto axis = [&](int d, int e, uint32_t stride, uint32_t (&off)[N1]) {   // local node; byte offsets along d
+    const int c = s.aligned[d] ? at.g[d] / PF - 1 + e : at.g[d] / PF;
+    const bool cell = c >= 0 && c < P.n[d];
+#pragma unroll
+    for (int j = 0; j < N1; ++j) {
+      const int v = PG * c + j - G.o[d];
+      off[j] = cell && v >= 0 && v < G.m[d] ? (uint32_t)v * stride : kNoPlane;
+    }
+    return s.aligned[d] ? (e ? 0 : PF) : 1;
+  };
+  const uint32_t x0 = xoff(0), x1 = xoff(1), x2 = xoff(2), x3 = PG == 2 ? xoff(3) : 0, x4 = PG == 2 ? xoff(4) : 0;
+  auto pair = [&](uint32_t o, double &a, double &b) {
+    const f64x2 v = __builtin_bit_cast(f64x2, __builtin_amdgcn_raw_buffer_load_b128(x, (int)o, 0, 0));
+    a = v.x;
+    b = v.y;
+  };
+  for (int ez = 0; ez < (DIM == 3 && s.aligned[2] ? 2 : 1); ++ez) {
+    uint32_t oz[N1];
+    const int lz = DIM == 3 ? axis(2, ez, sz, oz) : 0;
+    for (int ey = 0; ey < (s.aligned[1] ? 2 : 1); ++ey) {
+      uint32_t oy[N1];
+      const int ly = axis(1, ey, sy, oy);
+      const double *row = tab + (lz * F1 + ly) * F1 * ND;
+#pragma unroll
+      for (int k = 0; k < NZ; ++k) {
+        double v[N1][NX];
+#pragma unroll
+        for (int j = 0; j < N1; ++j) {
+          const uint32_t o = (DIM == 3 ? oz[k] : 0u) + oy[j];
+          if constexpr (PG == 1) {
+            v[j][0] = buf_ld64(x, o + x0);
+            v[j][1] = buf_ld64(x, o + x1);
+            v[j][2] = buf_ld64(x, o + x2);
+          } else if constexpr (O == 0) {
+            pair(o + x0, v[j][0], v[j][1]);
+            pair(o + x2, v[j][2], v[j][3]);
+            v[j][4] = buf_ld64(x, o + x4);
+          } else {
+            v[j][0] = buf_ld64(x, o + x0);
+            pair(o + x1, v[j][1], v[j][2]);
+            pair(o + x3, v[j][3], v[j][4]);
+          }
+        }
+#pragma unroll
+        for (int j = 0; j < N1; ++j) {
+          const double *c = row + (k * N1 + j) * N1;   // entries of row (lz, ly, 0); those of (.., a): c + a ND
+          double w[NX];
+#pragma unroll
+          for (int i = 0; i < NX; ++i) w[i] = in[i] ? v[j][i] : 0.0;
+          const double wl = lower ? w[PG] : 0.0, wu = upper ? w[PG] : 0.0;
+#pragma unroll
+          for (int i = 0; i < PG; ++i) y[0] = __builtin_fma(c[PF * ND + i], w[i], y[0]);
+          y[0] = __builtin_fma(c[PF * ND + PG], wl, y[0]);
+#pragma unroll
+          for (int a = 0; a < PF; ++a) {
+            y[a] = __builtin_fma(c[a * ND], wu, y[a]);
+#pragma unroll
+            for (int i = 1; i < N1; ++i) y[a] = __builtin_fma(c[a * ND + i], w[PG + i], y[a]);
+          }
+        }
+      }
+    }
+  }
 }
-__global__ __launch_bounds__(kDotThreads) void k_dot_part(int64_t n, const double *__restrict__ a,
-                                                          const double *__restrict__ b, double *__restrict__ part,
-                                                          const double *__restrict__ stop) {
-  if (stop && *stop != 0.0) return;
+
+// The nodes of a workgroup's thread: false past the segment's part on this XCD.
+__device__ __forceinline__ bool mf_thread_nodes(const MfPlan &P, int item, int &si, MfAt &at, int64_t &line) {
+  const int xcd = item & 7;
+  int j = item >> 3;
+  si = 0;
+  while (si < P.nseg - 1 && j >= P.seg[si].blocks) j -= P.seg[si++].blocks;
+  const MfSeg &s = P.seg[si];
+  const MfField &F = P.fld[s.f];
+  const int lo = (int)((int64_t)s.rows * xcd / 8), hi = (int)((int64_t)s.rows * (xcd + 1) / 8);
+  const int t = lo + j * kMfThreads + (int)threadIdx.x;
+  const bool on = t < hi;
+  int k = on ? t : lo < s.rows ? lo : 0;
+  at.i = s.first[0] + k % s.cnt[0];
+  at.g[0] = F.p * at.i;
+  k /= s.cnt[0];
+  const int b = s.first[1] + F.p * (k % s.cnt[1]), c = s.first[2] + F.p * (k / s.cnt[1]);
+  at.g[1] = b + F.o[1];
+  at.g[2] = c + F.o[2];
+  line = F.base + (int64_t)F.m[0] * (b + (int64_t)F.m[1] * c) - F.o[0] + at.g[0];   // row of the first node, if it has one
+  return on;
+}
+
+template <int DIM, int PF>
+__device__ __forceinline__ double mf_item(const MfPlan &P, const MfSeg &s, const MfAt &at, bool on, int64_t line,
+                                          const double *__restrict__ tab, const double *__restrict__ x,
+                                          double *__restrict__ q) {
+  double y[PF];
+#pragma unroll
+  for (int a = 0; a < PF; ++a) y[a] = 0.0;
+  for (int g = 0; g < P.nf; ++g) {
+    const MfField &G = P.fld[g];
+    const int t = P.tab[s.f][g];
+    if (t < 0 || G.rows == 0) continue;
+    const BufRsrc xg = buf_of(x + G.base, 8u * (uint32_t)G.rows);
+    if (G.p == 1) mf_rows<DIM, PF, 1, 0>(P, G, s, at, tab + t, xg, y);
+    else if (G.o[0] == 0) mf_rows<DIM, PF, 2, 0>(P, G, s, at, tab + t, xg, y);
+    else mf_rows<DIM, PF, 2, 1>(P, G, s, at, tab + t, xg, y);
+  }
+  const MfField &F = P.fld[s.f];
   double acc = 0.0;
-  for (int64_t i = (int64_t)blockIdx.x * kDotThreads + threadIdx.x; i < n; i += (int64_t)kDotBlocks * kDotThreads)
-    acc += a[i] * b[i];
-  const double s = block_sum(acc);
-  if (threadIdx.x == 0) part[blockIdx.x] = s;
-}
-__global__ __launch_bounds__(kDotThreads) void k_dot_final(const double *__restrict__ part, double *__restrict__ out,
-                                                           const double *__restrict__ stop) {
-  if (stop && *stop != 0.0) return;
-  const double s = block_sum(part[threadIdx.x]);
-  if (threadIdx.x == 0) *out = s;
-}
-
-// Device scalars of the block CG: kRz = <r,z> of the current direction,
-// kQp = <q,p>, kRzNew = the next <r,z>, kRr = ||r||^2; the stopping test
-// (k_cg_test) keeps the iteration count, the estimate ||r||, whether it
-// converged and kDone, which every kernel of an iteration reads at entry, so
-// iterations queued after the end return at once.
-enum { kRz = 0, kQp = 1, kRzNew = 2, kRr = 3, kDot = 4, kIt = 5, kEst = 6, kConv = 7, kDone = 8, kScalars = 9 };
-
-// it += 1 ; est = ||r|| ; converged = est <= rhs_test (cg.f90:323-407, RES_RES
-// and RES_RHS) ; done = converged or it >= maxit
-__global__ void k_cg_test(double *__restrict__ sc, double rhs_test, int maxit) {
-  if (sc[kDone] != 0.0) return;
-  const double it = sc[kIt] + 1.0;
-  const double est = sqrt(sc[kRr]);
-  const bool conv = est <= rhs_test;
-  sc[kIt] = it;
-  sc[kEst] = est;
-  sc[kConv] = conv ? 1.0 : 0.0;
-  sc[kDone] = (conv || it >= (double)maxit) ? 1.0 : 0.0;
-}
-// a new solve: no iteration made, not done
-__global__ void k_cg_reset(double *__restrict__ sc) {
-  sc[kIt] = 0.0;
-  sc[kEst] = 0.0;
-  sc[kConv] = 0.0;
-  sc[kDone] = 0.0;
+#pragma unroll
+  for (int a = 0; a < PF; ++a) {
+    const int v = at.g[0] + a - F.o[0];
+    if (on && v >= 0 && v < F.m[0]) {
+      q[line + a] = y[a];
+      acc += y[a] * x[line + a];
+    }
+  }
+  return acc;
 }
 
-// alpha = <r,z> / <q,p> (0 when <q,p> = 0, cg.f90:195-199); x += alpha p, r -= alpha q
-__global__ void k_cg_xr(int64_t n, const double *__restrict__ sc, double *__restrict__ x,
-                        const double *__restrict__ p, double *__restrict__ r, const double *__restrict__ q) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n || sc[kDone] != 0.0) return;
-  const double qp = sc[kQp];
-  const double alpha = qp != 0.0 ? sc[kRz] / qp : 0.0;
-  x[i] = x[i] + alpha * p[i];
-  r[i] = r[i] + (-alpha) * q[i];
+// q = A x from the element tables; partials <q, x> (part).  A workgroup takes 256
+// threads' nodes of one segment; each XCD a contiguous eighth of every segment.
+// 9 (y, z) lines of a cell, one plane of them in flight, all but the first read
+// from the L1 and L2; the element entries are scalar operands.  2 x 27 flops for
+// each of a node's 1 to 8 cells, but 8 B a row from memory instead of 12 B an
+// entry.  32^3 cells of Q2 and Q1 fields: 48 us for the four blocks' CSR rows, 33
+// us with a node a thread (loads of every other value: half of each line), 15 us
+// so.
+template <int DIM>
+__global__ __launch_bounds__(kMfThreads) void k_mf_product(const MfPlan *__restrict__ plan,
+                                                           const double *__restrict__ tab,
+                                                           const double *__restrict__ x, double *__restrict__ q,
+                                                           const CgState *S, double *part) {
+  if (S && S->done) return;
+  const MfPlan &P = *plan;
+  double acc[1] = {0.0};
+  for (int item = blockIdx.x; item < P.items; item += gridDim.x) {
+    int si;
+    MfAt at;
+    int64_t line;
+    const bool on = mf_thread_nodes(P, item, si, at, line);
+    const MfSeg &s = P.seg[si];
+    acc[0] += P.fld[s.f].p == 2 ? mf_item<DIM, 2>(P, s, at, on, line, tab, x, q)
+                                : mf_item<DIM, 1>(P, s, at, on, line, tab, x, q);
+  }
+  if (part) group_partials<1>(acc, part);
 }
-// z = invd o r (identity: z = r); p = beta p + z as scal then daxpy
-__global__ void k_cg_z(int64_t n, const double *__restrict__ invd, const double *__restrict__ r,
-                       double *__restrict__ z, const double *__restrict__ stop) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n || (stop && *stop != 0.0)) return;
-  z[i] = invd ? invd[i] * r[i] : r[i];
+
+// 1 / diagonal in the boxes' order, a row's cells in ascending order as in the
+// assembly; a zero pivot raises the flag
+__global__ __launch_bounds__(kMfThreads) void k_mf_invdiag(const MfPlan *__restrict__ plan,
+                                                           const double *__restrict__ tab, double *__restrict__ invd,
+                                                           int *__restrict__ bad) {
+  const MfPlan &P = *plan;
+  for (int item = blockIdx.x; item < P.items; item += gridDim.x) {
+    int si;
+    MfAt at;
+    int64_t line;
+    if (!mf_thread_nodes(P, item, si, at, line)) continue;
+    const MfSeg &s = P.seg[si];
+    const MfField &F = P.fld[s.f];
+    for (int a = 0; a < F.p; ++a) {
+      const int g[3] = {at.g[0] + a, at.g[1], at.g[2]};
+      if (g[0] < F.o[0] || g[0] >= F.o[0] + F.m[0]) continue;
+      double d = 0.0;
+      for (int b = 0; b < (1 << P.dim); ++b) {
+        int l = 0, stride = 1;
+        bool in = true;
+        for (int k = 0; k < P.dim; ++k) {
+          const int e = (b >> k) & 1, odd = g[k] % F.p;
+          const int c = odd ? g[k] / F.p : g[k] / F.p - 1 + e;
+          in = in && !(odd && e) && c >= 0 && c < P.n[k];
+          l += stride * (odd ? odd : e ? 0 : F.p);
+          stride *= F.p + 1;
+        }
+        if (in) d += tab[P.tab[s.f][s.f] + l * F.nd + l];
+      }
+      if (d == 0.0) atomicOr(bad, 1);
+      invd[line + a] = 1.0 / d;
+    }
+  }
 }
-// beta = (1 / <r,z>_old) <r,z>_new (cg.f90's order); p = beta p + z
-__global__ void k_cg_p(int64_t n, const double *__restrict__ sc, const double *__restrict__ z,
-                       double *__restrict__ p) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n || sc[kDone] != 0.0) return;
-  const double beta = (1.0 / sc[kRz]) * sc[kRzNew];
-  double v = beta * p[i];
-  p[i] = v + 1.0 * z[i];
+
+// A field's part of a block vector between the rows' and the box's order
+__global__ void k_mf_to_box(int32_t n, const int32_t *__restrict__ perm, const double *__restrict__ from,
+                            double *__restrict__ to) {
+  const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) to[perm[i]] = from[i];
 }
-// the new <r,z> becomes the current one (after every k_cg_p block read both)
-__global__ void k_cg_shift(double *__restrict__ sc) {
-  if (sc[kDone] == 0.0) sc[kRz] = sc[kRzNew];
+__global__ void k_mf_from_box(int32_t n, const int32_t *__restrict__ perm, const double *__restrict__ from,
+                              double *__restrict__ to) {
+  const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) to[i] = from[perm[i]];
 }
-// b - A x0 into r
-__global__ void k_sub(int64_t n, const double *__restrict__ b, double *__restrict__ r) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) r[i] = b[i] - r[i];
+
+// Values of block rows off .. off + rows of field f, kSpmvLanes lanes a row: an
+// entry's cells are those that hold both its nodes, at most two a direction,
+// found from their grid positions; the element entries are summed in ascending
+// order of the cells.  (One wavefront a row that searched each element entry's
+// column in the row took 2.5 ms for 32^3 cells of Q2 and Q1 fields, 0.5 ms here.)
+__global__ __launch_bounds__(256) void k_mf_assemble(const MfPlan *__restrict__ plan, int f, ColSet cs,
+                                                     const int32_t *__restrict__ rowptr,
+                                                     const int32_t *__restrict__ col,
+                                                     const double *__restrict__ tab, double *__restrict__ val) {
+  constexpr int LANES = 16;
+  const MfPlan &P = *plan;
+  const MfField &F = P.fld[f];
+  const int r = (int)(((int64_t)blockIdx.x * 256 + threadIdx.x) / LANES), sub = threadIdx.x % LANES;
+  if (r >= F.rows) return;
+  const int dim = P.dim;
+  auto grid = [&](const MfField &A, int row, int (&gi)[3]) {
+    int v = A.perm[row];
+    gi[0] = v % A.m[0] + A.o[0];
+    v /= A.m[0];
+    gi[1] = v % A.m[1] + A.o[1];
+    gi[2] = v / A.m[1] + A.o[2];
+  };
+  int gi[3];
+  grid(F, r, gi);
+  const int e1 = rowptr[F.off + r + 1];
+  for (int e = rowptr[F.off + r] + sub; e < e1; e += LANES) {
+    const int c = col[e];
+    int k = 0;   // the column's field: the last whose first row is not above it
+    for (int j = 1; j < cs.ng; ++j)
+      if (c >= cs.off[j] && cs.off[j] >= cs.off[k] && cs.rows[j] > 0) k = j;
+    const MfField &G = P.fld[cs.fld[k]];
+    int gj[3], c0[3], c1[3];
+    grid(G, c - cs.off[k], gj);
+    for (int d = 0; d < 3; ++d) {   // cells that hold both nodes along d
+      c0[d] = c1[d] = 0;
+      if (d < dim) {
+        c0[d] = max(max((gi[d] + F.p - 1) / F.p, (gj[d] + G.p - 1) / G.p) - 1, 0);
+        c1[d] = min(min(gi[d] / F.p, gj[d] / G.p), P.n[d] - 1);
+      }
+    }
+    double s = 0.0;
+    for (int z = c0[2]; z <= c1[2]; ++z)
+      for (int y = c0[1]; y <= c1[1]; ++y)
+        for (int x = c0[0]; x <= c1[0]; ++x) {
+          int l = gi[0] - F.p * x + (F.p + 1) * (gi[1] - F.p * y), m = gj[0] - G.p * x + (G.p + 1) * (gj[1] - G.p * y);
+          if (dim == 3) {
+            l += (F.p + 1) * (F.p + 1) * (gi[2] - F.p * z);
+            m += (G.p + 1) * (G.p + 1) * (gj[2] - G.p * z);
+          }
+          s += tab[cs.tab[k] + l * G.nd + m];
+        }
+    val[e] = s;
+  }
 }
+
+// --------------------------------------------------------------- block CG ---
+//
+// cg.f90:101-238 in three launches an iteration: the product with <q,p>; x, r
+// and <r,z>, ||r||^2; the stopping test, beta and p.  Scalars as in cg.hip: each
+// launch reduces the partial sums of the one before, the state alternates by
+// parity, launches after the end return at entry.  (One launch for each scalar
+// and vector operation took 89 of 137 us an iteration with 32^3 cells.)
+
+constexpr int kMfVecBlocks = 512;
+
+// partials <q, p> of a product that has none
+__global__ __launch_bounds__(kMfThreads) void k_mf_dot(int64_t n, const double *__restrict__ a,
+                                                       const double *__restrict__ b, const CgState *S, double *part) {
+  if (S && S->done) return;
+  double acc[1] = {0.0};
+  for (int64_t i = (int64_t)blockIdx.x * kMfThreads + threadIdx.x; i < n; i += (int64_t)gridDim.x * kMfThreads)
+    acc[0] += a[i] * b[i];
+  group_partials<1>(acc, part);
+}
+
+// r = b - q; p = z = M r; partials <r,z>, ||r||^2, ||b||^2
+__global__ __launch_bounds__(kMfThreads) void k_mf_start(int64_t n, const double *__restrict__ b,
+                                                         const double *__restrict__ q,
+                                                         const double *__restrict__ invd, double *__restrict__ r,
+                                                         double *__restrict__ p, double *part) {
+  double acc[3] = {0.0, 0.0, 0.0};
+  for (int64_t i = (int64_t)blockIdx.x * kMfThreads + threadIdx.x; i < n; i += (int64_t)gridDim.x * kMfThreads) {
+    const double bi = b[i], ri = bi - q[i], zi = invd ? invd[i] * ri : ri;
+    r[i] = ri;
+    p[i] = zi;
+    acc[0] += ri * zi;
+    acc[1] += ri * ri;
+    acc[2] += bi * bi;
+  }
+  group_partials<3>(acc, part);
+}
+
+// first state (RES_RES or RES_RHS, cg.f90:279-321); a zero pivot ends the solve
+__global__ __launch_bounds__(kMfThreads) void k_mf_begin(const double *part, int groups, double rtol, double atol,
+                                                         int crit, int maxit, const int *bad, CgState *S,
+                                                         CgResult *R) {
+  double v[3];
+  group_reduce<3>(part, groups, v);
+  if (threadIdx.x != 0) return;
+  CgState s{};
+  s.rtol = rtol;
+  s.atol = atol;
+  s.crit = crit;
+  s.maxit = maxit;
+  s.rz = v[0];
+  s.rnrm_m = sqrt(v[0]);
+  s.r0norm = s.rnorm = sqrt(v[1]);
+  s.bnorm = sqrt(v[2]);
+  s.rhs_test = rtol * (crit == FEMHIP_RES_RHS ? s.bnorm : s.r0norm) + atol;
+  s.done = bad && *bad;
+  S[0] = S[1] = s;
+  CgResult r{};
+  r.rhs_test = s.rhs_test;
+  r.rnorm = s.rnorm;
+  r.bnorm = s.bnorm;
+  r.done = s.done;
+  *R = r;
+}
+
+// alpha; x += alpha p, r -= alpha q; partials <r,z>, ||r||^2
+__global__ __launch_bounds__(kMfThreads) void k_mf_update(int64_t n, CgState *S, const double *part_in, int groups,
+                                                          const double *__restrict__ invd,
+                                                          const double *__restrict__ p,
+                                                          const double *__restrict__ q, double *__restrict__ x,
+                                                          double *__restrict__ r, double *part) {
+  if (S->done) return;
+  double red[1];
+  group_reduce<1>(part_in, groups, red);
+  const double alpha = red[0] != 0.0 ? S->rz / red[0] : 0.0;   // cg.f90:195-199
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    S->alpha = alpha;
+    S->pap = red[0];
+  }
+  double acc[2] = {0.0, 0.0};
+  for (int64_t i = (int64_t)blockIdx.x * kMfThreads + threadIdx.x; i < n; i += (int64_t)gridDim.x * kMfThreads) {
+    x[i] = x[i] + alpha * p[i];
+    const double ri = r[i] + (-alpha) * q[i];
+    r[i] = ri;
+    acc[0] += ri * (invd ? invd[i] * ri : ri);
+    acc[1] += ri * ri;
+  }
+  group_partials<2>(acc, part);
+}
+
+// stopping test (cg.f90:323-407), beta; p = z + beta p
+__global__ __launch_bounds__(kMfThreads) void k_mf_dir(int64_t n, CgState *S, int par, const double *part_in,
+                                                       int groups, const double *__restrict__ invd,
+                                                       const double *__restrict__ r, double *__restrict__ p,
+                                                       CgResult *R, CgResult *Rh) {
+  const CgState &cur = S[par];
+  const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
+  if (cur.done) {   // keep `done` sticky in both parity slots
+    if (lead) {
+      S[par ^ 1].done = 1;
+      if (Rh) *Rh = *R;
+    }
+    return;
+  }
+  double red[2], beta;
+  group_reduce<2>(part_in, groups, red);
+  if (cg_decide(cur, red, lead, S[par ^ 1], nullptr, R, Rh, beta)) return;
+  for (int64_t i = (int64_t)blockIdx.x * kMfThreads + threadIdx.x; i < n; i += (int64_t)gridDim.x * kMfThreads) {
+    const double zi = invd ? invd[i] * r[i] : r[i];
+    p[i] = beta * p[i] + zi;
+  }
+}
+
+// partials ||b - q||^2
+__global__ __launch_bounds__(kMfThreads) void k_mf_residual(int64_t n, const double *__restrict__ b,
+                                                            const double *__restrict__ q, double *part) {
+  double acc[1] = {0.0};
+  for (int64_t i = (int64_t)blockIdx.x * kMfThreads + threadIdx.x; i < n; i += (int64_t)gridDim.x * kMfThreads) {
+    const double ri = b[i] - q[i];
+    acc[0] += ri * ri;
+  }
+  group_partials<1>(acc, part);
+}
+__global__ __launch_bounds__(kMfThreads) void k_mf_sum(const double *part, int groups, double *out) {
+  double v[1];
+  group_reduce<1>(part, groups, v);
+  if (threadIdx.x == 0) *out = v[0];
+}
+
 // inverse of a diagonal block's diagonal (Jacobi on the block matrix); a
 // zero pivot raises the flag
 __global__ void k_block_invdiag(int32_t n, const int32_t *__restrict__ rowptr, const int32_t *__restrict__ col,
@@ -421,9 +773,24 @@ struct femhip_block_operator {
   bool have_phys = false, computed = false;
   DevBuf<double> tab, elvec, rhs;
   int32_t tab_off[kMaxFields][kMaxFields] = {}, vec_off[kMaxFields] = {};
-  DevBuf<double> x, r, z, p, q, invd, part, scal;
+  DevBuf<double> x, b, r, p, q, invd, part, part_u, scal;
+  DevBuf<CgState> st;
+  DevBuf<CgResult> res;
+  DevBuf<int> bad;
+  CgResult *h_res[2] = {nullptr, nullptr}, *d_res[2] = {nullptr, nullptr};   // pinned, mapped
+  hipEvent_t ev[2] = {nullptr, nullptr};
+  // products from the element tables
+  bool lat = false;
+  DevBuf<int32_t> perm[kMaxFields];
+  MfPlan h_plan{};
+  DevBuf<MfPlan> plan;
+  int gp = 1, gv = 1;                        // workgroups of the products and vector kernels
   int64_t ntot = 0;
   ~femhip_block_operator() {
+    for (auto *h : h_res)
+      if (h) (void)hipHostFree(h);
+    for (auto e : ev)
+      if (e) (void)hipEventDestroy(e);
     for (int f = 0; f < nf; ++f)
       if (field[f]) femhip_space_destroy(field[f]);
     if (ctx) ctx_release(ctx);
@@ -441,6 +808,8 @@ ColSet col_set(const femhip_block_operator &B, int f, int jb) {
     cs.nd[cs.ng] = B.field[g]->fe.nd;
     cs.off[cs.ng] = B.free_off[g];
     cs.tab[cs.ng] = B.tab_off[f][g];
+    cs.fld[cs.ng] = g;
+    cs.rows[cs.ng] = B.field[g]->n_free;
     ++cs.ng;
   }
   return cs;
@@ -549,9 +918,13 @@ void block_compute(femhip_block_operator &B, double *ms) {
         if (B.block[f] != ib || B.field[f]->n_free == 0) continue;
         const ColSet cs = col_set(B, f, jb);
         if (cs.ng == 0) continue;
-        hipLaunchKernelGGL(k_block_assemble, dim3((unsigned)B.field[f]->n_free), dim3(64), 0, st,
-                           face_tab(*B.field[f]), B.field[f]->n_free, B.free_off[f], B.field[f]->d_rep.p, cs,
-                           K.rowptr.p, K.col.p, B.tab.p, K.val.p);
+        if (B.lat)
+          hipLaunchKernelGGL(k_mf_assemble, dim3(nblocks((int64_t)B.field[f]->n_free * 16, 256)), dim3(256), 0, st,
+                             B.plan.p, f, cs, K.rowptr.p, K.col.p, B.tab.p, K.val.p);
+        else
+          hipLaunchKernelGGL(k_block_assemble, dim3((unsigned)B.field[f]->n_free), dim3(64), 0, st,
+                             face_tab(*B.field[f]), B.field[f]->n_free, B.free_off[f], B.field[f]->d_rep.p, cs,
+                             K.rowptr.p, K.col.p, B.tab.p, K.val.p);
         FH_HIP(hipGetLastError());
       }
     }
@@ -573,7 +946,7 @@ void block_compute(femhip_block_operator &B, double *ms) {
 }
 
 // y = A x over the block vectors (device pointers)
-void block_apply(femhip_block_operator &B, const double *x, double *y, const double *stop = nullptr) {
+void block_apply(femhip_block_operator &B, const double *x, double *y, const CgState *stop = nullptr) {
   hipStream_t st = B.ctx->stream;
   for (int ib = 0; ib < B.nb; ++ib) {
     int first = 1;
@@ -592,112 +965,204 @@ void block_apply(femhip_block_operator &B, const double *x, double *y, const dou
   }
 }
 
-// <a, b> into the device scalar `slot` (no host wait)
-void block_dot_dev(femhip_block_operator &B, const double *a, const double *b, int slot,
-                   const double *stop = nullptr) {
+// Boxes of the fields and the segments of the products; B.lat stays false
+// where a field's rows are no box.
+void plan_products(femhip_block_operator &B) {
+  MfPlan &P = B.h_plan;
+  const femhip_mesh_desc_t &m = B.field[0]->mesh;
+  P.nf = B.nf;
+  P.dim = m.dim;
+  for (int d = 0; d < 3; ++d) P.n[d] = d < m.dim ? m.n[d] : 1;
+  for (int f = 0; f < B.nf; ++f) {
+    const femhip_space &s = *B.field[f];
+    MfField &F = P.fld[f];
+    F.p = s.fe.order;
+    F.nd = s.fe.nd;
+    F.rows = s.n_free;
+    F.off = B.free_off[f];
+    F.base = B.boff[B.block[f]] + B.free_off[f];
+    for (int d = 0; d < 3; ++d) F.m[d] = 1;
+    if (s.n_free == 0) continue;
+    LatticeOp L;
+    if (s.fe.order > 2 || s.n_free > kLatticeMaxRows - 64 || !lattice_plan(s.mesh, B.ctx->num_cus, L) ||
+        !lattice_rows(s, L, B.perm[f]))
+      return;
+    for (int d = 0; d < m.dim; ++d) {
+      F.o[d] = L.g.o[d];
+      F.m[d] = L.g.m[d];
+    }
+    F.perm = B.perm[f].p;
+    for (int c = 0; c < (F.p == 2 ? 1 << (m.dim - 1) : 1); ++c) {   // bit d - 1: odd along d
+      MfSeg S{};
+      S.f = f;
+      for (int d = 0; d < 3; ++d) S.aligned[d] = S.cnt[d] = 1;
+      // along x a thread per cell vertex: the first may only have nodes after it
+      S.first[0] = F.p == 1 ? F.o[0] : 0;
+      S.cnt[0] = F.p == 1 ? F.m[0] : P.n[0] + (F.o[0] + F.m[0] > 2 * P.n[0] ? 1 : 0);
+      int64_t rows = S.cnt[0];
+      for (int d = 1; d < m.dim; ++d) {
+        const int odd = (c >> (d - 1)) & 1;
+        S.aligned[d] = !odd;
+        S.first[d] = F.p == 1 ? 0 : ((odd - F.o[d]) % 2 + 2) % 2;
+        S.cnt[d] = F.m[d] > S.first[d] ? (F.m[d] - S.first[d] + F.p - 1) / F.p : 0;
+        rows *= S.cnt[d];
+      }
+      S.rows = (int)rows;
+      if (S.rows == 0) continue;
+      S.blocks = (int)(((rows + 7) / 8 + kMfThreads - 1) / kMfThreads);
+      P.items += 8 * S.blocks;
+      P.seg[P.nseg++] = S;
+    }
+  }
+  if (P.nseg == 0) return;
+  auto cells = [](const MfSeg &s) { return s.aligned[0] + s.aligned[1] + s.aligned[2]; };
+  std::stable_sort(P.seg, P.seg + P.nseg, [&](const MfSeg &a, const MfSeg &b) { return cells(a) > cells(b); });
+  B.plan.alloc(1);
+  B.lat = true;
+}
+
+// the plan with the element tables' places (after set_physics)
+void upload_plan(femhip_block_operator &B) {
+  if (!B.lat) return;
+  for (int f = 0; f < B.nf; ++f)
+    for (int g = 0; g < B.nf; ++g) B.h_plan.tab[f][g] = B.coupling[f][g] ? B.tab_off[f][g] : -1;
+  FH_HIP(hipMemcpy(B.plan.p, &B.h_plan, sizeof(MfPlan), hipMemcpyHostToDevice));
+}
+
+// q = A x in the solver's order with partials <q, x>
+void solver_apply(femhip_block_operator &B, const double *x, double *q, const CgState *stop, double *part) {
   hipStream_t st = B.ctx->stream;
-  hipLaunchKernelGGL(k_dot_part, dim3(kDotBlocks), dim3(kDotThreads), 0, st, B.ntot, a, b, B.part.p, stop);
-  hipLaunchKernelGGL(k_dot_final, dim3(1), dim3(kDotThreads), 0, st, B.part.p, B.scal.p + slot, stop);
+  const dim3 T(kMfThreads);
+  if (!B.lat) {
+    block_apply(B, x, q, stop);
+    if (part) hipLaunchKernelGGL(k_mf_dot, dim3(B.gp), T, 0, st, B.ntot, q, x, stop, part);
+  } else if (B.h_plan.dim == 3) {
+    hipLaunchKernelGGL(k_mf_product<3>, dim3(B.gp), T, 0, st, B.plan.p, B.tab.p, x, q, stop, part);
+  } else {
+    hipLaunchKernelGGL(k_mf_product<2>, dim3(B.gp), T, 0, st, B.plan.p, B.tab.p, x, q, stop, part);
+  }
   FH_HIP(hipGetLastError());
 }
 
-double read_scalar(femhip_block_operator &B, int slot) {
-  double h = 0.0;
-  FH_HIP(hipMemcpyAsync(&h, B.scal.p + slot, sizeof(double), hipMemcpyDeviceToHost, B.ctx->stream));
-  FH_HIP(hipStreamSynchronize(B.ctx->stream));
-  return h;
+// A block vector into the solver's order, and back.
+void to_solver(femhip_block_operator &B, const double *from, double *to) {
+  hipStream_t st = B.ctx->stream;
+  if (!B.lat) {
+    FH_HIP(hipMemcpyAsync(to, from, sizeof(double) * (size_t)B.ntot, hipMemcpyDeviceToDevice, st));
+    return;
+  }
+  for (int f = 0; f < B.nf; ++f) {
+    const MfField &F = B.h_plan.fld[f];
+    if (F.rows)
+      hipLaunchKernelGGL(k_mf_to_box, dim3(nblocks(F.rows, 256)), dim3(256), 0, st, F.rows, F.perm, from + F.base,
+                         to + F.base);
+  }
+  FH_HIP(hipGetLastError());
+}
+void from_solver(femhip_block_operator &B, const double *from, double *to) {
+  hipStream_t st = B.ctx->stream;
+  if (!B.lat) {
+    FH_HIP(hipMemcpyAsync(to, from, sizeof(double) * (size_t)B.ntot, hipMemcpyDeviceToDevice, st));
+    return;
+  }
+  for (int f = 0; f < B.nf; ++f) {
+    const MfField &F = B.h_plan.fld[f];
+    if (F.rows)
+      hipLaunchKernelGGL(k_mf_from_box, dim3(nblocks(F.rows, 256)), dim3(256), 0, st, F.rows, F.perm, from + F.base,
+                         to + F.base);
+  }
+  FH_HIP(hipGetLastError());
 }
 
-double block_dot(femhip_block_operator &B, const double *a, const double *b) {
-  block_dot_dev(B, a, b, kDot);
-  return read_scalar(B, kDot);
-}
-
-constexpr int kBlockChunk = 8;   // iterations queued between two reads of the device state
+constexpr int kBlockChunk = 8;   // iterations queued at a time (even: the parity restarts at 0)
 
 // cg_solve_body (cg.f90:101-238) on the block operator with the RES_RES or
 // RES_RHS criterion (cg.f90:279-407), identity or Jacobi (the inverse
-// diagonals of the diagonal blocks) preconditioner; x holds x0
-void block_cg(femhip_block_operator &B, const femhip_cg_params_t &prm, const double *b, femhip_cg_result_t &res) {
+// diagonals of the diagonal blocks) preconditioner; q holds x0 and p the
+// right-hand side in block order, r the solution on return
+void block_cg(femhip_block_operator &B, const femhip_cg_params_t &prm, femhip_cg_result_t &res) {
   hipStream_t st = B.ctx->stream;
   const int64_t n = B.ntot;
-  const dim3 G(nblocks(n, 256)), T(256);
+  const dim3 G((unsigned)B.gv), T(kMfThreads);
   const bool jac = prm.preconditioner == FEMHIP_PREC_JACOBI;
   hipEvent_t e0, e1;
   FH_HIP(hipEventCreate(&e0));
   FH_HIP(hipEventCreate(&e1));
   FH_HIP(hipEventRecord(e0, st));
   if (jac) {
-    DevBuf<int> bad;
-    bad.alloc(1);
-    FH_HIP(hipMemsetAsync(bad.p, 0, sizeof(int), st));
-    for (int ib = 0; ib < B.nb; ++ib) {
-      const int32_t nr = B.nblk[ib];
-      if (nr == 0) continue;
-      FH_CHECK(B.blk[ib][ib].on, FEMHIP_ERR_ZERO_DIAGONAL, "diagonal block missing: Jacobi needs it");
-      hipLaunchKernelGGL(k_block_invdiag, dim3(nblocks(nr, 256)), T, 0, st, nr, B.blk[ib][ib].rowptr.p,
-                         B.blk[ib][ib].col.p, B.blk[ib][ib].val.p, B.invd.p + B.boff[ib], bad.p);
-      FH_HIP(hipGetLastError());
+    FH_HIP(hipMemsetAsync(B.bad.p, 0, sizeof(int), st));
+    for (int ib = 0; ib < B.nb; ++ib)
+      FH_CHECK(B.nblk[ib] == 0 || B.blk[ib][ib].on, FEMHIP_ERR_ZERO_DIAGONAL, "diagonal block missing: Jacobi needs it");
+    if (B.lat) {
+      hipLaunchKernelGGL(k_mf_invdiag, dim3((unsigned)B.gp), T, 0, st, B.plan.p, B.tab.p, B.invd.p, B.bad.p);
+    } else {
+      for (int ib = 0; ib < B.nb; ++ib)
+        if (B.nblk[ib] > 0)
+          hipLaunchKernelGGL(k_block_invdiag, dim3(nblocks(B.nblk[ib], 256)), T, 0, st, B.nblk[ib],
+                             B.blk[ib][ib].rowptr.p, B.blk[ib][ib].col.p, B.blk[ib][ib].val.p,
+                             B.invd.p + B.boff[ib], B.bad.p);
     }
-    int h_bad = 0;
-    FH_HIP(hipMemcpyAsync(&h_bad, bad.p, sizeof(int), hipMemcpyDeviceToHost, st));
-    FH_HIP(hipStreamSynchronize(st));
-    FH_CHECK(!h_bad, FEMHIP_ERR_ZERO_DIAGONAL, "op1 cannot be entrywise inverted; there exists a null diagonal entry");
+    FH_HIP(hipGetLastError());
   }
   const double *invd = jac ? B.invd.p : nullptr;
-  block_apply(B, B.x.p, B.r.p);
-  hipLaunchKernelGGL(k_sub, G, T, 0, st, n, b, B.r.p);
-  hipLaunchKernelGGL(k_cg_z, G, T, 0, st, n, invd, B.r.p, B.z.p, nullptr);
+  to_solver(B, B.q.p, B.x.p);
+  to_solver(B, B.p.p, B.b.p);
+  solver_apply(B, B.x.p, B.q.p, nullptr, nullptr);
+  hipLaunchKernelGGL(k_mf_start, G, T, 0, st, n, B.b.p, B.q.p, invd, B.r.p, B.p.p, B.part_u.p);
+  hipLaunchKernelGGL(k_mf_begin, dim3(1), T, 0, st, B.part_u.p, B.gv, prm.rtol, prm.atol, prm.stopping_criterion,
+                     prm.max_num_iterations, jac ? B.bad.p : nullptr, B.st.p, B.res.p);
   FH_HIP(hipGetLastError());
-  block_dot_dev(B, B.r.p, B.z.p, kRz);
-  FH_HIP(hipMemcpyAsync(B.p.p, B.z.p, sizeof(double) * (size_t)n, hipMemcpyDeviceToDevice, st));
-  const double rhs_test =
-      prm.stopping_criterion == FEMHIP_RES_RHS ? prm.rtol * std::sqrt(block_dot(B, b, b)) + prm.atol
-                                               : prm.rtol * std::sqrt(block_dot(B, B.r.p, B.r.p)) + prm.atol;
-  // alpha, beta and the stopping test stay on the device: the host queues
-  // kBlockChunk iterations and reads the state once per chunk; the kernels of
-  // iterations queued past the end return at entry (kDone)
-  hipLaunchKernelGGL(k_cg_reset, dim3(1), dim3(1), 0, st, B.scal.p);
-  const double *stop = B.scal.p + kDone;
-  double h[4] = {0.0, 0.0, 0.0, 0.0};   // kIt, kEst, kConv, kDone
-  static_assert(kEst == kIt + 1 && kConv == kIt + 2 && kDone == kIt + 3, "state slots are contiguous");
-  for (;;) {
+  // chunks, one ahead; the launches of iterations past the end return at entry
+  int64_t queued = 0;
+  auto push = [&](int slot) {
     for (int c = 0; c < kBlockChunk; ++c) {
-      block_apply(B, B.p.p, B.q.p, stop);
-      block_dot_dev(B, B.q.p, B.p.p, kQp, stop);
-      hipLaunchKernelGGL(k_cg_xr, G, T, 0, st, n, B.scal.p, B.x.p, B.p.p, B.r.p, B.q.p);
-      block_dot_dev(B, B.r.p, B.r.p, kRr, stop);
-      hipLaunchKernelGGL(k_cg_test, dim3(1), dim3(1), 0, st, B.scal.p, rhs_test, prm.max_num_iterations);
-      hipLaunchKernelGGL(k_cg_z, G, T, 0, st, n, invd, B.r.p, B.z.p, stop);
-      block_dot_dev(B, B.r.p, B.z.p, kRzNew, stop);
-      hipLaunchKernelGGL(k_cg_p, G, T, 0, st, n, B.scal.p, B.z.p, B.p.p);
-      hipLaunchKernelGGL(k_cg_shift, dim3(1), dim3(1), 0, st, B.scal.p);
+      const int par = c & 1;
+      solver_apply(B, B.p.p, B.q.p, B.st.p + par, B.part.p);
+      hipLaunchKernelGGL(k_mf_update, G, T, 0, st, n, B.st.p + par, B.part.p, B.gp, invd, B.p.p, B.q.p, B.x.p, B.r.p,
+                         B.part_u.p);
+      hipLaunchKernelGGL(k_mf_dir, G, T, 0, st, n, B.st.p, par, B.part_u.p, B.gv, invd, B.r.p, B.p.p, B.res.p,
+                         c == kBlockChunk - 1 ? B.d_res[slot] : nullptr);
       FH_HIP(hipGetLastError());
     }
-    FH_HIP(hipMemcpyAsync(h, B.scal.p + kIt, sizeof(h), hipMemcpyDeviceToHost, st));
-    FH_HIP(hipStreamSynchronize(st));
-    if (h[3] != 0.0) break;
+    FH_HIP(hipEventRecord(B.ev[slot], st));
+    queued += kBlockChunk;
+  };
+  push(0);
+  bool more = queued < prm.max_num_iterations;
+  if (more) push(1);
+  for (int slot = 0;; slot ^= 1) {
+    FH_HIP(hipEventSynchronize(B.ev[slot]));
+    if (B.h_res[slot]->done || !more) break;
+    more = queued < prm.max_num_iterations;
+    if (more) push(slot);
   }
-  const int it = (int)h[0];
-  const bool conv = h[2] != 0.0;
-  const double est = h[1];
   FH_HIP(hipEventRecord(e1, st));
-  FH_HIP(hipEventSynchronize(e1));
+  // true residual in FP64
+  solver_apply(B, B.x.p, B.q.p, nullptr, nullptr);
+  hipLaunchKernelGGL(k_mf_residual, G, T, 0, st, n, B.b.p, B.q.p, B.part_u.p);
+  hipLaunchKernelGGL(k_mf_sum, dim3(1), T, 0, st, B.part_u.p, B.gv, B.scal.p);
+  from_solver(B, B.x.p, B.r.p);
+  FH_HIP(hipGetLastError());
+  CgResult r;
+  double rr = 0.0;
+  int bad = 0;
+  FH_HIP(hipMemcpyAsync(&r, B.res.p, sizeof(r), hipMemcpyDeviceToHost, st));
+  FH_HIP(hipMemcpyAsync(&rr, B.scal.p, sizeof(rr), hipMemcpyDeviceToHost, st));
+  if (jac) FH_HIP(hipMemcpyAsync(&bad, B.bad.p, sizeof(bad), hipMemcpyDeviceToHost, st));
+  FH_HIP(hipStreamSynchronize(st));
   float t = 0.f;
   FH_HIP(hipEventElapsedTime(&t, e0, e1));
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
-  // true residual in FP64
-  block_apply(B, B.x.p, B.q.p);
-  hipLaunchKernelGGL(k_sub, G, T, 0, st, n, b, B.q.p);
-  res.true_residual = std::sqrt(block_dot(B, B.q.p, B.q.p));
-  res.rhs_norm = std::sqrt(block_dot(B, b, b));
-  res.num_iterations = it;
-  res.did_converge = conv ? 1 : 0;
+  FH_CHECK(!bad, FEMHIP_ERR_ZERO_DIAGONAL, "op1 cannot be entrywise inverted; there exists a null diagonal entry");
+  res.true_residual = std::sqrt(rr);
+  res.rhs_norm = r.bnorm;
+  res.num_iterations = r.iter;
+  res.did_converge = r.converged ? 1 : 0;
   res.outer_iterations = 0;
-  res.status = conv ? FEMHIP_OK : FEMHIP_ERR_NOT_CONVERGED;
-  res.error_estimate = est;
-  res.rhs_convergence_test = rhs_test;
+  res.status = r.converged ? FEMHIP_OK : FEMHIP_ERR_NOT_CONVERGED;
+  res.error_estimate = r.est;
+  res.rhs_convergence_test = r.rhs_test;
   res.solve_ms = t;
 }
 
@@ -770,15 +1235,22 @@ int femhip_block_operator_create(femhip_ctx_t *ctx, const femhip_block_layout_t 
       for (int f = 0; f < nf; ++f) build_reffe(B->fe[f], m.dim, B->field[f]->fe.order, 1, h, maxo + 1);
       build_block_patterns(*B);
       const size_t nt = (size_t)std::max<int64_t>(1, B->ntot);
-      B->rhs.alloc(nt);
-      B->x.alloc(nt);
-      B->r.alloc(nt);
-      B->z.alloc(nt);
-      B->p.alloc(nt);
-      B->q.alloc(nt);
-      B->invd.alloc(nt);
-      B->part.alloc(kDotBlocks);
-      B->scal.alloc(kScalars);
+      for (auto *v : {&B->rhs, &B->x, &B->b, &B->r, &B->p, &B->q, &B->invd}) v->alloc(nt);
+      plan_products(*B);
+      const int64_t rows = B->lat ? (int64_t)B->h_plan.items * kMfThreads : B->ntot;
+      B->gp = (int)std::min<int64_t>(B->lat ? 2048 : kMfVecBlocks, nblocks(rows, kMfThreads));
+      B->gv = (int)std::min<int64_t>(kMfVecBlocks, nblocks(B->ntot, kMfThreads));
+      B->part.alloc((size_t)B->gp);
+      B->part_u.alloc((size_t)3 * B->gv);
+      B->scal.alloc(1);
+      B->st.alloc(2);
+      B->res.alloc(1);
+      B->bad.alloc(1);
+      for (int k = 0; k < 2; ++k) {   // written by the GPU, read by the host: mapped, coherent
+        FH_HIP(hipHostMalloc((void **)&B->h_res[k], sizeof(CgResult), hipHostMallocMapped | hipHostMallocCoherent));
+        FH_HIP(hipHostGetDevicePointer((void **)&B->d_res[k], B->h_res[k], 0));
+        FH_HIP(hipEventCreateWithFlags(&B->ev[k], hipEventDisableTiming));
+      }
     } catch (...) {
       delete B;
       throw;
@@ -868,6 +1340,7 @@ int femhip_block_operator_set_physics(femhip_block_operator_t *B, const femhip_m
     FH_HIP(hipSetDevice(B->ctx->device));
     B->phys = *ph;
     upload_block_physics(*B);
+    upload_plan(*B);
     B->have_phys = true;
     B->computed = false;
     return FEMHIP_OK;
@@ -941,8 +1414,8 @@ int femhip_block_operator_apply(femhip_block_operator_t *B, const double *x, dou
     if (B->ntot == 0) return FEMHIP_OK;
     const size_t bytes = sizeof(double) * (size_t)B->ntot;
     hipStream_t st = B->ctx->stream;
-    FH_HIP(hipMemcpyAsync(B->z.p, x, bytes, hipMemcpyHostToDevice, st));
-    block_apply(*B, B->z.p, B->q.p);
+    FH_HIP(hipMemcpyAsync(B->p.p, x, bytes, hipMemcpyHostToDevice, st));
+    block_apply(*B, B->p.p, B->q.p);
     FH_HIP(hipMemcpyAsync(y, B->q.p, bytes, hipMemcpyDeviceToHost, st));
     FH_HIP(hipStreamSynchronize(st));
     return FEMHIP_OK;
@@ -972,16 +1445,11 @@ int femhip_block_operator_solve(femhip_block_operator_t *B, const femhip_cg_para
     }
     const size_t bytes = sizeof(double) * (size_t)B->ntot;
     hipStream_t st = B->ctx->stream;
-    const double *db = B->rhs.p;
-    DevBuf<double> bb;
-    if (b) {
-      bb.alloc((size_t)B->ntot);
-      FH_HIP(hipMemcpyAsync(bb.p, b, bytes, hipMemcpyHostToDevice, st));
-      db = bb.p;
-    }
-    FH_HIP(hipMemcpyAsync(B->x.p, x, bytes, hipMemcpyHostToDevice, st));
-    block_cg(*B, *prm, db, *res);
-    FH_HIP(hipMemcpyAsync(x, B->x.p, bytes, hipMemcpyDeviceToHost, st));
+    if (b) FH_HIP(hipMemcpyAsync(B->p.p, b, bytes, hipMemcpyHostToDevice, st));
+    else FH_HIP(hipMemcpyAsync(B->p.p, B->rhs.p, bytes, hipMemcpyDeviceToDevice, st));
+    FH_HIP(hipMemcpyAsync(B->q.p, x, bytes, hipMemcpyHostToDevice, st));
+    block_cg(*B, *prm, *res);
+    FH_HIP(hipMemcpyAsync(x, B->r.p, bytes, hipMemcpyDeviceToHost, st));
     FH_HIP(hipStreamSynchronize(st));
     return FEMHIP_OK;
   } catch (const Error &e) {

@@ -112,3 +112,94 @@ def test_block_operator_refuses_bad_layouts(env):
         with pytest.raises(F.FemhipError) as e:
             F.block_fe_affine_operator_t().create("CSR", [False], spaces, layout, di)
         assert e.value.code == 1
+
+
+EDGES = {
+    # threads past one workgroup of an eighth, free faces on every side, one cell thick, four fields
+    "2d_long": (2, (300, 5), [(2, "x0"), (1, "none")], [1, 2], None, (1.0, 2.0), 0.75, (1.0, 0.5)),
+    "2d_none": (2, (3, 11), [(2, "none"), (2, "boundary"), (1, "x0")], [1, 1, 2], None, (1.0, 2.0, 0.5), 0.75,
+                (1.0, 0.5, 0.2)),
+    "3d_none": (3, (6, 3, 5), [(2, "none"), (1, "x0")], [1, 2], None, (1.0, 2.0), 0.75, (1.0, 0.5)),
+    "3d_thin": (3, (1, 9, 2), [(2, "x0"), (1, "none")], [2, 1], None, (1.0, 2.0), 0.75, (1.0, 0.5)),
+    "3d_wide": (3, (40, 9, 4), [(2, "x0"), (1, "x0")], [1, 2], None, (1.0, 2.0), 0.75, (1.0, 0.5)),
+    "3d_empty_field": (3, (3, 4, 1), [(1, "boundary"), (2, "x0")], [1, 1], None, (1.0, 2.0), 0.75, (1.0, 0.5)),
+    "3d_four_fields": (3, (3, 4, 2), [(1, "x0"), (2, "boundary"), (1, "none"), (2, "x0")], [1, 2, 2, 1],
+                       [[1, 1, 0, 1], [0, 1, 1, 0], [1, 0, 1, 1], [1, 1, 1, 1]], (1.0, 2.0, 0.5, 3.0), 0.75,
+                       (1.0, 0.5, 0.0, 2.0)),
+}
+
+
+@pytest.mark.parametrize("name", list(EDGES))
+def test_products_from_element_tables(env, name):
+    """Assembly and CG on the fields' boxes at the edges of their threads and
+    faces: values as in the tests above; one CG iteration from a random guess
+    against the same step with the oracle's matrix (1e-12: one product and two
+    sums), whether or not the coupling is symmetric."""
+    CASES[name] = EDGES[name]
+    mf, oph, coupling, spaces, layout, op = _build(env, name)
+    del CASES[name]
+    op.compute()
+    for ib in range(1, mf.num_blocks + 1):
+        for jb in range(1, mf.num_blocks + 1):
+            irp, ja, val = mf.assemble_block(oph, coupling, ib, jb, symmetric_storage=False)
+            B = op.get_block(ib, jb)
+            assert np.array_equal(B.irp, irp) and np.array_equal(B.ja, ja), (ib, jb)
+            if len(val):
+                assert np.max(np.abs(B.val - val)) <= 1e-12 * np.max(np.abs(val)), (ib, jb)
+    irp, ja, val, rhs = mf.merged(oph, coupling)
+    rng = np.random.default_rng(3)
+    b, x0 = rng.standard_normal(len(rhs)), rng.standard_normal(len(rhs))
+    r = b - O.spmv(irp, ja, val, x0, False)
+    rows = np.repeat(np.arange(len(rhs)), np.diff(irp))
+    z = r / val[ja - 1 == rows]
+    q = O.spmv(irp, ja, val, z, False)
+    step = x0 + (r @ z) / (z @ q) * z
+    solver = F.iterative_linear_solver_t().create(env)
+    solver.set_type_from_string("CG")
+    solver.set_parameters_from_pl({"ILS_RTOL": 1e-30, "ILS_MAX_NUM_ITERATIONS": 1})
+    solver.set_operators(op.get_tangent(), F.jacobi_preconditioner_t(op))
+    x = solver.solve(b, x0)
+    assert solver.result["num_iterations"] == 1
+    assert np.linalg.norm(x - step) <= 1e-12 * np.linalg.norm(step)
+    res = np.linalg.norm(b - O.spmv(irp, ja, val, x, False))
+    assert abs(solver.result["true_residual"] - res) <= 1e-12 * (res + np.linalg.norm(b))
+
+
+def test_numbering_that_is_no_box(env):
+    """A field with a fixed node inside keeps the row-wise assembly and the CSR
+    product: the rows and columns left are those of the full operator."""
+    dim, n = 2, (6, 5)
+    tria = F.serial_triangulation_t().create(env, {
+        "STRUCT_HEX_MESH_GENERATOR_NUM_DIMS": dim, "STRUCT_HEX_MESH_GENERATOR_NUM_CELLS_X_DIM": list(n),
+        "STRUCT_HEX_MESH_GENERATOR_DOMAIN_LIMITS": [0, 1, 0, 1, 0, 0]})
+    full = [F.serial_fe_space_t().create(tria, order=o) for o in (2, 1)]
+    dofs = np.array(full[0].get_lst_dofs_gids())
+    nfree = int(dofs.max())
+    gone = 40   # an interior node's free id
+    new = np.where(dofs == gone, -(int(-dofs.min()) + 1), np.where(dofs > gone, dofs - 1, dofs)).astype(np.int32)
+    holed = [F.serial_fe_space_t().create(tria, order=2, lst_dofs_gids=new, num_free_dofs=nfree - 1,
+                                          num_fixed_dofs=int(-new.min())), full[1]]
+    mats, sols = [], []
+    for spaces in (full, holed):
+        op = F.block_fe_affine_operator_t()
+        op.create("CSR", [False], spaces, F.block_layout_t().create(2, [1, 2]),
+                  F.coupled_diffusion_discrete_integration_t((1.0, 2.0), 0.75, (1.0, 0.5)))
+        op.compute()
+        N = sum(op.block_sizes)
+        off = np.concatenate([[0], np.cumsum(op.block_sizes)])
+        A = np.zeros((N, N))
+        for i in (1, 2):
+            for j in (1, 2):
+                B = op.get_block(i, j)
+                r = np.repeat(np.arange(op.block_sizes[i - 1]), np.diff(B.irp))
+                A[off[i - 1] + r, off[j - 1] + B.ja - 1] = B.val
+        solver = F.iterative_linear_solver_t().create(env)
+        solver.set_type_from_string("CG")
+        solver.set_parameters_from_pl({"ILS_RTOL": 1e-12, "ILS_MAX_NUM_ITERATIONS": 2000})
+        solver.set_operators(op.get_tangent(), F.jacobi_preconditioner_t(op))
+        x = solver.solve()
+        ref = np.linalg.solve(A, op.get_translation())
+        assert solver.result["did_converge"] and np.linalg.norm(x - ref) <= 1e-10 * np.linalg.norm(ref)
+        mats.append(A)
+    keep = np.delete(np.arange(len(mats[0])), gone - 1)
+    assert np.array_equal(mats[1], mats[0][np.ix_(keep, keep)])
