@@ -641,7 +641,10 @@ int small_class(const BProb &P, BSmall &S) {
 // Each problem's path; tiles of the problems in the passes and the table of
 // their workgroups.  A workgroup takes about an eighth of what would fill every
 // CU once, within bounds: long marches repeat little, short ones leave no CU
-// waiting for the last problem.
+// waiting for the last problem (512 mixed problems: 8.2 ms, a quarter 9.6, a half
+// 12.3).  Each workgroup of a problem reads the partial sums of all of them, so
+// a problem has at most kMostGroups (four of 1000^2 cells: 30 ms with 570, 23.5).
+constexpr int kMostGroups = 192;
 void plan_passes(femhip_batch &B, const std::vector<BTables> &tabs) {
   const int count = (int)B.probs.size();
   std::vector<BSmall> small[kSmallClasses];
@@ -707,7 +710,7 @@ void plan_passes(femhip_batch &B, const std::vector<BTables> &tabs) {
       mesh.limits[2 * d + 1] = 1.0;
     }
     LatticeOp L;
-    FH_CHECK(lattice_plan(mesh, 0, L, kBatchThreads, per), FEMHIP_ERR_INVALID, "batch problem too large");
+    FH_CHECK(lattice_plan(mesh, 0, L, kBatchThreads, std::max(per, P.nrows / kMostGroups)), FEMHIP_ERR_INVALID, "batch problem too large");
     BSolve S{};
     S.g = L.g;
     S.dim = P.dim;

@@ -1391,10 +1391,6 @@ void prepare_host_slots(femhip_solver &s) {
       if (!e) FH_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
 }
 
-// One launch an iteration or two (cg_lattice.h).
-constexpr int32_t kOneLaunchRows = 400000;
-bool lattice_one_pass(int32_t n) { return n < kOneLaunchRows; }
-
 void prepare_lattice(femhip_solver &s) {
   femhip_operator &op = *s.op;
   hipStream_t st = s.ctx->stream;
@@ -1411,19 +1407,13 @@ void prepare_lattice(femhip_solver &s) {
     if (jac) s.invd.alloc(n);   // invD (FP64) or S (FP32_REFINED)
     if (mx) {
       for (auto *v : {&s.r32, &s.p32, &s.p32_alt, &s.q32, &s.d32}) v->alloc(n);
-      if (lattice_one_pass(n))
+      if (L.one)
         for (auto *v : {&s.r32_alt, &s.q32_alt}) v->alloc(n);
     } else {
       for (auto *v : {&s.r, &s.p, &s.p_alt}) v->alloc(n);
-      if (lattice_one_pass(n))
+      if (L.one)
         for (auto *v : {&s.r_alt, &s.q_alt}) v->alloc(n);
     }
-    if (L.ncomp > 1)   // rows between the components are no nodes: they stay zero
-      for (auto *v : {&s.r, &s.r_alt, &s.p, &s.p_alt, &s.q, &s.q_alt})
-        if (v->p) FH_HIP(hipMemsetAsync(v->p, 0, v->bytes(), st));
-    if (L.ncomp > 1)
-      for (auto *v : {&s.r32, &s.r32_alt, &s.p32, &s.p32_alt, &s.q32, &s.q32_alt, &s.d32})
-        if (v->p) FH_HIP(hipMemsetAsync(v->p, 0, v->bytes(), st));
     s.part_i.alloc((size_t)4 * s.g_mat);
     s.part_s.alloc((size_t)kSums * s.g_mat);   // the passes' sums, alternating
     s.part_u.alloc((size_t)kSums * std::max(s.g_mat, s.g_vec));
@@ -1636,7 +1626,7 @@ void enqueue_one(femhip_solver &s, int par, Launcher &L, const hipEvent_t *ev = 
     L.lds = lo.lds;
     const PairOf<double> p{{s.p.p, s.p_alt.p}};
     const PairOf<float> p32{{s.p32.p, s.p32_alt.p}};
-    const bool one = lattice_one_pass(n);
+    const bool one = lo.one;
     if (one && !mixed(s))
       L(s.lk.cg, GM, BL, lo.g, s.coef, s.q2tab, n, PairOf<double>{{s.r.p, s.r_alt.p}},
         PairOf<double>{{s.q.p, s.q_alt.p}}, p, s.x.p, sc, s.st.p, par, in, out, s.hist.p, s.res.p, rh);
@@ -2027,7 +2017,7 @@ void profile_lattice(femhip_solver &s, int32_t reps, double *ms_per_launch, doub
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   if (ms_per_launch) *ms_per_launch = ms / reps;
-  const bool one = lattice_one_pass(s.n);
+  const bool one = op.lat->one;
   const double values = s.coef.kq ? (double)op.space->fe.nq : s.coef.kc ? 1.0 : 0.0;
   if (bytes)
     *bytes = (double)s.n * (one ? (mx ? 32.0 : 64.0) + (sc ? 8.0 : 0.0) : (mx ? 36.0 : 72.0) + (sc ? mx ? 8.0 : 16.0 : 0.0)) +

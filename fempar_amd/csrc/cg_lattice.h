@@ -1,7 +1,7 @@
 // cg_lattice.h -- CG kernels on the lattice products (lattice.h); included by
 // cg.hip inside its namespaces, after the scalar state and the decisions.
 //
-// Two forms of an iteration, chosen by size (lattice_one_pass):
+// Two forms of an iteration, chosen by size (lattice_one):
 //
 // Two launches, the form of cg.f90:101-238:
 //   A: stopping test, x += alpha p, p = z + beta p and s = A p in one march over
@@ -24,7 +24,8 @@
 // those of the two-launch form: against long double at 20^3, alpha ||p|| after 39
 // iterations is off by 1.4e-8 (two reductions: 1.0e-8, the sequential sums of the
 // oracle: 9.7e-8).  72 B a row, and r and s alternate too; it saves a launch and
-// its wait, but its march holds twice the vectors in flight.
+// its wait, but its march holds twice the vectors in flight, and where memory
+// bounds it the two launches' 88 B in smaller workgroups are as fast.
 //
 // The FP32 iterations keep FP32 vectors of the scaled system S A S, but their
 // products are formed in FP64 from the same coefficients as the FP64 ones: only
@@ -42,7 +43,7 @@ __device__ __forceinline__ LatticeCell<DIM, P, KIND> lattice_cell(const CoefDev 
 }
 
 struct IoCg {
-  static constexpr int kKeep = 3;
+  static constexpr int kKeep = 3, kAhead3 = 1;
   struct Halo {
     double r, s, d, p;
   };
@@ -123,11 +124,12 @@ struct IoCg {
   }
 };
 
-#define FEMHIP_LATTICE_BOUNDS \
-  __launch_bounds__(lattice_threads(DIM, P, KIND == kElastic ? 3 : 1), lattice_waves(DIM, P, KIND == kElastic ? 3 : 1))
+#define FEMHIP_LATTICE_BOUNDS(ONE)                                         \
+  __launch_bounds__(lattice_threads(DIM, P, KIND == kElastic ? 3 : 1, ONE), \
+                    lattice_waves(DIM, P, KIND == kElastic ? 3 : 1, ONE))
 
 template <int DIM, int P, int KIND>
-__global__ FEMHIP_LATTICE_BOUNDS void k_lat_cg(Lattice g, CoefDev c, Q2Tab t, int32_t n, PairOf<double> r,
+__global__ FEMHIP_LATTICE_BOUNDS(true) void k_lat_cg(Lattice g, CoefDev c, Q2Tab t, int32_t n, PairOf<double> r,
                                                PairOf<double> s, PairOf<double> p, double *x, const double *invd,
                                                CgState *S, int par, const double *part_in, double *part_out,
                                                double *hist, CgResult *R, CgResult *Rh) {
@@ -150,7 +152,7 @@ __global__ FEMHIP_LATTICE_BOUNDS void k_lat_cg(Lattice g, CoefDev c, Q2Tab t, in
 }
 
 template <int DIM, int P, int KIND>
-__global__ FEMHIP_LATTICE_BOUNDS void k_lat_res(Lattice g, CoefDev c, Q2Tab t, int32_t n, int mode, int x_zero,
+__global__ FEMHIP_LATTICE_BOUNDS(true) void k_lat_res(Lattice g, CoefDev c, Q2Tab t, int32_t n, int mode, int x_zero,
                                                 const double *__restrict__ x, const double *__restrict__ b,
                                                 const double *__restrict__ invd, const double *__restrict__ sc,
                                                 double *__restrict__ r64, float *__restrict__ r32,
@@ -177,7 +179,7 @@ __global__ FEMHIP_LATTICE_BOUNDS void k_lat_res(Lattice g, CoefDev c, Q2Tab t, i
 // the folded x (ru = 1); the one after tests it and takes the direction from it
 // and the direction before last (ru = 2), which is still in the other set.
 template <int DIM, int P, int KIND>
-__global__ FEMHIP_LATTICE_BOUNDS void k_lat_rf(Lattice g, CoefDev c, Q2Tab t, int32_t n, PairOf<float> r,
+__global__ FEMHIP_LATTICE_BOUNDS(true) void k_lat_rf(Lattice g, CoefDev c, Q2Tab t, int32_t n, PairOf<float> r,
                                                PairOf<float> q, PairOf<float> p, float *d, double *__restrict__ x,
                                                const double *__restrict__ b, const double *__restrict__ sc, CgState *S,
                                                int par, const double *part_in, double *part_out, CgResult *R,
@@ -267,7 +269,7 @@ __global__ FEMHIP_LATTICE_BOUNDS void k_lat_rf(Lattice g, CoefDev c, Q2Tab t, in
 // ---- two launches an iteration ----
 
 struct IoCgA {
-  static constexpr int kKeep = 1;
+  static constexpr int kKeep = 1, kAhead3 = 1;
   struct Halo {
     double r, d, p;
   };
@@ -322,7 +324,7 @@ struct IoCgA {
 };
 
 template <int DIM, int P, int KIND>
-__global__ FEMHIP_LATTICE_BOUNDS void k_lat_a(Lattice g, CoefDev c, Q2Tab t, int32_t n, const double *r,
+__global__ FEMHIP_LATTICE_BOUNDS(false) void k_lat_a(Lattice g, CoefDev c, Q2Tab t, int32_t n, const double *r,
                                               const double *invd, PairOf<double> p, double *x, double *q, CgState *S,
                                               int par, const double *part_b, int gb, double *part, double *hist,
                                               CgResult *R, CgResult *Rh) {
@@ -401,7 +403,7 @@ __global__ __launch_bounds__(kThreads) void k_lat_b(int32_t n, double *__restric
 // FP32: p and r are those of the scaled system S A S (sc = S in FP64, null:
 // S = I), d the increment in its variables.
 struct IoRfA {
-  static constexpr int kKeep = 2;
+  static constexpr int kKeep = 2, kAhead3 = 1;
   struct Halo {
     double s;
     float r, p;
@@ -438,7 +440,7 @@ struct IoRfA {
 };
 
 template <int DIM, int P, int KIND>
-__global__ FEMHIP_LATTICE_BOUNDS void k_lat_rf_a(Lattice g, CoefDev c, Q2Tab t, int32_t n, const float *r,
+__global__ FEMHIP_LATTICE_BOUNDS(false) void k_lat_rf_a(Lattice g, CoefDev c, Q2Tab t, int32_t n, const float *r,
                                                  const double *sc, PairOf<float> p, float *d, float *q, double *x,
                                                  CgState *S, int par, const double *part_b, int gb, double *part,
                                                  CgResult *R, CgResult *Rh) {
@@ -480,7 +482,7 @@ __global__ FEMHIP_LATTICE_BOUNDS void k_lat_rf_a(Lattice g, CoefDev c, Q2Tab t, 
 
 // FP32 slot B: r -= alpha q (four rows a load), or after a fold the FP64 residual of the folded x
 template <int DIM, int P, int KIND>
-__global__ FEMHIP_LATTICE_BOUNDS void k_lat_rf_b(Lattice g, CoefDev c, Q2Tab t, int32_t n, float *__restrict__ r,
+__global__ FEMHIP_LATTICE_BOUNDS(false) void k_lat_rf_b(Lattice g, CoefDev c, Q2Tab t, int32_t n, float *__restrict__ r,
                                                  const float *__restrict__ q, const double *__restrict__ sc,
                                                  const double *__restrict__ b, const double *__restrict__ x, CgState *S,
                                                  int par, const double *part_a, int ga, double *part) {

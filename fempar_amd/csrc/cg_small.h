@@ -17,27 +17,6 @@
 constexpr int32_t kSmallMaxRows = 4096;
 constexpr int kSmallChunk = 1024;                     // iterations a launch
 
-// v plus the value of the lanes a DPP control names (no LDS round trip).
-template <int CTRL, int ROWS>
-__device__ __forceinline__ double dpp_add(double v) {
-  const uint64_t b = __builtin_bit_cast(uint64_t, v);
-  const int lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, CTRL, ROWS, 0xf, true);
-  const int hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32), CTRL, ROWS, 0xf, true);
-  return v + __builtin_bit_cast(double, (uint64_t)(uint32_t)lo | ((uint64_t)(uint32_t)hi << 32));
-}
-// Sum over each row of 16 lanes, in its last lane.
-__device__ __forceinline__ double row_sum15(double v) {
-  v = dpp_add<0x111, 0xf>(v);   // row_shr:1
-  v = dpp_add<0x112, 0xf>(v);   // row_shr:2
-  v = dpp_add<0x114, 0xf>(v);   // row_shr:4
-  return dpp_add<0x118, 0xf>(v);   // row_shr:8
-}
-// Sum over the wave, in lane 63.
-__device__ __forceinline__ double wave_sum63(double v) {
-  v = row_sum15(v);
-  v = dpp_add<0x142, 0xa>(v);      // row_bcast:15 to rows 1 and 3
-  return dpp_add<0x143, 0xc>(v);   // row_bcast:31 to rows 2 and 3
-}
 __device__ __forceinline__ double read_lane(double v, int lane) {
   const uint64_t b = __builtin_bit_cast(uint64_t, v);
   const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)b, lane);

@@ -104,9 +104,38 @@ struct LatticeShape {
   static constexpr bool PIPE = P == 1 && NC == 1;
 };
 
-// Largest workgroup and wanted waves a SIMD (registers 512 / waves) of the marches.
-__host__ __device__ constexpr int lattice_threads(int dim, int p, int nc) { return dim == 3 && p == 1 && nc == 1 ? 512 : 256; }
-__host__ __device__ constexpr int lattice_waves(int, int p, int nc) { return p == 1 && nc == 1 ? 4 : 2; }
+// Iterations in one launch or two (cg_lattice.h): us an iteration in one / two,
+// FP64 and FP32-refined.  3-D Q1, sin3 field: 24.9 / 31.7 and 28.6 / 29.4 at
+// 100^3, 39.2 / 48.3 and 40.6 / 41.7 at 128^3, 66 / 81 and 68 / 62 at 160^3 (cell
+// field there 84 / 75 and 53 / 51), 156 / 155 and 114 / 94 at 192^3.  2-D Q1: 19.7 /
+// 27.8 at 700,000 rows.  3-D Q2: 20.6 / 32 at 32^3, 34.0 / 38.0 and 33.5 / 37.0 at
+// 48^3 cells (857,000 rows), 56 / 54 and 53 / 49 at 64^3.  2-D Q2: 20.4 / 27.4 at
+// 400^2 cells, 48 / 50 at 800^2.  Elasticity: 26.6 / 27.8 and 23.7 / 26.0 at 64^3
+// (786,000 rows), 39 / 37 and 36 / 33 at 80^3.
+__host__ __device__ constexpr bool lattice_one(int64_t rows, int dim, int p, int nc) {
+  return rows < (dim == 3 && (p == 2 || nc > 1) ? 1000000 : 3000000);
+}
+// Largest workgroup and waves a SIMD (registers 512 / waves) of the marches.
+// One launch: one workgroup a CU, since each reads all workgroups' partial sums
+// at its start (128^3: 45 us an iteration with 768 workgroups of 256 threads, 39
+// with 256 of 768; 1001 x 700 Q1: 25 and 20), and registers for twice the
+// vectors; the cells of 3-D Q2 take all a wave can have.
+__host__ __device__ constexpr int lattice_threads(int dim, int p, int nc, bool one) {
+  return one ? (p == 1 && nc == 1 ? 768 : p == 2 && dim == 3 ? 256 : 512) : dim == 3 && p == 1 && nc == 1 ? 512 : 256;
+}
+__host__ __device__ constexpr int lattice_waves(int dim, int p, int nc, bool one) {
+  return one ? (p == 1 && nc == 1 ? 3 : p == 2 && dim == 3 ? 1 : 2) : p == 1 && nc == 1 ? 4 : 2;
+}
+// Largest tile for a size: smaller ones where a large one would leave CUs
+// without work (3-D Q1, 512 / 768 threads: 17.3 / 18.4 us at 80^3, 24.9 / 25.4 at
+// 100^3, 48 / 39 at 128^3; elasticity, 256 / 512: 13.4 / 15.0 at 36^3, 19.8 / 18.7 at 50^3).
+inline int lattice_tile(int64_t rows, int dim, int p, int nc) {
+  const bool one = lattice_one(rows, dim, p, nc);
+  const int most = lattice_threads(dim, p, nc, one);
+  if (one && nc > 1) return rows < 300000 ? 256 : most;
+  if (one && dim == 3 && p == 1) return rows < 1200000 ? 512 : most;
+  return most;
+}
 
 // What an Io keeps of a node from value() to out(), in doubles (kKeep, at most).
 constexpr int kLatticeKeep = 3;
@@ -125,8 +154,8 @@ inline int lattice_halo(int TX, int TY) {
 }
 
 // March of logical workgroup lb; false: it has no cells, and ready() was not called.
-// Cell: begin(cx, cy, in the mesh), prefetch(cz) and
-// advance() for its coefficient, bottom(u) with the nodes of the first plane,
+// Cell: begin(cx, cy, in the mesh), Next prefetch(cz) and
+// advance(next) for its coefficient, bottom(u) with the nodes of the first plane,
 // step(active, u, s): the P next planes in, the finished sums of the P planes
 // before the last of them out (this cell's share).
 // Io: Raw fetch(o) loads what the node at offset o needs; ready() then forms
@@ -135,6 +164,7 @@ inline int lattice_halo(int TX, int TY) {
 // this workgroup's); out<FULL>(o, keep, y) takes the finished sum y of the
 // node, with all of what value() kept (FULL) or only its value, keep[0].
 // halo(o) and halo_value(raw): the value alone, of a node past the tile.
+// kAhead3: planes loaded before they are used, in 3-D.
 template <int DIM, int P, class Cell, class Io>
 __device__ __forceinline__ bool lattice_march(const Lattice &g, int lb, Cell &cell, Io &io, double *lds) {
   constexpr int NC = Cell::kComps;
@@ -183,11 +213,15 @@ __device__ __forceinline__ bool lattice_march(const Lattice &g, int lb, Cell &ce
     const int gz = z - g.o[AX];
     return gz >= 0 && gz < g.m[AX] ? (uint32_t)gz * plane_bytes : kNoPlane;
   };
-  typename Io::Raw raw[NC][P][OWN];
-  typename Io::Halo hraw[NC][P];
+  constexpr int AHEAD = PIPE && DIM == 3 ? Io::kAhead3 : 1;
+  typename Io::Raw raws[AHEAD][NC][P][OWN];   // planes on their way
+  typename Io::Halo hraws[AHEAD][NC][P];
+  typename Cell::Next next_k[AHEAD];
   constexpr int KEEP = Io::kKeep;
   double *ring = lds + (PIPE ? 2 : 1) * half + (lane ? tid : 0);   // PIPE: [3][KEEP][cells], plane z in part z mod 3
-  auto fetch = [&](int z, int count) {   // planes z .. z + count - 1
+  auto fetch = [&](int slot, int z, int count) {   // planes z .. z + count - 1
+    auto &raw = raws[slot];
+    auto &hraw = hraws[slot];
 #pragma unroll
     for (int k = 0; k < NC; ++k)
 #pragma unroll
@@ -199,7 +233,9 @@ __device__ __forceinline__ bool lattice_march(const Lattice &g, int lb, Cell &ce
           hraw[k][c] = io.halo(base + hoff);
         }
   };
-  auto store = [&](double *U, int z, int count, int part) {
+  auto store = [&](int slot, double *U, int z, int count, int part) {
+    auto &raw = raws[slot];
+    auto &hraw = hraws[slot];
 #pragma unroll
     for (int k = 0; k < NC; ++k)
 #pragma unroll
@@ -278,15 +314,18 @@ __device__ __forceinline__ bool lattice_march(const Lattice &g, int lb, Cell &ce
       }
   };
 
-  fetch(P * zs, 1);
+  fetch(0, P * zs, 1);
   cell.begin(g, cx, cy, in_xy);
   if (!io.ready()) return true;   // the same for every workgroup
-  store(lds, P * zs, 1, 0);
+  store(0, lds, P * zs, 1, 0);
   double ub[NC][OWN];   // !PIPE: own nodes of the plane below the layer
-  if (PIPE) {
-    fetch(P * zs + 1, P);
-    cell.prefetch(g, zs, in_xy);
-  }
+  if (PIPE)
+#pragma unroll
+    for (int a = 0; a < AHEAD; ++a)
+      if (zs + a < z1) {
+        fetch(a, P * (zs + a) + 1, P);
+        next_k[a] = cell.prefetch(g, zs + a, in_xy);
+      }
   __syncthreads();
   {
     double u[NC][NPL];
@@ -308,28 +347,33 @@ __device__ __forceinline__ bool lattice_march(const Lattice &g, int lb, Cell &ce
       for (int i = 0; i < KEEP; ++i) keep[i] = ring[(part * KEEP + i) * cells];
     };
     int set = 1, next = 1;   // buffers; ring part of the plane stored next
-    for (int cz = zs; cz < z1; ++cz) {
-      double *U = lds + set * half, *C = U + P * LP;
-      store(U, P * cz + 1, P, next);
-      next = next == 2 ? 0 : next + 1;
-      cell.advance();
-      __syncthreads();
-      if (cz > zs) {
-        finish(lds + (set ^ 1) * half + P * LP, cz - 1, so_at, kept);
-        part = part == 2 ? 0 : part + 1;
-      }
-      if (cz + 1 < z1) {
-        fetch(P * (cz + 1) + 1, P);
-        cell.prefetch(g, cz + 1, in_xy);
-      }
-      double u[NC][P][NPL], s[NC][P][NPL];
+    for (int cb = zs; cb < z1; cb += AHEAD) {
 #pragma unroll
-      for (int c = 0; c < P; ++c) read_plane(U, c, u[0][c]);
-      cell.step(in_xy && cz < g.nc[AX], u, s);
-      share(C, s);
+      for (int a = 0; a < AHEAD; ++a) {
+        const int cz = cb + a;
+        if (cz >= z1) break;
+        double *U = lds + set * half, *C = U + P * LP;
+        store(a, U, P * cz + 1, P, next);
+        next = next == 2 ? 0 : next + 1;
+        cell.advance(next_k[a]);
+        __syncthreads();
+        if (cz > zs) {
+          finish(lds + (set ^ 1) * half + P * LP, cz - 1, so_at, kept);
+          part = part == 2 ? 0 : part + 1;
+        }
+        if (cz + AHEAD < z1) {
+          fetch(a, P * (cz + AHEAD) + 1, P);
+          next_k[a] = cell.prefetch(g, cz + AHEAD, in_xy);
+        }
+        double u[NC][P][NPL], s[NC][P][NPL];
 #pragma unroll
-      for (int j = 0; j < OWN; ++j) so[j] = s[0][0][(j / P) * N1 + j % P];
-      set ^= 1;
+        for (int c = 0; c < P; ++c) read_plane(U, c, u[0][c]);
+        cell.step(in_xy && cz < g.nc[AX], u, s);
+        share(C, s);
+#pragma unroll
+        for (int j = 0; j < OWN; ++j) so[j] = s[0][0][(j / P) * N1 + j % P];
+        set ^= 1;
+      }
     }
     __syncthreads();
     finish(lds + (set ^ 1) * half + P * LP, z1 - 1, so_at, kept);
@@ -338,11 +382,10 @@ __device__ __forceinline__ bool lattice_march(const Lattice &g, int lb, Cell &ce
     const double *Uo = U + (lane ? uat : 0);
     auto u_at = [&](int k, int c, int j) { return Uo[(k * P + c) * LP + (j / P) * LX + j % P]; };
     for (int cz = zs; cz < z1; ++cz) {
-      fetch(P * cz + 1, P);
-      cell.prefetch(g, cz, in_xy);
-      cell.advance();
+      fetch(0, P * cz + 1, P);
+      cell.advance(cell.prefetch(g, cz, in_xy));
       __syncthreads();   // the layer before has read U and C
-      store(U, P * cz + 1, P, 0);
+      store(0, U, P * cz + 1, P, 0);
       __syncthreads();
       double u[NC][P][NPL], s[NC][P][NPL];
 #pragma unroll
@@ -397,8 +440,11 @@ template <int DIM, int KIND>
 struct CellQ1 {
   static constexpr int kComps = 1, NPL = DIM == 3 ? 4 : 2, NV = 1 << DIM, NK = KIND == kCoefPoint ? NV : 1;
   CoefDev k;
-  double kv[NK], kn[NK];          // this layer's values, the next one's
-  double sz[2], sn[2];            // sines at the march's points
+  struct Next {                   // a layer's coefficient, loaded ahead
+    double v[KIND == kCoefSin3 ? 2 : NK];
+  };
+  double kv[NK];                  // this layer's values
+  double sz[2];                   // sines at the march's points
   double ka[2], kb[2], kc4[4];    // in-plane factors of the coefficient summed along x, y and the march
   double below[NPL], carry[NPL];  // modes of the plane below, unfinished sums of its modes
   int64_t col, plane;
@@ -428,26 +474,28 @@ struct CellQ1 {
 #pragma unroll
     for (int i = 0; i < NPL; ++i) carry[i] = 0.0;
   }
-  __device__ __forceinline__ void prefetch(const Lattice &g, int cz, bool in) {
+  __device__ __forceinline__ Next prefetch(const Lattice &g, int cz, bool in) const {
     const int z = min(cz, g.nc[DIM - 1] - 1);
     const int64_t at = col + plane * z;
+    Next n;
     if (KIND == kCoefCell) {
-      kn[0] = k.kc ? k.kc[at] : k.k0;
+      n.v[0] = k.kc ? k.kc[at] : k.k0;
     } else if (KIND == kCoefPoint) {
 #pragma unroll
-      for (int q = 0; q < NV; ++q) kn[q] = k.kq[q * k.cells + at];
+      for (int q = 0; q < NV; ++q) n.v[q % NK] = k.kq[q * k.cells + at];
     } else {
-      sn[0] = k.trig[k.toff[DIM - 1] + 2 * z].z;
-      sn[1] = k.trig[k.toff[DIM - 1] + 2 * z + 1].z;
+      n.v[0] = k.trig[k.toff[DIM - 1] + 2 * z].z;
+      n.v[1 % (KIND == kCoefSin3 ? 2 : NK)] = k.trig[k.toff[DIM - 1] + 2 * z + 1].z;
     }
+    return n;
   }
-  __device__ __forceinline__ void advance() {
+  __device__ __forceinline__ void advance(const Next &n) {
     if (KIND == kCoefSin3) {
-      sz[0] = sn[0];
-      sz[1] = sn[1];
+      sz[0] = n.v[0];
+      sz[1] = n.v[1 % (KIND == kCoefSin3 ? 2 : NK)];
     } else {
 #pragma unroll
-      for (int q = 0; q < NK; ++q) kv[q] = kn[q];
+      for (int q = 0; q < NK; ++q) kv[q] = n.v[q];
     }
   }
   // coefficient summed over the two points along direction d, at point (qe, qf)
@@ -572,8 +620,9 @@ struct CellElastic {
 #pragma unroll
       for (int i = 0; i < NPL; ++i) carry[c][i] = 0.0;
   }
-  __device__ __forceinline__ void prefetch(const Lattice &, int, bool) {}
-  __device__ __forceinline__ void advance() {}
+  struct Next {};
+  __device__ __forceinline__ Next prefetch(const Lattice &, int, bool) const { return {}; }
+  __device__ __forceinline__ void advance(const Next &) {}
   __device__ __forceinline__ void bottom(const double (&u)[3][NPL]) {
 #pragma unroll
     for (int c = 0; c < 3; ++c) CellQ1<3, kCoefCell>::modes(u[c], below[c]);
@@ -652,10 +701,14 @@ struct CellQ2 {
   static constexpr int kComps = 1, NPL = DIM == 3 ? 9 : 3, N = DIM == 3 ? 27 : 9;
   CoefDev k;
   Q2Tab t;
-  double kv, kn;
-  double sz[3], sn[3], kxy[NPL];
+  struct Next {                    // a layer's coefficient
+    double kv, sz[3];
+    int64_t at;
+  };
+  double kv;
+  double sz[3], kxy[NPL];
   double below[NPL], carry[NPL];   // the plane below interpolated in the plane, its unfinished sums
-  int64_t col, plane, at0, atn;
+  int64_t col, plane, at0;
 
   __device__ __forceinline__ void begin(const Lattice &g, int cx, int cy, bool in) {
     col = in ? cx + (int64_t)g.nc[0] * (DIM == 3 ? cy : 0) : 0;
@@ -669,21 +722,23 @@ struct CellQ2 {
 #pragma unroll
     for (int i = 0; i < NPL; ++i) carry[i] = 0.0;
   }
-  __device__ __forceinline__ void prefetch(const Lattice &g, int cz, bool in) {
+  __device__ __forceinline__ Next prefetch(const Lattice &g, int cz, bool in) const {
     const int z = min(cz, g.nc[DIM - 1] - 1);
-    atn = col + plane * z;
+    Next n{};
+    n.at = col + plane * z;
     if (KIND == kCoefCell) {
-      kn = k.kc ? k.kc[atn] : k.k0;
+      n.kv = k.kc ? k.kc[n.at] : k.k0;
     } else if (KIND == kCoefSin3) {
 #pragma unroll
-      for (int a = 0; a < 3; ++a) sn[a] = 0.5 * k.trig[k.toff[DIM - 1] + 3 * z + a].z;
+      for (int a = 0; a < 3; ++a) n.sz[a] = 0.5 * k.trig[k.toff[DIM - 1] + 3 * z + a].z;
     }
+    return n;
   }
-  __device__ __forceinline__ void advance() {
-    at0 = atn;
-    kv = kn;
+  __device__ __forceinline__ void advance(const Next &n) {
+    at0 = n.at;
+    kv = n.kv;
 #pragma unroll
-    for (int a = 0; a < 3; ++a) sz[a] = sn[a];
+    for (int a = 0; a < 3; ++a) sz[a] = n.sz[a];
   }
   __device__ __forceinline__ double at(int q) const {
     if (KIND == kCoefPoint) return k.kq[q * k.cells + at0];
@@ -797,6 +852,7 @@ struct CellQ2 {
 struct LatticeOp {
   Lattice g;
   int dim = 0, order = 0, ncomp = 1;
+  bool one = false;                 // an iteration in one launch
   int threads = 64, grid = 8;       // workgroup size and count
   size_t lds = 0;                   // bytes of LDS a workgroup
   bool identity = false;            // lattice rows are the operator's rows

@@ -65,7 +65,6 @@ __global__ void k_points_by_q(int64_t cells, int nq, const double *__restrict__ 
 
 template <int DIM, int P, int NC = 1>
 void split(LatticeOp &L, int cus, int max_threads, int cells) {
-  if (max_threads <= 0) max_threads = lattice_threads(DIM, P, NC);
   Lattice &g = L.g;
   const int e0 = g.E[0], e1 = DIM == 3 ? g.E[1] : 1, ez = g.E[DIM - 1];
   // Tile: the least lanes over all tiles.  Neighbouring tiles both compute the
@@ -103,7 +102,7 @@ void split(LatticeOp &L, int cus, int max_threads, int cells) {
     L.grid = g.tiles * g.nch;
     return;
   }
-  const int per_cu = std::max(1, std::min(256 * lattice_waves(DIM, P, NC) / L.threads, (int)(160 * 1024 / std::max<size_t>(1, L.lds))));
+  const int per_cu = std::max(1, std::min(256 * lattice_waves(DIM, P, NC, L.one) / L.threads, (int)(160 * 1024 / std::max<size_t>(1, L.lds))));
   const int64_t slots = (int64_t)per_cu * std::max(1, cus);
   double bestc = 1e300;
   for (int c = 1; c <= ez; ++c) {
@@ -145,6 +144,8 @@ bool lattice_plan(const femhip_mesh_desc_t &mesh, int cus, LatticeOp &L, int max
     if (rows * L.ncomp > INT32_MAX) return false;
   }
   g.stride = (int)rows;
+  L.one = lattice_one(rows * L.ncomp, dim, p, L.ncomp);
+  if (max_threads <= 0) max_threads = lattice_tile(rows * L.ncomp, dim, p, L.ncomp);
   if (dim == 2 && p == 1) split<2, 1>(L, cus, max_threads, cells);
   else if (dim == 2) split<2, 2>(L, cus, max_threads, cells);
   else if (p == 1 && L.ncomp == 3) split<3, 1, 3>(L, cus, max_threads, cells);
