@@ -242,6 +242,8 @@ __global__ __launch_bounds__(64) void k_batch_begin(const BSolve *__restrict__ p
 template <int DIM>
 __device__ __forceinline__ void batch_pass(const BSolve &P, int lb, const BPools &pl, CgState *S, int par, BOut *out,
                                            BCount *cnt, double *lds) {
+  double sums_in[kSums];
+  group_begin<kSums>(pl.part[par ^ 1] + P.poff, P.blocks, sums_in);
   const CgState &cur = S[par];
   CgState &next = S[par ^ 1];
   const bool lead = lb == 0 && threadIdx.x == 0;
@@ -249,7 +251,6 @@ __device__ __forceinline__ void batch_pass(const BSolve &P, int lb, const BPools
     if (lead) next.done = 1;
     return;
   }
-  const double *part_in = pl.part[par ^ 1] + P.poff;
   double *part_out = pl.part[par] + P.poff;
   const int set = cur.set;
   int64_t row0, rows;
@@ -258,7 +259,6 @@ __device__ __forceinline__ void batch_pass(const BSolve &P, int lb, const BPools
   const uint32_t b4 = 4u * (uint32_t)rows, b8 = 8u * (uint32_t)rows;
   CellQ1<DIM, kCoefCell> cell;
   cell.k = CoefDev{};
-  double alpha = 0.0, beta = 0.0;
   if (cur.ru == 1) {
     if (lead) {
       next = cur;
@@ -272,66 +272,33 @@ __device__ __forceinline__ void batch_pass(const BSolve &P, int lb, const BPools
     group_partials<2>(v, part_out, P.blocks, lb);
     return;
   }
-  CgResult unused;
-  if (cur.first == 1) {   // p = r
-    if (lead) {
-      next = cur;
-      next.first = 2;
-      next.set = set ^ 1;
-    }
-  } else if (cur.ru == 2) {
-    double rd[2];
-    group_reduce<2>(part_in, P.blocks, rd);
-    const RfStep step = rf_decide(cur, rd, lead, next, &unused);   // FP64 stopping test, beta
-    if (lead) {
-      next.first = 2;
-      next.set = set ^ 1;
-      if (step.done) {
-        out->iters = next.iter;
-        out->updates = next.updates;
-        out->conv = next.converged;
-        out->rnorm = next.rnorm;
-        out->t_end = (long long)wall_clock64();
-        atomicAdd(&cnt->done, 1);
-      }
-    }
-    if (step.done) return;
-    beta = step.beta;
-  } else {
-    double red[kSums];
-    group_reduce<kSums>(part_in, P.blocks, red);
-    const double rd[2] = {red[kSumNu], 0.0};
-    if (cur.first == 2) {   // no iteration made since the direction was set
-      if (lead) {
-        next = cur;
-        next.first = 0;
-        next.rz = red[kSumNu];
-      }
-    } else {
-      const RfStep step = rf_decide(cur, rd, lead, next, &unused);
-      if (step.fold) {   // back to the set of the direction before last
-        if (lead) {
-          next.ru = 1;
-          next.set = set ^ 1;
-        }
-        for (int64_t i = (int64_t)lb * kBatchThreads + threadIdx.x; i < P.nrows;
-             i += (int64_t)P.blocks * kBatchThreads) {
-          pl.x[P.xoff + i] += (double)pl.d[P.xoff + i];
-          pl.d[P.xoff + i] = 0.0f;
-        }
-        return;
-      }
-    }
-    pr_scalars(red, lead, next, alpha, beta);
-    if (lead) next.set = set ^ 1;
-  }
+  int act = kRfGo;
+  auto begin = [&](double &alpha, double &beta) {
+    CgResult unused;
+    act = rf_begin(cur, next, lead, sums_in, &unused, alpha, beta);
+    return act == kRfGo;
+  };
   const uint32_t old = cur.first == 1 ? 0 : b4;
-  IoRf io{buf_of(pl.r.v[set] + off, b4), buf_of(pl.q.v[set] + off, cur.ru == 2 ? 0 : old), buf_of(nullptr, 0),
-          buf_of(pl.p.v[set] + off, old), buf_of(pl.r.v[set ^ 1] + off, b4), buf_of(pl.q.v[set ^ 1] + off, b4),
-          buf_of(pl.p.v[set ^ 1] + off, b4), buf_of(pl.d + off, b4), false, alpha, beta, (float)alpha, (float)beta,
-          {0.0, 0.0, 0.0, 0.0, 0.0, 0.0}};
+  IoRf<decltype(begin)> io{buf_of(pl.r.v[set] + off, b4), buf_of(pl.q.v[set] + off, cur.ru == 2 ? 0 : old),
+                           buf_of(nullptr, 0), buf_of(pl.p.v[set] + off, old), buf_of(pl.r.v[set ^ 1] + off, b4),
+                           buf_of(pl.q.v[set ^ 1] + off, b4), buf_of(pl.p.v[set ^ 1] + off, b4),
+                           buf_of(pl.d + off, b4), false, begin, 0.0f, 0.0f, {0.0, 0.0, 0.0, 0.0, 0.0, 0.0}};
   for (int d = 0; d < DIM; ++d) cell.k.c[d] = P.cu[d];
-  lattice_march<DIM, 1>(w, lb, cell, io, lds);
+  if (!lattice_march<DIM, 1>(w, lb, cell, io, lds)) io.ready();   // no cells: the decision all the same
+  if (act == kRfFold)
+    for (int64_t i = (int64_t)lb * kBatchThreads + threadIdx.x; i < P.nrows; i += (int64_t)P.blocks * kBatchThreads) {
+      pl.x[P.xoff + i] += (double)pl.d[P.xoff + i];
+      pl.d[P.xoff + i] = 0.0f;
+    }
+  if (act == kRfDone && lead) {
+    out->iters = next.iter;
+    out->updates = next.updates;
+    out->conv = next.converged;
+    out->rnorm = next.rnorm;
+    out->t_end = (long long)wall_clock64();
+    atomicAdd(&cnt->done, 1);
+  }
+  if (act != kRfGo) return;
   group_partials<kSums>(io.sum, part_out, P.blocks, lb);
 }
 

@@ -52,12 +52,11 @@ struct IoCg {
   };
   const CgState &cur;
   CgState &next;
-  const double *part_in;
+  double (&part_in)[kSums];   // of group_begin
   double *hist;
   CgResult *R, *Rh;
   BufRsrc r, s, invd, p, rn, sn, pn, x;   // s and p have no bytes in the first pass: read as 0
   bool jac;
-  int groups;
   double alpha, beta;
   double sum[kSums];
 
@@ -83,7 +82,7 @@ struct IoCg {
       return true;
     }
     double red[kSums];
-    group_reduce<kSums>(part_in, groups, red);
+    group_end<kSums>(part_in, red);
     if (cur.first == 2) {   // no iteration made yet
       if (lead) {
         next = cur;
@@ -133,6 +132,8 @@ __global__ FEMHIP_LATTICE_BOUNDS(true) void k_lat_cg(Lattice g, CoefDev c, Q2Tab
                                                PairOf<double> s, PairOf<double> p, double *x, const double *invd,
                                                CgState *S, int par, const double *part_in, double *part_out,
                                                double *hist, CgResult *R, CgResult *Rh) {
+  double sums_in[kSums];
+  group_begin<kSums>(part_in, (int)gridDim.x, sums_in);
   const CgState &cur = S[par];
   if (cur.done) {   // keep `done` sticky in both parity slots
     if (blockIdx.x == 0 && threadIdx.x == 0) {
@@ -142,10 +143,10 @@ __global__ FEMHIP_LATTICE_BOUNDS(true) void k_lat_cg(Lattice g, CoefDev c, Q2Tab
     return;
   }
   const uint32_t bytes = 8u * (uint32_t)n, old = cur.first == 1 ? 0 : bytes;
-  IoCg io{cur, S[par ^ 1], part_in, hist, R, Rh, buf_of(r.v[par], bytes), buf_of(s.v[par], old),
+  IoCg io{cur, S[par ^ 1], sums_in, hist, R, Rh, buf_of(r.v[par], bytes), buf_of(s.v[par], old),
           buf_of(invd, invd ? bytes : 0), buf_of(p.v[par], old), buf_of(r.v[par ^ 1], bytes),
           buf_of(s.v[par ^ 1], bytes), buf_of(p.v[par ^ 1], bytes), buf_of(x, bytes), invd != nullptr,
-          (int)gridDim.x, 0.0, 0.0, {0.0, 0.0, 0.0, 0.0, 0.0, 0.0}};
+          0.0, 0.0, {0.0, 0.0, 0.0, 0.0, 0.0, 0.0}};
   auto cell = lattice_cell<DIM, P, KIND>(c, t);
   lattice_march<DIM, P>(g, lattice_block(g), cell, io, lattice_smem);
   group_partials<kSums>(io.sum, part_out);
@@ -184,6 +185,8 @@ __global__ FEMHIP_LATTICE_BOUNDS(true) void k_lat_rf(Lattice g, CoefDev c, Q2Tab
                                                const double *__restrict__ b, const double *__restrict__ sc, CgState *S,
                                                int par, const double *part_in, double *part_out, CgResult *R,
                                                CgResult *Rh) {
+  double sums_in[kSums];   // after an update pass only the first two count
+  group_begin<kSums>(part_in, (int)gridDim.x, sums_in);
   const CgState &cur = S[par];
   CgState &next = S[par ^ 1];
   const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
@@ -196,7 +199,6 @@ __global__ FEMHIP_LATTICE_BOUNDS(true) void k_lat_rf(Lattice g, CoefDev c, Q2Tab
   }
   const int set = cur.set;
   const uint32_t b4 = 4u * (uint32_t)n, b8 = 8u * (uint32_t)n;
-  double alpha = 0.0, beta = 0.0;
   if (cur.ru == 1) {
     if (lead) {
       next = cur;
@@ -210,59 +212,27 @@ __global__ FEMHIP_LATTICE_BOUNDS(true) void k_lat_rf(Lattice g, CoefDev c, Q2Tab
     group_partials<2>(out, part_out);
     return;
   }
-  if (cur.first == 1) {   // p = r
-    if (lead) {
-      next = cur;
-      next.first = 2;
-      next.set = set ^ 1;
-    }
-  } else if (cur.ru == 2) {
-    double rd[2];
-    group_reduce<2>(part_in, (int)gridDim.x, rd);
-    const RfStep step = rf_decide(cur, rd, lead, next, R);   // FP64 stopping test, beta
-    if (lead) {
-      next.first = 2;
-      next.set = set ^ 1;
-      if (Rh) *Rh = *R;
-    }
-    if (step.done) return;
-    beta = step.beta;
-  } else {
-    double red[kSums];
-    group_reduce<kSums>(part_in, (int)gridDim.x, red);
-    const double rd[2] = {red[kSumNu], 0.0};
-    if (cur.first == 2) {   // no iteration made since the direction was set
-      if (lead) {
-        next = cur;
-        next.first = 0;
-        next.rz = red[kSumNu];
-      }
-    } else {
-      const RfStep step = rf_decide(cur, rd, lead, next, R);
-      if (step.fold) {   // back to the set of the direction before last
-        if (lead) {
-          next.ru = 1;
-          next.set = set ^ 1;
-          if (Rh) *Rh = *R;
-        }
-        const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-        for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-          x[i] = new_x(x[i], d[i], sc, i);
-          d[i] = 0.0f;
-        }
-        return;
-      }
-    }
-    pr_scalars(red, lead, next, alpha, beta);
-    if (lead) next.set = set ^ 1;
-  }
-  if (lead && Rh) *Rh = *R;
+  int act = kRfGo;
+  auto begin = [&](double &alpha, double &beta) {
+    act = rf_begin(cur, next, lead, sums_in, R, alpha, beta);
+    if (lead && Rh) *Rh = *R;
+    return act == kRfGo;
+  };
   const uint32_t old = cur.first == 1 ? 0 : b4;
-  IoRf io{buf_of(r.v[set], b4), buf_of(q.v[set], cur.ru == 2 ? 0 : old), buf_of(sc, sc ? b8 : 0), buf_of(p.v[set], old),
-          buf_of(r.v[set ^ 1], b4), buf_of(q.v[set ^ 1], b4), buf_of(p.v[set ^ 1], b4), buf_of(d, b4), sc != nullptr,
-          alpha, beta, (float)alpha, (float)beta, {0.0, 0.0, 0.0, 0.0, 0.0, 0.0}};
+  IoRf<decltype(begin)> io{buf_of(r.v[set], b4), buf_of(q.v[set], cur.ru == 2 ? 0 : old), buf_of(sc, sc ? b8 : 0),
+                           buf_of(p.v[set], old), buf_of(r.v[set ^ 1], b4), buf_of(q.v[set ^ 1], b4),
+                           buf_of(p.v[set ^ 1], b4), buf_of(d, b4), sc != nullptr, begin, 0.0f, 0.0f,
+                           {0.0, 0.0, 0.0, 0.0, 0.0, 0.0}};
   auto cell = lattice_cell<DIM, P, KIND>(c, t);
-  lattice_march<DIM, P>(g, lattice_block(g), cell, io, lattice_smem);
+  if (!lattice_march<DIM, P>(g, lattice_block(g), cell, io, lattice_smem)) io.ready();   // no cells: the decision all the same
+  if (act == kRfFold) {
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
+      x[i] = new_x(x[i], d[i], sc, i);
+      d[i] = 0.0f;
+    }
+  }
+  if (act != kRfGo) return;
   group_partials<kSums>(io.sum, part_out);
 }
 

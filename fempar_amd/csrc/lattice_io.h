@@ -52,20 +52,40 @@ __device__ __forceinline__ void group_partials(double (&v)[NV], double *part, in
   }
 }
 // Sums of a launch's partials, in the same order in every workgroup: a wave
-// takes a whole sum.
+// takes a whole sum.  In two steps: the loads of the first need nothing but the
+// kernel's arguments, so they run beside those of the state.
 template <int NV>
-__device__ __forceinline__ void group_reduce(const double *part, int g, double (&v)[NV]) {
+__device__ __forceinline__ void group_begin(const double *part, int g, double (&a)[NV]) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int k = w + i * nw;
+    a[i] = 0.0;
+    if (k < NV)
+      for (int b = lane; b < g; b += 64) a[i] += part[k * g + b];
+  }
+}
+template <int NV>
+__device__ __forceinline__ void group_end(double (&a)[NV], double (&v)[NV]) {
   __shared__ double sm[NV];
-  const int lane = threadIdx.x & 63, nw = blockDim.x >> 6;
-  for (int k = threadIdx.x >> 6; k < NV; k += nw) {
-    double a = 0.0;
-    for (int b = lane; b < g; b += 64) a += part[k * g + b];
-    a = wave_sum63(a);
-    if (lane == 63) sm[k] = a;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int k = w + i * nw;
+    if (k < NV) {
+      const double s = wave_sum63(a[i]);
+      if (lane == 63) sm[k] = s;
+    }
   }
   __syncthreads();
 #pragma unroll
   for (int k = 0; k < NV; ++k) v[k] = sm[k];
+}
+template <int NV>
+__device__ __forceinline__ void group_reduce(const double *part, int g, double (&v)[NV]) {
+  double a[NV];
+  group_begin<NV>(part, g, a);
+  group_end<NV>(a, v);
 }
 template <int NV>
 __device__ __forceinline__ void group_partials(double (&v)[NV], double *part) {
@@ -152,8 +172,57 @@ struct IoRes {
   }
 };
 
+// What a pass of the FP32 one-launch form does, from its state and the sums of
+// the pass before (group_begin): an iteration with alpha and beta, the fold of a
+// reliable update, or nothing more.  `lead` writes the next state.
+enum { kRfGo, kRfFold, kRfDone };
+__device__ __forceinline__ int rf_begin(const CgState &cur, CgState &next, bool lead, double (&sums)[kSums],
+                                        CgResult *R, double &alpha, double &beta) {
+  const int other = cur.set ^ 1;
+  alpha = beta = 0.0;
+  if (cur.first == 1) {   // p = r
+    if (lead) {
+      next = cur;
+      next.first = 2;
+      next.set = other;
+    }
+    return kRfGo;
+  }
+  double red[kSums];
+  group_end<kSums>(sums, red);
+  if (cur.ru == 2) {
+    const double rd[2] = {red[0], red[1]};
+    const RfStep step = rf_decide(cur, rd, lead, next, R);   // FP64 stopping test, beta
+    if (lead) {
+      next.first = 2;
+      next.set = other;
+    }
+    beta = step.beta;
+    return step.done ? kRfDone : kRfGo;
+  }
+  const double rd[2] = {red[kSumNu], 0.0};
+  if (cur.first == 2) {   // no iteration made since the direction was set
+    if (lead) {
+      next = cur;
+      next.first = 0;
+      next.rz = red[kSumNu];
+    }
+  } else if (rf_decide(cur, rd, lead, next, R).fold) {   // back to the set of the direction before last
+    if (lead) {
+      next.ru = 1;
+      next.set = other;
+    }
+    return kRfFold;
+  }
+  pr_scalars(red, lead, next, alpha, beta);
+  if (lead) next.set = other;
+  return kRfGo;
+}
+
 // FP32 passes of the one-launch form: p, r, s are those of the scaled system S A S (sc = S in FP64,
-// null: S = I), d the increment in its variables.
+// null: S = I), d the increment in its variables.  begin(alpha, beta) takes the
+// pass's decision once the first loads are under way; false: no iteration.
+template <class Begin>
 struct IoRf {
   static constexpr int kKeep = 3;
   static constexpr int kAhead3 = 2;   // 40.6 against 42.0 us an iteration at 128^3, 32.4 against 35.9 with a cell field
@@ -166,10 +235,16 @@ struct IoRf {
   };
   BufRsrc r, q, sc, p, rn, qn, pn, d;   // q = S A S p; q and p have no bytes in the first pass: read as 0
   bool jac;
-  double alpha64, beta64;
+  Begin begin;
   float alpha, beta;
   double sum[kSums];
-  __device__ __forceinline__ bool ready() const { return true; }
+  __device__ __forceinline__ bool ready() {
+    double a = 0.0, b = 0.0;
+    const bool go = begin(a, b);
+    alpha = (float)a;
+    beta = (float)b;
+    return go;
+  }
   __device__ __forceinline__ Raw fetch(uint32_t o) const {
     return Raw{halo(o), buf_ld32(d, o)};
   }
