@@ -84,43 +84,26 @@ __device__ __forceinline__ int slice_row_index(const SlicedDev &m, int s, int la
   return ((m.meta[s] >> 28) & 1) ? m.srow[s * kSlice + lane] : s * kSlice + lane;
 }
 
-// Sum NV values over the block; every thread gets the result.
+// Fixed-order sums of a producer's g block partials (the same in every block),
+// in two steps as group_begin and group_end, but by all waves: these grids have
+// up to four workgroups a CU (a wave a sum: 2 us more an iteration at 80^3).  DPP
+// sums with one barrier in place of LDS permutes with three: 57 x 49 x 65 mapped
+// cells 20.7 -> 18.9 us an iteration.
 template <int NV>
-__device__ __forceinline__ void block_sum_all(double (&v)[NV]) {
-  __shared__ double sm[NV][kWaves];
-  __shared__ double out[NV];
-  for (int off = 32; off > 0; off >>= 1)
-    for (int k = 0; k < NV; ++k) v[k] += __shfl_down(v[k], off, 64);
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  if (lane == 0)
-    for (int k = 0; k < NV; ++k) sm[k][w] = v[k];
-  __syncthreads();
-  if (threadIdx.x == 0)
-    for (int k = 0; k < NV; ++k) {
-      double s = 0.0;
-      for (int i = 0; i < kWaves; ++i) s += sm[k][i];
-      out[k] = s;
-    }
-  __syncthreads();
-  for (int k = 0; k < NV; ++k) v[k] = out[k];
-  __syncthreads();
-}
-
-// Block partials of this launch: part[k * gridDim.x + blockIdx.x].
-template <int NV>
-__device__ __forceinline__ void write_partials(double (&v)[NV], double *part) {
-  block_sum_all<NV>(v);
-  if (threadIdx.x == 0)
-    for (int k = 0; k < NV; ++k) part[k * gridDim.x + blockIdx.x] = v[k];
-}
-
-// Fixed-order reduction of a producer's g block partials (same in every block).
-template <int NV>
-__device__ __forceinline__ void reduce_partials(const double *part, int g, double (&v)[NV]) {
+__device__ __forceinline__ void partials_begin(const double *part, int g, double (&v)[NV]) {
   for (int k = 0; k < NV; ++k) v[k] = 0.0;
   for (int b = threadIdx.x; b < g; b += kThreads)
     for (int k = 0; k < NV; ++k) v[k] += part[k * g + b];
-  block_sum_all<NV>(v);
+}
+template <int NV>
+__device__ __forceinline__ void partials_end(double (&v)[NV]) {
+  __shared__ double sm[NV][kWaves];
+  block_sums<kWaves, NV>(v, sm);
+}
+template <int NV>
+__device__ __forceinline__ void reduce_partials(const double *part, int g, double (&v)[NV]) {
+  partials_begin<NV>(part, g, v);
+  partials_end<NV>(v);
 }
 
 // logical block index giving each XCD (blocks dispatched round-robin over 8)
@@ -370,7 +353,7 @@ __global__ __launch_bounds__(kThreads) void k_init(SlicedDev m, const T *__restr
       acc[3] += (double)(bi * mb);
     }
   }
-  write_partials<4>(acc, part);
+  group_partials<4>(acc, part);
 }
 
 // one block: init_convergence_data (cg.f90:279-321).  A raised zero-pivot flag
@@ -456,7 +439,7 @@ __global__ __launch_bounds__(kThreads) void k_spmv(SlicedDev m, const T *__restr
     }
   }
   double red[2] = {(double)pq, (double)pp};
-  write_partials<2>(red, part);
+  group_partials<2>(red, part);
 }
 
 // alpha ; r -= alpha q ; partials <r,z>, ||r||^2 (x += alpha p is made by
@@ -466,6 +449,8 @@ template <typename T, typename A>
 __global__ __launch_bounds__(kThreads) void k_update(int32_t n, T *__restrict__ r, const T *__restrict__ q,
                                                      const T *__restrict__ invd, CgState *S, int par,
                                                      const double *part_s, int gs, double *part) {
+  double red[2];
+  partials_begin<2>(part_s, gs, red);
   if (S[par].done) return;
   const int64_t i0 = (int64_t)blockIdx.x * kThreads + threadIdx.x, stride = (int64_t)gridDim.x * kThreads;
   T rv[kPrefetch], qv[kPrefetch], dv[kPrefetch];
@@ -478,8 +463,7 @@ __global__ __launch_bounds__(kThreads) void k_update(int32_t n, T *__restrict__ 
       dv[k] = invd ? ld_nt(&invd[i]) : (T)1;
     }
   }
-  double red[2];
-  reduce_partials<2>(part_s, gs, red);
+  partials_end<2>(red);
   const double alpha = (red[0] != 0.0) ? S[par].rz / red[0] : 0.0;   // cg.f90:195-199
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     S[par].alpha = alpha;
@@ -500,7 +484,7 @@ __global__ __launch_bounds__(kThreads) void k_update(int32_t n, T *__restrict__ 
     if (i0 + k * stride < n) row(i0 + k * stride, rv[k], qv[k], dv[k]);
   for (int64_t i = i0 + kPrefetch * stride; i < n; i += stride) row(i, r[i], q[i], invd ? invd[i] : (T)1);
   double out[2] = {(double)rz, (double)rr};
-  write_partials<2>(out, part);
+  group_partials<2>(out, part);
 }
 
 // stopping test (cg.f90:323-407) ; beta ; x += alpha p ; p = z + beta p
@@ -512,6 +496,8 @@ __global__ __launch_bounds__(kThreads) void k_dir(int32_t n, T *__restrict__ x, 
                                                   const T *__restrict__ r, const T *__restrict__ invd, CgState *S,
                                                   int par, const double *part_u, int gu, double *hist, CgResult *R,
                                                   CgResult *Rh) {
+  double red[2];
+  partials_begin<2>(part_u, gu, red);
   const CgState &cur = S[par];
   if (cur.done) {   // keep `done` sticky in both parity slots
     if (blockIdx.x == 0 && threadIdx.x == 0) {
@@ -532,8 +518,7 @@ __global__ __launch_bounds__(kThreads) void k_dir(int32_t n, T *__restrict__ x, 
       dv[k] = invd ? ld_nt(&invd[i]) : (T)1;
     }
   }
-  double red[2];
-  reduce_partials<2>(part_u, gu, red);
+  partials_end<2>(red);
   double beta = 0.0;
   const bool done = cg_decide(cur, red, blockIdx.x == 0 && threadIdx.x == 0, S[par ^ 1], hist, R, Rh, beta);
   const T a = (T)cur.alpha;
@@ -593,7 +578,7 @@ __global__ __launch_bounds__(kThreads) void k_ru_init(SlicedDev m, const double 
       acc[3] += (double)(rf * rf);
     }
   }
-  write_partials<4>(acc, part);
+  group_partials<4>(acc, part);
 }
 
 __global__ __launch_bounds__(kThreads) void k_ru_init_fin(const double *part, int g, CgState *S, CgResult *R,
@@ -686,7 +671,7 @@ __global__ __launch_bounds__(kThreads, 4) void k_ru_spmv(SlicedDev m, SlicedDev 
       }
     }
   }
-  write_partials<3>(acc, part);
+  group_partials<3>(acc, part);
 }
 
 // slot 2: alpha ; r -= alpha q (partials <r,r> twice: <r,z> and ||r||^2), or
@@ -751,7 +736,7 @@ __global__ __launch_bounds__(kThreads) void k_ru_update(int32_t n, float *__rest
     if (i0 + k * stride < n) row(i0 + k * stride, rv[k], qv[k]);
   for (int64_t i = i0 + kPrefetch * stride; i < n; i += stride) row(i, r[i], q[i]);
   double out[2] = {(double)rr, (double)rr};
-  write_partials<2>(out, part);
+  group_partials<2>(out, part);
 }
 
 // slot 3: d += alpha p, then take the CG direction step p = r + beta p, or
@@ -934,7 +919,7 @@ __global__ __launch_bounds__(kThreads, 4) void k_rf_a(SlicedDev m, SlicedDev m32
     }
   }
   double out[2] = {(double)pq, (double)pp};
-  write_partials<2>(out, part);
+  group_partials<2>(out, part);
 }
 
 // SYM: the symmetric-diagonal copy, whose slice s holds rows 64 s .. 64 s + 63
@@ -963,7 +948,7 @@ __global__ __launch_bounds__(kThreads, 4) void k_rf_b(SlicedDev m, const double 
         acc[1] += ri * ri;
       }
     }
-    write_partials<2>(acc, part);
+    group_partials<2>(acc, part);
     return;
   }
   // the wave's slices kRfbGroup at a time, all their loads of r and q issued
@@ -1011,7 +996,7 @@ __global__ __launch_bounds__(kThreads, 4) void k_rf_b(SlicedDev m, const double 
       }
   }
   acc[0] = rr;
-  write_partials<2>(acc, part);
+  group_partials<2>(acc, part);
 }
 
 // ------------------------------------------------------------------ helpers ---
@@ -1210,7 +1195,7 @@ __global__ __launch_bounds__(kThreads) void k_true_res(SlicedDev m, const double
       acc[0] += ri * ri;
     }
   }
-  write_partials<1>(acc, part);
+  group_partials<1>(acc, part);
 }
 
 #include "cg_lattice.h"

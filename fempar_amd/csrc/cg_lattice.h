@@ -327,6 +327,8 @@ __global__ FEMHIP_LATTICE_BOUNDS(false) void k_lat_a(Lattice g, CoefDev c, Q2Tab
 __global__ __launch_bounds__(kThreads) void k_lat_b(int32_t n, double *__restrict__ r, const double *__restrict__ q,
                                                     const double *__restrict__ invd, CgState *S, int par,
                                                     const double *part_a, int ga, double *part) {
+  double red[2];
+  partials_begin<2>(part_a, ga, red);
   if (S[par].done) return;
   constexpr int K = 4;   // pairs a thread loads before it reduces the partials
   const int64_t i0 = (int64_t)blockIdx.x * kThreads + threadIdx.x, stride = (int64_t)gridDim.x * kThreads;
@@ -341,8 +343,7 @@ __global__ __launch_bounds__(kThreads) void k_lat_b(int32_t n, double *__restric
       dv[k] = invd ? reinterpret_cast<const double2 *>(invd)[i] : double2{1.0, 1.0};
     }
   }
-  double red[2];
-  group_reduce<2>(part_a, ga, red);
+  partials_end<2>(red);
   const double alpha = (red[0] != 0.0) ? S[par].rz / red[0] : 0.0;   // cg.f90:195-199
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     S[par].alpha = alpha;

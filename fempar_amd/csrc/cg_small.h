@@ -17,31 +17,6 @@
 constexpr int32_t kSmallMaxRows = 4096;
 constexpr int kSmallChunk = 1024;                     // iterations a launch
 
-__device__ __forceinline__ double read_lane(double v, int lane) {
-  const uint64_t b = __builtin_bit_cast(uint64_t, v);
-  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)b, lane);
-  const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(b >> 32), lane);
-  return __builtin_bit_cast(double, (uint64_t)lo | ((uint64_t)hi << 32));
-}
-
-// Sums over the workgroup, the same in every thread; sm: NV rows, free until
-// the second barrier after this one.
-template <int W, int NV>
-__device__ __forceinline__ void small_sums(double (&v)[NV], double (*sm)[W]) {
-  const int w = threadIdx.x >> 6;
-#pragma unroll
-  for (int k = 0; k < NV; ++k) v[k] = wave_sum63(v[k]);
-  if ((threadIdx.x & 63) == 63)
-#pragma unroll
-    for (int k = 0; k < NV; ++k) sm[k][w] = v[k];
-  __syncthreads();
-  static_assert(W <= 16 && NV <= 4, "a row of 16 lanes takes a sum");
-  const int lane = threadIdx.x & 63;
-  const double a = row_sum15(lane < 16 * NV && (lane & 15) < W ? sm[lane >> 4][lane & (W - 1)] : 0.0);
-#pragma unroll
-  for (int k = 0; k < NV; ++k) v[k] = read_lane(a, 16 * k + 15);
-}
-
 // Row `lane` of slice s as in slice_rows, its terms in the same order, x in LDS
 // (without that one's special cases, which hold more loads than fit here).
 __device__ __forceinline__ double small_row(const SlicedDev &m, const double *__restrict__ v, const double *x, int s, int lane) {
@@ -162,7 +137,7 @@ __global__ __launch_bounds__(T) void k_cg_small(SlicedDev m, const double *__res
         a2[1] += pi * pi;
       }
     }
-    small_sums<T / 64>(a2, sums);
+    block_sums<T / 64>(a2, sums);
     const double alpha = a2[0] != 0.0 ? cur.rz / a2[0] : 0.0;   // cg.f90:195-199
     cur.alpha = alpha;
     cur.pap = a2[0];
@@ -175,7 +150,7 @@ __global__ __launch_bounds__(T) void k_cg_small(SlicedDev m, const double *__res
         b2[0] += r[j] * (d[row[j]] * r[j]);
         b2[1] += r[j] * r[j];
       }
-    small_sums<T / 64>(b2, sums + 2);
+    block_sums<T / 64>(b2, sums + 2);
     const double rnorm = sqrt(b2[1]), beta = (1.0 / cur.rz) * b2[0];
     double est, rhs_test;
     cur.converged = cg_test(cur, ++cur.iter, b2, rnorm, est, rhs_test);

@@ -34,6 +34,31 @@ __device__ __forceinline__ double wave_sum63(double v) {
   v = dpp_add<0x142, 0xa>(v);      // row_bcast:15 to rows 1 and 3
   return dpp_add<0x143, 0xc>(v);   // row_bcast:31 to rows 2 and 3
 }
+__device__ __forceinline__ double read_lane(double v, int lane) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)b, lane);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(b >> 32), lane);
+  return __builtin_bit_cast(double, (uint64_t)lo | ((uint64_t)hi << 32));
+}
+
+// Sums over the workgroup, the same in every thread; sm: NV rows, free until
+// the second barrier after this one.
+template <int W, int NV>
+__device__ __forceinline__ void block_sums(double (&v)[NV], double (*sm)[W]) {
+  const int w = threadIdx.x >> 6;
+#pragma unroll
+  for (int k = 0; k < NV; ++k) v[k] = wave_sum63(v[k]);
+  if ((threadIdx.x & 63) == 63)
+#pragma unroll
+    for (int k = 0; k < NV; ++k) sm[k][w] = v[k];
+  __syncthreads();
+  static_assert(W <= 16 && NV <= 4, "a row of 16 lanes takes a sum");
+  const int lane = threadIdx.x & 63;
+  const double a = row_sum15(lane < 16 * NV && (lane & 15) < W ? sm[lane >> 4][lane & (W - 1)] : 0.0);
+#pragma unroll
+  for (int k = 0; k < NV; ++k) v[k] = read_lane(a, 16 * k + 15);
+}
+
 // Partial sums of workgroup lb of g: part[k * g + lb].
 template <int NV>
 __device__ __forceinline__ void group_partials(double (&v)[NV], double *part, int g, int lb) {
