@@ -1399,6 +1399,12 @@ void prepare_lattice(femhip_solver &s) {
       if (L.one)
         for (auto *v : {&s.r_alt, &s.q_alt}) v->alloc(n);
     }
+    if (op.structured) {   // its components start on whole slices: the rows between are no nodes and stay zero
+      for (auto *v : {&s.r, &s.r_alt, &s.p, &s.p_alt, &s.q, &s.q_alt})
+        if (v->p) FH_HIP(hipMemsetAsync(v->p, 0, v->bytes(), st));
+      for (auto *v : {&s.r32, &s.r32_alt, &s.p32, &s.p32_alt, &s.q32, &s.q32_alt, &s.d32})
+        if (v->p) FH_HIP(hipMemsetAsync(v->p, 0, v->bytes(), st));
+    }
     s.part_i.alloc((size_t)4 * s.g_mat);
     s.part_s.alloc((size_t)kSums * s.g_mat);   // the passes' sums, alternating
     s.part_u.alloc((size_t)kSums * std::max(s.g_mat, s.g_vec));

@@ -168,3 +168,22 @@ def test_serve_admission_order(env, policy, aging_s):
         assert small_first == (policy == "smallest" and aging_s == 0.0)
     finally:
         srv.free()
+
+
+def test_serve_reused_memory_and_padded_components(env):
+    """Sizes whose components do not fill whole slices, in both forms of an
+    iteration (70: more than a million rows), in a device block that an earlier
+    request has written: the rows between the components take no part."""
+    srv = F.serve_t(env, hbm_budget_bytes=4 << 30, max_active=1, setup_threads=1, rtol=RTOL)
+    try:
+        for n in (68, 70, 41, 72, 70):
+            print(f"[serve] padded components, n={n}", flush=True)
+            t = srv.submit(n, 50.0, 0.3)
+            res = srv.wait(t, timeout_s=60)
+            assert res["status"] == N.OK and res["did_converge"] == 1, (n, res)
+            assert res["true_residual"] <= 1.0001 * RTOL * res["rhs_norm"], n
+            x = srv.get_solution(t)
+            assert np.all(np.isfinite(x)) and np.linalg.norm(x) > 0
+            srv.release(t)
+    finally:
+        srv.free()
