@@ -106,7 +106,7 @@ def measure_config(F, env, n, order, di, rtol, steps, warmup, with_mixed=True, e
                      "first_step_s": first}
         if exact:
             out[prec]["error_vs_u"] = s.error_norms(exact)
-        # the CG SpMV of this configuration back to back (HIP events, 50 launches)
+        # the CG iterations of this configuration back to back (HIP events, 50 launches)
         sp_ms, sp_bytes = s.profile_spmv(50)
         out[prec]["spmv"] = {"kernel_ms": sp_ms, "algorithmic_bytes": sp_bytes, "GBs": sp_bytes / sp_ms / 1e6,
                              "frac_of_hbm_peak": sp_bytes / sp_ms / 1e6 / HBM_PEAK_GBS}
@@ -214,17 +214,17 @@ def run_batched(F, env, steps, rtol=1e-8):
            "latency_ms_max": float(lat.max()), "converged": int(np.sum(last["did_converge"])),
            "max_true_rel_residual": float(rel.max()), "threads_per_block": threads,
            "iterations_total": int(np.sum(last["num_iterations"]))}
-    # roofline of the solve launch: FP32 inner iterations of every problem,
-    # (4 3^d + 40) bytes per row and iteration (the diagonals once, ten 4-byte
-    # vector passes), over the launch time
-    dims = np.array([p[0] for p in problems])
-    per_row = 4.0 * 3.0 ** dims + 40.0
+    # roofline of the solve: FP32 inner iterations of every problem, 32 bytes
+    # per row and iteration (r, q, p and d read and written once; the products
+    # are formed from the cells), over the solve's time.  Problems solved in one
+    # workgroup keep these vectors on chip, so this is no lower bound for them.
+    per_row = 32.0
     alg = float(np.sum(np.asarray(last["num_iterations"], dtype=float) * np.asarray(last["num_dofs"], dtype=float)
                        * per_row))
     gbs = alg / (ms.mean() / 1e3) / 1e9
     out["roofline"] = {"bound": "hbm", "achieved": gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                        "frac": gbs / HBM_PEAK_GBS, "algorithmic_bytes": alg,
-                       "definition": "sum over problems of inner iterations x free DOFs x (4*3^d + 40) B / solve_ms"}
+                       "definition": "sum over problems of inner iterations x free DOFs x 32 B / solve_ms"}
     b.free()
     return out
 
@@ -260,9 +260,9 @@ def run_multifield(F, env, n=48, rtol=1e-10):
     nnz = int(np.sum(op.block_nnz))
     ndofs = op.num_rows
     it = r["num_iterations"]
-    # per iteration: every block's CSR (8 B value + 4 B column per entry, row
-    # pointers) once in the SpMV, and about 13 vector passes of 8 B per row
-    per_it = 12.0 * nnz + 4.0 * (ndofs + 2) + 104.0 * ndofs
+    # per iteration 13 vector passes of 8 B per row: product 2, x and r update
+    # 7 with M, direction 4 (the products are formed from the element tables)
+    per_it = 104.0 * ndofs
     out = {"workload": f"two fields on {n}^3 cells: Q2 + Q1, two blocks", "dofs": ndofs,
            "block_sizes": op.block_sizes, "nnz": nnz, "setup_s": setup_s,
            "t_assemble_ms": float(np.mean(asm)), "t_cg_ms": float(np.mean(sol)), "iterations": it,
@@ -299,8 +299,8 @@ def run_serving(F, env, count, rates=SERVE_RATES, rtol=1e-8, policy_rates=SERVE_
     server admits them as slots and HBM budget free up, first come first
     served ("rates") and, at policy_rates, smallest estimate first with a 2 s
     aging bound ("smallest_first").  Latency = arrival to solution on the
-    host.  Roofline: FP32 inner iterations x DOFs x 364 B (81 FP32 stencil
-    values and ten 4-byte vector passes per row) over the span."""
+    host.  Roofline: FP32 inner iterations x DOFs x 40 B (r, q, p and d read
+    and written once, the FP64 scaling read) over the span."""
     reqs = serving_requests(count)
     out = {"requests_per_rate": count, "rates": {}, "smallest_first": {}}
     for lam, policy in [(r, "fcfs") for r in rates] + [(r, "smallest") for r in policy_rates]:
@@ -317,7 +317,7 @@ def run_serving(F, env, count, rates=SERVE_RATES, rtol=1e-8, policy_rates=SERVE_
         lat = np.array([r["latency_ms"] for r in res])
         dofs = sum(r["num_dofs"] for r in res)
         span = end - arrivals[0]
-        alg = float(sum(r["num_iterations"] * r["num_dofs"] for r in res)) * 364.0
+        alg = float(sum(r["num_iterations"] * r["num_dofs"] for r in res)) * 40.0
         out["rates" if policy == "fcfs" else "smallest_first"][str(lam)] = {
             "p50_ms": float(np.percentile(lat, 50)), "p99_ms": float(np.percentile(lat, 99)),
             "hbm_GBs": alg / span / 1e9, "hbm_frac": alg / span / 1e9 / HBM_PEAK_GBS,
@@ -448,15 +448,15 @@ def main():
     ms_step = float(np.mean(wall) * 1e3)
     value = fes.num_free_dofs / float(np.mean(ta + tc))
 
-    # roofline of the dominant kernel (CG SpMV): HIP events around 50
-    # back-to-back launches on the solver stream (agrees with the kernel trace);
-    # beside it the event mean over the SpMVs of one solve, whose start events
-    # also hold each launch's dispatch latency
+    # roofline of the dominant kernel, one CG iteration with its product formed
+    # from the cells: HIP events around 50 back-to-back launches on the solver
+    # stream; beside it the event mean over the launches of one solve, whose
+    # start events also hold each launch's dispatch latency
     spmv_ms, spmv_bytes = s64.profile_spmv(50)
     insolve_ms, insolve_its, _ = s64.profile_cg()
     achieved = spmv_bytes / (spmv_ms * 1e-3) / 1e9
     traffic = None
-    tpath = os.path.join(ROOT, "profiles", f"spmv_traffic_poisson3d_q1_{n}.json")
+    tpath = os.path.join(ROOT, "profiles", f"cg_pass_traffic_poisson3d_q1_{n}.json")
     if os.path.exists(tpath):   # HBM bytes per launch from the committed rocprofv3 --pmc runs
         traffic = json.load(open(tpath)).get("FP64", {}).get("hbm_bytes_per_launch")
 
@@ -513,11 +513,11 @@ def main():
         "setup_s": t_setup, "warmup_step_s": t_first,
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS, "traffic": traffic,
-                     "traffic_source": (f"profiles/spmv_traffic_poisson3d_q1_{n}.json: rocprofv3 --pmc FETCH_SIZE and "
+                     "traffic_source": (f"profiles/cg_pass_traffic_poisson3d_q1_{n}.json: rocprofv3 --pmc FETCH_SIZE and "
                                         "WRITE_SIZE of this kernel at this size, calibrated by a plain copy; "
                                         "read from the committed file, not measured in this run")
                      if traffic is not None else None,
-                     "kernel": "k_spmv<double> (FP64 CG SpMV on the sliced solver copy)",
+                     "kernel": "k_lat_cg (one FP64 CG iteration: product from the cells, vector updates and sums)",
                      "kernel_ms": spmv_ms, "algorithmic_bytes": spmv_bytes,
                      "kernel_ms_in_solve_events": insolve_ms, "in_solve_launches": insolve_its},
         "mixed": mixed,

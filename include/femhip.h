@@ -236,10 +236,12 @@ int femhip_solver_create(femhip_ctx_t *ctx, femhip_operator_t *op, const femhip_
  * keep the solution on the device). */
 int femhip_solver_solve(femhip_solver_t *solver, const double *b, double *x, femhip_cg_result_t *res);
 /* Measurement aid (the reference's timer_t, Sources/Lib/timer.f90:42-207, has
- * no kernel-level counterpart): launches the solver's SpMV kernel `reps` times
- * on the context stream and reports the average launch duration from HIP
- * events and the kernel's algorithmic HBM bytes per launch (matrix stream +
- * row pointers + one read of p and one write of q). */
+ * no kernel-level counterpart): launches the solver's product `reps` times on
+ * the context stream and reports the average duration from HIP events and the
+ * algorithmic HBM bytes.  On a stored matrix that is the SpMV kernel (matrix
+ * stream + row pointers + one read of p and one write of q); where products are
+ * formed from the cells it is a whole CG iteration, which holds the product
+ * (every vector it reads and writes, and the coefficient's values). */
 int femhip_solver_profile_spmv(femhip_solver_t *solver, int32_t reps, double *ms_per_launch,
                                double *bytes_per_launch);
 /* Measurement aid: one device-resident solve (operator RHS, x0 = 0) launched
