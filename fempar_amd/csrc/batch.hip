@@ -910,6 +910,9 @@ int femhip_batch_create(femhip_ctx_t *ctx, int32_t count, const femhip_batch_pro
   } catch (const Error &e) {
     set_error(e.msg);
     return e.code;
+  } catch (const std::bad_alloc &) {
+    set_error("host allocation failed");
+    return FEMHIP_ERR_OOM;
   }
 }
 

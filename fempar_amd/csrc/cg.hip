@@ -15,7 +15,9 @@
 // state says `done`, every kernel returns at entry; the host launches
 // hipGraph-captured chunks of iterations and polls a small result block.
 //
-// The SpMV runs on the sliced diagonal/ELL copy of the CSR matrix (one
+// On the uniform mesh the products come from the cells (cg_lattice.h), and small
+// systems are solved by one workgroup (cg_small.h); the kernels above serve the
+// others.  Their SpMV runs on the sliced diagonal/ELL copy of the CSR matrix (one
 // wavefront per 64-row slice, column offsets of diagonal slices are
 // wave-uniform, so the matrix stream carries no indices), with each XCD given a
 // contiguous range of slices so that the +-plane neighbours of p stay in its L2.
