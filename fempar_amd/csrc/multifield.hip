@@ -616,6 +616,20 @@ __global__ __launch_bounds__(256) void k_mf_assemble(const MfPlan *__restrict__ 
 
 constexpr int kMfVecBlocks = 512;
 
+// Sums of a producer's block partials by all waves, in two steps as group_begin
+// and group_end: there are hundreds of them.
+template <int NV>
+__device__ __forceinline__ void partials_begin(const double *part, int g, double (&v)[NV]) {
+  for (int k = 0; k < NV; ++k) v[k] = 0.0;
+  for (int b = threadIdx.x; b < g; b += kMfThreads)
+    for (int k = 0; k < NV; ++k) v[k] += part[k * g + b];
+}
+template <int NV>
+__device__ __forceinline__ void partials_end(double (&v)[NV]) {
+  __shared__ double sm[NV][kMfThreads / 64];
+  block_sums<kMfThreads / 64, NV>(v, sm);
+}
+
 // partials <q, p> of a product that has none
 __global__ __launch_bounds__(kMfThreads) void k_mf_dot(int64_t n, const double *__restrict__ a,
                                                        const double *__restrict__ b, const CgState *S, double *part) {
@@ -676,9 +690,10 @@ __global__ __launch_bounds__(kMfThreads) void k_mf_update(int64_t n, CgState *S,
                                                           const double *__restrict__ p,
                                                           const double *__restrict__ q, double *__restrict__ x,
                                                           double *__restrict__ r, double *part) {
-  if (S->done) return;
   double red[1];
-  group_reduce<1>(part_in, groups, red);
+  partials_begin(part_in, groups, red);   // beside the state's load
+  if (S->done) return;
+  partials_end(red);
   const double alpha = red[0] != 0.0 ? S->rz / red[0] : 0.0;   // cg.f90:195-199
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     S->alpha = alpha;
@@ -700,6 +715,8 @@ __global__ __launch_bounds__(kMfThreads) void k_mf_dir(int64_t n, CgState *S, in
                                                        int groups, const double *__restrict__ invd,
                                                        const double *__restrict__ r, double *__restrict__ p,
                                                        CgResult *R, CgResult *Rh) {
+  double red[2], beta;
+  partials_begin(part_in, groups, red);
   const CgState &cur = S[par];
   const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
   if (cur.done) {   // keep `done` sticky in both parity slots
@@ -709,8 +726,7 @@ __global__ __launch_bounds__(kMfThreads) void k_mf_dir(int64_t n, CgState *S, in
     }
     return;
   }
-  double red[2], beta;
-  group_reduce<2>(part_in, groups, red);
+  partials_end(red);
   if (cg_decide(cur, red, lead, S[par ^ 1], nullptr, R, Rh, beta)) return;
   for (int64_t i = (int64_t)blockIdx.x * kMfThreads + threadIdx.x; i < n; i += (int64_t)gridDim.x * kMfThreads) {
     const double zi = invd ? invd[i] * r[i] : r[i];
