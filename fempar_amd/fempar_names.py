@@ -658,7 +658,7 @@ class block_fe_affine_operator_t:
 class batch_t:
     """Many independent Poisson problems (Q1, unit square/cube, constant k,
     f = f0 k d pi^2 prod sin(pi x), homogeneous Dirichlet) assembled in one launch
-    and solved in one persistent FP32-refined launch (femhip_batch_*)."""
+    and solved together by the FP32-refined CG (femhip_batch_*)."""
 
     def __init__(self, environment: environment_t, problems, rtol=1e-8, max_num_iterations=20000, delta=0.0):
         self._lib = N.load()

@@ -332,7 +332,7 @@ int femhip_block_operator_solve(femhip_block_operator_t *bop, const femhip_cg_pa
                                 double *x, femhip_cg_result_t *res);
 int femhip_block_operator_destroy(femhip_block_operator_t *bop);
 
-/* ---- batched form: many independent small problems in one persistent launch ----
+/* ---- batched form: many independent problems advanced together ----
  * Each problem is FEMPAR's test_poisson setting on its own mesh: Q1 on the unit
  * square/cube with n cells per direction, strong Dirichlet (g = 0) on the whole
  * boundary, constant coefficient k, source f = f0 k d pi^2 prod_i sin(pi x_i)
@@ -365,7 +365,8 @@ int femhip_batch_create(femhip_ctx_t *ctx, int32_t count, const femhip_batch_pro
                         const femhip_cg_params_t *params, femhip_batch_t **batch);
 /* Integrate + assemble every problem (one launch; FP64 and FP32 values, RHS, Jacobi). */
 int femhip_batch_assemble(femhip_batch_t *batch, double *ms);
-/* Solve every problem from x0 = 0 in one persistent, hipGraph-captured launch;
+/* Solve every problem from x0 = 0, the small ones in a workgroup each, the
+ * others one CG iteration of all of them in each launch (hipGraph chunks);
  * results (count entries, may be NULL) and elapsed device ms. */
 int femhip_batch_solve(femhip_batch_t *batch, femhip_batch_result_t *results, double *ms);
 /* Solution of problem i (num_dofs values, lexicographic free-node order = the
