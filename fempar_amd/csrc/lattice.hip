@@ -63,8 +63,9 @@ __global__ void k_points_by_q(int64_t cells, int nq, const double *__restrict__ 
   if (i < cells * nq) out[(i % nq) * cells + i / nq] = in[i];
 }
 
+// False where no tile fits max_threads: no default split would cover the box.
 template <int DIM, int P, int NC = 1>
-void split(LatticeOp &L, int cus, int max_threads, int cells) {
+bool split(LatticeOp &L, int cus, int max_threads, int cells) {
   Lattice &g = L.g;
   const int e0 = g.E[0], e1 = DIM == 3 ? g.E[1] : 1, ez = g.E[DIM - 1];
   // Tile: the least lanes over all tiles.  Neighbouring tiles both compute the
@@ -74,11 +75,14 @@ void split(LatticeOp &L, int cus, int max_threads, int cells) {
   for (int xt = 1; xt <= e0; ++xt) {
     const int TX = (e0 - 1 + xt - 1) / xt + 1;
     if (TX > max_threads) continue;
+    // A thread loads one halo node: narrow tiles (Q2, one or two cells along x) are
+    // cut short along y by their halo before the threads run out.
     int TY = std::min(max_threads / TX, e1);
-    if (TY < 2 && e1 > 1) continue;
+    if (DIM == 3) TY = std::min(TY, (max_threads - 1) / P - TX);
+    if (TY < std::min(e1, 2)) continue;
     const int yt = e1 > 1 ? (e1 - 1 + TY - 2) / (TY - 1) : 1;
     if (e1 > 1) TY = (e1 - 1 + yt - 1) / yt + 1;
-    const int lanes = std::max(TX * TY, lattice_halo<DIM, P>(TX, TY));   // a thread loads one halo node
+    const int lanes = std::max(TX * TY, lattice_halo<DIM, P>(TX, TY));
     if (lanes > max_threads) continue;
     const int waves = (lanes + 63) / 64;
     const double cost = (double)xt * yt * waves * (1.0 + 0.02 * xt);
@@ -92,6 +96,7 @@ void split(LatticeOp &L, int cus, int max_threads, int cells) {
     }
     if (TX <= 2) break;
   }
+  if (best == 1e300) return false;
   L.lds = lattice_lds<DIM, P, NC>(g.TX, g.TY) * sizeof(double);
   // Chunks of the march: each repeats one layer, so few long ones repeat
   // little and many short ones fill the chip; the fewest layers in turn on one
@@ -100,7 +105,7 @@ void split(LatticeOp &L, int cus, int max_threads, int cells) {
     const int layers = std::max(2, std::min(ez, cells / std::max(1, g.TX * g.TY)));
     g.nch = (ez + layers - 1) / layers;
     L.grid = g.tiles * g.nch;
-    return;
+    return true;
   }
   // One launch an iteration: at most one workgroup a CU, also where more would
   // fit (elasticity of 40 x 33 x 47 cells: 16.6 us with 288 of one layer, 15.2 with
@@ -121,12 +126,13 @@ void split(LatticeOp &L, int cus, int max_threads, int cells) {
   }
   const int blocks = g.tiles * g.nch;
   L.grid = (blocks + 7) / 8 * 8;
+  return true;
 }
 
 }  // namespace
 
 // Box of the free nodes of a structured mesh and its split.  False where the
-// free nodes are no box or an index would not fit.
+// free nodes are no box, an index would not fit or no tile covers the box.
 bool lattice_plan(const femhip_mesh_desc_t &mesh, int cus, LatticeOp &L, int max_threads, int cells) {
   const int dim = mesh.dim, p = mesh.order;
   L = LatticeOp{};
@@ -150,12 +156,11 @@ bool lattice_plan(const femhip_mesh_desc_t &mesh, int cus, LatticeOp &L, int max
   g.stride = (int)rows;
   L.one = lattice_one(rows * L.ncomp, dim, p, L.ncomp);
   if (max_threads <= 0) max_threads = lattice_tile(rows * L.ncomp, dim, p, L.ncomp);
-  if (dim == 2 && p == 1) split<2, 1>(L, cus, max_threads, cells);
-  else if (dim == 2) split<2, 2>(L, cus, max_threads, cells);
-  else if (p == 1 && L.ncomp == 3) split<3, 1, 3>(L, cus, max_threads, cells);
-  else if (p == 1) split<3, 1>(L, cus, max_threads, cells);
-  else split<3, 2>(L, cus, max_threads, cells);
-  return true;
+  if (dim == 2 && p == 1) return split<2, 1>(L, cus, max_threads, cells);
+  if (dim == 2) return split<2, 2>(L, cus, max_threads, cells);
+  if (p == 1 && L.ncomp == 3) return split<3, 1, 3>(L, cus, max_threads, cells);
+  if (p == 1) return split<3, 1>(L, cus, max_threads, cells);
+  return split<3, 2>(L, cus, max_threads, cells);
 }
 
 // The lattice row of every row of a space, perm, if each (cell, local DOF) of

@@ -166,3 +166,24 @@ def test_lattice_both_forms_and_limits(env):
     op.compute()
     x3 = s.solve()
     assert s.did_converge() and np.linalg.norm(x3 - x2) <= 1e-10 * np.linalg.norm(x2)
+
+
+@pytest.mark.parametrize("n,k,bc", [((1, 200, 20), "cell", "boundary"), ((2, 128, 8), "sin3", "boundary"),
+                                    ((1, 127, 4), "cell", "x0")])
+def test_thin_q2_boxes_match_oracle(env, n, k, bc):
+    """Q2 boxes one or two cells thick along x whose tiles are cut short by the
+    nodes after them, one a thread: every cell column is solved.  Solutions of a
+    matrix half an ulp off differ by 2e-13 at most (direct solves)."""
+    print(f"[lattice] thin {n} {k} {bc}", flush=True)
+    osp, oph, op = _build(env, n, 2, k, bc)
+    op.compute()
+    irp, ja, val, rhs = osp.assemble(oph, True)
+    assert len(rhs) == op.n > 4096
+    ref, _ = O.cg(irp, ja, val, rhs, True, precond="jacobi", rtol=1e-12, maxit=20000)
+    bound = 125 * np.finfo(float).eps
+    for precision, rtol, tol in (("FP64", 1e-12, 1e-10), ("FP32_REFINED", 1e-10, 1e-8)):
+        s, x = _solve(env, op, precision, "jacobi", rtol)
+        assert s.did_converge() and np.linalg.norm(x - ref) <= tol * np.linalg.norm(ref), precision
+        r = rhs - O.spmv(irp, ja, val, x, True)
+        rounding = bound * np.linalg.norm(O.spmv(irp, ja, np.abs(val), np.abs(x), True))
+        assert abs(s.result["true_residual"] - np.linalg.norm(r)) <= rounding
