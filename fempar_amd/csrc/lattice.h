@@ -76,8 +76,8 @@ __device__ __forceinline__ void buf_st32(BufRsrc r, uint32_t o8, float v) {
 }
 
 // The part of a lattice that logical workgroup lb reads, as a lattice of its
-// own planes: row0 is its first row (vectors of any length then keep 30-bit
-// byte offsets, as long as a chunk's planes do).
+// own planes: row0 is its first row.  Vectors of any length then keep 30-bit
+// byte offsets, as a chunk's planes do: lattice_plan with `cells` bounds its layers.
 __device__ __forceinline__ Lattice lattice_window(const Lattice &g, int dim, int p, int lb, int64_t &row0, int64_t &rows) {
   Lattice w = g;
   const int a = dim - 1, chunk = lb / g.tiles;

@@ -102,7 +102,11 @@ bool split(LatticeOp &L, int cus, int max_threads, int cells) {
   // little and many short ones fill the chip; the fewest layers in turn on one
   // CU wins.
   if (cus <= 0) {
-    const int layers = std::max(2, std::min(ez, cells / std::max(1, g.TX * g.TY)));
+    // the planes a chunk reads stay within 30-bit byte offsets (lattice_window)
+    const int64_t plane = (int64_t)g.m[0] * (DIM == 3 ? g.m[1] : 1);
+    const int64_t most = (kLatticeMaxRows / plane - 1) / P - 1;
+    if (most < 1) return false;
+    const int layers = (int)std::min<int64_t>(most, std::max(2, std::min(ez, cells / std::max(1, g.TX * g.TY))));
     g.nch = (ez + layers - 1) / layers;
     L.grid = g.tiles * g.nch;
     return true;

@@ -95,3 +95,35 @@ def test_batch_paths_match_oracle(env, problems):
         x_ref, _ = O.cg(irp, ja, val, rhs, False, precond="jacobi", rtol=1e-12, maxit=20000)
         assert np.linalg.norm(x - x_ref) <= 1e-5 * np.linalg.norm(x_ref), (dim, n)
     b.free()
+
+
+def test_batch_problem_beyond_one_window(env):
+    """A cube of 513^3 rows (1.08 GB a vector, more than 30-bit byte offsets reach)
+    beside a small problem.  The source is the operator's lowest eigenvector, so the
+    solution is known in closed form and its relative error is at most the
+    relative residual, 1e-8 (and 1e-12 of rounding)."""
+    n = 514
+    print(f"[batch] one problem of {(n - 1) ** 3} rows", flush=True)
+    b = F.batch_t(env, [(3, n, 2.0, 0.5), (2, 40, 1.0, 1.0)], rtol=1e-8)
+    b.assemble()
+    res = b.solve()
+    print(f"[batch] solved in {res['ms']:.2f} ms, {res['num_iterations'].tolist()}", flush=True)
+    assert np.all(res["did_converge"] == 1)
+    for i, (dim, n, f0) in enumerate(((3, n, 0.5), (2, 40, 1.0))):
+        h, g = 1.0 / n, 0.5 - 0.5 / np.sqrt(3.0)
+        c = np.cos(np.pi * h)
+        stiff, mass = 2.0 * (1.0 - c) / h, h * (2.0 + c) / 3.0        # of sin(pi x) at a node, by its value there
+        load = h * ((1.0 - g) * np.cos(np.pi * h * g) + g * np.cos(np.pi * h * (1.0 - g)))
+        scale = f0 * dim * np.pi ** 2 * load ** dim / (dim * stiff * mass ** (dim - 1))
+        s = np.sin(np.pi * h * np.arange(1, n))
+        ref = scale * s
+        for _ in range(dim - 1):
+            ref = np.multiply.outer(s, ref)
+        x = b.get_solution(i).reshape(ref.shape)
+        norm = np.linalg.norm(ref)
+        x -= ref
+        assert np.linalg.norm(x) <= (1e-8 + 1e-12) * norm, (dim, n)
+        # no row is left out: the first and the last planes by themselves
+        for plane in (0, n // 2, n - 2):
+            assert np.linalg.norm(x[plane]) <= (1e-8 + 1e-12) * norm and np.linalg.norm(ref[plane]) > 0.0
+    b.free()

@@ -69,3 +69,30 @@ def test_tiles_cover_boxes(order):
             L = plan((nx, ny), order, 1, bc)
             assert L
             check_tiles(L, 768)
+
+
+def window_rows(L, chunk):
+    """lattice_window of lattice.h: rows of the whole planes that a chunk of the march reads."""
+    g, a, p = L.g, L.dim - 1, L.order
+    z0, z1 = g.E[a] * chunk // g.nch, g.E[a] * (chunk + 1) // g.nch
+    first, last = max(p * max(z0 - 1, 0) - g.o[a], 0), min(p * z1 - g.o[a], g.m[a] - 1)
+    return max(last - first + 1, 0) * (g.m[0] * g.m[1] if L.dim == 3 else g.m[0])
+
+
+@pytest.mark.parametrize("dim,sizes", [
+    (2, (130, 1000, 2048, 4095, 4096)),
+    (3, (25, 100, 400, 512, 513, 514, 515, 600, 647, 813, 814, 1000, 1030, 1290, 1291))])
+def test_batch_windows_keep_their_byte_offsets(dim, sizes):
+    """The passes of a batch read vectors of any length through windows of at
+    most 2^30 bytes: larger ones would reach the offsets that stand for `outside'.
+    Cells a workgroup as plan_passes asks for them."""
+    for n in sizes:
+        rows = (n - 1) ** dim
+        for per in (1024, 16384):
+            L = plan((n,) * dim, 1, 1, N.BC_ALL_BOUNDARY, cus=0, max_threads=256, cells=max(per, rows // 192))
+            assert L, n
+            check_tiles(L, 256)
+            chunks = [window_rows(L, c) for c in range(L.g.nch)]
+            assert 8 * max(chunks) <= 1 << 30, n
+            assert sum(chunks) >= rows
+    assert plan((1292,) * 3, 1, 1, N.BC_ALL_BOUNDARY, cus=0, max_threads=256, cells=16384) is None   # rows past 2^31
