@@ -1968,8 +1968,9 @@ void profiled_solve(femhip_solver &s, double *spmv_ms, int32_t *iterations) {
 }
 
 // Times `reps` CG iterations (vector updates and product) in a state that never
-// converges, with zero vectors and sums, so x stays; bytes: every vector read
-// and written as in cg_lattice.h, and the coefficient values.
+// converges, with zero vectors and sums, so x stays; the result block and the
+// history's first entry, which every iteration writes, are put back.  bytes:
+// every vector read and written as in cg_lattice.h, and the coefficient values.
 void profile_lattice(femhip_solver &s, int32_t reps, double *ms_per_launch, double *bytes) {
   hipStream_t st = s.ctx->stream;
   const femhip_operator &op = *s.op;
@@ -1980,6 +1981,10 @@ void profile_lattice(femhip_solver &s, int32_t reps, double *ms_per_launch, doub
   h.delta = -1.0;
   h.maxit = INT32_MAX;
   h.crit = FEMHIP_RES_RES;
+  CgResult last;
+  double hist0 = 0.0;
+  FH_HIP(hipMemcpyAsync(&last, s.res.p, sizeof(last), hipMemcpyDeviceToHost, st));
+  FH_HIP(hipMemcpyAsync(&hist0, s.hist.p, sizeof(hist0), hipMemcpyDeviceToHost, st));
   FH_HIP(hipMemcpyAsync(s.st.p, &h, sizeof(h), hipMemcpyHostToDevice, st));
   FH_HIP(hipStreamSynchronize(st));
   const bool mx = mixed(s);
@@ -2004,7 +2009,9 @@ void profile_lattice(femhip_solver &s, int32_t reps, double *ms_per_launch, doub
   FH_HIP(hipEventRecord(e0, st));
   for (int k = 0; k < reps; ++k) launch();
   FH_HIP(hipEventRecord(e1, st));
-  FH_HIP(hipEventSynchronize(e1));
+  FH_HIP(hipMemcpyAsync(s.res.p, &last, sizeof(last), hipMemcpyHostToDevice, st));
+  FH_HIP(hipMemcpyAsync(s.hist.p, &hist0, sizeof(hist0), hipMemcpyHostToDevice, st));
+  FH_HIP(hipStreamSynchronize(st));
   float ms = 0.f;
   FH_HIP(hipEventElapsedTime(&ms, e0, e1));
   (void)hipEventDestroy(e0);
