@@ -1757,11 +1757,16 @@ void push_chunk(femhip_solver &s, int slot, int size_idx = 0) {
   FH_HIP(hipEventRecord(s.ev[slot], st));
 }
 
+// Whether a solve's passes are more than its iterations: the lattice passes take
+// each decision one pass later, and a reliable update of a refined form (at most
+// one an iteration) spends up to three.  The device ends those solves.
+bool ends_late(const femhip_solver &s) { return s.lat || mixed(s); }
+
 }  // namespace
 
 int64_t solver_pass_budget(const femhip_solver &s) {
   const int64_t maxit = s.prm.max_num_iterations;
-  return s.lat ? 4 * maxit + 8 : maxit;
+  return ends_late(s) ? 4 * maxit + 8 : maxit;
 }
 
 namespace {
@@ -1797,10 +1802,8 @@ void iterate(femhip_solver &s, int maxit) {
     FH_HIP(hipEventSynchronize(s.ev[c.slot]));
     const CgResult r = *s.h_res[c.slot];
     if (r.done) break;
-    // budget queued: wait for the rest.  The lattice passes take each decision
-    // one pass later, and an update of their refined form (at most one an
-    // iteration) spends three: there the device ends the solve, and chunks go
-    // on until it has.
+    // budget queued: wait for the rest; where the device ends the solve, chunks
+    // go on until it has
     if (queued >= solver_pass_budget(s)) continue;
     double need = 1e30;              // iterations still needed
     if (prev_it >= 0 && r.prog_it > prev_it && r.prog > 0.0 && prev > r.prog && r.rhs_test > 0.0) {
@@ -1813,7 +1816,7 @@ void iterate(femhip_solver &s, int maxit) {
     }
     static const char *plan_env = getenv("FEMHIP_TAIL_CHUNKS");   // 0: always full chunks
     if (plan_env && atoi(plan_env) == 0) need = 1e30;
-    const double rest = std::min(need, s.lat ? (double)maxit - r.prog_it + 4.0 : 1e30) -
+    const double rest = std::min(need, ends_late(s) ? (double)maxit - r.prog_it + 4.0 : 1e30) -
                         (double)(queued - r.prog_it);   // beyond what is queued
     if (nq > 0 && rest <= 0.0) continue;
     push(rest > kChunk ? 0 : 1);
