@@ -1925,8 +1925,11 @@ void solve(femhip_solver &s, bool x_zero, femhip_cg_result_t *out) {
 }
 
 // One device-resident solve (b = the operator's RHS, x0 = 0) launched kernel
-// by kernel with events around every SpMV; returns the mean SpMV duration over
-// the iterations that ran (launches queued after convergence return at entry).
+// by kernel with events around every product, until the device ends it; returns
+// the mean product duration over the iterations that ran, on the lattice over the
+// passes that ran: in the one-launch form one more than the iterations and three
+// more for an update, in the other one more for an update.  Launches queued after
+// the end return at entry.
 void profiled_solve(femhip_solver &s, double *spmv_ms, int32_t *iterations) {
   hipStream_t st = s.ctx->stream;
   load_vector(s, s.b.p, s.op->rhs.p, hipMemcpyDeviceToDevice);
@@ -1938,7 +1941,7 @@ void profiled_solve(femhip_solver &s, double *spmv_ms, int32_t *iterations) {
   int launched = 0;
   bool done = false;
   try {
-    while (!done && launched < s.prm.max_num_iterations) {
+    while (!done && launched < solver_pass_budget(s)) {
       for (int i = 0; i < kChunk; ++i, ++launched) {
         hipEvent_t e[2];
         FH_HIP(hipEventCreate(&e[0]));
@@ -1954,14 +1957,16 @@ void profiled_solve(femhip_solver &s, double *spmv_ms, int32_t *iterations) {
     }
     CgResult r;
     FH_HIP(hipMemcpy(&r, s.res.p, sizeof(r), hipMemcpyDeviceToHost));
-    const int it = std::min(r.iter, launched);
+    int passes = r.iter;   // 0: ended by the initial residual or a zero pivot
+    if (s.lat && passes > 0) passes += s.op->lat->one ? 3 * r.updates + 1 : r.updates;   // FP64: no updates
+    passes = std::min(passes, launched);
     double sum = 0.0;
-    for (int k = 0; k < it; ++k) {
+    for (int k = 0; k < passes; ++k) {
       float ms = 0.f;
       FH_HIP(hipEventElapsedTime(&ms, ev[(size_t)2 * k], ev[(size_t)2 * k + 1]));
       sum += ms;
     }
-    *spmv_ms = it > 0 ? sum / it : 0.0;
+    *spmv_ms = passes > 0 ? sum / passes : 0.0;
     *iterations = r.iter;
   } catch (...) {
     for (auto e : ev) (void)hipEventDestroy(e);

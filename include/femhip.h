@@ -248,7 +248,8 @@ int femhip_solver_profile_spmv(femhip_solver_t *solver, int32_t reps, double *ms
  * kernel by kernel, with HIP events around every SpMV on the solver's stream;
  * mean SpMV duration over the iterations that ran (inside the CG sequence,
  * with the vector kernels in between), the iteration count, and the SpMV's
- * algorithmic bytes per launch. */
+ * algorithmic bytes per launch.  Where products are formed from the cells the
+ * mean is over the passes that ran, those of reliable updates among them. */
 int femhip_solver_profile_cg(femhip_solver_t *solver, double *spmv_ms, int32_t *iterations,
                              double *bytes_per_launch);
 /* copy the last solution to the host (n values) */

@@ -53,3 +53,19 @@ def test_profile_spmv_keeps_the_solve(env, name):
     again = s.get_error_estimate_history_convergence_test()   # of the profiled solve: the same one
     assert len(again) == its and np.max(np.abs(again / hist - 1.0)) <= 1e-7
     assert np.linalg.norm(s.get_solution() - x) <= 1e-10 * np.linalg.norm(x)
+
+
+@pytest.mark.parametrize("precision", ["FP64", "FP32_REFINED"])
+@pytest.mark.parametrize("name", SYSTEMS)
+def test_profile_cg_runs_to_the_limit(env, name, precision):
+    """A limit that is a whole number of chunks: the passes that decide an
+    iteration after it, and those of an update, are launched all the same."""
+    print(f"[profile] cg {name} {precision}", flush=True)
+    op = _operator(env, name)
+    s = _solver(env, op, ILS_RTOL=1e-14, ILS_MAX_NUM_ITERATIONS=32, FEMHIP_PRECISION=precision)
+    s.solve_resident()
+    assert not s.did_converge() and s.get_num_iterations() == 32
+    x = s.get_solution()
+    ms, count, _ = s.profile_cg()
+    assert ms > 0 and count == 32
+    assert np.linalg.norm(s.get_solution() - x) <= 1e-10 * np.linalg.norm(x)
