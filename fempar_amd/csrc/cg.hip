@@ -1343,13 +1343,53 @@ int32_t lattice_min_rows(const femhip_solver &s) {
   return fe.order == 1 ? 2049 : 1025;
 }
 
+// Whether the march is as fast as the stored matrix.  Its layers are applied one
+// after the other, so a long box of small cross-section leaves lanes and CUs idle
+// for most of an iteration, and one of few layers and very many tiles reads as many
+// partial sums in every workgroup.  Both times in us an iteration, fitted to solves
+// of 1016 boxes of 300 to 3 million rows, a third of them long, in both precisions:
+// within 20 to 28 % for eight in ten.  Of 1898 solves the cells had been slower by
+// more than 10 % in 431 (134 times at worst); by the rule the slower side is
+// taken in 50, at a loss of 7 % at the median of the wrong ones, 1.96 times at most.
+//                                         cells            stored
+//   2-D Q1 4 x 100,000 cells, FP64 / FP32  204 / 272        24 / 21
+//   2-D Q2 1 x 38,616, point values        233 / 453        15 / 14
+//   3-D Q1 2 x 2 x 100,000, FP64           269              48
+//   3-D Q2 1 x 1 x 5777                     87 / 107         15 / 14
+//   2-D Q1 51 x 10,739                      41 / 42          36 / 26
+//   3-D Q1 23 x 4 x 25,925                  90 / 107        253 / 169
+// Boxes of sides near one size keep the cells.  A twentieth is granted to them,
+// since they need no layout of the matrix.
+bool lattice_pays(const femhip_solver &s) {
+  const femhip_operator &op = *s.op;
+  const LatticeOp &L = *op.lat;
+  const bool mx = mixed(s), points = op.tab_kind == 0 && op.phys.k_kind == FEMHIP_K_QPOINT;
+  // a layer: 2-D Q1, 2-D Q2, 3-D Q1, elasticity, 3-D Q2; FP64, FP32; one value a cell or sines, point values
+  static const double layer_us[5][2][2] = {{{0.6, 0.6}, {0.8, 0.9}},
+                                           {{1.4, 1.5}, {2.0, 3.1}},
+                                           {{0.75, 0.95}, {1.0, 1.8}},
+                                           {{1.8, 1.8}, {2.2, 2.2}},
+                                           {{3.4, 9.3}, {4.4, 10.7}}};
+  const int family = L.dim == 2 ? L.order - 1 : L.order == 2 ? 4 : L.ncomp == 3 ? 3 : 2;
+  const double n = (double)op.n, entries = (double)op.nnz_full;
+  double cells = 8.0 + layer_us[family][mx][points] * L.rounds * L.layers + n * (mx ? 7e-6 : 13e-6);
+  if (L.one) cells += 7e-3 * L.rounds * L.grid;   // partial sums
+  if (points) cells += 8.0 * (double)op.space->ncells * op.space->fe.nq / 5e6;
+  double stored;
+  if (!mx && op.n <= kSmallMaxRows && op.nnz_full <= kSmallEntries)   // one workgroup (cg_small.h)
+    stored = 2.5 + 0.25 * entries / n + 1e-4 * entries;
+  else
+    stored = (op.n <= 4096 ? 9.5 : 11.0) + 0.3 * entries / n + entries * (mx ? 1e-6 : 2e-6) + n * 15e-6;
+  return cells <= 1.05 * stored;
+}
+
 // Whether a solver forms its products from the cells: scalar Poisson and vector
 // Q1 elasticity on the uniform mesh (lattice_operator), in FP64 and FP32_REFINED.
 // FP32_STRICT and the FP32 integration are defined by their stored FP32 matrix.
 bool wants_lattice(femhip_solver &s) {
   if (s.op->structured) return true;   // has no other form
   if (!s.op->space || strict(s) || (mixed(s) && fp32_integration())) return false;
-  return s.op->n >= lattice_min_rows(s) && lattice_operator(*s.op);
+  return s.op->n >= lattice_min_rows(s) && lattice_operator(*s.op) && lattice_pays(s);
 }
 
 void drop_graphs(femhip_solver &s) {
@@ -1441,7 +1481,7 @@ void prepare(femhip_solver &s) {
   femhip_operator &op = *s.op;
   FH_CHECK(op.computed, FEMHIP_ERR_STATE, "solve before fe_affine_operator%compute");
   const bool lat = wants_lattice(s);
-  if (s.prepared && lat != s.lat) {   // the operator's mesh was moved since: other layout, other buffers
+  if (s.prepared && lat != s.lat) {   // mesh moved or another kind of coefficient since: other layout, other buffers
     FH_HIP(hipStreamSynchronize(s.ctx->stream));
     drop_graphs(s);
     s.prepared = false;

@@ -862,6 +862,7 @@ struct LatticeOp {
   int threads = 64, grid = 8;       // workgroup size and count
   size_t lds = 0;                   // bytes of LDS a workgroup
   bool identity = false;            // lattice rows are the operator's rows
+  int rounds = 1, layers = 1;       // workgroups a CU's slot takes in turn, layers each marches
 };
 // cus > 0: chunks that fill that many CUs; otherwise of about `cells` cells a workgroup
 bool lattice_plan(const femhip_mesh_desc_t &mesh, int cus, LatticeOp &L, int max_threads = 0, int cells = 0);

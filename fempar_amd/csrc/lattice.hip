@@ -130,6 +130,8 @@ bool split(LatticeOp &L, int cus, int max_threads, int cells) {
   }
   const int blocks = g.tiles * g.nch;
   L.grid = (blocks + 7) / 8 * 8;
+  L.rounds = (int)((blocks + slots - 1) / slots);
+  L.layers = (ez + g.nch - 1) / g.nch + (g.nch > 1 ? 1 : 0);
   return true;
 }
 

@@ -14,7 +14,8 @@ class Lattice(C.Structure):
 
 class LatticeOp(C.Structure):
     _fields_ = [("g", Lattice), ("dim", C.c_int), ("order", C.c_int), ("ncomp", C.c_int), ("one", C.c_bool),
-                ("threads", C.c_int), ("grid", C.c_int), ("lds", C.c_size_t), ("identity", C.c_bool)]
+                ("threads", C.c_int), ("grid", C.c_int), ("lds", C.c_size_t), ("identity", C.c_bool),
+                ("rounds", C.c_int), ("layers", C.c_int)]
 
 
 def plan(n, order, ncomp, bc, cus=256, max_threads=0, cells=0):
