@@ -30,7 +30,8 @@
 // stamped with the device wall clock.
 // (One workgroup a problem whatever its size leaves the end of a batch to the
 // largest, each at the rate of one CU: 512 problems up to 256^2 and 48^3 took
-// 67 ms of solving, now 8.4 ms; one 40^3 24 ms, now 0.46 ms.)
+// 66 ms of solving to 1e-8 and 110 ms to 1e-10, now 8.2 and 13.0 ms; one 40^3 23.5
+// and 39 ms, now 0.44 and 0.76 ms.)
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -597,9 +598,10 @@ int small_class(const BProb &P, BSmall &S) {
 // Each problem's path; tiles of the problems in the passes and the table of
 // their workgroups.  A workgroup takes about an eighth of what would fill every
 // CU once, within bounds: long marches repeat little, short ones leave no CU
-// waiting for the last problem (512 mixed problems: 8.2 ms, a quarter 9.6, a half
-// 12.3).  Each workgroup of a problem reads the partial sums of all of them, so
-// a problem has at most kMostGroups (four of 1000^2 cells: 30 ms with 570, 23.5).
+// waiting for the last problem (512 mixed problems to 1e-8: 8.2 ms, a quarter 9.6, a
+// half 12.3).  Each workgroup of a problem reads the partial sums of all of them, so
+// a problem has at most kMostGroups, or as many as its tiles and windows need (four
+// of 1000^2 cells: 33.3 ms with 570, 23.0; the mixed problems 8.2 either way).
 constexpr int kMostGroups = 192;
 void plan_passes(femhip_batch &B, const std::vector<BTables> &tabs) {
   const int count = (int)B.probs.size();

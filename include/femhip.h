@@ -364,7 +364,9 @@ typedef struct femhip_batch femhip_batch_t;
  * factor (0: 0.1); precision must be FEMHIP_PRECISION_FP32_REFINED. */
 int femhip_batch_create(femhip_ctx_t *ctx, int32_t count, const femhip_batch_problem_t *problems,
                         const femhip_cg_params_t *params, femhip_batch_t **batch);
-/* Integrate + assemble every problem (one launch; FP64 and FP32 values, RHS, Jacobi). */
+/* Integrate + assemble every problem: its FP64 diagonals, which
+ * femhip_batch_get_problem_matrix returns, and its right-hand side, which the
+ * solve uses (two launches: the 1-D load integrals, then the rows). */
 int femhip_batch_assemble(femhip_batch_t *batch, double *ms);
 /* Solve every problem from x0 = 0, the small ones in a workgroup each, the
  * others one CG iteration of all of them in each launch (hipGraph chunks);

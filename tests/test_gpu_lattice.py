@@ -3,8 +3,8 @@
 Sizes at the edges of the workgroup tiles and chunks (one cell more or less
 than a tile, thin and long boxes, a single layer), 2-D and 3-D, Q1 and Q2, one
 coefficient a cell, the closed form and point values, the two Dirichlet kinds
-(the free nodes' box with and without its last planes), both preconditioners
-and both forms of an iteration (below and above 400,000 rows).
+(the free nodes' box with and without its last planes) and both preconditioners,
+with iterations in one launch (in two: test_gpu_lattice_two_launches.py).
 
 Gates: FP64 solutions to 1e-12 within 1e-10 relative of the oracle's, in no more
 than 2 % + 2 of its iterations; FP32-refined within 1e-8 (the gates of test_gpu_parity)."""
